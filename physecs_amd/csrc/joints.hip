@@ -44,6 +44,7 @@ struct JointArgs {
     float4* jRow;
     const float4 *bpos, *bquat, *dcom, *dinvI, *dvel;
     float4 *bvel, *pvel, *pang;
+    const float4* brec;
     const int32_t* order;                                     // joints sorted by colour
     float h;
 };
@@ -321,12 +322,12 @@ __device__ __forceinline__ JBodies joint_bodies(const JointArgs& a, int j) {
     B.b0 = a.jB0[j]; B.b1 = a.jB1[j];
     B.im0 = 0.f; B.im1 = 0.f; B.I0 = mzero(); B.I1 = mzero();
     if (B.b0 >= 0) {
-        B.im0 = a.bvel[bv(B.b0, BV_CV)].w;
-        B.I0 = mk_m3(xyz(a.bvel[bv(B.b0, BV_I0)]), xyz(a.bvel[bv(B.b0, BV_I1)]), xyz(a.bvel[bv(B.b0, BV_I2)]));
+        B.im0 = a.brec[br(B.b0, BR_COM)].w;
+        B.I0 = mk_m3(xyz(a.brec[br(B.b0, BR_I0)]), xyz(a.brec[br(B.b0, BR_I1)]), xyz(a.brec[br(B.b0, BR_I2)]));
     }
     if (B.b1 >= 0) {
-        B.im1 = a.bvel[bv(B.b1, BV_CV)].w;
-        B.I1 = mk_m3(xyz(a.bvel[bv(B.b1, BV_I0)]), xyz(a.bvel[bv(B.b1, BV_I1)]), xyz(a.bvel[bv(B.b1, BV_I2)]));
+        B.im1 = a.brec[br(B.b1, BR_COM)].w;
+        B.I1 = mk_m3(xyz(a.brec[br(B.b1, BR_I0)]), xyz(a.brec[br(B.b1, BR_I1)]), xyz(a.brec[br(B.b1, BR_I2)]));
     }
     return B;
 }
@@ -654,7 +655,7 @@ static JointArgs make_jargs(World& w, float h) {
     a.jPar0 = w.jPar0.p; a.jPar1 = w.jPar1.p; a.jGear = w.jGear.p; a.jGearInit = w.jGearInit.p;
     a.jB0 = w.jB0.p; a.jB1 = w.jB1.p; a.jR0 = w.jR0.p; a.jR1 = w.jR1.p; a.jRow = w.jRow.p;
     a.bpos = w.bpos.p; a.bquat = w.bquat.p; a.dcom = w.dcom.p; a.dinvI = w.dinvI.p; a.dvel = w.dvel.p;
-    a.bvel = w.bvel.p; a.pvel = w.pvel.p; a.pang = w.pang.p;
+    a.bvel = w.bvel.p; a.brec = w.brec.p; a.pvel = w.pvel.p; a.pang = w.pang.p;
     a.order = w.jOrder.p;
     a.h = h;
     return a;

@@ -86,14 +86,18 @@ struct PinnedInts {
 };
 
 constexpr int WAVE = 64;
-// What a contact or joint solve reads and writes for one dynamic body, in one 128-byte
-// record (one cache line): solver v and w (velocityTemp), component v after the velocity
-// integration (.w = inverse mass), component w, and the columns of the world inverse
-// inertia of the substep (massTemp's R * invI * R^T). Bodies are gathered by index, so
-// one line per body instead of one per array.
-enum { BV_V = 0, BV_W = 1, BV_CV = 2, BV_CW = 3, BV_I0 = 4, BV_I1 = 5, BV_I2 = 6, BV_WORDS = 8 };
-constexpr int CONTACT_ROW_FIELDS = 9;   // float4 rows per contact point (sRow)
+// What a contact or joint solve reads and writes for one dynamic body, gathered by index:
+// solver v (.w = inverse mass) and w (velocityTemp), 32 bytes.
+enum { BV_V = 0, BV_W = 1, BV_WORDS = 2 };
 __host__ __device__ __forceinline__ int bv(int body, int field) { return BV_WORDS * body + field; }
+// What the substep's contact and joint rows are built from, in one 128-byte record (one
+// cache line) per dynamic body: centre of mass in the world (.w = inverse mass),
+// orientation, component v and w before the velocity integration (.w = x and y of w after
+// it), and the columns of the world inverse inertia (massTemp's R * invI * R^T; the first's
+// .w = z of w after the integration).
+enum { BR_COM = 0, BR_Q, BR_V, BR_W, BR_I0, BR_I1, BR_I2, BR_WORDS = 8 };
+__host__ __device__ __forceinline__ int br(int body, int field) { return BR_WORDS * body + field; }
+constexpr int CONTACT_ROW_FIELDS = 7;   // float4 rows per contact point (sRow)
 constexpr int JOINT_MAX_ROWS = 7;      // a prismatic joint with its limit and drive rows
 // substep-loop execution: one launch per colour and pass; one cooperative launch per step
 // (grid barriers between colours); one dependency-driven launch per pass
@@ -178,7 +182,7 @@ struct World {
     DBuf<float4> dvel, dang;             // D component velocity (dvel.w = invMass)
     DBuf<float4> dcom;                   // D local com (w = kinematic ? 1 : 0)
     DBuf<float4> dinvI;                  // 3 x D columns of the local inverse inertia
-    DBuf<float4> bvel;                   // BV_WORDS per dynamic body (record layout below)
+    DBuf<float4> bvel, brec;             // BV_WORDS and BR_WORDS per dynamic body
     DBuf<float4> pvel, pang;             // D pseudo velocities (pang.w = constraint count)
     DBuf<float4> winvI;                  // 3 x D world inverse inertia (massTemp)
 
@@ -256,7 +260,8 @@ struct World {
     DBuf<int32_t> worldMStart;           // W first manifold of each world
 
     // manifolds, solve (colour) order
-    DBuf<int32_t> sB0, sB1, sFlags, sA0, sA1;   // sFlags: numPoints | soft<<8 | color<<16
+    DBuf<int2> sB, sA;                   // per slot: its sides' dynamic bodies (-1: none) and internal bodies
+    DBuf<int32_t> sFlags, sMode;         // sFlags: numPoints | soft<<8 | color<<16; sMode: the substep's
     DBuf<int32_t> sCanon;                // canonical index
     DBuf<int32_t> batchLoc, batchList, batchN;   // runs of small colours: LDS slots of their bodies
     DBuf<int32_t> colorPack;             // the colouring's read-back, packed by k_color_start
@@ -264,9 +269,9 @@ struct World {
     bool batchLdsSet = false;            // k_solve_batch's LDS limit raised on this world's device
     DBuf<float4> sN;                     // normal, friction
     DBuf<float2> sSoft;                  // frequency, damping
-    DBuf<float4> sR0, sR1;               // 4 x M: r0 local + targetVelocity, r1 local
-    DBuf<float4> sRow;                   // 5 x 4 x M per-substep rows
-    DBuf<float4> sLam;                   // 4 x M: lambda N, lambda T, target velocity
+    DBuf<float4> sR;                     // 4 x M x 2 sides: local anchor + targetVelocity
+    DBuf<float4> sRow;                   // 4 x CONTACT_ROW_FIELDS x M per-substep rows
+    DBuf<float2> sLam;                   // 4 x M: lambda N, lambda T
 
     // contact cache (canonical order, double-buffered)
     DBuf<uint64_t> cacheKey[2];

@@ -269,9 +269,9 @@ __global__ __launch_bounds__(256) void k_setup(
     const int32_t* __restrict__ mfPrev, const int32_t* __restrict__ prevNum,
     const float4* __restrict__ prevLp, int prevCap, uint64_t* __restrict__ curKey,
     int32_t* __restrict__ curTri, int32_t* __restrict__ curNum,
-    float4* __restrict__ curLp, int32_t* __restrict__ sB0, int32_t* __restrict__ sB1, int32_t* __restrict__ sA0,
-    int32_t* __restrict__ sA1, int32_t* __restrict__ sFlags, int32_t* __restrict__ sCanon, float4* __restrict__ sN,
-    float2* __restrict__ sSoft, float4* __restrict__ sR0, float4* __restrict__ sR1, int32_t* __restrict__ sWorld) {
+    float4* __restrict__ curLp, int2* __restrict__ sB, int2* __restrict__ sA, int32_t* __restrict__ sFlags,
+    int32_t* __restrict__ sCanon, float4* __restrict__ sN, float2* __restrict__ sSoft, float4* __restrict__ sR,
+    int32_t* __restrict__ sWorld) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= M) return;
     const int s = rank[m];
@@ -329,19 +329,17 @@ __global__ __launch_bounds__(256) void k_setup(
             }
             if (!found) tv = -rest * relN;
             r0o = f4(r0, tv);
-            r1o = f4(r1, 0.f);
+            r1o = f4(r1, tv);   // each side's lane carries the target velocity into its row
             curLp[(size_t)k * Mcap + m] = r0o;
         }
-        sR0[(size_t)k * Mcap + s] = r0o;
-        sR1[(size_t)k * Mcap + s] = r1o;
+        sR[2 * ((size_t)k * Mcap + s)] = r0o;
+        sR[2 * ((size_t)k * Mcap + s) + 1] = r1o;
     }
     curKey[m] = key;
     curTri[m] = tri;
     curNum[m] = num | (mfColor[m] << CACHE_COLOR_SHIFT) | CACHE_HAS_COLOR;
-    sB0[s] = b0;
-    sB1[s] = b1;
-    sA0[s] = a0;
-    sA1[s] = a1;
+    sB[s] = make_int2(b0, b1);
+    sA[s] = make_int2(a0, a1);
     sFlags[s] = num | (soft ? 256 : 0) | (mfColor[m] << 16);
     sCanon[s] = m;
     sN[s] = f4(n, friction);
@@ -384,31 +382,53 @@ void sv_color_points(World& w, int nColors) {
 }
 
 // ------------------------------------------------------------------ substep pieces
-// Contact rows of point k of manifold slot s, field f at ((k * R_NF + f) * Mcap + s):
-// r0 x n (.w = c), r1 x n (.w = inverse effective mass N), tangent (.w = inverse
-// effective mass T), r0 x t (.w = effective mass N, 1 / invN), r1 x t (.w = the bias
-// 0.1 c / h), and the rows times the bodies' world inverse inertia, as preSolve keeps them
-// (src/ContactConstraints.cpp:21-24): r0xnt (.w = beta c / h of a soft contact), r1xnt
-// (.w = invN + gamma / h of a soft contact), r0xtt, r1xtt. Everything here is fixed for the
-// substep, so the solve's arithmetic on it is done once, with the operations and in the
-// order ContactConstraints::solve does it (src/ContactConstraints.cpp:54-68). Per point
-// also (lambda N, lambda T, target velocity) in sLam.
-enum { R_R0XN = 0, R_R1XN, R_T, R_R0XT, R_R1XT, R_R0XNT, R_R1XNT, R_R0XTT, R_R1XTT, R_NF };
-static_assert(R_NF == CONTACT_ROW_FIELDS, "sRow holds CONTACT_ROW_FIELDS float4 per point");
-#define ROW(f, k) a.sRow[((size_t)((k) * R_NF + (f))) * a.Mcap + s]
+// Every contact kernel gives a manifold to two adjacent lanes, one per body: lane i works
+// on side i & 1 of manifold slot i >> 1. A side's lane loads its own body and its own rows,
+// computes its half of each relative velocity and updates its own body; the halves meet
+// through DPP lane moves. A launch of one colour of the 32k scene holds about a wave per
+// ten SIMDs, so its time is one wave's chain of instructions: k_solve is 718 of them instead
+// of 1,076 with a lane per manifold, at 98 registers instead of 208, and took 4.26 us per
+// colour launch of the settled 32k scene instead of 5.63 (a run of small colours in
+// k_solve_batch 17.1 us instead of 24.8; a large colour of 1,024 worlds 8.4 instead of 10.4).
+//
+// Contact rows of point k of side lane i, field f at ((k * RS_NF + f) * Mcap) * 2 + i, so
+// a wave's loads are contiguous: r x n (.w = target velocity), the row times the body's
+// world inverse inertia, as preSolve keeps it (src/ContactConstraints.cpp:21-24; .w = the
+// effective mass 1 / invN, or invN + gamma / h of a soft contact), and I * (r x t) (.w =
+// the bias 0.1 c / h, or beta c / h of a soft contact). Side 0's vectors are stored
+// negated: both sides then add to the relative velocity and subtract the impulse, and
+// negation changes no other bit of a product or a sum's magnitude. Per point also the
+// tangent (.w = the friction impulse of one pass). The friction row reads the component
+// velocities (src/ContactConstraints.cpp:92-101), which no pass changes, so its impulse
+// rv / invT is fixed for the substep like the terms of src/ContactConstraints.cpp:54-68:
+// all are computed here, once, with the operations and in the order of the solve. 7 float4
+// per point instead of 9, and the solve reads no component velocity.
+enum { RS_N = 0, RS_NT, RS_TT, RS_NF };
+static_assert(2 * RS_NF + 1 == CONTACT_ROW_FIELDS, "sRow holds CONTACT_ROW_FIELDS float4 per point");
+#define ROW(f, k) a.sRow[((size_t)((k) * RS_NF + (f)) * a.Mcap) * 2 + i]
+#define ROWT(k) a.sRow[(size_t)(8 * RS_NF + (k)) * a.Mcap + s]
 #define LAM(k) a.sLam[(size_t)(k) * a.Mcap + s]
+// sMode: what the solve has to know of a slot this substep: points, softness, and the points
+// whose normal or friction row has no mass (invN or invT is 0) and is left out
+enum { MODE_NUM = 255, MODE_SOFT = 256, MODE_SKIP_N = 1 << 16, MODE_SKIP_T = 1 << 20 };
+// a pass over the contacts: with the bias; without the soft contacts (relaxation); the
+// substep's first (the lambdas are 0) and last (nothing reads them afterwards)
+enum { PASS_BIAS = 1, PASS_SKIP_SOFT = 2, PASS_FIRST = 4, PASS_LAST = 8 };
 
 struct SubArgs {
     int M, Mcap, D, nColors, substeps, iterations;
     float h, g;
-    const int32_t *sB0, *sB1, *sA0, *sA1, *sFlags, *colorStart;
-    const float4 *sN, *sR0, *sR1;
+    const int32_t *sB, *sA;               // 2 per slot: the sides' dynamic bodies (-1) and internal bodies
+    const int32_t *sFlags, *colorStart;
+    const float4 *sN, *sR;
     const float2* sSoft;
-    float4 *sRow, *sLam;
+    float4* sRow;
+    float2* sLam;
+    int32_t* sMode;
     float4 *bpos, *bquat;                 // body poses (dynamic bodies come first)
     float4 *dvel, *dang;                  // component velocity at the start of the substep (dvel.w = invMass)
-    float4* bvel;                         // per dynamic body: solver v, w (velocityTemp), component
-                                          // v, w after gravity + gyroscopic term (friction reads them)
+    float4* bvel;                         // per dynamic body: solver v (.w = invMass), w (velocityTemp)
+    float4* brec;                         // per dynamic body: what its contact rows are built from
     const float4 *dcom, *dinvI;
     float4 *pvel, *pang;                  // pseudo velocities (pang.w = constraint count)
     // dependency-driven passes: per body, the colours of its manifolds (2 x 64 bits); a work
@@ -422,6 +442,18 @@ struct SubArgs {
     int xctlWords;                        // words of xctl cleared by k_prepare
 };
 
+// the even (side 0) or the odd (side 1) lane's value in both lanes of a pair
+__device__ __forceinline__ float side0(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xA0, 0xf, 0xf, true));   // quad_perm 0,0,2,2
+}
+__device__ __forceinline__ float side1(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xF5, 0xf, 0xf, true));   // quad_perm 1,1,3,3
+}
+__device__ __forceinline__ f3 side0(f3 v) { return mk3(side0(v.x), side0(v.y), side0(v.z)); }
+__device__ __forceinline__ f3 side1(f3 v) { return mk3(side1(v.x), side1(v.y), side1(v.z)); }
+// side 0's half of a relative velocity carries a minus sign
+__device__ __forceinline__ f3 signed_of(f3 v, int side) { return side ? v : neg(v); }
+
 __device__ __forceinline__ m3 world_inv_inertia(const SubArgs& a, int b) {
     m3 rot = mat3_cast(q4(a.bquat[b]));
     m3 invI = mk_m3(xyz(a.dinvI[3 * b]), xyz(a.dinvI[3 * b + 1]), xyz(a.dinvI[3 * b + 2]));
@@ -429,71 +461,75 @@ __device__ __forceinline__ m3 world_inv_inertia(const SubArgs& a, int b) {
 }
 
 // update contact rows (src/Physecs.cpp:368-426) then preSolve (src/ContactConstraints.cpp:4-31)
-// of one manifold; the world inverse inertia is rebuilt with the same operations as massTemp.
-__device__ void prepare_manifold(const SubArgs& a, int s) {
-    int b0 = a.sB0[s], b1 = a.sB1[s], a0 = a.sA0[s], a1 = a.sA1[s];
-    int num = a.sFlags[s] & 255;
-    f3 n = xyz(a.sN[s]);
-    qf q0 = q4(a.bquat[a0]), q1 = q4(a.bquat[a1]);
-    f3 com0 = s3(0.f), v0 = s3(0.f), w0 = s3(0.f), com1 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-    float im0 = 0.f, im1 = 0.f;
-    m3 I0 = mzero(), I1 = mzero();
-    if (b0 >= 0) {
-        com0 = add(xyz(a.bpos[a0]), qrot(q0, xyz(a.dcom[b0])));
-        float4 vv = a.dvel[b0];
-        v0 = xyz(vv); im0 = vv.w; w0 = xyz(a.dang[b0]);
-        I0 = world_inv_inertia(a, b0);
+// of one side of a manifold. Everything of the body comes from its record (integrate_velocity),
+// one 128-byte line per side; gathered from the bodies' six arrays, with the inertia and the
+// centre of mass rebuilt per manifold, the kernel was bound by those gathers: 58 us on 295k
+// manifolds of 218k bodies instead of 25 (and 10 more for the bodies' records in the write-back).
+__device__ void prepare_side(const SubArgs& a, int i) {
+    const int s = i >> 1, side = i & 1;
+    const int b = a.sB[i], flags = a.sFlags[s], num = flags & 255;
+    const f3 n = xyz(a.sN[s]);
+    qf q;
+    f3 com = s3(0.f), v = s3(0.f), w = s3(0.f), cv = s3(0.f), cw = s3(0.f);
+    float im = 0.f;
+    m3 I = mzero();
+    if (b >= 0) {
+        const float4 *r = a.brec + br(b, 0), rc = r[BR_COM], rv = r[BR_V], rw = r[BR_W], i0 = r[BR_I0];
+        q = q4(r[BR_Q]);
+        com = xyz(rc); im = rc.w;
+        v = xyz(rv); w = xyz(rw);
+        I = mk_m3(xyz(i0), xyz(r[BR_I1]), xyz(r[BR_I2]));
+        cv = add(v, mul(a.h, mk3(0.f, -a.g, 0.f)));   // as integrate_velocity
+        cw = mk3(rv.w, rw.w, i0.w);
+    } else {
+        q = q4(a.bquat[a.sA[i]]);
     }
-    if (b1 >= 0) {
-        com1 = add(xyz(a.bpos[a1]), qrot(q1, xyz(a.dcom[b1])));
-        float4 vv = a.dvel[b1];
-        v1 = xyz(vv); im1 = vv.w; w1 = xyz(a.dang[b1]);
-        I1 = world_inv_inertia(a, b1);
-    }
-    float nn = dot(n, n);
-    const int sflags = a.sFlags[s];
-    const bool soft = (sflags & 256) != 0;
+    const float nn = dot(n, n), imSum = side0(im) + side1(im);
+    const bool soft = (flags & 256) != 0;
     const float2 sp = a.sSoft[s];
     const float h = a.h;
+    int mode = num | (soft ? MODE_SOFT : 0);
     for (int k = 0; k < num; ++k) {
-        f3 r0 = qrot(q0, xyz(a.sR0[(size_t)k * a.Mcap + s]));
-        f3 r1 = qrot(q1, xyz(a.sR1[(size_t)k * a.Mcap + s]));
-        f3 cp0 = add(com0, r0), cp1 = add(com1, r1);
-        float cn = dot(sub(cp1, cp0), n);
-        f3 r0xn = cross(r0, n), r1xn = cross(r1, n);
-        f3 rel = sub(sub(add(v1, cross(w1, r1)), v0), cross(w0, r0));
-        float relN = dot(rel, n);
+        const float4 anchor = a.sR[2 * (size_t)k * a.Mcap + i];
+        const f3 r = qrot(q, xyz(anchor));
+        const f3 cp = add(com, r);
+        const float cn = dot(sub(side1(cp), side0(cp)), n);
+        const f3 rxn = cross(r, n);
+        const f3 wxr = cross(w, r);
+        const f3 rel = sub(sub(side1(add(v, wxr)), side0(v)), side0(wxr));
+        const float relN = dot(rel, n);
         f3 t = sub(rel, mul(relN, n));
-        float tl = length(t);
+        const float tl = length(t);
         if (tl != 0.f) t = divs(t, tl);
-        f3 r0xt = cross(r0, t), r1xt = cross(r1, t);
-        f3 r0xnt = mulmv(I0, r0xn), r1xnt = mulmv(I1, r1xn), r0xtt = mulmv(I0, r0xt), r1xtt = mulmv(I1, r1xt);
-        float invN = nn * (im0 + im1) + dot(r0xn, r0xnt) + dot(r1xn, r1xnt);
-        float invT = dot(t, t) * (im0 + im1) + dot(r0xt, r0xtt) + dot(r1xt, r1xtt);
+        const f3 rxt = cross(r, t);
+        const f3 rxnt = mulmv(I, rxn), rxtt = mulmv(I, rxt);
+        const float dn = dot(rxn, rxnt), dt = dot(rxt, rxtt);
+        const float invN = nn * imSum + side0(dn) + side1(dn);
+        const float invT = dot(t, t) * imSum + side0(dt) + side1(dt);
         // src/ContactConstraints.cpp:54-68 on the substep's fixed values
         const float effMass = 1.f / invN;
         const float bias = 0.1f * cn / h;
-        float softA = 0.f, softB = 0.f;
+        float termA = effMass, termB = bias;
         if (soft) {
             float af = 2.f * 3.14159265358979323846f * sp.x;
             float stiffness = af * af * effMass;
             float damping = 2.f * af * sp.y * effMass;
             float gamma = 1.f / (damping + h * stiffness);
             float beta = h * stiffness / (damping + h * stiffness);
-            softA = beta * cn / h;
-            softB = invN + gamma / h;
+            termA = invN + gamma / h;
+            termB = beta * cn / h;
         }
-        ROW(R_R0XN, k) = f4(r0xn, cn);
-        ROW(R_R1XN, k) = f4(r1xn, invN);
-        ROW(R_T, k) = f4(t, invT);
-        ROW(R_R0XT, k) = f4(r0xt, effMass);
-        ROW(R_R1XT, k) = f4(r1xt, bias);
-        ROW(R_R0XNT, k) = f4(r0xnt, softA);
-        ROW(R_R1XNT, k) = f4(r1xnt, softB);
-        ROW(R_R0XTT, k) = f4(r0xtt, 0.f);
-        ROW(R_R1XTT, k) = f4(r1xtt, 0.f);
-        LAM(k) = make_float4(0.f, 0.f, a.sR0[(size_t)k * a.Mcap + s].w, 0.f);   // lambdas start at 0
+        // the friction impulse of one pass, on the component velocities
+        const float ct = dot(signed_of(t, side), cv), cr = dot(signed_of(rxt, side), cw);
+        const float rvT = side0(ct + cr) + side1(ct) + side1(cr);
+        if (invN == 0.f) mode |= MODE_SKIP_N << k;
+        if (invT == 0.f) mode |= MODE_SKIP_T << k;
+        ROW(RS_N, k) = f4(signed_of(rxn, side), anchor.w);
+        ROW(RS_NT, k) = f4(signed_of(rxnt, side), termA);
+        ROW(RS_TT, k) = f4(signed_of(rxtt, side), termB);
+        if (side == 0) ROWT(k) = f4(t, rvT / invT);
     }
+    if (side == 0) a.sMode[s] = mode;
 }
 
 // src/MathUtil.h:10-21
@@ -505,175 +541,144 @@ __device__ __forceinline__ f3 solve33(const m3& A, f3 b) {
     return mk3(id * dot(b, c12), id * dot(A.c0, cross(b, A.c2)), id * dot(A.c0, cross(A.c1, b)));
 }
 
-// integrate velocities of one body, src/Physecs.cpp:443-468
-__device__ void integrate_velocity(const SubArgs& a, int d) {
-    if (a.dcom[d].w != 0.f) return;   // kinematic
-    m3 rot = mat3_cast(q4(a.bquat[d]));
+// integrate velocities of one body, src/Physecs.cpp:443-468, from its component velocities;
+// and its record for the substep's contact and joint rows
+__device__ void integrate_velocity(const SubArgs& a, int d, float4 vv, f3 ang) {
+    const float4 cm = a.dcom[d];
+    if (cm.w != 0.f) return;   // kinematic
+    const qf q = q4(a.bquat[d]);
+    m3 rot = mat3_cast(q);
     m3 invRot = transpose(rot);
-    float4 vv = a.dvel[d];
     f3 v = add(xyz(vv), mul(a.h, mk3(0.f, -a.g, 0.f)));
     m3 invI = mk_m3(xyz(a.dinvI[3 * d]), xyz(a.dinvI[3 * d + 1]), xyz(a.dinvI[3 * d + 2]));
-    f3 wl = mulmv(invRot, xyz(a.dang[d]));
+    f3 wl = mulmv(invRot, ang);
     m3 I = inverse(invI);
     f3 Iw = mulmv(I, wl);
     f3 f = mul(a.h, cross(wl, Iw));
     m3 J = madd(I, mscale(a.h, msub(mulmm(matrixCross3(wl), I), matrixCross3(Iw))));
     wl = sub(wl, solve33(J, f));
     f3 w = mulmv(rot, wl);
-    a.bvel[bv(d, BV_CV)] = f4(v, vv.w);
-    a.bvel[bv(d, BV_CW)] = f4(w, 0.f);
-    a.bvel[bv(d, BV_V)] = f4(v, 0.f);
+    a.bvel[bv(d, BV_V)] = f4(v, vv.w);
     a.bvel[bv(d, BV_W)] = f4(w, 0.f);
-    const m3 wI = world_inv_inertia(a, d);   // the inertia prepare_manifold uses this substep
-    a.bvel[bv(d, BV_I0)] = f4(wI.c0, 0.f);
-    a.bvel[bv(d, BV_I1)] = f4(wI.c1, 0.f);
-    a.bvel[bv(d, BV_I2)] = f4(wI.c2, 0.f);
+    const m3 wI = world_inv_inertia(a, d);   // massTemp of the substep
+    float4* r = a.brec + br(d, 0);
+    r[BR_COM] = f4(add(xyz(a.bpos[d]), qrot(q, xyz(cm))), vv.w);
+    r[BR_Q] = f4q(q);
+    r[BR_V] = f4(xyz(vv), w.x);
+    r[BR_W] = f4(ang, w.y);
+    r[BR_I0] = f4(wI.c0, w.z);
+    r[BR_I1] = f4(wI.c1, 0.f);
+    r[BR_I2] = f4(wI.c2, 0.f);
     a.pvel[d] = make_float4(0.f, 0.f, 0.f, 0.f);
     a.pang[d] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// One manifold's normal then friction rows, src/ContactConstraints.cpp:33-124. Manifolds of
-// one colour touch disjoint dynamic bodies, so a colour is solved in parallel exactly as a
-// sequential pass over it would be.
-// Everything one manifold's solve reads except the bodies' solver velocities: the
-// manifold's rows, normal, friction, cached target velocities and lambdas, and both
-// bodies' inverse masses and component velocities. All of it is fixed for the whole pass.
-struct MInputs {
-    int num, b0, b1;
+// Everything one side's solve reads except its body's solver velocities: the manifold's
+// mode, normal (with the side's sign) and friction, and its rows, tangents and lambdas. All
+// of it is fixed for the whole pass.
+struct SideIn {
+    int num, mode, b;
     bool soft;
-    f3 n;
-    float friction, im0, im1;
-    f3 cv0, cw0, cv1, cw1;
-    float4 row[4][R_NF], lam[4];
+    f3 sn;
+    float friction;
+    float4 row[4][RS_NF], t[4];
+    float2 lam[4];
 };
 
-// the manifold's own inputs: flags, bodies, normal; point slots' rows and lambdas (all four
-// slots when ALL, else slot 0 with the flags and slots 1-3 once the point count is known)
-template <bool ALL>
-__device__ __forceinline__ void load_own(const SubArgs& a, int s, MInputs& in) {
-    const int flags = a.sFlags[s];
-    in.soft = (flags & 256) != 0;
-    in.num = flags & 255;
-    in.b0 = a.sB0[s];
-    in.b1 = a.sB1[s];
-    const float4 nf = a.sN[s];
-    in.n = xyz(nf);
-    in.friction = nf.w;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (ALL || k == 0 || k < in.num) {
-#pragma unroll
-            for (int f = 0; f < R_NF; ++f) in.row[k][f] = ROW(f, k);
-            in.lam[k] = LAM(k);
-        }
-    }
-}
-
 // EAGER loads point slot 0's rows (every manifold has a first point) with the manifold's
-// flags and body indices, without waiting for the point count; slots 1-3 wait for the
-// count, in the same round of loads as the body records (which wait for the body indices
+// mode and body index, without waiting for the point count; slots 1-3 wait for the count,
+// in the same round of loads as the body's velocities (which wait for the body index
 // anyway), so unused slots cost no traffic and the solve still takes two dependent rounds.
 template <bool EAGER = false>
-__device__ __forceinline__ void load_inputs(const SubArgs& a, int s, MInputs& in) {
-    int flags = a.sFlags[s];
-    in.soft = (flags & 256) != 0;
-    in.num = flags & 255;
-    in.b0 = a.sB0[s];
-    in.b1 = a.sB1[s];
-    float4 nf = a.sN[s];
-    in.n = xyz(nf);
+__device__ __forceinline__ void load_side(const SubArgs& a, int i, int pass, SideIn& in) {
+    const int s = i >> 1;
+    in.mode = a.sMode[s];
+    in.soft = (in.mode & MODE_SOFT) != 0;
+    in.num = in.mode & MODE_NUM;
+    in.b = a.sB[i];
+    const float4 nf = a.sN[s];
+    in.sn = signed_of(xyz(nf), i & 1);
     in.friction = nf.w;
-    in.im0 = 0.f; in.im1 = 0.f;
-    in.cv0 = s3(0.f); in.cw0 = s3(0.f); in.cv1 = s3(0.f); in.cw1 = s3(0.f);
-    if (in.b0 >= 0) {
-        float4 c = a.bvel[bv(in.b0, BV_CV)];
-        in.im0 = c.w; in.cv0 = xyz(c); in.cw0 = xyz(a.bvel[bv(in.b0, BV_CW)]);
-    }
-    if (in.b1 >= 0) {
-        float4 c = a.bvel[bv(in.b1, BV_CV)];
-        in.im1 = c.w; in.cv1 = xyz(c); in.cw1 = xyz(a.bvel[bv(in.b1, BV_CW)]);
-    }
-    // all rows of the manifold are loaded before any dependent arithmetic (memory-level
+    // all rows of the side are loaded before any dependent arithmetic (memory-level
     // parallelism); unused point slots are never read back
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if ((EAGER && k == 0) || k < in.num) {
 #pragma unroll
-            for (int f = 0; f < R_NF; ++f) in.row[k][f] = ROW(f, k);
-            in.lam[k] = LAM(k);
+            for (int f = 0; f < RS_NF; ++f) in.row[k][f] = ROW(f, k);
+            in.t[k] = ROWT(k);
+            in.lam[k] = (pass & PASS_FIRST) ? make_float2(0.f, 0.f) : LAM(k);
         }
     }
 }
 
-// ContactConstraints::solve (src/ContactConstraints.cpp:33-124) of one manifold on the
-// bodies' solver velocities v0, w0, v1, w1 (updated in place); stores the accumulated
-// lambdas in the manifold's rows. The effective mass, the bias and a soft contact's terms
-// come from the rows (computed once per substep with the same operations).
-__device__ __forceinline__ void solve_core(const SubArgs& a, int s, const MInputs& in, bool useBias, float h, f3& v0,
-                                           f3& w0, f3& v1, f3& w1) {
-    (void)h;
-    const int num = in.num, b0 = in.b0, b1 = in.b1;
-    const f3 n = in.n;
-    const float im0 = in.im0, im1 = in.im1;
+// ContactConstraints::solve (src/ContactConstraints.cpp:33-124) of one side of a manifold,
+// normal then friction rows, on its body's solver velocities (v.w = invMass; updated in
+// place); the even lane stores the accumulated lambdas. Manifolds of one colour touch
+// disjoint dynamic bodies, so a colour is solved in parallel exactly as a sequential pass
+// over it would be. Both lanes of the pair run it together.
+__device__ __forceinline__ void solve_side(const SubArgs& a, int i, const SideIn& in, int pass, float4& v4, f3& w) {
+    const int s = i >> 1, num = in.num;
+    const bool moves = in.b >= 0;
+    const float im = (i & 1) ? v4.w : -v4.w;
+    f3 v = xyz(v4);
     float lN[4], lT[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k >= num) break;
         const float4* r = in.row[k];
         lN[k] = in.lam[k].x;
-        float invN = r[R_R1XN].w;
-        if (invN == 0.f) continue;
-        f3 r0xn = xyz(r[R_R0XN]), r1xn = xyz(r[R_R1XN]);
-        float rv = dot(neg(n), v0) + dot(neg(r0xn), w0) + dot(n, v1) + dot(r1xn, w1);
+        if (in.mode & (MODE_SKIP_N << k)) continue;
+        const float p = dot(in.sn, v), q = dot(xyz(r[RS_N]), w);
+        const float rv = side0(p + q) + side1(p) + side1(q);
         float lambda;
-        if (in.soft) lambda = (rv + r[R_R0XNT].w) / r[R_R1XNT].w;
-        else lambda = (rv - in.lam[k].z + (useBias ? r[R_R1XT].w : 0.f)) * r[R_R0XT].w;
-        float prev = lN[k];
+        if (in.soft) lambda = (rv + r[RS_TT].w) / r[RS_NT].w;
+        else lambda = (rv - r[RS_N].w + ((pass & PASS_BIAS) ? r[RS_TT].w : 0.f)) * r[RS_NT].w;
+        const float prev = lN[k];
         lN[k] = lN[k] + lambda;
         lN[k] = gmin(lN[k], 0.f);
         lambda = lN[k] - prev;
-        if (b0 >= 0) { v0 = add(v0, mul(lambda * im0, n)); w0 = add(w0, mul(lambda, xyz(r[R_R0XNT]))); }
-        if (b1 >= 0) { v1 = sub(v1, mul(lambda * im1, n)); w1 = sub(w1, mul(lambda, xyz(r[R_R1XNT]))); }
+        if (moves) {   // the normal with side 1's sign times -im or im: the side's own sign
+            v = sub(v, mul(lambda * im, signed_of(in.sn, i & 1)));
+            w = sub(w, mul(lambda, xyz(r[RS_NT])));
+        }
     }
-    // friction rows read the component velocities (src/ContactConstraints.cpp:142-152)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k >= num) break;
-        const float4* r = in.row[k];
         lT[k] = in.lam[k].y;
-        float invT = r[R_T].w;
-        if (invT == 0.f) continue;
-        f3 t = xyz(r[R_T]), r0xt = xyz(r[R_R0XT]), r1xt = xyz(r[R_R1XT]);
-        float rv = dot(neg(t), in.cv0) + dot(neg(r0xt), in.cw0) + dot(t, in.cv1) + dot(r1xt, in.cw1);
-        float lambda = rv / invT;
-        float limit = in.friction * lN[k];
-        float prev = lT[k];
-        lT[k] = lT[k] + lambda;
+        if (in.mode & (MODE_SKIP_T << k)) continue;
+        const float limit = in.friction * lN[k];
+        const float prev = lT[k];
+        lT[k] = lT[k] + in.t[k].w;
         lT[k] = gclamp(lT[k], limit, -limit);
-        lambda = lT[k] - prev;
-        if (b0 >= 0) { v0 = add(v0, mul(lambda * im0, t)); w0 = add(w0, mul(lambda, xyz(r[R_R0XTT]))); }
-        if (b1 >= 0) { v1 = sub(v1, mul(lambda * im1, t)); w1 = sub(w1, mul(lambda, xyz(r[R_R1XTT]))); }
+        const float lambda = lT[k] - prev;
+        if (moves) {
+            v = sub(v, mul(lambda * im, xyz(in.t[k])));
+            w = sub(w, mul(lambda, xyz(in.row[k][RS_TT])));
+        }
     }
+    v4 = f4(v, v4.w);
+    if ((i & 1) || (pass & PASS_LAST)) return;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k >= num) break;
-        *reinterpret_cast<float2*>(&LAM(k)) = make_float2(lN[k], lT[k]);
+        LAM(k) = make_float2(lN[k], lT[k]);
     }
 }
 
-// one manifold of a colour launch: every other manifold touching its bodies is in another
-// launch, so plain accesses see the previous colours' results
+// one side of a manifold of a colour launch: every other manifold touching its body is in
+// another launch, so plain accesses see the previous colours' results
 template <bool EAGER = false>
-__device__ void solve_manifold(const SubArgs& a, int s, bool useBias, float h, bool skipSoft) {
-    MInputs in;
-    load_inputs<EAGER>(a, s, in);
-    if (skipSoft && in.soft) return;
-    f3 v0 = s3(0.f), w0 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-    if (in.b0 >= 0) { v0 = xyz(a.bvel[bv(in.b0, BV_V)]); w0 = xyz(a.bvel[bv(in.b0, BV_W)]); }
-    if (in.b1 >= 0) { v1 = xyz(a.bvel[bv(in.b1, BV_V)]); w1 = xyz(a.bvel[bv(in.b1, BV_W)]); }
-    solve_core(a, s, in, useBias, h, v0, w0, v1, w1);
-    if (in.b0 >= 0) { a.bvel[bv(in.b0, BV_V)] = f4(v0, 0.f); a.bvel[bv(in.b0, BV_W)] = f4(w0, 0.f); }
-    if (in.b1 >= 0) { a.bvel[bv(in.b1, BV_V)] = f4(v1, 0.f); a.bvel[bv(in.b1, BV_W)] = f4(w1, 0.f); }
+__device__ void solve_lane(const SubArgs& a, int i, int pass) {
+    SideIn in;
+    load_side<EAGER>(a, i, pass, in);
+    if ((pass & PASS_SKIP_SOFT) && in.soft) return;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    f3 w = s3(0.f);
+    if (in.b >= 0) { v = a.bvel[bv(in.b, BV_V)]; w = xyz(a.bvel[bv(in.b, BV_W)]); }
+    solve_side(a, i, in, pass, v, w);
+    if (in.b >= 0) { a.bvel[bv(in.b, BV_V)] = v; a.bvel[bv(in.b, BV_W)] = f4(w, 0.f); }
 }
 
 // integrate positions of one body, src/Physecs.cpp:494-511
@@ -697,29 +702,36 @@ __device__ void integrate_position(const SubArgs& a, int d) {
     a.bquat[d] = f4q(q);
 }
 
-// write back, src/Physecs.cpp:523-530
-__device__ void write_back(const SubArgs& a, int d) {
+// write back, src/Physecs.cpp:523-530, and, when another substep follows (next), its
+// velocity integration: one launch over the bodies between two substeps
+__device__ void write_back(const SubArgs& a, int d, bool next) {
     if (a.dcom[d].w != 0.f) return;
-    float4 v = a.bvel[bv(d, BV_V)];
-    a.dvel[d] = make_float4(v.x, v.y, v.z, a.dvel[d].w);
-    a.dang[d] = a.bvel[bv(d, BV_W)];
+    const float4 v = a.bvel[bv(d, BV_V)], w = a.bvel[bv(d, BV_W)];
+    a.dvel[d] = v;
+    a.dang[d] = w;
+    if (next) integrate_velocity(a, d, v, xyz(w));
 }
 
 // ------------------------------------------------------------------ discrete kernels
-__global__ __launch_bounds__(256) void k_prepare(SubArgs a, int sub) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < (a.iterations + 1) * FLOW_QUEUES) a.tickets[i] = 0;
-    if (i == 0) a.barrier[0] = 0;
-    for (int j = i; j < a.xctlWords; j += gridDim.x * blockDim.x) a.xctl[j] = 0;
-    if (sub == 0 && i < FLOW_QUEUES) a.qDone[i] = 0;
-    if (i < a.M) prepare_manifold(a, i);
-    else if (i - a.M < a.D) integrate_velocity(a, i - a.M);
+// the first substep's velocity integration
+__global__ __launch_bounds__(256) void k_integrate_velocities(SubArgs a) {
+    const int d = blockIdx.x * blockDim.x + threadIdx.x;
+    if (d < a.D) integrate_velocity(a, d, a.dvel[d], xyz(a.dang[d]));
 }
-// XCD-homed slots. Workgroups are dispatched round-robin to the 8 XCDs (workgroup b on XCD
-// b % 8), each with its own L2. k_prepare writes slot s's rows from workgroup s / 256, so
-// from XCD (s / 256) % 8, the slot's home; the colour launches give each workgroup a chunk
-// of BLOCK slots homed on its own XCD, so the rows (and the lambdas, rewritten in place every
-// pass) are read from that XCD's L2 rather than from memory. Chunk k holds slots
+
+__global__ __launch_bounds__(256) void k_prepare(SubArgs a, int sub) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
+    for (int j = i; j < (a.iterations + 1) * FLOW_QUEUES; j += nth) a.tickets[j] = 0;
+    if (i == 0) a.barrier[0] = 0;
+    for (int j = i; j < a.xctlWords; j += nth) a.xctl[j] = 0;
+    if (sub == 0 && i < FLOW_QUEUES) a.qDone[i] = 0;
+    if (i < 2 * a.M) prepare_side(a, i);
+}
+// XCD-homed lanes. Workgroups are dispatched round-robin to the 8 XCDs (workgroup b on XCD
+// b % 8), each with its own L2. k_prepare writes side lane i's rows from workgroup i / 256, so
+// from XCD (i / 256) % 8, the lane's home; the colour launches give each workgroup a chunk
+// of BLOCK lanes homed on its own XCD, so the rows (and the lambdas, rewritten in place every
+// pass) are read from that XCD's L2 rather than from memory. Chunk k holds lanes
 // [k * BLOCK, (k + 1) * BLOCK); its home is (k / q) % 8 with q = 256 / BLOCK chunks per
 // prepare workgroup, so home-x chunks come in runs of q, one run every 8q chunks. Workgroup
 // b (XCD x = b % 8) takes the (b / 8)-th home-x chunk at or after chunk k0.
@@ -730,11 +742,12 @@ __device__ __forceinline__ int homed_chunk(int b, int k0, int q) {
     return period * (m / q) + q * x + (m % q);
 }
 
+// side lanes [begin, end) of one colour (both even)
 template <int BLOCK, bool EAGER>
-__global__ __launch_bounds__(BLOCK) void k_solve(SubArgs a, int begin, int end, int useBias, float h, int skipSoft) {
+__global__ __launch_bounds__(BLOCK) void k_solve(SubArgs a, int begin, int end, int pass) {
     const int k = homed_chunk(blockIdx.x, begin / BLOCK, 256 / BLOCK);
-    int s = k * BLOCK + threadIdx.x;
-    if (s >= begin && s < end) solve_manifold<EAGER>(a, s, useBias != 0, h, skipSoft != 0);
+    const int i = k * BLOCK + threadIdx.x;
+    if (i >= begin && i < end) solve_lane<EAGER>(a, i, pass);
 }
 
 // ------------------------------------------------------------------ one launch per pass
@@ -765,16 +778,18 @@ __device__ __forceinline__ void st_agent3(float4* p, f3 v) {
     __hip_atomic_store(q + 2, __float_as_uint(v.z), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the solve of one manifold whose fixed inputs are loaded, on velocities at the coherence point
-__device__ __forceinline__ void solve_coherent(const SubArgs& a, int s, const MInputs& in, bool useBias, float h,
-                                              bool skipSoft) {
-    if (skipSoft && in.soft) return;
-    f3 v0 = s3(0.f), w0 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-    if (in.b0 >= 0) { v0 = ld_agent3(&a.bvel[bv(in.b0, BV_V)]); w0 = ld_agent3(&a.bvel[bv(in.b0, BV_W)]); }
-    if (in.b1 >= 0) { v1 = ld_agent3(&a.bvel[bv(in.b1, BV_V)]); w1 = ld_agent3(&a.bvel[bv(in.b1, BV_W)]); }
-    solve_core(a, s, in, useBias, h, v0, w0, v1, w1);
-    if (in.b0 >= 0) { st_agent3(&a.bvel[bv(in.b0, BV_V)], v0); st_agent3(&a.bvel[bv(in.b0, BV_W)], w0); }
-    if (in.b1 >= 0) { st_agent3(&a.bvel[bv(in.b1, BV_V)], v1); st_agent3(&a.bvel[bv(in.b1, BV_W)], w1); }
+// the solve of one side whose fixed inputs are loaded, on velocities at the coherence point
+// (the inverse mass beside them never changes)
+__device__ __forceinline__ void solve_coherent(const SubArgs& a, int i, const SideIn& in, int pass) {
+    if ((pass & PASS_SKIP_SOFT) && in.soft) return;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    f3 w = s3(0.f);
+    if (in.b >= 0) {
+        v = f4(ld_agent3(&a.bvel[bv(in.b, BV_V)]), a.bvel[bv(in.b, BV_V)].w);
+        w = ld_agent3(&a.bvel[bv(in.b, BV_W)]);
+    }
+    solve_side(a, i, in, pass, v, w);
+    if (in.b >= 0) { st_agent3(&a.bvel[bv(in.b, BV_V)], xyz(v)); st_agent3(&a.bvel[bv(in.b, BV_W)], w); }
 }
 
 // grid barrier number `target` / gridDim.x of the substep: every workgroup has arrived
@@ -797,27 +812,25 @@ __device__ __forceinline__ void pass_barrier(int32_t* count, int target, int32_t
     __syncthreads();
 }
 
-__global__ __launch_bounds__(PASS_THREADS) void k_solve_pass(SubArgs a, int nColors, int useBias, float h,
-                                                            int skipSoft, int barrierBase) {
+__global__ __launch_bounds__(PASS_THREADS) void k_solve_pass(SubArgs a, int nColors, int pass, int barrierBase) {
     const int tid = blockIdx.x * PASS_THREADS + threadIdx.x;
     const int nth = gridDim.x * PASS_THREADS;
-    const bool bias = useBias != 0, skip = skipSoft != 0;
-    int s = a.colorStart[0] + tid, e = a.colorStart[1];
-    MInputs in;
-    bool have = s < e;
-    if (have) load_inputs<true>(a, s, in);
+    int i = 2 * a.colorStart[0] + tid, e = 2 * a.colorStart[1];
+    SideIn in;
+    bool have = i < e;
+    if (have) load_side<true>(a, i, pass, in);
     for (int c = 0; c < nColors; ++c) {
-        if (have) solve_coherent(a, s, in, bias, h, skip);
-        for (int s2 = s + nth; s2 < e; s2 += nth) {
-            MInputs in2;
-            load_inputs<true>(a, s2, in2);
-            solve_coherent(a, s2, in2, bias, h, skip);
+        if (have) solve_coherent(a, i, in, pass);
+        for (int i2 = i + nth; i2 < e; i2 += nth) {
+            SideIn in2;
+            load_side<true>(a, i2, pass, in2);
+            solve_coherent(a, i2, in2, pass);
         }
         if (c + 1 == nColors) break;
-        s = e + tid;                 // the next colour starts where this one ends
-        e = a.colorStart[c + 2];
-        have = s < e;
-        if (have) load_inputs<true>(a, s, in);
+        i = e + tid;                 // the next colour starts where this one ends
+        e = 2 * a.colorStart[c + 2];
+        have = i < e;
+        if (have) load_side<true>(a, i, pass, in);
         pass_barrier(a.barrier, barrierBase + (c + 1) * (int)gridDim.x, a.flowErr);
     }
 }
@@ -843,19 +856,19 @@ constexpr int XPASS_MAX_GRID = 248; // at most 31 workgroups per XCD: a byte nev
 
 __device__ __forceinline__ f3 ld_l2_3(const float4* p) { return ld_agent3(p); }
 
-__device__ __forceinline__ void solve_xcd(const SubArgs& a, int s, const MInputs& in, bool useBias, float h,
-                                          bool skipSoft) {
-    if (skipSoft && in.soft) return;
-    f3 v0 = s3(0.f), w0 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-    if (in.b0 >= 0) { v0 = ld_l2_3(&a.bvel[bv(in.b0, BV_V)]); w0 = ld_l2_3(&a.bvel[bv(in.b0, BV_W)]); }
-    if (in.b1 >= 0) { v1 = ld_l2_3(&a.bvel[bv(in.b1, BV_V)]); w1 = ld_l2_3(&a.bvel[bv(in.b1, BV_W)]); }
-    solve_core(a, s, in, useBias, h, v0, w0, v1, w1);
-    if (in.b0 >= 0) { a.bvel[bv(in.b0, BV_V)] = f4(v0, 0.f); a.bvel[bv(in.b0, BV_W)] = f4(w0, 0.f); }
-    if (in.b1 >= 0) { a.bvel[bv(in.b1, BV_V)] = f4(v1, 0.f); a.bvel[bv(in.b1, BV_W)] = f4(w1, 0.f); }
+__device__ __forceinline__ void solve_xcd(const SubArgs& a, int i, const SideIn& in, int pass) {
+    if ((pass & PASS_SKIP_SOFT) && in.soft) return;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    f3 w = s3(0.f);
+    if (in.b >= 0) {
+        v = f4(ld_l2_3(&a.bvel[bv(in.b, BV_V)]), a.bvel[bv(in.b, BV_V)].w);
+        w = ld_l2_3(&a.bvel[bv(in.b, BV_W)]);
+    }
+    solve_side(a, i, in, pass, v, w);
+    if (in.b >= 0) { a.bvel[bv(in.b, BV_V)] = v; a.bvel[bv(in.b, BV_W)] = f4(w, 0.f); }
 }
 
-__global__ __launch_bounds__(XPASS_THREADS) void k_solve_xpass(SubArgs a, int nColors, int useBias, float h,
-                                                              int skipSoft, int32_t* ctl) {
+__global__ __launch_bounds__(XPASS_THREADS) void k_solve_xpass(SubArgs a, int nColors, int pass, int32_t* ctl) {
     __shared__ int sRank, sP;
     unsigned long long* reg = reinterpret_cast<unsigned long long*>(ctl);
     if (threadIdx.x == 0) {
@@ -889,23 +902,22 @@ __global__ __launch_bounds__(XPASS_THREADS) void k_solve_xpass(SubArgs a, int nC
     if (P == 0) return;            // another XCD's workgroup (or registration failed)
     const int tid = sRank * XPASS_THREADS + threadIdx.x;
     const int nth = P * XPASS_THREADS;
-    const bool bias = useBias != 0, skip = skipSoft != 0;
-    int s = a.colorStart[0] + tid, e = a.colorStart[1];
-    MInputs in;
-    bool have = s < e;
-    if (have) load_inputs<true>(a, s, in);
+    int i = 2 * a.colorStart[0] + tid, e = 2 * a.colorStart[1];
+    SideIn in;
+    bool have = i < e;
+    if (have) load_side<true>(a, i, pass, in);
     for (int c = 0; c < nColors; ++c) {
-        if (have) solve_xcd(a, s, in, bias, h, skip);
-        for (int s2 = s + nth; s2 < e; s2 += nth) {
-            MInputs in2;
-            load_inputs<true>(a, s2, in2);
-            solve_xcd(a, s2, in2, bias, h, skip);
+        if (have) solve_xcd(a, i, in, pass);
+        for (int i2 = i + nth; i2 < e; i2 += nth) {
+            SideIn in2;
+            load_side<true>(a, i2, pass, in2);
+            solve_xcd(a, i2, in2, pass);
         }
         if (c + 1 == nColors) break;
-        s = e + tid;
-        e = a.colorStart[c + 2];
-        have = s < e;
-        if (have) load_inputs<true>(a, s, in);
+        i = e + tid;
+        e = 2 * a.colorStart[c + 2];
+        have = i < e;
+        if (have) load_side<true>(a, i, pass, in);
         pass_barrier(ctl + 2, (c + 1) * P, a.flowErr);
     }
 }
@@ -918,11 +930,11 @@ __global__ __launch_bounds__(XPASS_THREADS) void k_solve_xpass(SubArgs a, int nC
 // global memory. k_batch_map gives each run its bodies (batchList, from 2S on) and each
 // manifold side its LDS slot (batchLoc, 2 per solve slot; -1 for a static side), once per
 // step: a run's slots never change within the step.
-constexpr int BATCH_THREADS = 512;      // k_solve's register footprint allows 2 waves per SIMD
+constexpr int BATCH_THREADS = 1024;     // two lanes per manifold; 4 waves per SIMD at 128 registers
 constexpr int BATCH_MAP_THREADS = 1024;
 constexpr int BATCH_HASH = 8192;        // LDS hash of body -> slot: at least twice a run's bodies
 constexpr int BATCH_MAX_GROUPS = 16;
-constexpr int BATCH_MAX_MANIFOLDS = 1264;   // 2 x 1264 bodies x 64 B of records in LDS
+constexpr int BATCH_MAX_MANIFOLDS = 1264;   // 2 x 1264 bodies x 32 B of velocities in LDS
 constexpr int BATCH_MAX_COLOURS = 128;
 
 struct BatchGroups {
@@ -934,8 +946,7 @@ __device__ __forceinline__ uint32_t batch_hash(int b) { return ((uint32_t)b * 26
 
 // One workgroup, every run in turn: the run's bodies get slots 0..n-1 in first-claim order
 // (the order does not reach the arithmetic) through an LDS hash table with linear probing.
-__global__ __launch_bounds__(BATCH_MAP_THREADS) void k_batch_map(BatchGroups g, const int32_t* __restrict__ sB0,
-                                                                 const int32_t* __restrict__ sB1,
+__global__ __launch_bounds__(BATCH_MAP_THREADS) void k_batch_map(BatchGroups g, const int32_t* __restrict__ sB,
                                                                  int32_t* __restrict__ batchLoc,
                                                                  int32_t* __restrict__ batchList,
                                                                  int32_t* __restrict__ batchN) {
@@ -948,8 +959,7 @@ __global__ __launch_bounds__(BATCH_MAP_THREADS) void k_batch_map(BatchGroups g, 
         if (threadIdx.x == 0) count = 0;
         __syncthreads();
         for (int i = threadIdx.x; i < sides; i += BATCH_MAP_THREADS) {
-            const int sl = S + (i >> 1);
-            const int b = (i & 1) ? sB1[sl] : sB0[sl];
+            const int b = sB[2 * S + i];
             if (b < 0) continue;
             uint32_t h = batch_hash(b);
             for (int probe = 0; probe < BATCH_HASH; ++probe) {   // the table is never full
@@ -966,15 +976,14 @@ __global__ __launch_bounds__(BATCH_MAP_THREADS) void k_batch_map(BatchGroups g, 
         }
         __syncthreads();
         for (int i = threadIdx.x; i < sides; i += BATCH_MAP_THREADS) {
-            const int sl = S + (i >> 1);
-            const int b = (i & 1) ? sB1[sl] : sB0[sl];
+            const int b = sB[2 * S + i];
             int slot = -1;
             if (b >= 0) {
                 uint32_t h = batch_hash(b);
                 for (int probe = 0; probe < BATCH_HASH && hk[h] != b; ++probe) h = (h + 1) & (BATCH_HASH - 1);
                 slot = hv[h];
             }
-            batchLoc[2 * sl + (i & 1)] = slot;
+            batchLoc[2 * S + i] = slot;
         }
         if (threadIdx.x == 0) batchN[q] = count;
         __syncthreads();
@@ -989,71 +998,58 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The run's bodies' records (solver v and w, component v and w with the inverse mass:
-// BV_V..BV_CW) are gathered into LDS once per launch, so a manifold's solve needs only its
-// own rows from global memory: slot 0's with the flags, slots 1-3 once the point count is
-// known (one CU's load bandwidth bounds these launches, so unused slots are not read). Each
-// colour's rows are loaded before the barrier that waits for the previous colour's
-// velocities, so their latency overlaps the wait.
-constexpr int BATCH_BODY_F4 = BV_CW + 1;
+// The run's bodies' velocities (solver v with the inverse mass, and w) are gathered into
+// LDS once per launch, so a manifold's solve needs only its own rows from global memory:
+// slot 0's with the mode, slots 1-3 once the point count is known (one CU's load bandwidth
+// bounds these launches, so unused slots are not read). Each colour's rows are loaded
+// before the barrier that waits for the previous colour's velocities, so their latency
+// overlaps the wait.
 __global__ __launch_bounds__(BATCH_THREADS) void k_solve_batch(SubArgs a, int c0, int c1, int S,
                                                                const int32_t* __restrict__ batchLoc,
                                                                const int32_t* __restrict__ batchList,
-                                                               const int32_t* __restrict__ batchN, int useBias, float h,
-                                                               int skipSoft) {
-    extern __shared__ float4 rec[];       // [BATCH_BODY_F4][n]: record field f of body slot i at f * n + i
-    __shared__ int32_t cs[BATCH_MAX_COLOURS + 1];   // the run's colour starts
+                                                               const int32_t* __restrict__ batchN, int pass) {
+    extern __shared__ float4 rec[];       // [n] solver v, then [n] solver w of the run's bodies
+    __shared__ int32_t cs[BATCH_MAX_COLOURS + 1];   // the run's colour starts, in side lanes
     const int n = *batchN;
     const int32_t* list = batchList + 2 * S;
-    for (int i = threadIdx.x; i <= c1 - c0; i += BATCH_THREADS) cs[i] = a.colorStart[c0 + i];
+    for (int i = threadIdx.x; i <= c1 - c0; i += BATCH_THREADS) cs[i] = 2 * a.colorStart[c0 + i];
     for (int i = threadIdx.x; i < n; i += BATCH_THREADS) {
         const int b = list[i];
-#pragma unroll
-        for (int f = 0; f < BATCH_BODY_F4; ++f) rec[f * n + i] = a.bvel[bv(b, f)];
+        rec[i] = a.bvel[bv(b, BV_V)];
+        rec[n + i] = a.bvel[bv(b, BV_W)];
     }
     __syncthreads();
-    auto solve = [&](int s, MInputs& in, int2 l) {
-        if (skipSoft && in.soft) return;
-        f3 v0 = s3(0.f), w0 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-        in.im0 = 0.f; in.im1 = 0.f;
-        in.cv0 = s3(0.f); in.cw0 = s3(0.f); in.cv1 = s3(0.f); in.cw1 = s3(0.f);
-        if (in.b0 >= 0) {
-            v0 = xyz(rec[BV_V * n + l.x]); w0 = xyz(rec[BV_W * n + l.x]);
-            const float4 c = rec[BV_CV * n + l.x];
-            in.im0 = c.w; in.cv0 = xyz(c); in.cw0 = xyz(rec[BV_CW * n + l.x]);
-        }
-        if (in.b1 >= 0) {
-            v1 = xyz(rec[BV_V * n + l.y]); w1 = xyz(rec[BV_W * n + l.y]);
-            const float4 c = rec[BV_CV * n + l.y];
-            in.im1 = c.w; in.cv1 = xyz(c); in.cw1 = xyz(rec[BV_CW * n + l.y]);
-        }
-        solve_core(a, s, in, useBias != 0, h, v0, w0, v1, w1);
-        if (in.b0 >= 0) { rec[BV_V * n + l.x] = f4(v0, 0.f); rec[BV_W * n + l.x] = f4(w0, 0.f); }
-        if (in.b1 >= 0) { rec[BV_V * n + l.y] = f4(v1, 0.f); rec[BV_W * n + l.y] = f4(w1, 0.f); }
+    auto solve = [&](int i, const SideIn& in, int l) {
+        if ((pass & PASS_SKIP_SOFT) && in.soft) return;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        f3 w = s3(0.f);
+        if (in.b >= 0) { v = rec[l]; w = xyz(rec[n + l]); }
+        solve_side(a, i, in, pass, v, w);
+        if (in.b >= 0) { rec[l] = v; rec[n + l] = f4(w, 0.f); }
     };
     for (int c = 0; c < c1 - c0; ++c) {
         const int e = cs[c + 1];
-        int s = cs[c] + (int)threadIdx.x;
-        MInputs in;
-        int2 l = make_int2(-1, -1);
-        const bool have = s < e;
+        int i = cs[c] + (int)threadIdx.x;
+        SideIn in;
+        int l = -1;
+        const bool have = i < e;
         if (have) {
-            load_own<false>(a, s, in);
-            l = *reinterpret_cast<const int2*>(batchLoc + 2 * s);
+            load_side(a, i, pass, in);
+            l = batchLoc[i];
         }
         lds_barrier();   // the previous colour's velocities are in LDS
-        if (have) solve(s, in, l);
-        // colours larger than the workgroup: a thread's manifolds of one colour share no body
-        for (s += BATCH_THREADS; s < e; s += BATCH_THREADS) {
-            load_own<false>(a, s, in);
-            solve(s, in, *reinterpret_cast<const int2*>(batchLoc + 2 * s));
+        if (have) solve(i, in, l);
+        // colours larger than the workgroup: a lane's manifolds of one colour share no body
+        for (i += BATCH_THREADS; i < e; i += BATCH_THREADS) {
+            load_side(a, i, pass, in);
+            solve(i, in, batchLoc[i]);
         }
     }
     lds_barrier();
     for (int i = threadIdx.x; i < n; i += BATCH_THREADS) {
         const int b = list[i];
-        a.bvel[bv(b, BV_V)] = rec[BV_V * n + i];
-        a.bvel[bv(b, BV_W)] = rec[BV_W * n + i];
+        a.bvel[bv(b, BV_V)] = rec[i];
+        a.bvel[bv(b, BV_W)] = rec[n + i];
     }
 }
 
@@ -1081,12 +1077,11 @@ __global__ void k_world_ranges(int M, int W, const int32_t* __restrict__ sFlags,
     if (s == M - 1 || ((sFlags[s + 1] >> 16) & 127) != c || sWorld[s + 1] != wd) wcE[c * W + wd] = s + 1;
 }
 
-// One wave per world: a world's colour holds a few dozen manifolds, and the solve's
-// register footprint allows 8 waves per CU, so one-wave workgroups keep 8 worlds resident
-// per CU (when their LDS fits). Rows are loaded eagerly: these colours are latency-bound.
+// One wave per world: a world's colour holds a few dozen manifolds, two lanes each, and
+// one-wave workgroups keep many worlds resident per CU (when their LDS fits). Rows are
+// loaded eagerly: these colours are latency-bound.
 constexpr int WORLD_THREADS = 64;
-__global__ __launch_bounds__(WORLD_THREADS) void k_world_pass(SubArgs a, WorldPassArgs p, int useBias, float h,
-                                                               int skipSoft) {
+__global__ __launch_bounds__(WORLD_THREADS) void k_world_pass(SubArgs a, WorldPassArgs p, int pass) {
     extern __shared__ float4 wv[];        // [n] solver v, then [n] solver w of the world's bodies
     const int wd = p.list[blockIdx.x];
     const int d0 = p.wDyn[wd], n = p.wDyn[wd + 1] - d0;
@@ -1097,18 +1092,17 @@ __global__ __launch_bounds__(WORLD_THREADS) void k_world_pass(SubArgs a, WorldPa
     }
     __syncthreads();
     for (int c = 0; c < p.nColors; ++c) {
-        const int S = p.wcS[c * p.W + wd], E = p.wcE[c * p.W + wd];
-        for (int s = S + (int)threadIdx.x; s < E; s += WORLD_THREADS) {
-            MInputs in;
-            load_inputs<true>(a, s, in);
-            if (skipSoft && in.soft) continue;
-            const int l0 = in.b0 - d0, l1 = in.b1 - d0;
-            f3 v0 = s3(0.f), w0 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-            if (in.b0 >= 0) { v0 = xyz(wv[l0]); w0 = xyz(wv[n + l0]); }
-            if (in.b1 >= 0) { v1 = xyz(wv[l1]); w1 = xyz(wv[n + l1]); }
-            solve_core(a, s, in, useBias != 0, h, v0, w0, v1, w1);
-            if (in.b0 >= 0) { wv[l0] = f4(v0, 0.f); wv[n + l0] = f4(w0, 0.f); }
-            if (in.b1 >= 0) { wv[l1] = f4(v1, 0.f); wv[n + l1] = f4(w1, 0.f); }
+        const int S = 2 * p.wcS[c * p.W + wd], E = 2 * p.wcE[c * p.W + wd];
+        for (int i = S + (int)threadIdx.x; i < E; i += WORLD_THREADS) {
+            SideIn in;
+            load_side<true>(a, i, pass, in);
+            if ((pass & PASS_SKIP_SOFT) && in.soft) continue;
+            const int l = in.b - d0;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            f3 w = s3(0.f);
+            if (in.b >= 0) { v = wv[l]; w = xyz(wv[n + l]); }
+            solve_side(a, i, in, pass, v, w);
+            if (in.b >= 0) { wv[l] = v; wv[n + l] = f4(w, 0.f); }
         }
         __syncthreads();
     }
@@ -1147,16 +1141,15 @@ __device__ __forceinline__ int colours_below(const uint64_t* used, int b, int c)
 // microseconds between XCDs.
 //
 // The solve order is the colour order's, so the arithmetic is exactly that of one launch
-// per colour. Waves take 64 manifolds at a time, in solve order, from the pass's ticket: a
+// per colour. Waves take 32 manifolds at a time, in solve order, from the pass's ticket: a
 // manifold waits only on manifolds of lower solve positions held by waves already running,
 // so the waits resolve in order. Every wait is bounded; one that runs out sets flowErr and
 // gives up (the host reports the error) rather than hang.
 constexpr int FLOW_SPIN_LIMIT = 1 << 18;   // ~0.5 s of polling: a wait this long is a bug
 
 struct FlowArgs {
-    int pass;
-    int useBias, skipSoft;
-    float h;
+    int index;                             // the pass within its substep
+    int pass;                              // PASS_* flags
     uint32_t epoch;                        // unique per launch (24 bits used)
     uint64_t* pub;                         // 6 words per body
     int xcdScope;                          // 1: a queue per XCD, 0: one queue
@@ -1186,10 +1179,10 @@ __device__ __forceinline__ bool read_pub(const FlowArgs& f, int b, uint32_t ver,
 // Hands body b's velocities on after one of its manifolds: to the next manifold of the
 // pass (published under version ver), or, after its last manifold of the pass, to the
 // kernels after the pass (the plain solver velocities, written back at the launch's end).
-__device__ __forceinline__ void hand_on(const SubArgs& a, const FlowArgs& f, int b, bool last, uint32_t ver, f3 v,
+__device__ __forceinline__ void hand_on(const SubArgs& a, const FlowArgs& f, int b, bool last, uint32_t ver, float4 v,
                                         f3 w) {
     if (last) {
-        a.bvel[bv(b, BV_V)] = f4(v, 0.f);
+        a.bvel[bv(b, BV_V)] = v;
         a.bvel[bv(b, BV_W)] = f4(w, 0.f);
         return;
     }
@@ -1211,51 +1204,48 @@ __global__ __launch_bounds__(256) void k_solve_flow(SubArgs a, FlowArgs f) {
     }
     const int qb = f.qStart[queue], qn = f.qStart[queue + 1] - qb;
     const uint32_t vbase = (f.epoch & 0xffffffu) << 8;
-    const bool useBias = f.useBias != 0, skipSoft = f.skipSoft != 0;
     int done = 0;
     for (;;) {
         int base = 0;
-        if (lane == 0) base = atomicAdd(a.tickets + f.pass * FLOW_QUEUES + queue, WAVE);
+        if (lane == 0) base = atomicAdd(a.tickets + f.index * FLOW_QUEUES + queue, WAVE / 2);
         base = __shfl(base, 0);
         if (base >= qn) break;
-        const int idx = base + lane;
-        bool pending = idx < qn;
-        const int s = pending ? (f.qList ? f.qList[qb + idx] : qb + idx) : 0;
-        MInputs in;
-        int r0 = 0, r1 = 0;
-        bool last0 = false, last1 = false;
-        f3 v0 = s3(0.f), w0 = s3(0.f), v1 = s3(0.f), w1 = s3(0.f);
-        bool have0 = true, have1 = true;
+        const int idx = base + (lane >> 1);
+        bool pending = idx < qn;           // the same in both lanes of a pair
+        const int i = 2 * (pending ? (f.qList ? f.qList[qb + idx] : qb + idx) : 0) + (lane & 1);
+        SideIn in;
+        int r = 0;
+        bool last = false, have = true;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        f3 w = s3(0.f);
         if (pending) {
             // everything but the bodies' solver velocities is fixed for the pass: loaded
             // before the wait, off the critical path
-            load_inputs(a, s, in);
-            const int c = a.sFlags[s] >> 16;
-            if (in.b0 >= 0) {
-                r0 = colours_below(a.used, in.b0, c);
-                last0 = r0 == colours_of(a.used, in.b0) - 1;
-                have0 = r0 == 0;
-                if (have0) { v0 = xyz(a.bvel[bv(in.b0, BV_V)]); w0 = xyz(a.bvel[bv(in.b0, BV_W)]); }
-            }
-            if (in.b1 >= 0) {
-                r1 = colours_below(a.used, in.b1, c);
-                last1 = r1 == colours_of(a.used, in.b1) - 1;
-                have1 = r1 == 0;
-                if (have1) { v1 = xyz(a.bvel[bv(in.b1, BV_V)]); w1 = xyz(a.bvel[bv(in.b1, BV_W)]); }
+            load_side(a, i, f.pass, in);
+            const int c = a.sFlags[i >> 1] >> 16;
+            if (in.b >= 0) {
+                r = colours_below(a.used, in.b, c);
+                last = r == colours_of(a.used, in.b) - 1;
+                have = r == 0;
+                v = a.bvel[bv(in.b, BV_V)];   // the velocities only when have; the inverse mass always
+                w = xyz(a.bvel[bv(in.b, BV_W)]);
             }
         }
         int spins = 0;
         while (__ballot(pending)) {
             if (pending) {
-                if (!have0) have0 = read_pub(f, in.b0, vbase | (uint32_t)r0, v0, w0);
-                if (!have1) have1 = read_pub(f, in.b1, vbase | (uint32_t)r1, v1, w1);
-                if (have0 && have1) {
+                if (!have) {
+                    f3 pv;
+                    have = read_pub(f, in.b, vbase | (uint32_t)r, pv, w);
+                    v = f4(pv, v.w);
+                }
+                const bool both = __builtin_amdgcn_mov_dpp((int)have, 0xB1, 0xf, 0xf, true) != 0 && have;   // quad_perm 1,0,3,2
+                if (both) {
                     // a soft manifold in the relaxation passes its bodies' velocities on
-                    if (!(skipSoft && in.soft)) solve_core(a, s, in, useBias, f.h, v0, w0, v1, w1);
-                    if (in.b0 >= 0) hand_on(a, f, in.b0, last0, vbase | (uint32_t)(r0 + 1), v0, w0);
-                    if (in.b1 >= 0) hand_on(a, f, in.b1, last1, vbase | (uint32_t)(r1 + 1), v1, w1);
+                    if (!((f.pass & PASS_SKIP_SOFT) && in.soft)) solve_side(a, i, in, f.pass, v, w);
+                    if (in.b >= 0) hand_on(a, f, in.b, last, vbase | (uint32_t)(r + 1), v, w);
                     pending = false;
-                    ++done;
+                    done += lane & 1;
                 } else if (++spins > FLOW_SPIN_LIMIT) {
                     atomicOr(a.flowErr, 1);
                     pending = false;
@@ -1299,9 +1289,9 @@ __global__ __launch_bounds__(256) void k_integrate_positions(SubArgs a) {
     int d = blockIdx.x * blockDim.x + threadIdx.x;
     if (d < a.D) integrate_position(a, d);
 }
-__global__ __launch_bounds__(256) void k_writeback(SubArgs a) {
+__global__ __launch_bounds__(256) void k_writeback(SubArgs a, int next) {
     int d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d < a.D) write_back(a, d);
+    if (d < a.D) write_back(a, d, next != 0);
 }
 
 // ------------------------------------------------------------------ persistent kernel
@@ -1312,27 +1302,27 @@ __global__ __launch_bounds__(256) void k_step_persistent(SubArgs a) {
     cg::grid_group grid = cg::this_grid();
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int nth = gridDim.x * blockDim.x;
+    for (int d = tid; d < a.D; d += nth) integrate_velocity(a, d, a.dvel[d], xyz(a.dang[d]));
+    grid.sync();
     for (int sub = 0; sub < a.substeps; ++sub) {
-        for (int i = tid; i < a.M + a.D; i += nth) {
-            if (i < a.M) prepare_manifold(a, i);
-            else integrate_velocity(a, i - a.M);
-        }
+        for (int i = tid; i < 2 * a.M; i += nth) prepare_side(a, i);
         grid.sync();
         for (int it = 0; it < a.iterations; ++it) {
             for (int c = 0; c < a.nColors; ++c) {
-                int b = a.colorStart[c], e = a.colorStart[c + 1];
-                for (int s = b + tid; s < e; s += nth) solve_manifold(a, s, true, a.h, false);
+                const int b = 2 * a.colorStart[c], e = 2 * a.colorStart[c + 1];
+                for (int i = b + tid; i < e; i += nth) solve_lane(a, i, PASS_BIAS | (it == 0 ? PASS_FIRST : 0));
                 grid.sync();
             }
         }
         for (int d = tid; d < a.D; d += nth) integrate_position(a, d);
         grid.sync();
         for (int c = 0; c < a.nColors; ++c) {
-            int b = a.colorStart[c], e = a.colorStart[c + 1];
-            for (int s = b + tid; s < e; s += nth) solve_manifold(a, s, false, 0.f, true);
+            const int b = 2 * a.colorStart[c], e = 2 * a.colorStart[c + 1];
+            for (int i = b + tid; i < e; i += nth)
+                solve_lane(a, i, PASS_SKIP_SOFT | PASS_LAST | (a.iterations == 0 ? PASS_FIRST : 0));
             grid.sync();
         }
-        for (int d = tid; d < a.D; d += nth) write_back(a, d);
+        for (int d = tid; d < a.D; d += nth) write_back(a, d, sub + 1 < a.substeps);
         grid.sync();
     }
 }
@@ -1477,8 +1467,7 @@ int sv_color(World& w, int M) {
                        w.dang.p, w.dcom.p, w.D, w.mfPrev.p, w.cacheNum[prv].p, w.cacheLp[prv].p, w.manifoldCap,
                        w.cacheKey[cur].p, w.cacheTri[cur].p,
                        w.cacheNum[cur].p, w.cacheLp[cur].p,
-                       w.sB0.p, w.sB1.p, w.sA0.p, w.sA1.p, w.sFlags.p, w.sCanon.p, w.sN.p, w.sSoft.p, w.sR0.p,
-                       w.sR1.p, w.sWorld.p);
+                       w.sB.p, w.sA.p, w.sFlags.p, w.sCanon.p, w.sN.p, w.sSoft.p, w.sR.p, w.sWorld.p);
     PGX_LAUNCH_CHECK();
     return nColors;
 }
@@ -1489,11 +1478,11 @@ static SubArgs make_args(World& w, int M, float dt) {
     a.nColors = (int)w.colorStartHost.size() - 1;
     a.substeps = w.substeps; a.iterations = w.iterations;
     a.h = dt / w.substeps; a.g = w.g;
-    a.sB0 = w.sB0.p; a.sB1 = w.sB1.p; a.sA0 = w.sA0.p; a.sA1 = w.sA1.p; a.sFlags = w.sFlags.p;
+    a.sB = (const int32_t*)w.sB.p; a.sA = (const int32_t*)w.sA.p; a.sFlags = w.sFlags.p;
     a.colorStart = w.colorCount.p;
-    a.sN = w.sN.p; a.sR0 = w.sR0.p; a.sR1 = w.sR1.p; a.sSoft = w.sSoft.p; a.sRow = w.sRow.p; a.sLam = w.sLam.p;
+    a.sN = w.sN.p; a.sR = w.sR.p; a.sSoft = w.sSoft.p; a.sRow = w.sRow.p; a.sLam = w.sLam.p; a.sMode = w.sMode.p;
     a.bpos = w.bpos.p; a.bquat = w.bquat.p; a.dvel = w.dvel.p; a.dang = w.dang.p;
-    a.bvel = w.bvel.p; a.dcom = w.dcom.p; a.dinvI = w.dinvI.p;
+    a.bvel = w.bvel.p; a.brec = w.brec.p; a.dcom = w.dcom.p; a.dinvI = w.dinvI.p;
     a.pvel = w.pvel.p; a.pang = w.pang.p;
     a.used = w.usedMask.p; a.tickets = w.tickets.p; a.flowErr = w.flowErr.p; a.qDone = w.qDone.p;
     a.barrier = w.passBarrier.p;
@@ -1523,7 +1512,8 @@ static int pass_blocks(World& w, int maxColour) {
         PGX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, w.device));
         w.passBlocksMax = std::max(1, std::min(cus, perCU * cus));
     }
-    const int want = w.persistentBlocksWanted > 0 ? w.persistentBlocksWanted : div_up(std::max(maxColour, 1), PASS_THREADS);
+    const int want = w.persistentBlocksWanted > 0 ? w.persistentBlocksWanted
+                                                  : div_up(2 * std::max(maxColour, 1), PASS_THREADS);
     return std::max(1, std::min(want, w.passBlocksMax));
 }
 
@@ -1538,7 +1528,7 @@ static int xpass_blocks(World& w, int maxColour) {
         w.xpassBlocksMax = std::max(8, std::min(XPASS_MAX_GRID, perCU * cus));
     }
     const int perXcd = w.persistentBlocksWanted > 0 ? div_up(w.persistentBlocksWanted, 8)
-                                                    : div_up(std::max(maxColour, 1), XPASS_THREADS);
+                                                    : div_up(2 * std::max(maxColour, 1), XPASS_THREADS);
     return std::max(8, std::min(8 * perXcd, w.xpassBlocksMax));
 }
 
@@ -1574,7 +1564,7 @@ bool sv_world_pass_fits(World& w) {
 
 // one colour [b, e) in workgroups of `block` threads; with events, stamped from the
 // launch's own dispatch packet
-// Workgroups of a colour launch over slots [b, e) in chunks of bs homed on their XCD
+// Workgroups of a colour launch over side lanes [b, e) in chunks of bs homed on their XCD
 // (homed_chunk): 8 per round, as many rounds as the XCD with the most chunks needs.
 static int homed_blocks(int b, int e, int bs) {
     const int q = 256 / bs, period = 8 * q, k0 = b / bs, k1 = (e - 1) / bs + 1;   // chunks [k0, k1)
@@ -1588,11 +1578,11 @@ static int homed_blocks(int b, int e, int bs) {
 }
 
 static void launch_solve(int block, bool eager, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const SubArgs& a, int b,
-                         int e, int useBias, float h, int skipSoft) {
+                         int e, int pass) {
     auto go = [&](auto kernel, int bs) {
-        const int nb = homed_blocks(b, e, bs);
-        if (e0) hipExtLaunchKernelGGL(kernel, dim3(nb), dim3(bs), 0, s, e0, e1, 0, a, b, e, useBias, h, skipSoft);
-        else hipLaunchKernelGGL(kernel, dim3(nb), dim3(bs), 0, s, a, b, e, useBias, h, skipSoft);
+        const int nb = homed_blocks(2 * b, 2 * e, bs);
+        if (e0) hipExtLaunchKernelGGL(kernel, dim3(nb), dim3(bs), 0, s, e0, e1, 0, a, 2 * b, 2 * e, pass);
+        else hipLaunchKernelGGL(kernel, dim3(nb), dim3(bs), 0, s, a, 2 * b, 2 * e, pass);
     };
     if (eager) {
         if (block == 256) go(k_solve<256, true>, 256);
@@ -1615,7 +1605,7 @@ void sv_presize(World& w) {
         w.batchN.alloc(BATCH_MAX_GROUPS);
         if (!w.batchLdsSet) {
             PGX_HIP(hipFuncSetAttribute((const void*)k_solve_batch, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)(2 * BATCH_BODY_F4 * sizeof(float4) * BATCH_MAX_MANIFOLDS)));
+                                        (int)(4 * sizeof(float4) * BATCH_MAX_MANIFOLDS)));
             w.batchLdsSet = true;
         }
     }
@@ -1634,7 +1624,7 @@ void sv_substeps(World& w, int M, float dt) {
         if (w.timing) PGX_HIP(hipEventRecord(w.ev[7], s));
         return;
     }
-    int nbP = div_up(std::max(M + w.D, 1), 256), nbD = div_up(std::max(w.D, 1), 256);
+    int nbP = div_up(2 * (long)std::max(M, 1), 256), nbD = div_up(std::max(w.D, 1), 256);
     int nColors = a.nColors;
     const bool flow = w.execMode == EXEC_FLOW || w.execMode == EXEC_FLOW_XCD;
     FlowArgs f{};
@@ -1680,7 +1670,7 @@ void sv_substeps(World& w, int M, float dt) {
     w.lastFlowPasses = flow && M > 0 ? w.substeps * (w.iterations + 1) : 0;
     // waves of the dependency-driven pass: enough to hold every manifold at once, at most
     // what the chip keeps resident comfortably; on XCD queues, 64 workgroups per XCD
-    const int flowBlocks = f.xcdScope ? 64 * w.nXcd : std::max(1, std::min(div_up(std::max(M, 1), 256), 2048));
+    const int flowBlocks = f.xcdScope ? 64 * w.nXcd : std::max(1, std::min(div_up(2 * (long)std::max(M, 1), 256), 2048));
     // launch groups of the colour passes: (first colour, end colour, batched run index + 1);
     // a run holds consecutive colours of at most colorBatch manifolds each, at most
     // BATCH_MAX_MANIFOLDS in all (its bodies' velocities fit in LDS), two colours or more
@@ -1706,7 +1696,7 @@ void sv_substeps(World& w, int M, float dt) {
     }
     if (bg.n > 0) {   // the runs' body slots, fixed for the step
         sv_presize(w);
-        hipLaunchKernelGGL(k_batch_map, dim3(1), dim3(BATCH_MAP_THREADS), 0, s, bg, w.sB0.p, w.sB1.p, w.batchLoc.p,
+        hipLaunchKernelGGL(k_batch_map, dim3(1), dim3(BATCH_MAP_THREADS), 0, s, bg, a.sB, w.batchLoc.p,
                            w.batchList.p, w.batchN.p);
         PGX_LAUNCH_CHECK();
     }
@@ -1719,13 +1709,14 @@ void sv_substeps(World& w, int M, float dt) {
         for (int c = 0; c < nColors; ++c) maxColour = std::max(maxColour, w.colorStartHost[c + 1] - w.colorStartHost[c]);
         passGrid = onePass ? pass_blocks(w, maxColour) : xpass_blocks(w, maxColour);
     }
-    auto pass = [&](bool rec, int useBias, float h, int skipSoft) {
+    auto pass = [&](bool rec, int flags) {
         const int p = passIndex++;
+        if (p == 0) flags |= PASS_FIRST;
         if (M == 0) return;
         if (xcdPass) {
             int nc = nColors;
             int32_t* ctl = w.xpassCtl.p + XPASS_CTL * p;
-            void* args[] = {&a, &nc, &useBias, &h, &skipSoft, &ctl};
+            void* args[] = {&a, &nc, &flags, &ctl};
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (rec) {
                 solve_events(w, -1, &e0, &e1);
@@ -1741,7 +1732,7 @@ void sv_substeps(World& w, int M, float dt) {
             // once per workgroup; the count is cleared by k_prepare
             int base = p * (nColors - 1) * passGrid;
             int nc = nColors;
-            void* args[] = {&a, &nc, &useBias, &h, &skipSoft, &base};
+            void* args[] = {&a, &nc, &flags, &base};
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (rec) {
                 solve_events(w, -1, &e0, &e1);
@@ -1753,7 +1744,7 @@ void sv_substeps(World& w, int M, float dt) {
             return;
         }
         if (flow) {
-            f.pass = p; f.useBias = useBias; f.skipSoft = skipSoft; f.h = h;
+            f.index = p; f.pass = flags;
             f.epoch = ++w.flowEpoch;
             if (rec) {
                 hipEvent_t e0, e1;
@@ -1776,10 +1767,9 @@ void sv_substeps(World& w, int M, float dt) {
                 const bool first = k == 0 || w.worldListHost[0].empty(), last = k == 1 || w.worldListHost[1].empty();
                 if (rec && (first || last))
                     hipExtLaunchKernelGGL(k_world_pass, dim3(nw), dim3(WORLD_THREADS), worldLds[k], s,
-                                          first ? e0 : nullptr, last ? e1 : nullptr, 0, a, q, useBias, h, skipSoft);
+                                          first ? e0 : nullptr, last ? e1 : nullptr, 0, a, q, flags);
                 else
-                    hipLaunchKernelGGL(k_world_pass, dim3(nw), dim3(WORLD_THREADS), worldLds[k], s, a, q, useBias, h,
-                                       skipSoft);
+                    hipLaunchKernelGGL(k_world_pass, dim3(nw), dim3(WORLD_THREADS), worldLds[k], s, a, q, flags);
             }
             return;
         }
@@ -1789,40 +1779,42 @@ void sv_substeps(World& w, int M, float dt) {
             if (g.z) {
                 const int q = g.z - 1;
                 // 2 bodies per manifold at most
-                const size_t lds = 2 * BATCH_BODY_F4 * sizeof(float4) * (size_t)(bg.E[q] - bg.S[q]);
+                const size_t lds = 4 * sizeof(float4) * (size_t)(bg.E[q] - bg.S[q]);
                 if (rec) {   // a run of colours [g.x, g.y), stamped from its dispatch packet
                     hipEvent_t e0, e1;
                     solve_events(w, g.x, &e0, &e1, g.y);
                     hipExtLaunchKernelGGL(k_solve_batch, dim3(1), dim3(BATCH_THREADS), lds, s, e0, e1, 0, a, g.x, g.y,
-                                          bg.S[q], w.batchLoc.p, w.batchList.p, w.batchN.p + q, useBias, h, skipSoft);
+                                          bg.S[q], w.batchLoc.p, w.batchList.p, w.batchN.p + q, flags);
                 } else {
                     hipLaunchKernelGGL(k_solve_batch, dim3(1), dim3(BATCH_THREADS), lds, s, a, g.x, g.y, bg.S[q],
-                                       w.batchLoc.p, w.batchList.p, w.batchN.p + q, useBias, h, skipSoft);
+                                       w.batchLoc.p, w.batchList.p, w.batchN.p + q, flags);
                 }
                 continue;
             }
             const int c = g.x, b = w.colorStartHost[c], e = w.colorStartHost[c + 1];
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (rec) solve_events(w, c, &e0, &e1);
-            launch_solve(w.tune.solveBlock, e - b <= w.tune.eagerMax, s, e0, e1, a, b, e, useBias, h, skipSoft);
+            launch_solve(w.tune.solveBlock, e - b <= w.tune.eagerMax, s, e0, e1, a, b, e, flags);
         }
     };
     jt_step_setup(w);
+    hipLaunchKernelGGL(k_integrate_velocities, dim3(nbD), dim3(256), 0, s, a);
     for (int sub = 0; sub < w.substeps; ++sub) {
         const bool rec = w.timing && sub == 0;
         passIndex = 0;
-        // rows + preSolve of the contacts, velocity integration; then the joint rows, whose
+        // rows + preSolve of the contacts (the velocities were integrated before the first
+        // substep and by the write-back before each other one); then the joint rows, whose
         // preSolve follows the contacts' (src/Physecs.cpp:430-479)
-        hipLaunchKernelGGL(k_prepare, dim3(nbP), dim3(256), 0, s, a, sub);
+        if (M > 0) hipLaunchKernelGGL(k_prepare, dim3(nbP), dim3(256), 0, s, a, sub);
         jt_update(w, a.h);
         jt_colors(w, a.h, 0, false);
         for (int it = 0; it < w.iterations; ++it) {
-            pass(rec, 1, a.h, 0);
+            pass(rec, PASS_BIAS);
             jt_colors(w, a.h, 1, it == 0);   // joint colours after the contacts (Physecs.cpp:482-490)
         }
         hipLaunchKernelGGL(k_integrate_positions, dim3(nbD), dim3(256), 0, s, a);
-        pass(rec, 0, 0.f, 1);
-        hipLaunchKernelGGL(k_writeback, dim3(nbD), dim3(256), 0, s, a);
+        pass(rec, PASS_SKIP_SOFT | PASS_LAST);
+        hipLaunchKernelGGL(k_writeback, dim3(nbD), dim3(256), 0, s, a, sub + 1 < w.substeps ? 1 : 0);
         PGX_LAUNCH_CHECK();
     }
 }

@@ -305,7 +305,7 @@ void world_set_dyn_ranges(World& w, const std::vector<int32_t>& dynWorld) {
 void world_alloc_derived(World& w, const pgx_config* cfg, int nTrimesh) {
     const int D = w.D, C = w.C, W = w.W;
     w.refitReady.alloc(std::max(1, w.nDynCol));
-    w.bvel.alloc(BV_WORDS * (size_t)D); w.pvel.alloc(D); w.pang.alloc(D); w.winvI.alloc(3 * (size_t)D);
+    w.bvel.alloc(BV_WORDS * (size_t)D); w.brec.alloc(BR_WORDS * (size_t)D); w.pvel.alloc(D); w.pang.alloc(D); w.winvI.alloc(3 * (size_t)D);
     w.cbmin.alloc(C); w.cbmax.alloc(C);
     // broadphase buffers
     w.worldBoundsI.alloc(16);
@@ -355,8 +355,8 @@ void world_alloc_derived(World& w, const pgx_config* cfg, int nTrimesh) {
     }
 
     w.colorKeys.alloc(M); w.colorPerm.alloc(M); w.colorRank.alloc(M); w.colorCount.alloc(160); w.colorPoints.alloc(160);
-    w.sB0.alloc(M); w.sB1.alloc(M); w.sFlags.alloc(M); w.sA0.alloc(M); w.sA1.alloc(M); w.sCanon.alloc(M);
-    w.sN.alloc(M); w.sSoft.alloc(M); w.sR0.alloc(4 * M); w.sR1.alloc(4 * M); w.sRow.alloc(4 * CONTACT_ROW_FIELDS * M); w.sLam.alloc(4 * M);
+    w.sB.alloc(M); w.sA.alloc(M); w.sFlags.alloc(M); w.sMode.alloc(M); w.sCanon.alloc(M);
+    w.sN.alloc(M); w.sSoft.alloc(M); w.sR.alloc(8 * M); w.sRow.alloc(4 * CONTACT_ROW_FIELDS * M); w.sLam.alloc(4 * M);
     for (int k = 0; k < 2; ++k) {
         w.cacheKey[k].alloc(M); w.cacheTri[k].alloc(M); w.cacheNum[k].alloc(M); w.cacheLp[k].alloc(4 * M);
     }
@@ -504,22 +504,22 @@ int pgx_world_create(const pgx_config* cfg, const pgx_scene_desc* sc, pgx_world*
 static void release_world(World& w) {
     DBuf<float4>* f4s[] = {&w.bpos, &w.bquat, &w.dvel, &w.dang, &w.dcom, &w.dinvI, &w.bvel, &w.pvel,
                            &w.pang, &w.winvI, &w.cparams, &w.clpos, &w.clquat, &w.cmat, &w.cbmin, &w.cbmax,
-                           &w.leafMin, &w.leafMax, &w.nodeMin, &w.nodeMax, &w.npNormal, &w.npPts, &w.sN, &w.sR0,
-                           &w.sR1, &w.sRow, &w.sLam, &w.cacheLp[0], &w.cacheLp[1]};
+                           &w.leafMin, &w.leafMax, &w.nodeMin, &w.nodeMax, &w.npNormal, &w.npPts, &w.sN, &w.sR,
+                           &w.sRow, &w.brec, &w.cacheLp[0], &w.cacheLp[1]};
     for (auto* b : f4s) b->release();
     DBuf<int32_t>* i32s[] = {&w.cbody, &w.cworld, &w.clocal, &w.cflags, &w.ctype, &w.cindex, &w.worldColStart,
                              &w.colOfLocal, &w.mvals, &w.leafFlags, &w.leafParent, &w.leafEsc, &w.nodeChild,
                              &w.nodeParent, &w.nodeEsc, &w.nodeFlags, &w.nodeCounter, &w.worldRoot, &w.worldStop,
                              &w.pvals, &w.counters, &w.npNum, &w.npIndex, &w.mfPair, &w.mfB0, &w.mfB1, &w.mfColor,
-                             &w.colorPerm, &w.colorRank, &w.colorCount, &w.worldMStart, &w.sB0, &w.sB1, &w.sFlags, &w.sA0,
-                             &w.sA1, &w.sCanon, &w.cacheNum[0], &w.cacheNum[1], &w.sortT.valt, &w.scanT.sums,
+                             &w.colorPerm, &w.colorRank, &w.colorCount, &w.worldMStart, &w.sFlags, &w.sMode,
+                             &w.sCanon, &w.cacheNum[0], &w.cacheNum[1], &w.sortT.valt, &w.scanT.sums,
                              &w.dynCols, &w.staticCols, &w.worldStaticStart, &w.refitReady};
     for (auto* b : i32s) b->release();
     DBuf<uint64_t>* u64s[] = {&w.mkeys, &w.pkeys, &w.mfKey, &w.claim, &w.usedMask, &w.colorKeys, &w.cacheKey[0],
                               &w.cacheKey[1], &w.nonColliding, &w.sortT.kalt};
     for (auto* b : u64s) b->release();
     w.bentity.release(); w.centity.release(); w.worldBoundsI.release(); w.sortT.hist.release(); w.sortT.scan.sums.release();
-    w.nodeRange.release(); w.sSoft.release();
+    w.nodeRange.release(); w.sSoft.release(); w.sLam.release(); w.sB.release(); w.sA.release();
     DBuf<int32_t>* ji[] = {&w.jType, &w.jA0, &w.jA1, &w.jB0, &w.jB1, &w.jRowFlags, &w.jNRows, &w.jOrder};
     for (auto* b : ji) b->release();
     DBuf<float4>* jf[] = {&w.jP0, &w.jQ0, &w.jP1, &w.jQ1, &w.jDrive, &w.jR0, &w.jR1, &w.jRow};
@@ -1646,20 +1646,19 @@ int pgx_world_get_manifolds(pgx_world* h, int32_t* keys, int32_t* ints, float* f
         *n = M;
         if (M == 0) return PGX_OK;
         size_t Mc = w.manifoldCap;
-        std::vector<int32_t> canon(M), b0(M), b1(M), flags(M), mfPair(M), mfSrc(M), mfTri(M);
+        std::vector<int32_t> canon(M), flags(M), mfPair(M), mfSrc(M), mfTri(M);
         std::vector<uint64_t> mkey(M);
-        std::vector<float4> sn(M), r0(4 * Mc), r1(4 * Mc);
+        std::vector<int2> sb(M);
+        std::vector<float4> sn(M), rr(8 * Mc);
         PGX_HIP(hipMemcpy(canon.data(), w.sCanon.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
-        PGX_HIP(hipMemcpy(b0.data(), w.sB0.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
-        PGX_HIP(hipMemcpy(b1.data(), w.sB1.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
+        PGX_HIP(hipMemcpy(sb.data(), w.sB.p, sizeof(int2) * M, hipMemcpyDeviceToHost));
         PGX_HIP(hipMemcpy(flags.data(), w.sFlags.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
         PGX_HIP(hipMemcpy(mfPair.data(), w.mfPair.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
         PGX_HIP(hipMemcpy(mfSrc.data(), w.mfSrc.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
         PGX_HIP(hipMemcpy(mfTri.data(), w.mfTri.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost));
         PGX_HIP(hipMemcpy(mkey.data(), w.mfKey.p, sizeof(uint64_t) * M, hipMemcpyDeviceToHost));
         PGX_HIP(hipMemcpy(sn.data(), w.sN.p, sizeof(float4) * M, hipMemcpyDeviceToHost));
-        PGX_HIP(hipMemcpy(r0.data(), w.sR0.p, sizeof(float4) * 4 * Mc, hipMemcpyDeviceToHost));
-        PGX_HIP(hipMemcpy(r1.data(), w.sR1.p, sizeof(float4) * 4 * Mc, hipMemcpyDeviceToHost));
+        PGX_HIP(hipMemcpy(rr.data(), w.sR.p, sizeof(float4) * 8 * Mc, hipMemcpyDeviceToHost));
         // narrowphase points: the pair slots, then the triangle-mesh manifold slots
         std::vector<float4> pts(8 * ((size_t)w.lastPairs + w.lastMeshSlots));
         if (w.lastPairs)
@@ -1686,7 +1685,7 @@ int pgx_world_get_manifolds(pgx_world* h, int32_t* keys, int32_t* ints, float* f
                 keys[5 * s + 4] = mfTri[m];
             }
             if (ints) {
-                ints[4 * s] = b0[s]; ints[4 * s + 1] = b1[s]; ints[4 * s + 2] = num; ints[4 * s + 3] = flags[s] >> 16;
+                ints[4 * s] = sb[s].x; ints[4 * s + 1] = sb[s].y; ints[4 * s + 2] = num; ints[4 * s + 3] = flags[s] >> 16;
             }
             if (floats) {
                 float* o = floats + 56 * (size_t)s;
@@ -1697,7 +1696,7 @@ int pgx_world_get_manifolds(pgx_world* h, int32_t* keys, int32_t* ints, float* f
                     float4 a = pts[8 * (size_t)p + 2 * k2], b = pts[8 * (size_t)p + 2 * k2 + 1];
                     float* q = o + 4 + 6 * k2;
                     q[0] = a.x; q[1] = a.y; q[2] = a.z; q[3] = b.x; q[4] = b.y; q[5] = b.z;
-                    float4 ra = r0[(size_t)k2 * Mc + s], rb = r1[(size_t)k2 * Mc + s];
+                    float4 ra = rr[2 * ((size_t)k2 * Mc + s)], rb = rr[2 * ((size_t)k2 * Mc + s) + 1];
                     float* t = o + 28 + 7 * k2;
                     t[0] = ra.x; t[1] = ra.y; t[2] = ra.z; t[3] = rb.x; t[4] = rb.y; t[5] = rb.z; t[6] = ra.w;
                 }
