@@ -648,6 +648,7 @@ __device__ bool collide(int t0, float4 g0, f3 p0, qf q0, int t1, float4 g1, f3 p
 
 #include "np_convex.h"
 #include "np_trimesh.h"
+#include "np_wave.h"
 
 namespace pgx {
 
@@ -770,45 +771,42 @@ __global__ __launch_bounds__(256) void k_narrowphase(
     }
 }
 
-// Pairs with a convex mesh: a fixed grid of `lanes` threads walks the list; lane l owns
-// EPA workspace l. The list length is read on the device, so no host round trip.
+// Pairs with a convex mesh, a wave per pair (np_wave.h): a fixed grid of CONVEX_WAVES waves,
+// what the chip holds of their 14 KB of LDS each, walks the list. The list length is read on
+// the device, so no host round trip.
+constexpr int CONVEX_WAVES = 2816;
 __global__ __launch_bounds__(64) void k_narrowphase_convex(
     const int32_t* __restrict__ nHeavyP, const int32_t* __restrict__ heavy, const uint64_t* __restrict__ pkeys,
     int localBits, const int32_t* __restrict__ worldColStart, const int32_t* __restrict__ colOfLocal,
     const int32_t* __restrict__ cbody, const int32_t* __restrict__ ctype, const float4* __restrict__ cparams,
     const float4* __restrict__ clpos, const float4* __restrict__ clquat, const float4* __restrict__ bpos,
-    const float4* __restrict__ bquat, ConvexView cv, double* epaV, double* epaFN, int32_t* epaFI, int32_t* epaE,
-    int lanes, int32_t* __restrict__ npNum, float4* __restrict__ npNormal, float4* __restrict__ npPts,
-    int32_t* __restrict__ errors) {
-    int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    if (lane >= lanes) return;
-    int nHeavy = *nHeavyP;
-    EpaWs ws;
-    ws.vd = epaV + lane; ws.fn = epaFN + lane; ws.fi = epaFI + lane; ws.ed = epaE + lane;
-    ws.L = (size_t)lanes;
-    ws.overflow = false;
-    uint64_t lmask = (1ull << localBits) - 1;
-    for (int h = lane; h < nHeavy; h += lanes) {
-        int p = heavy[h];
-        uint64_t key = pkeys[p];
-        int wd = (int)(key >> (2 * localBits));
-        int base = worldColStart[wd];
-        int c0 = colOfLocal[base + (int)((key >> localBits) & lmask)];
-        int c1 = colOfLocal[base + (int)(key & lmask)];
-        int b0 = cbody[c0], b1 = cbody[c1];
-        qf bq0 = q4(bquat[b0]), bq1 = q4(bquat[b1]);
-        f3 p0 = add(xyz(bpos[b0]), qrot(bq0, xyz(clpos[c0])));
-        qf q0 = qmul(bq0, q4(clquat[c0]));
-        f3 p1 = add(xyz(bpos[b1]), qrot(bq1, xyz(clpos[c1])));
-        qf q1 = qmul(bq1, q4(clquat[c1]));
+    const float4* __restrict__ bquat, ConvexView cv, int32_t* __restrict__ npNum, float4* __restrict__ npNormal,
+    float4* __restrict__ npPts, int32_t* __restrict__ errors) {
+    __shared__ WaveMem M;
+    const int nHeavy = *nHeavyP;
+    const uint64_t lmask = (1ull << localBits) - 1;
+    for (int h = blockIdx.x; h < nHeavy; h += gridDim.x) {
+        const int p = heavy[h];
+        const uint64_t key = pkeys[p];
+        const int base = worldColStart[(int)(key >> (2 * localBits))];
+        const int c0 = colOfLocal[base + (int)((key >> localBits) & lmask)];
+        const int c1 = colOfLocal[base + (int)(key & lmask)];
+        const int b0 = cbody[c0], b1 = cbody[c1];
+        const qf bq0 = q4(bquat[b0]), bq1 = q4(bquat[b1]);
+        const f3 p0 = add(xyz(bpos[b0]), qrot(bq0, xyz(clpos[c0])));
+        const qf q0 = qmul(bq0, q4(clquat[c0]));
+        const f3 p1 = add(xyz(bpos[b1]), qrot(bq1, xyz(clpos[c1])));
+        const qf q1 = qmul(bq1, q4(clquat[c1]));
         Mf m;
-        bool ovf = false;
-        bool hit = collide_convex(ctype[c0], cparams[c0], p0, q0, ctype[c1], cparams[c1], p1, q1, cv, ws, m, ovf);
+        bool ovf;
+        const bool hit = collide_convex_w(ctype[c0], cparams[c0], p0, q0, ctype[c1], cparams[c1], p1, q1, cv, M, m, ovf);
+        if (threadIdx.x != 0) continue;
         if (ovf) atomicAdd(errors, 1);
-        int num = hit ? m.numPoints : 0;
+        const int num = hit ? m.numPoints : 0;
         npNum[p] = num;
         if (num) {
             npNormal[p] = f4(m.normal, 0.f);
+#pragma unroll
             for (int k = 0; k < 4; ++k)
                 if (k < num) {
                     npPts[8 * (size_t)p + 2 * k] = f4(m.pts[k].p0, 0.f);
@@ -1192,28 +1190,52 @@ __global__ __launch_bounds__(64) void k_mesh_query(MeshArgs A, int32_t* tmWs, in
     }
 }
 
-// pass 2, one lane per (pair, candidate triangle): the per-shape test, its contact record
-__global__ __launch_bounds__(64) void k_mesh_test(MeshArgs A, double* epaV, double* epaFN, int32_t* epaFI,
-                                                  int32_t* epaE, int epaLanes, const int32_t* __restrict__ candTotal,
-                                                  int candCap, const int32_t* __restrict__ cand,
+// pass 2, the per-shape test of every (pair, candidate triangle), its contact record. A wave
+// takes a run of candidates, as few as spreads them over MESH_TEST_WAVES waves: the closed
+// forms one per lane, then the convex bodies' GJK and EPA one after another, the whole wave
+// on each (with a lane each, 125 us for 2,048 hulls on a terrain, 304 B of scratch per lane).
+constexpr int MESH_TEST_WAVES = 4096;
+__global__ __launch_bounds__(64) void k_mesh_test(MeshArgs A, const int32_t* __restrict__ candTotal, int candCap,
+                                                  const int32_t* __restrict__ cand,
                                                   const int32_t* __restrict__ pairOf, MeshRecs recs) {
-    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    if (lane >= epaLanes) return;
+    __shared__ WaveMem M;
+    const int lane = threadIdx.x;
     const int total = min(*candTotal, candCap);
-    EpaWs ews;
-    ews.vd = epaV + lane; ews.fn = epaFN + lane; ews.fi = epaFI + lane; ews.ed = epaE + lane;
-    ews.L = (size_t)epaLanes;
-    for (int k = lane; k < total; k += epaLanes) {
-        MeshPair m;
-        SupConvex sc;
-        mesh_pair(A, pairOf[k], m, sc);
-        MeshCtx mc{&A.tv, m.mi};
-        ews.overflow = false;
-        TCI ci;
-        bool epaErr = false;
-        bool hit = mesh_test(m.tb, m.g, m.lpos, m.lor, sc, mc, cand[k], ews, ci, epaErr);
-        if (epaErr) atomicAdd(A.errors, 1);
-        recs.store(k, hit, ci);
+    const int waves = gridDim.x;
+    const int run = min(WAVE, max(1, (total + waves - 1) / waves));
+    for (long first = (long)blockIdx.x * run; first < total; first += (long)waves * run) {
+        const int k = (int)first + lane;
+        const bool mine = lane < run && k < total;
+        int h = 0, ti = 0;
+        bool convex = false;
+        if (mine) {
+            MeshPair m;
+            SupConvex sc;
+            h = pairOf[k];
+            ti = cand[k];
+            mesh_pair(A, h, m, sc);
+            convex = m.tb == PGX_CONVEX_MESH;
+            if (!convex) {
+                const MeshCtx mc{&A.tv, m.mi};
+                TCI ci;
+                const bool hit = mesh_test_closed(m.tb, m.g, m.lpos, m.lor, mc, ti, ci);
+                recs.store(k, hit, ci);
+            }
+        }
+        for (uint64_t todo = __ballot(convex); todo; todo &= todo - 1) {
+            const int l = first_lane(todo), kc = (int)first + l;
+            MeshPair m;
+            SupConvex sc;
+            mesh_pair(A, __builtin_amdgcn_readlane(h, l), m, sc);
+            const MeshCtx mc{&A.tv, m.mi};
+            TCI ci;
+            bool ovf = false;
+            const bool hit = mesh_test_convex_w(sc, mc, __builtin_amdgcn_readlane(ti, l), M, ci, ovf);
+            if (lane == 0) {
+                if (ovf) atomicAdd(A.errors, 1);
+                recs.store(kc, hit, ci);
+            }
+        }
     }
 }
 
@@ -1263,7 +1285,9 @@ constexpr int MTD_MBITS = 8;   // manifold index within a pair: at most TM_MAXCA
 
 __device__ __forceinline__ float manifold_mtd(const Mf& m) {   // src/Physecs.cpp:663-670
     float mtd = 0;
-    for (int i = 0; i < m.numPoints; i++) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (i >= m.numPoints) break;
         float dist = dot(sub(m.pts[i].p0, m.pts[i].p1), m.normal);
         if (dist > mtd) mtd = dist;
     }
@@ -1362,18 +1386,11 @@ __global__ __launch_bounds__(64) void k_mtd_walk(MtdArgs A, ConvexView cv) {
     }
 }
 
-// pass 2: the pairs with a convex mesh, a fixed grid of `lanes` threads; lane l owns EPA
-// workspace l
-__global__ __launch_bounds__(64) void k_mtd_convex(MtdArgs A, ConvexView cv, double* epaV, double* epaFN,
-                                                   int32_t* epaFI, int32_t* epaE, int lanes) {
-    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    if (lane >= lanes) return;
+// pass 2: the pairs with a convex mesh, a wave per pair
+__global__ __launch_bounds__(64) void k_mtd_convex(MtdArgs A, ConvexView cv) {
+    __shared__ WaveMem M;
     const int n = min(A.counts[1], A.listCap);
-    EpaWs ws;
-    ws.vd = epaV + lane; ws.fn = epaFN + lane; ws.fi = epaFI + lane; ws.ed = epaE + lane;
-    ws.L = (size_t)lanes;
-    ws.overflow = false;
-    for (int h = lane; h < n; h += lanes) {
+    for (int h = blockIdx.x; h < n; h += gridDim.x) {
         const int2 qc = A.convexPairs[h];
         int t, wd;
         float4 g;
@@ -1382,8 +1399,9 @@ __global__ __launch_bounds__(64) void k_mtd_convex(MtdArgs A, ConvexView cv, dou
         mtd_query(A, qc.x, t, g, pos, q, wd);
         mtd_collider_pose(A, qc.y, cp, cq);
         Mf m;
-        bool ovf = false;
-        const bool hit = collide_convex(A.ctype[qc.y], A.cparams[qc.y], cp, cq, t, g, pos, q, cv, ws, m, ovf);
+        bool ovf;
+        const bool hit = collide_convex_w(A.ctype[qc.y], A.cparams[qc.y], cp, cq, t, g, pos, q, cv, M, m, ovf);
+        if (threadIdx.x != 0) continue;
         if (ovf) atomicAdd(A.counts + 3, 1);
         if (hit && m.numPoints > 0) mtd_put(A, atomicAdd(A.counts, 1), qc.x, qc.y, 0, m);
     }
@@ -1452,15 +1470,14 @@ void np_mtd_launch(World& w, const MtdArgs& A) {
     hipLaunchKernelGGL(k_mtd_walk, dim3(div_up(A.n, 64)), dim3(64), 0, w.stream, A, cv);
     PGX_LAUNCH_CHECK();
     if (w.nConvex > 0) {
-        hipLaunchKernelGGL(k_mtd_convex, dim3(div_up(w.epaLanes, 64)), dim3(64), 0, w.stream, A, cv, w.epaV.p,
-                           w.epaFN.p, w.epaFI.p, w.epaE.p, w.epaLanes);
+        hipLaunchKernelGGL(k_mtd_convex, dim3(CONVEX_WAVES), dim3(64), 0, w.stream, A, cv);
         PGX_LAUNCH_CHECK();
     }
     if (w.nTriMesh > 0) {
         const TriMeshView tv{w.tmVerts.p, w.tmTris.p, w.tmTriN.p, w.tmTriC.p, w.tmNodes.p, w.tmMesh.p};
         const MeshRecs recs{A.recs, (size_t)A.recLanes * TM_MAXCAND};
         hipLaunchKernelGGL(k_mtd_mesh, dim3(div_up(A.recLanes, 64)), dim3(64), 0, w.stream, A, cv, tv, w.tmWs.p,
-                           w.meshLanes, recs, w.epaV.p, w.epaFN.p, w.epaFI.p, w.epaE.p, w.epaLanes);
+                           w.meshLanes, recs, w.epaV.p, w.epaFN.p, w.epaFI.p, w.epaE.p, A.recLanes);
         PGX_LAUNCH_CHECK();
     }
 }
@@ -1533,11 +1550,10 @@ void np_run(World& w, int nPairs) {
     }
     if (w.nConvex > 0) {
         ConvexView cv{w.cvVerts.p, w.cvMesh.p, w.cvFace.p, w.cvFaceIdx.p, w.cvFaceN.p, w.cvFaceC.p};
-        hipLaunchKernelGGL(k_narrowphase_convex, dim3(div_up(w.epaLanes, 64)), dim3(64), 0, w.stream,
+        hipLaunchKernelGGL(k_narrowphase_convex, dim3(CONVEX_WAVES), dim3(64), 0, w.stream,
                            w.counters.p + 8, w.heavy.p, w.pkeys.p, w.localBits, w.worldColStart.p, w.colOfLocal.p,
                            w.cbody.p, w.ctype.p, w.cparams.p, w.clpos.p, w.clquat.p, w.bpos.p, w.bquat.p, cv,
-                           w.epaV.p, w.epaFN.p, w.epaFI.p, w.epaE.p, w.epaLanes, w.npNum.p, w.npNormal.p, w.npPts.p,
-                           w.counters.p + 9);
+                           w.npNum.p, w.npNormal.p, w.npPts.p, w.counters.p + 9);
         PGX_LAUNCH_CHECK();
     }
     if (w.nTriMesh > 0) {
@@ -1552,9 +1568,8 @@ void np_run(World& w, int nPairs) {
         hipLaunchKernelGGL(k_mesh_query, dim3(div_up(w.meshLanes, 64)), dim3(64), 0, w.stream, A, w.tmWs.p,
                            w.meshLanes, w.counters.p + 13, w.tmCandCap, w.tmCand.p, w.tmPairOf.p, w.tmCandOff.p,
                            w.tmCandCount.p, w.meshCount.p);
-        hipLaunchKernelGGL(k_mesh_test, dim3(div_up(w.epaLanes, 64)), dim3(64), 0, w.stream, A, w.epaV.p, w.epaFN.p,
-                           w.epaFI.p, w.epaE.p, w.epaLanes, w.counters.p + 13, w.tmCandCap, w.tmCand.p, w.tmPairOf.p,
-                           recs);
+        hipLaunchKernelGGL(k_mesh_test, dim3(MESH_TEST_WAVES), dim3(64), 0, w.stream, A, w.counters.p + 13,
+                           w.tmCandCap, w.tmCand.p, w.tmPairOf.p, recs);
         hipLaunchKernelGGL(k_mesh_emit, dim3(div_up(w.meshLanes, 64)), dim3(64), 0, w.stream, A, w.tmWs.p,
                            w.meshLanes, w.tmCandOff.p, w.tmCandCount.p, recs, w.npNum.p, w.npNormal.p, w.npPts.p,
                            w.npTri.p, w.meshFirst.p, w.meshCount.p, w.counters.p + 11, w.mmCap, w.pairCap);

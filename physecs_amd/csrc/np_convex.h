@@ -7,10 +7,9 @@
 // them the same way.
 //
 // Pairs with a convex mesh on either side are taken out of the one-pair-per-lane
-// primitive kernel into a list and solved by k_narrowphase_convex, a grid-stride kernel
-// of a fixed number of lanes. The EPA polytope of every lane lives in a device workspace
-// laid out lane-interleaved (element e of lane l at e * lanes + l), so that the lanes of a
-// wave walking the same face or vertex index read one contiguous line.
+// primitive kernel into a list and solved a wave per pair (np_wave.h). The single-lane forms
+// here serve the yes/no overlap tests and, with a polytope workspace laid out
+// lane-interleaved (element e of lane l at e * lanes + l), the triangle-mesh MTD queries.
 // Included by narrowphase.hip (shares its clipping and box-face routines).
 #pragma once
 
@@ -371,202 +370,5 @@ struct MeshRef {
     __device__ f3 vert(int i) const { return xyz(cv->verts[info.x + i]); }
     __device__ f3 face_vert(int2 fc, int k) const { return vert(cv->faceIdx[fc.x + k]); }
 };
-
-// src/Collision.cpp:352-410
-__device__ void convex_convex_contacts(f3 pos0, qf or0, const MeshRef& m0, f3 s0, f3 pos1, qf or1,
-                                       const MeshRef& m1, f3 s1, f3 normal, CPt* cps, int& numPoints) {
-    int f0 = 0;
-    float maxDot = 0.f;
-    for (int i = 0; i < m0.nfaces(); ++i) {
-        float d = dot(normal, world_face_normal(or0, m0.fnormal(i), s0));
-        if (d > maxDot) { maxDot = d; f0 = i; }
-    }
-    int f1 = 0;
-    float minDot = 0.f;
-    for (int i = 0; i < m1.nfaces(); ++i) {
-        float d = dot(normal, world_face_normal(or1, m1.fnormal(i), s1));
-        if (d < minDot) { minDot = d; f1 = i; }
-    }
-    int2 F0 = m0.face(f0), F1 = m1.face(f1);
-    m3 worldToC0 = transpose(mat3_cast(or0));
-    f3 refOrig = mulv(s0, m0.fcentroid(f0));
-    f3 u0 = normalize(sub(mulv(s0, m0.face_vert(F0, 0)), refOrig));
-    f3 u1 = normalize(divv(m0.fnormal(f0), s0));
-    f3 u2 = cross(u0, u1);
-    m3 c0ToRef = transpose(mk_m3(u0, u1, u2));
-    m3 worldToRef = mulmm(c0ToRef, worldToC0);
-    f2 clip[16];
-    f2 poly[CVX_MAXPOLY];
-    int nc = F0.y < 16 ? F0.y : 16;
-    for (int i = 0; i < nc; ++i) {
-        f3 v = mulmv(c0ToRef, mulv(s0, m0.face_vert(F0, i)));
-        clip[i] = mk2(v.z, v.x);
-    }
-    int n = F1.y < 16 ? F1.y : 16;
-    for (int i = 0; i < n; ++i) {
-        f3 v = mulmv(worldToRef, sub(add(pos1, qrot(or1, mulv(s1, m1.face_vert(F1, i)))), pos0));
-        poly[i] = mk2(v.z, v.x);
-    }
-    clip_polygon_n<CVX_MAXPOLY>(poly, n, clip, nc);
-    f3 incOrig = mulmv(worldToRef, sub(add(pos1, qrot(or1, mulv(s1, m1.fcentroid(f1)))), pos0));
-    f3 incNormal = mulmv(worldToRef, qrot(or1, normalize(divv(m1.fnormal(f1), s1))));
-    m3 refToWorld = transpose(worldToRef);
-    polygon_polygon_face_contacts(pos0, refToWorld, refOrig, u1, incOrig, incNormal, poly, n, 2, 0, cps, numPoints);
-}
-
-// src/Collision.cpp:694-785
-__device__ void capsule_convex_contacts(f3 p0L, f3 p1L, float radius, f3 meshPos, const m3& c2w, const MeshRef& m,
-                                        f3 scale, Mf& res) {
-    int fi = 0;
-    float minDot = 0.f;
-    for (int i = 0; i < m.nfaces(); ++i) {
-        float d = dot(res.normal, normalize(mulmv(c2w, divv(m.fnormal(i), scale))));
-        if (d < minDot) { minDot = d; fi = i; }
-    }
-    int2 F = m.face(fi);
-    f3 refOrig = mulv(scale, m.fcentroid(fi));
-    f3 u0 = normalize(sub(mulv(scale, m.face_vert(F, 0)), refOrig));
-    f3 u1 = normalize(divv(m.fnormal(fi), scale));
-    f3 u2 = cross(u0, u1);
-    m3 convexToRef = transpose(mk_m3(u0, u1, u2));
-    f2 clip[16];
-    int nc = F.y < 16 ? F.y : 16;
-    for (int i = 0; i < nc; ++i) {
-        f3 v = mulmv(convexToRef, mulv(scale, m.face_vert(F, i)));
-        clip[i] = mk2(v.z, v.x);
-    }
-    f3 p0Ref = mulmv(convexToRef, p0L), p1Ref = mulmv(convexToRef, p1L);
-    f2 line0 = mk2(p0Ref.z, p0Ref.x), line1 = mk2(p1Ref.z, p1Ref.x);
-    if (clip_line_n(line0, line1, clip, nc)) {
-        m3 refToWorld = mulmm(c2w, transpose(convexToRef));
-        float distToPlane = dot(refOrig, u1);
-        float y0, y1;
-        float distX = p0Ref.z - p1Ref.z, distY = p0Ref.x - p1Ref.x;
-        float adx = gabs(distX), ady = gabs(distY);
-        if (adx && adx >= ady) {
-            y0 = gmix(p0Ref.y, p1Ref.y, (p0Ref.z - line0.x) / distX);
-            y1 = gmix(p1Ref.y, p0Ref.y, (p1Ref.z - line1.x) / -distX);
-        } else if (ady > adx) {
-            y0 = gmix(p0Ref.y, p1Ref.y, (p0Ref.x - line0.y) / distY);
-            y1 = gmix(p1Ref.y, p0Ref.y, (p1Ref.x - line1.y) / -distY);
-        } else {
-            y0 = p0Ref.y;
-            y1 = p1Ref.y;
-        }
-        y0 -= radius;
-        y1 -= radius;
-        int n = 0;
-        if (y0 < distToPlane) {
-            f3 p = mk3(line0.y, y0, line0.x), on = mk3(line0.y, distToPlane, line0.x);
-            res.pts[n].p0 = add(meshPos, mulmv(refToWorld, p));
-            res.pts[n].p1 = add(meshPos, mulmv(refToWorld, on));
-            ++n;
-        }
-        if (y1 < distToPlane) {
-            f3 p = mk3(line1.y, y1, line1.x), on = mk3(line1.y, distToPlane, line1.x);
-            res.pts[n].p0 = add(meshPos, mulmv(refToWorld, p));
-            res.pts[n].p1 = add(meshPos, mulmv(refToWorld, on));
-            ++n;
-        }
-        res.numPoints = n;
-    } else {
-        res.numPoints = 0;
-    }
-}
-
-// src/Collision.cpp:808-871
-__device__ void box_convex_contacts(f3 boxCenter, const m3& basis, f3 he, f3 cpos, qf cor, const MeshRef& m,
-                                    f3 scale, f3 normal, CPt* cps, int& numPoints) {
-    int boxAxis = 0;
-    float boxAxisSign = 0.f, maxDot = 0.f;
-    for (int i = 0; i < 3; ++i) {
-        float d = dot(normal, col(basis, i));
-        float ad = gabs(d);
-        if (ad > maxDot) { maxDot = ad; boxAxis = i; boxAxisSign = d < 0 ? -1.f : 1.f; }
-    }
-    int fi = 0;
-    float minDot = 0.f;
-    for (int i = 0; i < m.nfaces(); ++i) {
-        float d = dot(normal, world_face_normal(cor, m.fnormal(i), scale));
-        if (d < minDot) { minDot = d; fi = i; }
-    }
-    int2 F = m.face(fi);
-    int cx = (boxAxis + 1) % 3, cy = (boxAxis + 2) % 3;
-    m3 worldToBox = transpose(basis);
-    f2 poly[CVX_MAXPOLY];
-    int n = F.y < 16 ? F.y : 16;
-    for (int i = 0; i < n; ++i) {
-        f3 v = mulmv(worldToBox, sub(add(cpos, qrot(cor, mulv(scale, m.face_vert(F, i)))), boxCenter));
-        poly[i] = mk2(at(v, cx), at(v, cy));
-    }
-    float hx = at(he, cx), hy = at(he, cy);
-    f2 clip[4] = {mk2(hx, hy), mk2(hx, -hy), mk2(-hx, -hy), mk2(-hx, hy)};
-    clip_polygon_n<CVX_MAXPOLY>(poly, n, clip, 4);
-    f3 incOrig = mulmv(worldToBox, sub(add(cpos, qrot(cor, mulv(scale, m.fcentroid(fi)))), boxCenter));
-    f3 incNormal = normalize(mulmv(worldToBox, qrot(cor, divv(m.fnormal(fi), scale))));
-    polygon_box_face_contacts_n<CVX_MAXPOLY>(boxCenter, basis, boxAxis, (int)boxAxisSign, he, incOrig, incNormal,
-                                             poly, n, cx, cy, cps, numPoints);
-}
-
-// one pair with a convex mesh on either side (src/Collision.cpp:895-1016); flips as the
-// reference's dispatcher does
-__device__ bool collide_convex(int t0, float4 g0, f3 p0, qf q0, int t1, float4 g1, f3 p1, qf q1,
-                               const ConvexView& cv, EpaWs& ws, Mf& m, bool& epaOverflow) {
-    m.numPoints = 0;
-    ws.overflow = false;
-    bool flipRes = false;
-    if (t0 == PGX_CONVEX_MESH && t1 != PGX_CONVEX_MESH) {   // mirrored: solve (other, convex) and flip
-        int tt = t0; t0 = t1; t1 = tt;
-        float4 gg = g0; g0 = g1; g1 = gg;
-        f3 pp = p0; p0 = p1; p1 = pp;
-        qf qq = q0; q0 = q1; q1 = qq;
-        flipRes = true;
-    }
-    MeshRef m1{&cv, cv.mesh[(int)g1.w]};
-    SupConvex b{p1, mat3_cast(q1), mk3(g1.x, g1.y, g1.z), cv.verts + m1.info.x, m1.info.y};
-    GjkV s[4];
-    bool hit = false;
-    if (t0 == PGX_SPHERE) {                                  // src/Collision.cpp:488-499
-        SupSphere a{p0, g0.x};
-        if (gjk(a, b, sub(p1, p0), s)) {
-            m.normal = epa(a, b, s, ws, m.pts[0].p0, m.pts[0].p1);
-            m.numPoints = 1;
-            hit = true;
-        }
-    } else if (t0 == PGX_CAPSULE) {                          // src/Collision.cpp:787-806
-        f3 axis = qrot(q0, mk3(0.f, 1.f, 0.f));
-        SupCapsule a{p0, axis, g0.x, g0.y};
-        if (gjk(a, b, sub(p1, p0), s)) {
-            m.normal = epa(a, b, s, ws, m.pts[0].p0, m.pts[0].p1);
-            m3 w2c = inverse(b.l2w);
-            f3 p = mulmv(w2c, sub(p0, p1));
-            f3 axisLc = mulmv(w2c, axis);
-            capsule_convex_contacts(add(p, mul(axisLc, g0.x)), sub(p, mul(axisLc, g0.x)), g0.y, p1, b.l2w, m1,
-                                    b.scale, m);
-            if (!m.numPoints) m.numPoints = 1;
-            hit = true;
-        }
-    } else if (t0 == PGX_BOX) {                              // src/Collision.cpp:873-887
-        SupBox a{p0, mat3_cast(q0), mk3(g0.x, g0.y, g0.z)};
-        if (gjk(a, b, sub(p1, p0), s)) {
-            m.normal = epa(a, b, s, ws, m.pts[0].p0, m.pts[0].p1);
-            box_convex_contacts(p0, a.l2w, a.he, p1, q1, m1, b.scale, m.normal, m.pts, m.numPoints);
-            if (!m.numPoints) m.numPoints = 1;
-            hit = true;
-        }
-    } else {                                                 // src/Collision.cpp:412-426
-        MeshRef m0{&cv, cv.mesh[(int)g0.w]};
-        SupConvex a{p0, mat3_cast(q0), mk3(g0.x, g0.y, g0.z), cv.verts + m0.info.x, m0.info.y};
-        if (gjk(a, b, sub(p1, p0), s)) {
-            m.normal = epa(a, b, s, ws, m.pts[0].p0, m.pts[0].p1);
-            convex_convex_contacts(p0, q0, m0, a.scale, p1, q1, m1, b.scale, m.normal, m.pts, m.numPoints);
-            if (!m.numPoints) m.numPoints = 1;
-            hit = true;
-        }
-    }
-    epaOverflow = ws.overflow;
-    if (flipRes) flip(m);
-    return hit;
-}
 
 }  // namespace pgx

@@ -362,11 +362,8 @@ struct SupTriangle {
     }
 };
 
-__device__ bool convex_tri(const SupConvex& sc, f3 a, f3 b, f3 c, f3 centroid, EpaWs& ews, TCI& ci) {   // :616-697
-    SupTriangle st{a, b, c};
-    GjkV s[4];
-    if (!gjk(sc, st, sub(centroid, sc.pos), s)) return false;
-    ci.normal = epa(sc, st, s, ews, ci.cpBody, ci.cpTri);
+// the contact's distance and the triangle feature its point lies on (:640-697)
+__device__ __forceinline__ void convex_tri_feature(f3 a, f3 b, f3 c, TCI& ci) {
     ci.distance = dot(sub(ci.cpTri, ci.cpBody), ci.normal);
     f3 v0 = sub(b, a), v1 = sub(c, a), v2 = sub(ci.cpTri, a);
     float d00 = dot(v0, v0), d01 = dot(v0, v1), d11 = dot(v1, v1), d20 = dot(v2, v0), d21 = dot(v2, v1);
@@ -397,6 +394,14 @@ __device__ bool convex_tri(const SupConvex& sc, f3 a, f3 b, f3 c, f3 centroid, E
             ci.feature = TF_FACE;
         }
     }
+}
+
+__device__ bool convex_tri(const SupConvex& sc, f3 a, f3 b, f3 c, f3 centroid, EpaWs& ews, TCI& ci) {   // :616-697
+    SupTriangle st{a, b, c};
+    GjkV s[4];
+    if (!gjk(sc, st, sub(centroid, sc.pos), s)) return false;
+    ci.normal = epa(sc, st, s, ews, ci.cpBody, ci.cpTri);
+    convex_tri_feature(a, b, c, ci);
     return true;
 }
 
@@ -754,22 +759,28 @@ __device__ int mesh_query(int t, float4 g, f3 localPos, qf localOr, const Convex
     return nc;
 }
 
-// the per-shape test of one candidate triangle ti (src/CollisionTriangleMesh.cpp:886-903)
-__device__ bool mesh_test(int t, float4 g, f3 localPos, qf localOr, const SupConvex& sc, const MeshCtx& mc, int ti,
-                          EpaWs& ews, TCI& ci, bool& epaErr) {
+// the per-shape test of one candidate triangle ti (src/CollisionTriangleMesh.cpp:886-903):
+// the shapes with a closed form
+__device__ bool mesh_test_closed(int t, float4 g, f3 localPos, qf localOr, const MeshCtx& mc, int ti, TCI& ci) {
     int4 ix = mc.tri(ti);
     f3 a = mc.vert(ix.x), b = mc.vert(ix.y), c = mc.vert(ix.z);
     f3 n = mc.n(ti);
     ci.featureIndex = 0; ci.boxFeature = 0; ci.boxAxis = 0;
-    bool hit;
-    if (t == PGX_SPHERE) hit = sphere_tri(localPos, g.x, a, b, c, n, ci);
-    else if (t == PGX_CAPSULE) hit = capsule_tri(localPos, localOr, g.x, g.y, a, b, c, n, ci);
-    else if (t == PGX_BOX) hit = box_tri(localPos, localOr, mk3(g.x, g.y, g.z), a, b, c, n, ci);
-    else {
-        hit = convex_tri(sc, a, b, c, mc.c(ti), ews, ci);
-        if (ews.overflow) epaErr = true;
-    }
     ci.tri = ti;
+    if (t == PGX_SPHERE) return sphere_tri(localPos, g.x, a, b, c, n, ci);
+    if (t == PGX_CAPSULE) return capsule_tri(localPos, localOr, g.x, g.y, a, b, c, n, ci);
+    return box_tri(localPos, localOr, mk3(g.x, g.y, g.z), a, b, c, n, ci);
+}
+
+// and all shapes, in one lane
+__device__ bool mesh_test(int t, float4 g, f3 localPos, qf localOr, const SupConvex& sc, const MeshCtx& mc, int ti,
+                          EpaWs& ews, TCI& ci, bool& epaErr) {
+    if (t != PGX_CONVEX_MESH) return mesh_test_closed(t, g, localPos, localOr, mc, ti, ci);
+    int4 ix = mc.tri(ti);
+    ci.featureIndex = 0; ci.boxFeature = 0; ci.boxAxis = 0;
+    ci.tri = ti;
+    const bool hit = convex_tri(sc, mc.vert(ix.x), mc.vert(ix.y), mc.vert(ix.z), mc.c(ti), ews, ci);
+    if (ews.overflow) epaErr = true;
     return hit;
 }
 

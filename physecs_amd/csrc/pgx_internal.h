@@ -106,11 +106,10 @@ constexpr int JOINT_MAX_ROWS = 7;      // a prismatic joint with its limit and d
 enum { EXEC_COLORS = 0, EXEC_COOPERATIVE = 1, EXEC_FLOW = 2, EXEC_FLOW_XCD = 3, EXEC_WORLDS = 4, EXEC_PASS = 5, EXEC_XPASS = 6 };
 constexpr int FLOW_QUEUES = 8;         // queues of a dependency-driven pass: at most one per XCD
 constexpr int WORLD_SMALL = 256;       // per-world passes: worlds up to this many dynamic bodies share a launch
-// convex narrowphase: EPA polytope capacity per lane and lanes of the convex kernel
+// convex narrowphase: EPA polytope capacity
 constexpr int EPA_MAXV = 104;          // 4 simplex vertices + at most 100 insertions
 constexpr int EPA_MAXF = 256;          // > 2 * EPA_MAXV - 4, the face count of a closed triangulation
 constexpr int EPA_MAXE = 128;          // horizon (loose) edges of one insertion
-constexpr int EPA_LANES = 65536;
 constexpr int CVX_MAX_FACE_VERTS = 16;
 // triangle-mesh narrowphase: per-lane capacities and lanes
 constexpr int TM_MAXCAND = 256;        // triangles overlapping one body's local bounds
@@ -292,8 +291,7 @@ struct World {
     DBuf<int2> cvFace;
     DBuf<int32_t> cvFaceIdx;
     DBuf<int32_t> heavy;               // pairs with a convex mesh (filled by the primitive kernel)
-    int epaLanes = 0;                  // lanes of the convex kernel = EPA workspaces
-    DBuf<double> epaV, epaFN;
+    DBuf<double> epaV, epaFN;          // the triangle-mesh MTD queries' polytopes, a lane each
     DBuf<int32_t> epaFI, epaE;
     // static triangle meshes: vertices, triangles in the BVH build's order (mesh-local
     // vertex indices), triangle normals / centroids, BVH nodes (2 float4 each: {min,

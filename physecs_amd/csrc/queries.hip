@@ -283,8 +283,13 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
     A.recLanes = 1;
     A.recs = nullptr;
     if (w.nTriMesh > 0) {
-        A.recLanes = std::max(1, std::min({w.meshLanes, w.epaLanes, 8192}));
+        A.recLanes = std::max(1, std::min(w.meshLanes, 8192));
         w.qRecs.alloc((size_t)(TM_CI_WORDS + 1) * TM_MAXCAND * A.recLanes);
+        if (w.nConvex > 0) {   // convex query shapes against triangles: a polytope per lane
+            const size_t L = (size_t)A.recLanes;
+            w.epaV.alloc(9 * EPA_MAXV * L); w.epaFN.alloc(3 * EPA_MAXF * L);
+            w.epaFI.alloc(3 * EPA_MAXF * L); w.epaE.alloc(2 * EPA_MAXE * L);
+        }
         A.recs = w.qRecs.p;
     }
     A.qPrm = w.qShape.p; A.qPos = w.qShape.p + n; A.qQuat = w.qShape.p + 2 * (size_t)n; A.qType = w.qType.p;

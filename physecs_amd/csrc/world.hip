@@ -432,10 +432,6 @@ void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
         w.nConvex = sc->n_convex;
         upload(w.cvVerts, cvv, s); upload(w.cvMesh, cvm, s); upload(w.cvFace, cvf, s);
         upload(w.cvFaceIdx, cvfi, s); upload(w.cvFaceN, cvn, s); upload(w.cvFaceC, cvc, s);
-        w.epaLanes = EPA_LANES;
-        size_t L = (size_t)w.epaLanes;
-        w.epaV.alloc(9 * EPA_MAXV * L); w.epaFN.alloc(3 * EPA_MAXF * L);
-        w.epaFI.alloc(3 * EPA_MAXF * L); w.epaE.alloc(2 * EPA_MAXE * L);
     }
     if (sc->n_trimesh > 0) {
         w.tmMaxDepth = upload_triangle_meshes(w, sc, s);
@@ -450,12 +446,6 @@ void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
         w.tmCand.alloc(w.tmCandCap); w.tmPairOf.alloc(w.tmCandCap);
         w.tmRecs.alloc((size_t)(TM_CI_WORDS + 1) * w.tmCandCap);
         w.tmCandOff.alloc(w.pairCap); w.tmCandCount.alloc(w.pairCap);
-        if (w.epaLanes < w.meshLanes) {   // convex bodies against triangles need EPA state per lane
-            w.epaLanes = w.meshLanes;
-            size_t L = (size_t)w.epaLanes;
-            w.epaV.alloc(9 * EPA_MAXV * L); w.epaFN.alloc(3 * EPA_MAXF * L);
-            w.epaFI.alloc(3 * EPA_MAXF * L); w.epaE.alloc(2 * EPA_MAXE * L);
-        }
     }
     // creation-time bounds: no margin (src/Physecs.cpp:32)
     bp_compute_bounds(w, false);
