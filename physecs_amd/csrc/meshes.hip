@@ -221,10 +221,33 @@ BuiltMesh load_mesh(const void* cache, size_t len, const float* vp, int nv, cons
     return m;
 }
 
+// Whether the depth-first walk, left child first, meets the triangles in index order, as the
+// build leaves them (a cache may hold any tree that passes load_mesh's checks).
+static bool leaves_in_order(const BuiltMesh& m) {
+    auto asi = [](float f) { int i; std::memcpy(&i, &f, sizeof i); return i; };
+    std::vector<int> todo{0};
+    int next = 0;
+    while (!todo.empty()) {
+        const int n = todo.back();
+        todo.pop_back();
+        const int count = asi(m.nodes[2 * n].w), index = asi(m.nodes[2 * n + 1].w);
+        if (count == 0) {
+            todo.push_back(index + 1);
+            todo.push_back(index);
+        } else {
+            if (index < next) return false;
+            next = index + count;
+        }
+        if (todo.size() > m.nodes.size()) return false;   // not a tree
+    }
+    return true;
+}
+
 int upload_triangle_meshes(World& w, const pgx_scene_desc* sc, hipStream_t s) {
     std::vector<float4> verts, triN, triC, nodes;
     std::vector<int4> tris, meshes;
     int maxDepth = 0;
+    w.tmInOrder = true;
     for (int m = 0; m < sc->n_trimesh; ++m) {
         int v0 = sc->tri_vert_start[m], nv = sc->tri_vert_start[m + 1] - v0;
         int t0 = sc->tri_start[m], nt = sc->tri_start[m + 1] - t0;
@@ -236,6 +259,7 @@ int upload_triangle_meshes(World& w, const pgx_scene_desc* sc, hipStream_t s) {
         const BuiltMesh bm = cache ? load_mesh(cache, sc->tri_bvh_cache_bytes[m], vp, nv, ip, nt)
                                    : build_mesh(vp, nv, ip, nt);
         maxDepth = std::max(maxDepth, bm.depth);
+        w.tmInOrder = w.tmInOrder && leaves_in_order(bm);
         int vbase = (int)verts.size(), tbase = (int)tris.size(), nbase = (int)nodes.size() / 2;
         meshes.push_back(make_int4(vbase, nv, tbase, nbase));
         for (int i = 0; i < nv; ++i) verts.push_back(make_float4(vp[3 * i], vp[3 * i + 1], vp[3 * i + 2], 0.f));

@@ -10,6 +10,7 @@
 #include "pgx_internal.h"
 #include "shape_bounds.h"
 #include <iterator>
+#include <type_traits>
 
 namespace pgx {
 
@@ -647,8 +648,8 @@ __device__ bool collide(int t0, float4 g0, f3 p0, qf q0, int t1, float4 g1, f3 p
 }  // namespace pgx
 
 #include "np_convex.h"
-#include "np_trimesh.h"
 #include "np_wave.h"
+#include "np_trimesh.h"
 
 namespace pgx {
 
@@ -1089,21 +1090,34 @@ __global__ __launch_bounds__(64) void k_triggers(
 }
 
 // ------------------------------------------------------------------ triangle-mesh pairs
-// Everything the three mesh passes read.
+// What the passes over mesh pairs read, for the step's pairs and the MTD queries' alike.
 struct MeshArgs {
-    const int32_t* nMeshP;                 // number of mesh pairs (device)
-    const int32_t* meshPairs;              // their pair slots
+    const int32_t* nPairs;                 // number of mesh pairs (device)
+    int maxPairs;                          // and how many of them are listed
+    const int32_t* stepPairs;              // the step's: pair slots,
+    const int2* queryPairs;                // or (query, collider)
     const uint64_t* pkeys;
     int localBits;
     const int32_t *worldColStart, *colOfLocal, *cbody, *ctype;
     const float4 *cparams, *clpos, *clquat, *bpos, *bquat;
+    const float4 *qPrm, *qPos, *qQuat;
+    const int32_t* qType;
     ConvexView cv;
     TriMeshView tv;
+    int inOrder;                           // World::tmInOrder
     int32_t* errors;                       // capacity and EPA errors
+    // candidates (triangle, pair), each pair's block of them, their records; the convex ones
+    // that GJK hit, with their simplex (36 floats, word f of hit i at f * candCap + i)
+    int32_t* candTotal;
+    int candCap;
+    int32_t *cand, *pairOf, *candOff, *candCount;
+    MeshRecs recs;
+    int32_t *hitTotal, *hitList;
+    float* simplex;
 };
 
 struct MeshPair {
-    int p, tb;
+    int p, c, tb;                          // pair slot or query; the mesh's collider; the body's shape
     bool flip;
     float4 g;
     f3 pos0, pos1, lpos;
@@ -1111,169 +1125,242 @@ struct MeshPair {
     int4 mi;
 };
 
-// mesh pair h: the body collider and the mesh, their world poses, the body in the mesh's
-// frame. src/Collision.cpp:897-906: a mesh on side 0 is solved as (other, mesh) and flipped.
-// False for a mesh-mesh pair (no routine).
-__device__ bool mesh_pair(const MeshArgs& A, int h, MeshPair& m, SupConvex& sc) {
-    m.p = A.meshPairs[h];
-    uint64_t key = A.pkeys[m.p];
-    uint64_t lmask = (1ull << A.localBits) - 1;
-    int wd = (int)(key >> (2 * A.localBits));
-    int base = A.worldColStart[wd];
-    int c0 = A.colOfLocal[base + (int)((key >> A.localBits) & lmask)];
-    int c1 = A.colOfLocal[base + (int)(key & lmask)];
-    int t0 = A.ctype[c0], t1 = A.ctype[c1];
-    if (t0 == PGX_TRIANGLE_MESH && t1 == PGX_TRIANGLE_MESH) return false;
-    m.flip = t0 == PGX_TRIANGLE_MESH;
-    int cb = m.flip ? c1 : c0, cm = m.flip ? c0 : c1;
-    int bb = A.cbody[cb], bm = A.cbody[cm];
-    qf qb = q4(A.bquat[bb]), qm = q4(A.bquat[bm]);
-    m.pos0 = add(xyz(A.bpos[bb]), qrot(qb, xyz(A.clpos[cb])));
-    m.or0 = qmul(qb, q4(A.clquat[cb]));
-    m.pos1 = add(xyz(A.bpos[bm]), qrot(qm, xyz(A.clpos[cm])));
-    m.or1 = qmul(qm, q4(A.clquat[cm]));
-    m.tb = A.ctype[cb];
-    m.g = A.cparams[cb];
-    m.mi = A.tv.mesh[(int)A.cparams[cm].w];
+__device__ __forceinline__ void collider_pose(const MeshArgs& A, int c, f3& pos, qf& q) {
+    const int b = A.cbody[c];
+    const qf bq = q4(A.bquat[b]);
+    pos = add(xyz(A.bpos[b]), qrot(bq, xyz(A.clpos[c])));
+    q = qmul(bq, q4(A.clquat[c]));
+}
+
+// mesh pair h: the body collider (or query shape) and the mesh, their world poses, the body
+// in the mesh's frame. src/Collision.cpp:897-906: a mesh on side 0 is solved as (other, mesh)
+// and flipped. False for a mesh-mesh pair (no routine).
+template <bool QUERY>
+__device__ __forceinline__ bool mesh_pair(const MeshArgs& A, int h, MeshPair& m, SupConvex& sc) {
+    if (QUERY) {
+        const int2 qc = A.queryPairs[h];
+        m.p = qc.x;
+        m.c = qc.y;
+        m.flip = true;
+        m.tb = A.qType[m.p];
+        m.g = A.qPrm[m.p];
+        m.pos0 = xyz(A.qPos[m.p]);
+        m.or0 = q4(A.qQuat[m.p]);
+    } else {
+        m.p = A.stepPairs[h];
+        const uint64_t key = A.pkeys[m.p];
+        const uint64_t lmask = (1ull << A.localBits) - 1;
+        const int base = A.worldColStart[(int)(key >> (2 * A.localBits))];
+        const int c0 = A.colOfLocal[base + (int)((key >> A.localBits) & lmask)];
+        const int c1 = A.colOfLocal[base + (int)(key & lmask)];
+        const int t0 = A.ctype[c0], t1 = A.ctype[c1];
+        if (t0 == PGX_TRIANGLE_MESH && t1 == PGX_TRIANGLE_MESH) return false;
+        m.flip = t0 == PGX_TRIANGLE_MESH;
+        const int cb = m.flip ? c1 : c0;
+        m.c = m.flip ? c0 : c1;
+        collider_pose(A, cb, m.pos0, m.or0);
+        m.tb = A.ctype[cb];
+        m.g = A.cparams[cb];
+    }
+    collider_pose(A, m.c, m.pos1, m.or1);
+    m.mi = A.tv.mesh[(int)A.cparams[m.c].w];
     mesh_local(m.tb, m.g, m.pos0, m.or0, m.pos1, m.or1, A.cv, m.lpos, m.lor, sc);
     return true;
 }
 
-// exclusive prefix of n over the wave and the wave's total
-__device__ __forceinline__ int wave_scan(int n, int& total) {
-    const int lane = threadIdx.x & (WAVE - 1);
-    int incl = n;
-    for (int o = 1; o < WAVE; o <<= 1) {
-        int t = __shfl_up(incl, o);
-        if (lane >= o) incl += t;
+// Places in a list for the waves of a block, n[wave] each: one atomic per block. (One per
+// wave, on one address, served some 65 per us: 47 us for the 3,071 pairs of 2,048 hulls and
+// 1,024 capsules on a terrain, more than the query itself.) Every wave of the block calls it.
+template <int WAVES>
+__device__ __forceinline__ int block_reserve(int32_t* counter, int n) {
+    __shared__ int count[WAVES], first;
+    const int wave = threadIdx.x / WAVE;
+    if (wave_lane() == 0) count[wave] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int total = 0;
+        for (int k = 0; k < WAVES; ++k) total += count[k];
+        first = total ? atomicAdd(counter, total) : 0;
     }
-    total = __shfl(incl, WAVE - 1);
-    return incl - n;
+    __syncthreads();
+    int at = first;
+    for (int k = 0; k < wave; ++k) at += count[k];
+    __syncthreads();   // read before the block's next turn
+    return at;
 }
 
-// pass 1, one lane per mesh pair: the BVH query, and a block of candidate slots (triangle,
-// pair) reserved for the pair with one atomic per wave
-__global__ __launch_bounds__(64) void k_mesh_query(MeshArgs A, int32_t* tmWs, int lanes, int32_t* __restrict__ candTotal,
-                                                   int candCap, int32_t* __restrict__ cand,
-                                                   int32_t* __restrict__ pairOf, int32_t* __restrict__ candOff,
-                                                   int32_t* __restrict__ candCount, int32_t* __restrict__ meshCount) {
-    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nMesh = *A.nMeshP;
-    MeshWs ws{tmWs + lane, (size_t)lanes};
-    for (int h0 = lane & ~(WAVE - 1); h0 < nMesh; h0 += lanes) {   // the same trip count for a whole wave
-        const int h = h0 + (lane & (WAVE - 1));
+// pass 1, a wave per pair: the BVH query, and a block of candidate slots reserved for the
+// pair. Queries without room are counted on (their caller provides it and asks again).
+constexpr int MESH_BLOCK_WAVES = 8, MESH_BLOCKS = 512;
+template <bool QUERY>
+__global__ __launch_bounds__(MESH_BLOCK_WAVES * 64) void k_mesh_query(MeshArgs A, int32_t* __restrict__ meshCount) {
+    __shared__ QueryMem mem[MESH_BLOCK_WAVES];
+    const int n = min(*A.nPairs, A.maxPairs), lane = wave_lane(), wave = threadIdx.x / WAVE;
+    QueryMem& S = mem[wave];
+    for (int h0 = blockIdx.x * MESH_BLOCK_WAVES; h0 < n; h0 += gridDim.x * MESH_BLOCK_WAVES) {
+        const int h = h0 + wave;
         int nc = 0;
-        if (h < nMesh) {
+        if (h < n) {
             MeshPair m;
             SupConvex sc;
-            meshCount[A.meshPairs[h]] = 0;
-            if (mesh_pair(A, h, m, sc)) {
-                MeshCtx mc{&A.tv, m.mi};
-                nc = mesh_query(m.tb, m.g, m.lpos, m.lor, A.cv, mc, ws);
-                if (nc < 0) { atomicAdd(A.errors, 1); nc = 0; }
+            const bool ok = mesh_pair<QUERY>(A, h, m, sc);
+            if (!QUERY && lane == 0) meshCount[m.p] = 0;
+            if (ok) {
+                const MeshCtx mc{&A.tv, m.mi};
+                nc = mesh_query(m.tb, m.g, m.lpos, m.lor, A.cv, mc, A.inOrder != 0, S);
+                if (nc < 0) {
+                    if (lane == 0) atomicAdd(A.errors, 1);
+                    nc = 0;
+                }
             }
         }
-        int total;
-        int off = wave_scan(nc, total);
-        int base = 0;
-        if ((lane & (WAVE - 1)) == WAVE - 1 && total) base = atomicAdd(candTotal, total);
-        base = __shfl(base, WAVE - 1) + off;
-        if (h < nMesh) {
-            if (base + nc > candCap) { atomicAdd(A.errors, 1); nc = 0; }
-            for (int i = 0; i < nc; ++i) {
-                cand[base + i] = ws.cand(i);
-                pairOf[base + i] = h;
-            }
-            candOff[h] = base;
-            candCount[h] = nc;
+        const int base = block_reserve<MESH_BLOCK_WAVES>(A.candTotal, nc);
+        if (h >= n) continue;
+        if (base + nc > A.candCap) {
+            if (!QUERY && lane == 0) atomicAdd(A.errors, 1);
+            nc = 0;
+        }
+        for (int i = lane; i < nc; i += WAVE) {
+            A.cand[base + i] = S.cand[i];
+            A.pairOf[base + i] = h;
+        }
+        if (lane == 0) {
+            A.candOff[h] = base;
+            A.candCount[h] = nc;
         }
     }
 }
 
-// pass 2, the per-shape test of every (pair, candidate triangle), its contact record. A wave
-// takes a run of candidates, as few as spreads them over MESH_TEST_WAVES waves: the closed
-// forms one per lane, then the convex bodies' GJK and EPA one after another, the whole wave
-// on each (with a lane each, 125 us for 2,048 hulls on a terrain, 304 B of scratch per lane).
-constexpr int MESH_TEST_WAVES = 4096;
-__global__ __launch_bounds__(64) void k_mesh_test(MeshArgs A, const int32_t* __restrict__ candTotal, int candCap,
-                                                  const int32_t* __restrict__ cand,
-                                                  const int32_t* __restrict__ pairOf, MeshRecs recs) {
-    __shared__ WaveMem M;
-    const int lane = threadIdx.x;
-    const int total = min(*candTotal, candCap);
-    const int waves = gridDim.x;
-    const int run = min(WAVE, max(1, (total + waves - 1) / waves));
-    for (long first = (long)blockIdx.x * run; first < total; first += (long)waves * run) {
-        const int k = (int)first + lane;
-        const bool mine = lane < run && k < total;
-        int h = 0, ti = 0;
-        bool convex = false;
-        if (mine) {
+// pass 2, a lane per (pair, candidate triangle): the closed forms and their contact records;
+// for a convex mesh GJK, its hits listed with their simplex
+constexpr int MESH_TEST_BLOCKS = 2048;
+template <bool QUERY, bool CONVEX>
+__global__ __launch_bounds__(64) void k_mesh_test(MeshArgs A) {
+    const int total = min(*A.candTotal, A.candCap);
+    // whole waves go round together, so the appends see whole waves
+    for (int base = blockIdx.x * WAVE; base < total; base += gridDim.x * WAVE) {
+        const int k = base + (int)threadIdx.x;
+        bool solved = false;
+        GV va, vb, vc, vd;
+        if (k < total) {
             MeshPair m;
             SupConvex sc;
-            h = pairOf[k];
-            ti = cand[k];
-            mesh_pair(A, h, m, sc);
-            convex = m.tb == PGX_CONVEX_MESH;
-            if (!convex) {
-                const MeshCtx mc{&A.tv, m.mi};
-                TCI ci;
-                const bool hit = mesh_test_closed(m.tb, m.g, m.lpos, m.lor, mc, ti, ci);
-                recs.store(k, hit, ci);
-            }
-        }
-        for (uint64_t todo = __ballot(convex); todo; todo &= todo - 1) {
-            const int l = first_lane(todo), kc = (int)first + l;
-            MeshPair m;
-            SupConvex sc;
-            mesh_pair(A, __builtin_amdgcn_readlane(h, l), m, sc);
+            mesh_pair<QUERY>(A, A.pairOf[k], m, sc);
             const MeshCtx mc{&A.tv, m.mi};
             TCI ci;
-            bool ovf = false;
-            const bool hit = mesh_test_convex_w(sc, mc, __builtin_amdgcn_readlane(ti, l), M, ci, ovf);
-            if (lane == 0) {
-                if (ovf) atomicAdd(A.errors, 1);
-                recs.store(kc, hit, ci);
+            ci.tri = A.cand[k];
+            const int4 ix = mc.tri(ci.tri);
+            const f3 a = mc.vert(ix.x), b = mc.vert(ix.y), c = mc.vert(ix.z);
+            bool hit;
+            if (CONVEX && m.tb == PGX_CONVEX_MESH) {
+                hit = solved = gjk_w(sc, SupTriangle{a, b, c}, sub(mc.c(ci.tri), sc.pos), va, vb, vc, vd);
+            } else {
+                hit = mesh_test_closed(m.tb, m.g, m.lpos, m.lor, a, b, c, mc.n(ci.tri), ci);
+                if (hit) A.recs.store(k, ci);
+            }
+            A.recs.rec(k, TM_CI_WORDS) = hit ? 1 : 0;
+        }
+        if (CONVEX && __ballot(solved)) {
+            const int i = wave_append(A.hitTotal, solved);
+            if (solved) {
+                A.hitList[i] = k;
+                float* s = A.simplex + i;
+                const size_t cap = (size_t)A.candCap;
+                int f = 0;
+                auto put = [&](const GV& g) {
+                    for (const f3& v : {g.pos, g.sp0, g.sp1}) {
+                        s[cap * f] = v.x; s[cap * (f + 1)] = v.y; s[cap * (f + 2)] = v.z;
+                        f += 3;
+                    }
+                };
+                put(va); put(vb); put(vc); put(vd);
             }
         }
     }
 }
 
-// pass 3, one lane per mesh pair: the pair's hit records in candidate order, a block of
-// manifold slots (one atomic per wave), the emission passes
-__global__ __launch_bounds__(64) void k_mesh_emit(MeshArgs A, int32_t* tmWs, int lanes,
-                                                  const int32_t* __restrict__ candOff,
-                                                  const int32_t* __restrict__ candCount, MeshRecs recs,
-                                                  int32_t* __restrict__ npNum, float4* __restrict__ npNormal,
-                                                  float4* __restrict__ npPts, int32_t* __restrict__ npTri,
-                                                  int32_t* __restrict__ meshFirst, int32_t* __restrict__ meshCount,
-                                                  int32_t* __restrict__ slotCounter, int mmCap, int pairCap) {
-    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nMesh = *A.nMeshP;
-    MeshWs ws{tmWs + lane, (size_t)lanes};
-    for (int h0 = lane & ~(WAVE - 1); h0 < nMesh; h0 += lanes) {
-        const int h = h0 + (lane & (WAVE - 1));
-        int nct = 0;
+// pass 3, a wave per listed triangle: EPA and the contact record
+template <bool QUERY>
+__global__ __launch_bounds__(64) void k_mesh_epa(MeshArgs A) {
+    __shared__ WaveMem M;
+    const int n = *A.hitTotal;
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const int k = A.hitList[i];
         MeshPair m;
         SupConvex sc;
-        bool ok = h < nMesh && mesh_pair(A, h, m, sc);
-        if (ok) {
-            const int off = candOff[h], nc = candCount[h];
-            for (int i = 0; i < nc; ++i)
-                if (recs.hit(off + i)) ws.order(nct++) = off + i;
+        mesh_pair<QUERY>(A, A.pairOf[k], m, sc);
+        const MeshCtx mc{&A.tv, m.mi};
+        TCI ci;
+        ci.tri = A.cand[k];
+        ci.featureIndex = 0; ci.boxFeature = 0; ci.boxAxis = 0;
+        const int4 ix = mc.tri(ci.tri);
+        const f3 a = mc.vert(ix.x), b = mc.vert(ix.y), c = mc.vert(ix.z);
+        // word `lane` of the simplex per lane, then in every lane
+        const float word = A.simplex[(size_t)A.candCap * min((int)threadIdx.x, 35) + i];
+        auto get = [&](int f) {
+            return GV{mk3(lane_read(word, f), lane_read(word, f + 1), lane_read(word, f + 2)),
+                      mk3(lane_read(word, f + 3), lane_read(word, f + 4), lane_read(word, f + 5)),
+                      mk3(lane_read(word, f + 6), lane_read(word, f + 7), lane_read(word, f + 8))};
+        };
+        bool ovf;
+        ci.normal = epa_w(hull_of(sc), SupTriangle{a, b, c}, get(0), get(9), get(18), get(27), M, ci.cpBody, ci.cpTri, ovf);
+        convex_tri_feature(a, b, c, ci);
+        if (threadIdx.x == 0) {
+            if (ovf) atomicAdd(A.errors, 1);
+            A.recs.store(k, ci);
         }
-        int total;
-        int pre = wave_scan(nct, total);
-        int base = 0;
-        if ((lane & (WAVE - 1)) == WAVE - 1 && total) base = atomicAdd(slotCounter, total);
-        const int slot = __shfl(base, WAVE - 1) + pre;
-        if (!ok || nct == 0) continue;
-        if (slot + nct > mmCap) { atomicAdd(A.errors, 1); continue; }
-        MeshCtx mc{&A.tv, m.mi};
+    }
+}
+
+// pass 4, a wave per pair: its hit records in candidate order into S; their number
+__device__ __forceinline__ int mesh_hits(const MeshArgs& A, int off, int nc, EmitMem& S) {
+    const int lane = wave_lane();
+    int nct = 0;
+    for (int first = 0; first < nc; first += WAVE) {
+        const int i = first + lane;
+        const bool hit = i < nc && A.recs.hit(off + i);
+        const uint64_t hits = __ballot(hit);
+        if (hit) {
+            S.order[nct + __popcll(hits & lanes_below())] = i;
+            S.feature[i] = A.recs.feature(off + i);
+            S.dist[i] = A.recs.dist(off + i);
+        }
+        nct += (int)__popcll(hits);
+    }
+    wave_sync();
+    return nct;
+}
+
+// and the emission passes: the step's manifolds go to a block of slots per pair
+template <bool CONVEX>
+__global__ __launch_bounds__(MESH_BLOCK_WAVES * 64) void k_mesh_emit(MeshArgs A, int32_t* __restrict__ npNum,
+                                                  float4* __restrict__ npNormal, float4* __restrict__ npPts,
+                                                  int32_t* __restrict__ npTri, int32_t* __restrict__ meshFirst,
+                                                  int32_t* __restrict__ meshCount, int32_t* __restrict__ slotCounter,
+                                                  int mmCap, int pairCap) {
+    __shared__ EmitMem mem[MESH_BLOCK_WAVES];
+    const int n = min(*A.nPairs, A.maxPairs), lane = wave_lane(), wave = threadIdx.x / WAVE;
+    EmitMem& S = mem[wave];
+    for (int h0 = blockIdx.x * MESH_BLOCK_WAVES; h0 < n; h0 += gridDim.x * MESH_BLOCK_WAVES) {
+        const int h = h0 + wave;
+        const int off = h < n ? A.candOff[h] : 0;
+        const int nct = h < n ? mesh_hits(A, off, A.candCount[h], S) : 0;
+        const int slot = block_reserve<MESH_BLOCK_WAVES>(slotCounter, nct);
+        if (nct == 0) continue;
+        if (slot + nct > mmCap) {
+            if (lane == 0) atomicAdd(A.errors, 1);
+            continue;
+        }
+        MeshPair m;
+        SupConvex sc;
+        mesh_pair<false>(A, h, m, sc);
+        const MeshCtx mc{&A.tv, m.mi};
         MeshOut out{npNum, npNormal, npPts, npTri, pairCap + slot, slot, 0, m.flip};
-        mesh_emit(m.tb, m.g, m.lpos, m.lor, m.pos1, m.or1, mc, A.cv, ws, recs, nct, out);
-        meshFirst[m.p] = slot;
-        meshCount[m.p] = out.n;
+        mesh_emit<CONVEX>(m.tb, m.g, m.lpos, m.lor, m.pos1, m.or1, mc, A.cv, S, A.recs, (size_t)off, nct, out);
+        if (lane == 0) {
+            meshFirst[m.p] = slot;
+            meshCount[m.p] = out.n;
+        }
     }
 }
 
@@ -1294,12 +1381,15 @@ __device__ __forceinline__ float manifold_mtd(const Mf& m) {   // src/Physecs.cp
     return mtd;
 }
 
-__device__ __forceinline__ void mtd_put(const MtdArgs& A, int slot, int q, int c, int k, const Mf& m) {
+__device__ __forceinline__ void mtd_store(const MtdArgs& A, int slot, int q, int c, int k, float4 res) {
     if (slot >= A.cap) return;
     A.keys[slot] = ((uint64_t)(uint32_t)q << (A.cbits + MTD_MBITS)) | ((uint64_t)(uint32_t)c << MTD_MBITS) |
                    (uint64_t)k;
     A.vals[slot] = slot;
-    A.res[slot] = f4(m.normal, manifold_mtd(m));
+    A.res[slot] = res;
+}
+__device__ __forceinline__ void mtd_put(const MtdArgs& A, int slot, int q, int c, int k, const Mf& m) {
+    mtd_store(A, slot, q, c, k, f4(m.normal, manifold_mtd(m)));
 }
 
 __device__ __forceinline__ void mtd_query(const MtdArgs& A, int i, int& t, float4& g, f3& pos, qf& q, int& wd) {
@@ -1407,62 +1497,81 @@ __global__ __launch_bounds__(64) void k_mtd_convex(MtdArgs A, ConvexView cv) {
     }
 }
 
-// the manifolds of one (query, mesh) pair: the mesh is the collider, geom0, so the pair is
+// pass 3, the pairs with a triangle mesh, in the step's mesh passes: the manifolds of one
+// (query, mesh) pair; the mesh is the collider, geom0, so the pair is
 // solved as (query, mesh) and flipped (src/Collision.cpp:897-901)
 struct MtdOut {
-    const MtdArgs* A;
-    int q, c, n;
-    __device__ void emit(Mf& m, int) {
+    float4* res;          // LDS: the pair's results
+    int n;
+    __device__ __forceinline__ void emit(Mf& m, int) {   // the same manifold in every lane
         if (m.numPoints <= 0) return;
         m.normal = neg(m.normal);
-        for (int i = 0; i < m.numPoints; ++i) { f3 t = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = t; }
-        mtd_put(*A, atomicAdd(A->counts, 1), q, c, n, m);
+        swap_sides(m);
+        if (wave_lane() == 0) res[n] = f4(m.normal, manifold_mtd(m));
         ++n;
     }
 };
 
-// pass 3: the pairs with a triangle mesh, one lane per pair: the mesh BVH query, the
-// per-triangle tests into the lane's own block of TM_MAXCAND contact records (a buffer of
-// recLanes * TM_MAXCAND records), the emission passes (the step's three mesh passes in one
-// lane)
-__global__ __launch_bounds__(64) void k_mtd_mesh(MtdArgs A, ConvexView cv, TriMeshView tv, int32_t* tmWs,
-                                                 int wsLanes, MeshRecs recs, double* epaV, double* epaFN,
-                                                 int32_t* epaFI, int32_t* epaE, int epaLanes) {
-    const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-    if (lane >= A.recLanes) return;
-    const int n = min(A.counts[2], A.listCap);
-    MeshWs ws{tmWs + lane, (size_t)wsLanes};
-    EpaWs ews;
-    ews.vd = epaV + lane; ews.fn = epaFN + lane; ews.fi = epaFI + lane; ews.ed = epaE + lane;
-    ews.L = (size_t)epaLanes;
-    ews.overflow = false;
-    for (int h = lane; h < n; h += A.recLanes) {
-        const int2 qc = A.meshPairs[h];
-        int t, wd;
-        float4 g;
-        f3 pos, mpos, lpos;
-        qf q, mq, lor;
-        mtd_query(A, qc.x, t, g, pos, q, wd);
-        mtd_collider_pose(A, qc.y, mpos, mq);
-        SupConvex sc;
-        mesh_local(t, g, pos, q, mpos, mq, cv, lpos, lor, sc);
-        const MeshCtx mc{&tv, tv.mesh[(int)A.cparams[qc.y].w]};
-        const int nc = mesh_query(t, g, lpos, lor, cv, mc, ws);
-        if (nc < 0) { atomicAdd(A.counts + 3, 1); continue; }
-        const int base = lane * TM_MAXCAND;
-        int nct = 0;
-        for (int j = 0; j < nc; ++j) {
-            TCI ci;
-            bool epaErr = false;
-            ews.overflow = false;
-            const bool hit = mesh_test(t, g, lpos, lor, sc, mc, ws.cand(j), ews, ci, epaErr);
-            if (epaErr) atomicAdd(A.counts + 3, 1);
-            recs.store(base + j, hit, ci);
-            if (hit) ws.order(nct++) = base + j;
+template <bool CONVEX>
+__global__ __launch_bounds__(MESH_BLOCK_WAVES * 64) void k_mtd_mesh_emit(MeshArgs A, MtdArgs Q) {
+    __shared__ EmitMem mem[MESH_BLOCK_WAVES];
+    __shared__ float4 results[MESH_BLOCK_WAVES][TM_MAXCAND];
+    const int n = min(*A.nPairs, A.maxPairs), wave = threadIdx.x / WAVE;
+    EmitMem& S = mem[wave];
+    for (int h0 = blockIdx.x * MESH_BLOCK_WAVES; h0 < n; h0 += gridDim.x * MESH_BLOCK_WAVES) {
+        const int h = h0 + wave;
+        const int off = h < n ? A.candOff[h] : 0;
+        const int nct = h < n ? mesh_hits(A, off, A.candCount[h], S) : 0;
+        MtdOut out{results[wave], 0};
+        MeshPair m;
+        if (nct) {
+            SupConvex sc;
+            mesh_pair<true>(A, h, m, sc);
+            const MeshCtx mc{&A.tv, m.mi};
+            mesh_emit<CONVEX>(m.tb, m.g, m.lpos, m.lor, m.pos1, m.or1, mc, A.cv, S, A.recs, (size_t)off, nct, out);
         }
-        MtdOut out{&A, qc.x, qc.y, 0};
-        mesh_emit(t, g, lpos, lor, mpos, mq, mc, cv, ws, recs, nct, out);
+        const int base = block_reserve<MESH_BLOCK_WAVES>(Q.counts, out.n);
+        for (int k = wave_lane(); k < out.n; k += WAVE) mtd_store(Q, base + k, m.p, m.c, k, out.res[k]);
+        wave_sync();   // the results are read before the wave's next pair overwrites them
     }
+}
+
+// the passes up to the emission
+template <bool QUERY>
+static void mesh_passes(World& w, const MeshArgs& A) {
+    hipLaunchKernelGGL(k_mesh_query<QUERY>, dim3(MESH_BLOCKS), dim3(MESH_BLOCK_WAVES * 64), 0, w.stream, A, w.meshCount.p);
+    if (w.nConvex > 0) {
+        hipLaunchKernelGGL((k_mesh_test<QUERY, true>), dim3(MESH_TEST_BLOCKS), dim3(64), 0, w.stream, A);
+        hipLaunchKernelGGL(k_mesh_epa<QUERY>, dim3(CONVEX_WAVES), dim3(64), 0, w.stream, A);
+    } else {
+        hipLaunchKernelGGL((k_mesh_test<QUERY, false>), dim3(MESH_TEST_BLOCKS), dim3(64), 0, w.stream, A);
+    }
+    PGX_LAUNCH_CHECK();
+}
+
+static MeshArgs mesh_args(World& w, MeshBuffers& b) {
+    MeshArgs A{};
+    A.pkeys = w.pkeys.p; A.localBits = w.localBits;
+    A.worldColStart = w.worldColStart.p; A.colOfLocal = w.colOfLocal.p; A.cbody = w.cbody.p; A.ctype = w.ctype.p;
+    A.cparams = w.cparams.p; A.clpos = w.clpos.p; A.clquat = w.clquat.p; A.bpos = w.bpos.p; A.bquat = w.bquat.p;
+    A.cv = ConvexView{w.cvVerts.p, w.cvMesh.p, w.cvFace.p, w.cvFaceIdx.p, w.cvFaceN.p, w.cvFaceC.p};
+    A.tv = TriMeshView{w.tmVerts.p, w.tmTris.p, w.tmTriN.p, w.tmTriC.p, w.tmNodes.p, w.tmMesh.p};
+    A.inOrder = w.tmInOrder ? 1 : 0;
+    A.candCap = b.candCap;
+    A.cand = b.cand.p; A.pairOf = b.pairOf.p; A.candOff = b.candOff.p; A.candCount = b.candCount.p;
+    A.recs = MeshRecs{b.recs.p, (size_t)b.candCap};
+    A.hitList = b.hitList.p; A.simplex = b.simplex.p;
+    return A;
+}
+
+// buffers for the mesh pairs' passes: `pairs` pairs, `cands` candidate triangles
+void np_mesh_buffers(World& w, MeshBuffers& b, size_t pairs, size_t cands) {
+    b.candOff.alloc(pairs); b.candCount.alloc(pairs);
+    if ((size_t)b.candCap >= cands) return;
+    b.cand.alloc(cands); b.pairOf.alloc(cands);
+    b.recs.alloc((size_t)(TM_CI_WORDS + 1) * cands);
+    if (w.nConvex > 0) { b.hitList.alloc(cands); b.simplex.alloc(36 * cands); }
+    b.candCap = (int)cands;
 }
 
 void np_mtd_launch(World& w, const MtdArgs& A) {
@@ -1474,10 +1583,13 @@ void np_mtd_launch(World& w, const MtdArgs& A) {
         PGX_LAUNCH_CHECK();
     }
     if (w.nTriMesh > 0) {
-        const TriMeshView tv{w.tmVerts.p, w.tmTris.p, w.tmTriN.p, w.tmTriC.p, w.tmNodes.p, w.tmMesh.p};
-        const MeshRecs recs{A.recs, (size_t)A.recLanes * TM_MAXCAND};
-        hipLaunchKernelGGL(k_mtd_mesh, dim3(div_up(A.recLanes, 64)), dim3(64), 0, w.stream, A, cv, tv, w.tmWs.p,
-                           w.meshLanes, recs, w.epaV.p, w.epaFN.p, w.epaFI.p, w.epaE.p, A.recLanes);
+        MeshArgs M = mesh_args(w, w.qMesh);
+        M.nPairs = A.counts + 2; M.maxPairs = A.listCap; M.queryPairs = A.meshPairs;
+        M.qPrm = A.qPrm; M.qPos = A.qPos; M.qQuat = A.qQuat; M.qType = A.qType;
+        M.errors = A.counts + 3; M.candTotal = A.counts + 4; M.hitTotal = A.counts + 5;
+        mesh_passes<true>(w, M);
+        hipLaunchKernelGGL(w.nConvex > 0 ? k_mtd_mesh_emit<true> : k_mtd_mesh_emit<false>, dim3(MESH_BLOCKS),
+                           dim3(MESH_BLOCK_WAVES * 64), 0, w.stream, M, A);
         PGX_LAUNCH_CHECK();
     }
 }
@@ -1557,22 +1669,14 @@ void np_run(World& w, int nPairs) {
         PGX_LAUNCH_CHECK();
     }
     if (w.nTriMesh > 0) {
-        MeshArgs A;
-        A.nMeshP = w.counters.p + 10; A.meshPairs = w.meshPairs.p; A.pkeys = w.pkeys.p; A.localBits = w.localBits;
-        A.worldColStart = w.worldColStart.p; A.colOfLocal = w.colOfLocal.p; A.cbody = w.cbody.p; A.ctype = w.ctype.p;
-        A.cparams = w.cparams.p; A.clpos = w.clpos.p; A.clquat = w.clquat.p; A.bpos = w.bpos.p; A.bquat = w.bquat.p;
-        A.cv = ConvexView{w.cvVerts.p, w.cvMesh.p, w.cvFace.p, w.cvFaceIdx.p, w.cvFaceN.p, w.cvFaceC.p};
-        A.tv = TriMeshView{w.tmVerts.p, w.tmTris.p, w.tmTriN.p, w.tmTriC.p, w.tmNodes.p, w.tmMesh.p};
-        A.errors = w.counters.p + 12;
-        MeshRecs recs{w.tmRecs.p, (size_t)w.tmCandCap};
-        hipLaunchKernelGGL(k_mesh_query, dim3(div_up(w.meshLanes, 64)), dim3(64), 0, w.stream, A, w.tmWs.p,
-                           w.meshLanes, w.counters.p + 13, w.tmCandCap, w.tmCand.p, w.tmPairOf.p, w.tmCandOff.p,
-                           w.tmCandCount.p, w.meshCount.p);
-        hipLaunchKernelGGL(k_mesh_test, dim3(MESH_TEST_WAVES), dim3(64), 0, w.stream, A, w.counters.p + 13,
-                           w.tmCandCap, w.tmCand.p, w.tmPairOf.p, recs);
-        hipLaunchKernelGGL(k_mesh_emit, dim3(div_up(w.meshLanes, 64)), dim3(64), 0, w.stream, A, w.tmWs.p,
-                           w.meshLanes, w.tmCandOff.p, w.tmCandCount.p, recs, w.npNum.p, w.npNormal.p, w.npPts.p,
-                           w.npTri.p, w.meshFirst.p, w.meshCount.p, w.counters.p + 11, w.mmCap, w.pairCap);
+        MeshArgs A = mesh_args(w, w.stepMesh);
+        A.nPairs = w.counters.p + 10; A.maxPairs = w.pairCap; A.stepPairs = w.meshPairs.p;
+        A.errors = w.counters.p + 12; A.candTotal = w.counters.p + 13; A.hitTotal = w.counters.p + 2;
+        mesh_passes<false>(w, A);
+        hipLaunchKernelGGL(w.nConvex > 0 ? k_mesh_emit<true> : k_mesh_emit<false>, dim3(MESH_BLOCKS),
+                           dim3(MESH_BLOCK_WAVES * 64), 0, w.stream, A,
+                           w.npNum.p, w.npNormal.p, w.npPts.p, w.npTri.p, w.meshFirst.p, w.meshCount.p,
+                           w.counters.p + 11, w.mmCap, w.pairCap);
         PGX_LAUNCH_CHECK();
     }
 }

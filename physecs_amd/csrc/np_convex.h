@@ -1,5 +1,5 @@
-// Convex-mesh narrowphase on the device: GJK (src/GJK.h:131-292), EPA (src/EPA.h:9-186)
-// and the convex contact generators (src/Collision.cpp:352-426,488-499,694-887,
+// Convex-mesh narrowphase on the device: GJK (src/GJK.h:131-292); with np_wave.h, EPA
+// (src/EPA.h:9-186) and the convex contact generators (src/Collision.cpp:352-426,488-499,694-887,
 // src/ContactsUtil.cpp:109-204), operation for operation with the reference, including
 // its mixed precision: simplex and polytope vertices are doubles, every support query
 // narrows its direction to float, and the float helpers the reference feeds with double
@@ -7,9 +7,8 @@
 // them the same way.
 //
 // Pairs with a convex mesh on either side are taken out of the one-pair-per-lane
-// primitive kernel into a list and solved a wave per pair (np_wave.h). The single-lane forms
-// here serve the yes/no overlap tests and, with a polytope workspace laid out
-// lane-interleaved (element e of lane l at e * lanes + l), the triangle-mesh MTD queries.
+// primitive kernel into a list and solved a wave per pair (np_wave.h). The single-lane GJK
+// here serves the yes/no overlap tests.
 // Included by narrowphase.hip (shares its clipping and box-face routines).
 #pragma once
 
@@ -153,147 +152,7 @@ __device__ bool gjk(const S0& s0, const S1& s1, f3 startDir, GjkV* s) {         
     return false;
 }
 
-// ------------------------------------------------------------------ EPA
-// one lane's polytope in the lane-interleaved workspace
-struct EpaWs {
-    double* vd;       // 9 doubles per vertex: pos, sp0, sp1
-    int* fi;          // 3 ints per face
-    double* fn;       // 3 doubles per face (unit normal)
-    int* ed;          // 2 ints per loose edge
-    size_t L;         // lanes
-    int nv, nf;
-    bool overflow;
-    __device__ double& V(int v, int c) { return vd[(size_t)(v * 9 + c) * L]; }
-    __device__ int& FI(int f, int k) { return fi[(size_t)(f * 3 + k) * L]; }
-    __device__ double& FN(int f, int c) { return fn[(size_t)(f * 3 + c) * L]; }
-    __device__ int& E(int e, int k) { return ed[(size_t)(e * 2 + k) * L]; }
-    __device__ d3 pos(int v) { return mkd(V(v, 0), V(v, 1), V(v, 2)); }
-    __device__ d3 normal(int f) { return mkd(FN(f, 0), FN(f, 1), FN(f, 2)); }
-    __device__ void putV(int v, const GjkV& g) {
-        V(v, 0) = g.pos.x; V(v, 1) = g.pos.y; V(v, 2) = g.pos.z;
-        V(v, 3) = g.sp0.x; V(v, 4) = g.sp0.y; V(v, 5) = g.sp0.z;
-        V(v, 6) = g.sp1.x; V(v, 7) = g.sp1.y; V(v, 8) = g.sp1.z;
-    }
-    __device__ GjkV getV(int v) {
-        GjkV g;
-        g.pos = mkd(V(v, 0), V(v, 1), V(v, 2));
-        g.sp0 = mkd(V(v, 3), V(v, 4), V(v, 5));
-        g.sp1 = mkd(V(v, 6), V(v, 7), V(v, 8));
-        return g;
-    }
-    __device__ void create_face(int i0, int i1, int i2) {              // src/EPA.h:24-34
-        if (nf >= EPA_MAXF) { overflow = true; return; }
-        d3 n = dcross(dsub(pos(i0), pos(i1)), dsub(pos(i2), pos(i1)));
-        double len = dlength(n);
-        if (len) n = ddivs(n, len);
-        FI(nf, 0) = i0; FI(nf, 1) = i1; FI(nf, 2) = i2;
-        FN(nf, 0) = n.x; FN(nf, 1) = n.y; FN(nf, 2) = n.z;
-        ++nf;
-    }
-    __device__ void copy_face(int dst, int src) {
-        for (int k = 0; k < 3; ++k) { FI(dst, k) = FI(src, k); FN(dst, k) = FN(src, k); }
-    }
-    __device__ double face_distance(int f) { return ddot(pos(FI(f, 0)), normal(f)); }   // src/EPA.h:41-43
-};
-
-template <class S0, class S1>
-__device__ f3 epa(const S0& s0, const S1& s1, GjkV* s, EpaWs& P, f3& cp0, f3& cp1) {   // src/EPA.h:171-186
-    P.nv = 4; P.nf = 0; P.overflow = false;
-    for (int i = 0; i < 4; ++i) P.putV(i, s[i]);
-    {   // EpaPolytope(GjkSimplex&), src/EPA.h:50-66
-        d3 n = dcross(dsub(s[0].pos, s[1].pos), dsub(s[2].pos, s[1].pos));
-        if (ddot(dsub(s[3].pos, s[0].pos), n) < 0) {
-            P.create_face(0, 1, 2); P.create_face(3, 1, 0); P.create_face(3, 2, 1); P.create_face(3, 0, 2);
-        } else {
-            P.create_face(0, 2, 1); P.create_face(3, 2, 0); P.create_face(3, 1, 2); P.create_face(3, 0, 1);
-        }
-    }
-    float minDist = 0.f;
-    d3 normal = mkd(0, 0, 0);
-    int faceIndex = 0;
-    for (int it = 0; it < 100 && !P.overflow; ++it) {
-        // findClosestFace: a float running minimum compared against double distances (:68-79)
-        minDist = __builtin_inff();
-        for (int f = 0; f < P.nf; ++f) {
-            double d = P.face_distance(f);
-            if (d < (double)minDist) { minDist = (float)d; normal = P.normal(f); faceIndex = f; }
-        }
-        GjkV v = mdiff(s0, s1, narrow(normal));
-        if (ddot(v.pos, normal) - (double)minDist < (double)0.00001f) break;
-        // insertVertex (:81-120)
-        if (P.nv >= EPA_MAXV) { P.overflow = true; break; }
-        int ne = 0;
-        for (int f = P.nf - 1; f >= 0; --f) {
-            if (ddot(P.normal(f), dsub(v.pos, P.pos(P.FI(f, 0)))) > 0) {
-                int e[3][2] = {{P.FI(f, 0), P.FI(f, 1)}, {P.FI(f, 1), P.FI(f, 2)}, {P.FI(f, 2), P.FI(f, 0)}};
-                bool found[3] = {false, false, false};
-                for (int j = 0; j < 3; ++j)
-                    for (int k = ne - 1; k >= 0; --k)
-                        if (P.E(k, 0) == e[j][1] && P.E(k, 1) == e[j][0]) {
-                            found[j] = true;
-                            P.E(k, 0) = P.E(ne - 1, 0);
-                            P.E(k, 1) = P.E(ne - 1, 1);
-                            --ne;
-                            break;
-                        }
-                for (int j = 0; j < 3; ++j)
-                    if (!found[j]) {
-                        if (ne >= EPA_MAXE) { P.overflow = true; break; }
-                        P.E(ne, 0) = e[j][0];
-                        P.E(ne, 1) = e[j][1];
-                        ++ne;
-                    }
-                P.copy_face(f, P.nf - 1);
-                --P.nf;
-            }
-        }
-        int vi = P.nv++;
-        P.putV(vi, v);
-        for (int k = 0; k < ne; ++k) P.create_face(vi, P.E(k, 0), P.E(k, 1));
-    }
-    // getClosestPoints (:122-168), including proj = normal + distance (:133)
-    int fa = P.FI(faceIndex, 0), fb = P.FI(faceIndex, 1), fc = P.FI(faceIndex, 2);
-    GjkV a = P.getV(fa), b = P.getV(fb), c = P.getV(fc);
-    d3 proj = dadds(P.normal(faceIndex), P.face_distance(faceIndex));
-    f3 v0 = narrow(dsub(b.pos, a.pos)), v1 = narrow(dsub(c.pos, a.pos)), v2 = narrow(dsub(proj, a.pos));
-    double d00 = dot(v0, v0), d01 = dot(v0, v1), d11 = dot(v1, v1), d20 = dot(v2, v0), d21 = dot(v2, v1);
-    double denom = d00 * d11 - d01 * d01;
-    double u, vv, w;
-    if (denom) {
-        vv = (d20 * d11 - d21 * d01) / denom;
-        w = (d00 * d21 - d01 * d20) / denom;
-        u = 1.0 - vv - w;
-    } else {
-        w = 0;
-        if (d00) { vv = d20 / d00; u = 1.0 - vv; }
-        else { vv = 0; u = 1.0; }
-    }
-    cp0 = narrow(dadd(dadd(dmul(u, a.sp0), dmul(vv, b.sp0)), dmul(w, c.sp0)));
-    cp1 = narrow(dadd(dadd(dmul(u, a.sp1), dmul(vv, b.sp1)), dmul(w, c.sp1)));
-    return narrow(normal);
-}
-
 // ------------------------------------------------------------------ contact generation
-template <int CAP>
-__device__ void clip_polygon_n(f2* poly, int& n, const f2* clip, int nclip) {   // src/Clipping.cpp:21-53
-    f2 out[CAP];
-    for (int e = 0; e < nclip; ++e) {
-        f2 a = clip[e], b = clip[(e + 1) % nclip];
-        int m = 0;
-        for (int i = 0; i < n; ++i) {
-            int j = (i + 1) == n ? 0 : i + 1;
-            bool ii = inside(poly[i], a, b), ji = inside(poly[j], a, b);
-            if (ii && ji) { if (m < CAP) out[m++] = poly[j]; }
-            else if (ii) { if (m < CAP) out[m++] = intersect2(poly[i], poly[j], a, b); }
-            else if (ji) {
-                if (m < CAP) out[m++] = intersect2(poly[i], poly[j], a, b);
-                if (m < CAP) out[m++] = poly[j];
-            }
-        }
-        n = m;
-        for (int i = 0; i < m; ++i) poly[i] = out[i];
-    }
-}
 __device__ bool clip_line_n(f2& p0, f2& p1, const f2* clip, int nclip) {        // src/Clipping.cpp:55-71
     for (int i = 0; i < nclip; ++i) {
         int j = (i + 1) % nclip;
@@ -304,59 +163,6 @@ __device__ bool clip_line_n(f2& p0, f2& p1, const f2* clip, int nclip) {        
         else return false;
     }
     return true;
-}
-
-// src/ContactsUtil.cpp:109-204
-__device__ void polygon_polygon_face_contacts(f3 refPos, const m3& refToWorld, f3 refOrig, f3 refNormal,
-                                              f3 incOrig, f3 incNormal, const f2* poly, int n, int cx, int cy,
-                                              CPt* cps, int& numPoints) {
-    f3 pen[CVX_MAXPOLY];
-    int np = 0;
-    float distRef = dot(refOrig, refNormal);
-    f3 dir = mk3(0.f, 1.f, 0.f);
-    for (int i = 0; i < n; ++i) {
-        f3 p3 = mk3(poly[i].y, 0.f, poly[i].x);
-        float distance = dot(sub(incOrig, p3), incNormal) / dot(dir, incNormal);
-        if (distance < distRef + 1e-4f) {
-            p3.y = distance;
-            pen[np++] = p3;
-        }
-    }
-    auto emit = [&](int slot, int idx) {
-        f3 on = pen[idx];
-        on.y = distRef;
-        cps[slot].p0 = add(refPos, mulmv(refToWorld, on));
-        cps[slot].p1 = add(refPos, mulmv(refToWorld, pen[idx]));
-    };
-    if (np > 4) {
-        emit(0, 0);
-        float maxD = 0.f;
-        int maxDi = 0;
-        for (int i = 0; i < np; ++i) {
-            f3 d = sub(pen[i], pen[0]);
-            float dd = dot(d, d);
-            if (dd > maxD) { maxD = dd; maxDi = i; }
-        }
-        emit(1, maxDi);
-        float maxA = 0.f, minA = 0.f;
-        int maxAi = 0, minAi = 0;
-        for (int i = 0; i < np; ++i) {
-            f3 ca = sub(pen[0], pen[i]), cb = sub(pen[maxDi], pen[i]);
-            float area = det2(mk2(at(ca, cx), at(ca, cy)), mk2(at(cb, cx), at(cb, cy)));
-            if (area > maxA) { maxA = area; maxAi = i; }
-        }
-        emit(2, maxAi);
-        for (int i = 0; i < np; ++i) {
-            f3 da = sub(pen[0], pen[i]), db = sub(pen[maxDi], pen[i]);
-            float area = det2(mk2(at(da, cx), at(da, cy)), mk2(at(db, cx), at(db, cy)));
-            if (area < minA) { minA = area; minAi = i; }
-        }
-        emit(3, minAi);
-        numPoints = 4;
-    } else {
-        for (int i = 0; i < np; ++i) emit(i, i);
-        numPoints = np;
-    }
 }
 
 __device__ __forceinline__ f3 world_face_normal(qf q, f3 n, f3 scale) { return normalize(qrot(q, divv(n, scale))); }

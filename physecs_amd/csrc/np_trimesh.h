@@ -1,19 +1,20 @@
 // Triangle-mesh narrowphase on the device: physecs::collisionTriangleMesh
-// (src/CollisionTriangleMesh.cpp:882-956) for one (body collider, static mesh) pair per
-// lane -- the body's mesh-local AABB queries the mesh BVH depth first (left child first,
-// src/TriangleMesh.cpp:163-192), every overlapping triangle is tested
-// (sphere/capsule/box closed forms, GJK/EPA for convex meshes, :44-121,221-396,616-697),
-// face contacts are emitted in reverse order with swap-removal, the rest are ordered with
-// std::sort's own introsort and emitted unless their feature's vertices were already
-// covered (:906-953). The triangle distance routines follow src/GeomUtil.cpp:61-127,469-665.
+// (src/CollisionTriangleMesh.cpp:882-956) of (body collider, static mesh) pairs -- the body's
+// mesh-local AABB queries the mesh BVH (overlapBvh, src/TriangleMesh.cpp:163-192), every
+// overlapping triangle is tested (sphere/capsule/box closed forms, GJK/EPA for convex
+// meshes, :44-121,221-396,616-697), face contacts are emitted in reverse order with
+// swap-removal, the rest are ordered with std::sort's own introsort and emitted unless their
+// feature's vertices were already covered (:906-953). The triangle distance routines follow
+// src/GeomUtil.cpp:61-127,469-665.
 //
-// Three passes: each pair queries the BVH and reserves a block of candidate triangles;
-// every (pair, candidate) is tested by a lane of its own (contact records stored flat,
-// one per candidate); each pair then emits its manifolds from its records. Per-lane state
-// of the query and emission passes (candidate triangles, the contact order, covered
-// vertices) lives in a lane-interleaved workspace (word w of lane l at w * lanes + l). A
-// pair's manifolds go to a block of slots reserved with one atomic add, in emission
-// order. Included by narrowphase.hip after np_convex.h.
+// Four passes: the BVH query, a wave per pair (64 nodes at a time); the closed forms and GJK,
+// a lane per (pair, candidate triangle); EPA, a wave per triangle that GJK hit; the emission,
+// a wave per pair (hull faces and polygon corners one per lane). For 2,048 hulls and 1,024
+// capsules on a terrain they take 20 + 41 + 26 + 54 us; a lane per pair ran the few thousand
+// pairs as a few waves, 83 us of query, 125 us of tests with EPA and 251 us of emission. One
+// launch for all of it, a wave per pair, took 184 us: the tests of a pair's triangles are
+// then a chain, and a capsule's few triangles leave most lanes idle.
+// Included by narrowphase.hip after np_wave.h.
 #pragma once
 #include "introsort.h"
 
@@ -38,27 +39,16 @@ struct TCI {                 // TriangleContactInfo (:22-36)
     int feature, featureIndex, boxFeature, boxAxis;
 };
 
-// per-lane workspace of the query and emission passes
-struct MeshWs {
-    int32_t* w;              // lane's first word
-    size_t L;
-    __device__ int& cand(int i) { return w[(size_t)i * L]; }
-    __device__ int& order(int i) { return w[(size_t)(TM_MAXCAND + i) * L]; }
-    __device__ int& voided(int i) { return w[(size_t)(2 * TM_MAXCAND + i) * L]; }
-};
-
 // contact records, one per candidate triangle: word f of record k at f * cap + k (word
 // TM_CI_WORDS: 1 if the triangle test hit)
 struct MeshRecs {
     int32_t* w;
     size_t cap;
-    __device__ int& rec(int k, int f) const { return w[(size_t)f * cap + k]; }
-    __device__ bool hit(int k) const { return rec(k, TM_CI_WORDS) != 0; }
-    __device__ float dist(int k) const { return __int_as_float(rec(k, 10)); }
-    __device__ int feature(int k) const { return rec(k, 11); }
-    __device__ void store(int k, bool h, const TCI& t) const {
-        rec(k, TM_CI_WORDS) = h ? 1 : 0;
-        if (!h) return;
+    __device__ int& rec(size_t k, int f) const { return w[(size_t)f * cap + k]; }
+    __device__ bool hit(size_t k) const { return rec(k, TM_CI_WORDS) != 0; }
+    __device__ float dist(size_t k) const { return __int_as_float(rec(k, 10)); }
+    __device__ int feature(size_t k) const { return rec(k, 11); }
+    __device__ void store(size_t k, const TCI& t) const {
         rec(k, 0) = t.tri;
         rec(k, 1) = __float_as_int(t.normal.x); rec(k, 2) = __float_as_int(t.normal.y); rec(k, 3) = __float_as_int(t.normal.z);
         rec(k, 4) = __float_as_int(t.cpBody.x); rec(k, 5) = __float_as_int(t.cpBody.y); rec(k, 6) = __float_as_int(t.cpBody.z);
@@ -66,7 +56,7 @@ struct MeshRecs {
         rec(k, 10) = __float_as_int(t.distance);
         rec(k, 11) = t.feature; rec(k, 12) = t.featureIndex; rec(k, 13) = t.boxFeature | (t.boxAxis << 8);
     }
-    __device__ TCI load(int k) const {
+    __device__ TCI load(size_t k) const {
         TCI t;
         t.tri = rec(k, 0);
         t.normal = mk3(__int_as_float(rec(k, 1)), __int_as_float(rec(k, 2)), __int_as_float(rec(k, 3)));
@@ -79,14 +69,29 @@ struct MeshRecs {
     }
 };
 
-// index array over the contact order (record indices), compared by distance
-// (TriangleContactInfo::operator<)
+// the query's LDS: the BVH nodes still to visit, the candidate triangles
+constexpr int TM_NODES = 512;
+struct QueryMem {
+    int nodes[TM_NODES];
+    int cand[TM_MAXCAND];
+};
+// the emission's: the clipped polygons, the hit candidates in contact order with their
+// distance and feature, the covered vertices
+struct EmitMem {
+    WavePoly P;
+    int order[TM_MAXCAND], feature[TM_MAXCAND];
+    float dist[TM_MAXCAND];
+    int voided[3 * TM_MAXCAND];
+};
+
+// index array over the contact order (candidate indices), compared by distance
+// (TriangleContactInfo::operator<); every lane runs the sort alike. Distances that are not
+// numbers can lead its unguarded scans past the array: they stop there.
 struct OrderArr {
-    MeshWs* ws;
-    const MeshRecs* recs;
-    __device__ int get(int i) { return ws->order(i); }
-    __device__ void set(int i, int v) { ws->order(i) = v; }
-    __device__ bool less(int a, int b) { return recs->dist(a) < recs->dist(b); }
+    EmitMem& S;
+    __device__ __forceinline__ int get(int i) { return i >= 0 && i < TM_MAXCAND ? S.order[i] : -1; }
+    __device__ __forceinline__ void set(int i, int v) { if (i >= 0 && i < TM_MAXCAND && v >= 0) S.order[i] = v; }
+    __device__ __forceinline__ bool less(int a, int b) { return a >= 0 && b >= 0 && S.dist[a] < S.dist[b]; }
 };
 
 // ------------------------------------------------------------------ GeomUtil (triangles)
@@ -396,15 +401,6 @@ __device__ __forceinline__ void convex_tri_feature(f3 a, f3 b, f3 c, TCI& ci) {
     }
 }
 
-__device__ bool convex_tri(const SupConvex& sc, f3 a, f3 b, f3 c, f3 centroid, EpaWs& ews, TCI& ci) {   // :616-697
-    SupTriangle st{a, b, c};
-    GjkV s[4];
-    if (!gjk(sc, st, sub(centroid, sc.pos), s)) return false;
-    ci.normal = epa(sc, st, s, ews, ci.cpBody, ci.cpTri);
-    convex_tri_feature(a, b, c, ci);
-    return true;
-}
-
 // ------------------------------------------------------------------ contact generation
 struct MeshCtx {
     const TriMeshView* tv;
@@ -416,36 +412,38 @@ struct MeshCtx {
 };
 
 // the triangle's face frame (u0 toward vertex 0, u1 = normal) and its clip triangle in
-// (z, x), listed backwards (:132-146)
-__device__ void tri_frame(const MeshCtx& mc, int t, bool normalizeN, f3& refOrig, f3& u1, m3& meshToRef, f2* clip) {
-    int4 ix = mc.tri(t);
+// (z, x), listed backwards (:132-146): clip corner `lane` in lanes 0-2
+__device__ __forceinline__ void tri_frame(const MeshCtx& mc, int t, bool normalizeN, f3& refOrig, f3& u1, m3& meshToRef,
+                                          f2& clip) {
+    const int4 ix = mc.tri(t);
+    const int lane = wave_lane();
     refOrig = mc.c(t);
-    f3 u0 = normalize(sub(mc.vert(ix.x), refOrig));
+    const f3 u0 = normalize(sub(mc.vert(ix.x), refOrig));
     u1 = normalizeN ? normalize(mc.n(t)) : mc.n(t);
-    f3 u2 = cross(u0, u1);
+    const f3 u2 = cross(u0, u1);
     meshToRef = transpose(mk_m3(u0, u1, u2));
-    int iv[3] = {ix.x, ix.y, ix.z};
-    for (int i = 0; i < 3; i++) {
-        f3 v = mulmv(meshToRef, mc.vert(iv[i]));
-        clip[3 - i - 1] = mk2(v.z, v.x);
-    }
+    const f3 v = mulmv(meshToRef, mc.vert(lane == 0 ? ix.z : lane == 1 ? ix.y : ix.x));
+    clip = mk2(v.z, v.x);
 }
 
-__device__ void gen_sphere(f3 pos1, qf or1, const TCI& ci, Mf& m) {   // :73-81
+__device__ __forceinline__ void gen_sphere(f3 pos1, qf or1, const TCI& ci, Mf& m) {   // :73-81
     m.normal = qrot(or1, ci.normal);
     m.numPoints = 1;
     m.pts[0].p0 = add(pos1, qrot(or1, ci.cpBody));
     m.pts[0].p1 = add(pos1, qrot(or1, ci.cpTri));
 }
 
-__device__ bool gen_capsule_face(f3 pos0, qf or0, float hh0, float r0, f3 pos1, qf or1, const MeshCtx& mc,
+__device__ __forceinline__ bool gen_capsule_face(f3 pos0, qf or0, float hh0, float r0, f3 pos1, qf or1, const MeshCtx& mc,
                                  const TCI& ci, Mf& m) {   // :123-217; false when nothing is pushed
     f3 dir = qrot(or0, mk3(0.f, 1.f, 0.f));
     f3 p0l = sub(pos0, mul(dir, hh0)), p1l = add(pos0, mul(dir, hh0));
     f3 refOrig, u1;
     m3 meshToRef;
+    f2 corner;
+    tri_frame(mc, ci.tri, true, refOrig, u1, meshToRef, corner);
     f2 clip[3];
-    tri_frame(mc, ci.tri, true, refOrig, u1, meshToRef, clip);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) clip[i] = mk2(lane_read(corner.x, i), lane_read(corner.y, i));
     f3 p0Ref = mulmv(meshToRef, p0l), p1Ref = mulmv(meshToRef, p1l);
     f2 line0 = mk2(p0Ref.z, p0Ref.x), line1 = mk2(p1Ref.z, p1Ref.x);
     if (!clip_line_n(line0, line1, clip, 3)) return false;
@@ -467,37 +465,36 @@ __device__ bool gen_capsule_face(f3 pos0, qf or0, float hh0, float r0, f3 pos1, 
     }
     y0 -= r0;
     y1 -= r0;
-    int n = 0;
     m.normal = mulmv(meshToWorld, ci.normal);
-    if (y0 < distToPlane) {
-        f3 p = mk3(line0.y, y0, line0.x), on = mk3(line0.y, distToPlane, line0.x);
-        m.pts[n].p0 = add(pos1, mulmv(refToWorld, p));
-        m.pts[n].p1 = add(pos1, mulmv(refToWorld, on));
-        ++n;
+    const bool k0 = y0 < distToPlane, k1 = y1 < distToPlane;
+    CPt a, b;
+    a.p0 = add(pos1, mulmv(refToWorld, mk3(line0.y, y0, line0.x)));
+    a.p1 = add(pos1, mulmv(refToWorld, mk3(line0.y, distToPlane, line0.x)));
+    b.p0 = add(pos1, mulmv(refToWorld, mk3(line1.y, y1, line1.x)));
+    b.p1 = add(pos1, mulmv(refToWorld, mk3(line1.y, distToPlane, line1.x)));
+    if (!k0 && !k1) {
+        a.p0 = add(pos1, mulmv(meshToWorld, ci.cpBody));
+        a.p1 = add(pos1, mulmv(meshToWorld, ci.cpTri));
     }
-    if (y1 < distToPlane) {
-        f3 p = mk3(line1.y, y1, line1.x), on = mk3(line1.y, distToPlane, line1.x);
-        m.pts[n].p0 = add(pos1, mulmv(refToWorld, p));
-        m.pts[n].p1 = add(pos1, mulmv(refToWorld, on));
-        ++n;
-    }
-    if (!n) {
-        n = 1;
-        m.pts[0].p0 = add(pos1, mulmv(meshToWorld, ci.cpBody));
-        m.pts[0].p1 = add(pos1, mulmv(meshToWorld, ci.cpTri));
-    }
-    m.numPoints = n;
+    m.pts[0] = !k0 && k1 ? b : a;
+    m.pts[1] = b;
+    m.numPoints = k0 && k1 ? 2 : 1;
     return true;
 }
 
-__device__ void gen_box_tri_face(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf meshOr, const MeshCtx& mc,
-                                 const TCI& ci, Mf& m) {   // :398-467
-    m3 basis = mat3_cast(boxOr);
-    f3 tn = mc.n(ci.tri);
+__device__ __forceinline__ void swap_sides(Mf& m) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (i < m.numPoints) { const f3 t = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = t; }
+}
+
+__device__ __forceinline__ void clip_box_tri(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf meshOr, const MeshCtx& mc,
+                                             const TCI& ci, FaceClip& F, Mf& m) {   // :398-467
+    const m3 basis = mat3_cast(boxOr);
+    const f3 tn = mc.n(ci.tri);
     f3 refOrig, u1;
     m3 meshToRef;
-    f2 clip[3];
-    tri_frame(mc, ci.tri, true, refOrig, u1, meshToRef, clip);
+    tri_frame(mc, ci.tri, true, refOrig, u1, meshToRef, F.clip);
     int incAxis = 0;
     float incSign = 0.f;
     if (ci.boxFeature == BF_FACE) {
@@ -511,58 +508,49 @@ __device__ void gen_box_tri_face(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf mesh
             if (ad > maxDot) { maxDot = ad; incAxis = i; incSign = d > 0 ? -1.f : 1.f; }
         }
     }
-    int ia1 = (incAxis + 1) % 3, ia2 = (incAxis + 2) % 3;
-    f3 ui = col(basis, incAxis), ua = col(basis, ia1), ub = col(basis, ia2);
-    f3 incOrig = mulmv(meshToRef, add(boxPos, mul(mul(ui, at(he, incAxis)), incSign)));
-    f3 A = mul(ua, at(he, ia1)), B = mul(ub, at(he, ia2)), nA = mul(neg(ua), at(he, ia1));
-    f3 pp[4] = {add(incOrig, mulmv(meshToRef, add(A, B))), add(incOrig, mulmv(meshToRef, add(nA, B))),
-                add(incOrig, mulmv(meshToRef, sub(nA, B))), add(incOrig, mulmv(meshToRef, sub(A, B)))};
-    f2 poly[CVX_MAXPOLY];
-    for (int i = 0; i < 4; ++i) poly[i] = mk2(pp[i].z, pp[i].x);
-    int n = 4;
-    clip_polygon_n<CVX_MAXPOLY>(poly, n, clip, 3);
-    f3 incNormal = mulmv(meshToRef, ui);
-    m3 meshToWorld = mat3_cast(meshOr);
-    m3 refToWorld = mulmm(meshToWorld, transpose(meshToRef));
-    m3 negM = mk_m3(neg(meshToWorld.c0), neg(meshToWorld.c1), neg(meshToWorld.c2));
+    const int ia1 = (incAxis + 1) % 3, ia2 = (incAxis + 2) % 3, lane = wave_lane();
+    const f3 ui = col(basis, incAxis), ua = col(basis, ia1), ub = col(basis, ia2);
+    const f3 incOrig = mulmv(meshToRef, add(boxPos, mul(mul(ui, at(he, incAxis)), incSign)));
+    const f3 A = mul(ua, at(he, ia1)), B = mul(ub, at(he, ia2)), nA = mul(neg(ua), at(he, ia1));
+    // corners A + B, nA + B, nA - B, A - B
+    const f3 side = lane == 0 || lane == 3 ? A : nA;
+    const f3 pp = add(incOrig, mulmv(meshToRef, lane < 2 ? add(side, B) : sub(side, B)));
+    F.p = mk2(pp.z, pp.x);
+    F.n = 4;
+    F.nclip = 3;
+    F.incOrig = incOrig;
+    F.incNormal = mulmv(meshToRef, ui);
+    const m3 meshToWorld = mat3_cast(meshOr);
+    const m3 negM = mk_m3(neg(meshToWorld.c0), neg(meshToWorld.c1), neg(meshToWorld.c2));
     m.normal = mulmv(negM, tn);
-    polygon_polygon_face_contacts(meshPos, refToWorld, refOrig, u1, incOrig, incNormal, poly, n, 2, 0, m.pts,
-                                  m.numPoints);
-    for (int i = 0; i < m.numPoints; ++i) { f3 t = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = t; }
+    F.polygon_frame(meshPos, mulmm(meshToWorld, transpose(meshToRef)), refOrig, u1);
 }
 
-__device__ void gen_box_face_tri(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf meshOr, const MeshCtx& mc,
-                                 const TCI& ci, Mf& m) {   // :469-512
-    m3 basis = mat3_cast(boxOr);
-    m3 meshToBox = transpose(basis);
-    int refAxis = ci.boxAxis;
-    f3 tc = mc.c(ci.tri), tn = mc.n(ci.tri);
-    float refSign = dot(col(basis, refAxis), sub(tc, boxPos)) < 0 ? -1.f : 1.f;
-    int cx = (refAxis + 1) % 3, cy = (refAxis + 2) % 3;
-    int4 ix = mc.tri(ci.tri);
-    int iv[3] = {ix.x, ix.y, ix.z};
-    f2 poly[CVX_MAXPOLY];
-    for (int i = 0; i < 3; ++i) {
-        f3 v = mulmv(meshToBox, sub(mc.vert(iv[i]), boxPos));
-        poly[i] = mk2(at(v, cx), at(v, cy));
-    }
-    float hx = at(he, cx), hy = at(he, cy);
-    f2 clip[4] = {mk2(hx, hy), mk2(hx, -hy), mk2(-hx, -hy), mk2(-hx, hy)};
-    int n = 3;
-    clip_polygon_n<CVX_MAXPOLY>(poly, n, clip, 4);
-    f3 incOrig = mulmv(meshToBox, sub(tc, boxPos));
-    f3 incNormal = mulmv(meshToBox, tn);
-    m3 meshToWorld = mat3_cast(meshOr);
-    m.normal = mulmv(meshToWorld, mul(refSign, col(basis, refAxis)));
-    polygon_box_face_contacts_n<CVX_MAXPOLY>(boxPos, basis, refAxis, (int)refSign, he, incOrig, incNormal, poly, n,
-                                             cx, cy, m.pts, m.numPoints);
-    for (int i = 0; i < m.numPoints; ++i) {
-        m.pts[i].p0 = add(meshPos, mulmv(meshToWorld, m.pts[i].p0));
-        m.pts[i].p1 = add(meshPos, mulmv(meshToWorld, m.pts[i].p1));
-    }
+__device__ __forceinline__ void clip_tri_box(f3 boxPos, qf boxOr, f3 he, qf meshOr, const MeshCtx& mc, const TCI& ci,
+                                             FaceClip& F, Mf& m) {   // :469-512
+    const m3 basis = mat3_cast(boxOr);
+    const m3 meshToBox = transpose(basis);
+    const int refAxis = ci.boxAxis, lane = wave_lane();
+    const f3 tc = mc.c(ci.tri), tn = mc.n(ci.tri);
+    const float refSign = dot(col(basis, refAxis), sub(tc, boxPos)) < 0 ? -1.f : 1.f;
+    const int cx = (refAxis + 1) % 3, cy = (refAxis + 2) % 3;
+    const int4 ix = mc.tri(ci.tri);
+    const f3 v = mulmv(meshToBox, sub(mc.vert(lane == 0 ? ix.x : lane == 1 ? ix.y : ix.z), boxPos));
+    F.p = mk2(at(v, cx), at(v, cy));
+    F.n = 3;
+    F.clip = lane_rectangle(at(he, cx), at(he, cy));
+    F.nclip = 4;
+    F.incOrig = mulmv(meshToBox, sub(tc, boxPos));
+    F.incNormal = mulmv(meshToBox, tn);
+    m.normal = mulmv(mat3_cast(meshOr), mul(refSign, col(basis, refAxis)));
+    F.refPos = boxPos;
+    F.basis = basis;
+    F.he = he;
+    F.axis = refAxis;
+    F.axisSign = (int)refSign;
 }
 
-__device__ void gen_box_edge_tri_edge(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf meshOr, const MeshCtx& mc,
+__device__ __forceinline__ void gen_box_edge_tri_edge(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf meshOr, const MeshCtx& mc,
                                       const TCI& ci, Mf& m) {   // :514-542
     m3 basis = mat3_cast(boxOr);
     int boxAxis = ci.boxAxis;
@@ -587,88 +575,52 @@ __device__ void gen_box_edge_tri_edge(f3 boxPos, qf boxOr, f3 he, f3 meshPos, qf
     m.pts[0].p1 = add(meshPos, mulmv(meshToWorld, p1));
 }
 
-__device__ void gen_convex_tri_face(f3 cpos, qf cor, const MeshRef& cm, f3 scale, f3 meshPos, qf meshOr,
-                                    const MeshCtx& mc, const TCI& ci, Mf& m) {   // :699-757
-    f3 tn = mc.n(ci.tri);
+__device__ __forceinline__ void clip_convex_tri(f3 cpos, qf cor, const MeshRef& cm, f3 scale, f3 meshPos, qf meshOr,
+                                                const MeshCtx& mc, const TCI& ci, FaceClip& F, Mf& m) {   // :699-757
+    const f3 tn = mc.n(ci.tri);
     f3 refOrig, u1;
     m3 meshToRef;
-    f2 clip[3];
-    tri_frame(mc, ci.tri, false, refOrig, u1, meshToRef, clip);
-    int fi = 0;   // the reference leaves the index unset when no face has a negative dot
-    float minDot = 0.f;
-    for (int i = 0; i < cm.nfaces(); ++i) {
-        float d = dot(tn, normalize(qrot(cor, divv(cm.fnormal(i), scale))));
-        if (d < minDot) { minDot = d; fi = i; }
-    }
-    int2 F = cm.face(fi);
-    f2 poly[CVX_MAXPOLY];
-    int n = F.y < CVX_MAX_FACE_VERTS ? F.y : CVX_MAX_FACE_VERTS;
-    for (int i = 0; i < n; ++i) {
-        f3 v = mulmv(meshToRef, add(cpos, qrot(cor, mulv(scale, cm.face_vert(F, i)))));
-        poly[i] = mk2(v.z, v.x);
-    }
-    clip_polygon_n<CVX_MAXPOLY>(poly, n, clip, 3);
-    f3 incOrig = mulmv(meshToRef, add(cpos, qrot(cor, mulv(scale, cm.fcentroid(fi)))));
-    f3 incNormal = mulmv(meshToRef, qrot(cor, normalize(divv(cm.fnormal(fi), scale))));
-    m3 meshToWorld = mat3_cast(meshOr);
-    m3 refToWorld = mulmm(meshToWorld, transpose(meshToRef));
-    m3 negM = mk_m3(neg(meshToWorld.c0), neg(meshToWorld.c1), neg(meshToWorld.c2));
+    tri_frame(mc, ci.tri, false, refOrig, u1, meshToRef, F.clip);
+    F.nclip = 3;
+    // the reference leaves the index unset when no face has a negative dot: 0 here
+    const int fi = wave_face(cm.nfaces(), [&](int i) { return -dot(tn, normalize(qrot(cor, divv(cm.fnormal(i), scale)))); });
+    const int2 Fc = cm.face(fi);
+    F.n = Fc.y < CVX_MAX_FACE_VERTS ? Fc.y : CVX_MAX_FACE_VERTS;
+    const f3 v = mulmv(meshToRef, add(cpos, qrot(cor, mulv(scale, lane_face_vert(cm, Fc, F.n)))));
+    F.p = mk2(v.z, v.x);
+    F.incOrig = mulmv(meshToRef, add(cpos, qrot(cor, mulv(scale, cm.fcentroid(fi)))));
+    F.incNormal = mulmv(meshToRef, qrot(cor, normalize(divv(cm.fnormal(fi), scale))));
+    const m3 meshToWorld = mat3_cast(meshOr);
+    const m3 negM = mk_m3(neg(meshToWorld.c0), neg(meshToWorld.c1), neg(meshToWorld.c2));
     m.normal = mulmv(negM, tn);
-    polygon_polygon_face_contacts(meshPos, refToWorld, refOrig, u1, incOrig, incNormal, poly, n, 2, 0, m.pts,
-                                  m.numPoints);
-    for (int i = 0; i < m.numPoints; ++i) { f3 t = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = t; }
+    F.polygon_frame(meshPos, mulmm(meshToWorld, transpose(meshToRef)), refOrig, u1);
 }
 
-__device__ void gen_convex_face_tri(f3 cpos, qf cor, const MeshRef& cm, f3 scale, f3 meshPos, qf meshOr,
-                                    const MeshCtx& mc, const TCI& ci, Mf& m) {   // :759-824
-    m3 convexToMesh = mat3_cast(cor);
-    m3 meshToConvex = transpose(convexToMesh);
-    int fi = 0;   // unset in the reference when no face has a positive dot
-    float maxDot = 0.f;
-    for (int i = 0; i < cm.nfaces(); ++i) {
-        float d = dot(ci.normal, normalize(qrot(cor, divv(cm.fnormal(i), scale))));
-        if (d > maxDot) { maxDot = d; fi = i; }
-    }
-    int2 F = cm.face(fi);
-    f3 refOrig = mulv(scale, cm.fcentroid(fi));
-    f3 u0 = normalize(sub(mulv(scale, cm.face_vert(F, 0)), refOrig));
-    f3 u1 = normalize(divv(cm.fnormal(fi), scale));
-    f3 u2 = cross(u0, u1);
-    m3 convexToRef = transpose(mk_m3(u0, u1, u2));
-    m3 meshToRef = mulmm(convexToRef, meshToConvex);
-    f2 clip[CVX_MAX_FACE_VERTS];
-    int nc = F.y < CVX_MAX_FACE_VERTS ? F.y : CVX_MAX_FACE_VERTS;
-    for (int i = 0; i < nc; ++i) {
-        f3 v = mulmv(convexToRef, mulv(scale, cm.face_vert(F, i)));
-        clip[i] = mk2(v.z, v.x);
-    }
-    int4 ix = mc.tri(ci.tri);
-    int iv[3] = {ix.x, ix.y, ix.z};
-    f2 poly[CVX_MAXPOLY];
-    for (int i = 0; i < 3; ++i) {
-        f3 v = mulmv(meshToRef, sub(mc.vert(iv[i]), cpos));
-        poly[i] = mk2(v.z, v.x);
-    }
-    int n = 3;
-    clip_polygon_n<CVX_MAXPOLY>(poly, n, clip, nc);
-    f3 incOrig = mulmv(meshToRef, sub(mc.c(ci.tri), cpos));
-    f3 incNormal = mulmv(meshToRef, mc.n(ci.tri));
-    m3 meshToWorld = mat3_cast(meshOr);
-    m3 refToMesh = transpose(meshToRef);
-    polygon_polygon_face_contacts(cpos, refToMesh, refOrig, u1, incOrig, incNormal, poly, n, 2, 0, m.pts,
-                                  m.numPoints);
-    if (m.numPoints) {
-        for (int i = 0; i < m.numPoints; ++i) {
-            m.pts[i].p0 = add(meshPos, mulmv(meshToWorld, m.pts[i].p0));
-            m.pts[i].p1 = add(meshPos, mulmv(meshToWorld, m.pts[i].p1));
-        }
-        m.normal = mulmv(mulmm(meshToWorld, convexToMesh), u1);
-    } else {
-        m.normal = mulmv(meshToWorld, ci.normal);
-        m.numPoints = 1;
-        m.pts[0].p0 = add(meshPos, mulmv(meshToWorld, ci.cpBody));
-        m.pts[0].p1 = add(meshPos, mulmv(meshToWorld, ci.cpTri));
-    }
+__device__ __forceinline__ void clip_tri_convex(f3 cpos, qf cor, const MeshRef& cm, f3 scale, qf meshOr,
+                                                const MeshCtx& mc, const TCI& ci, FaceClip& F, Mf& m) {   // :759-824
+    const m3 convexToMesh = mat3_cast(cor);
+    const m3 meshToConvex = transpose(convexToMesh);
+    // unset in the reference when no face has a positive dot: 0 here
+    const int fi = wave_face(cm.nfaces(), [&](int i) { return dot(ci.normal, normalize(qrot(cor, divv(cm.fnormal(i), scale)))); });
+    const int2 Fc = cm.face(fi);
+    const f3 refOrig = mulv(scale, cm.fcentroid(fi));
+    const f3 u0 = normalize(sub(mulv(scale, cm.face_vert(Fc, 0)), refOrig));
+    const f3 u1 = normalize(divv(cm.fnormal(fi), scale));
+    const f3 u2 = cross(u0, u1);
+    const m3 convexToRef = transpose(mk_m3(u0, u1, u2));
+    const m3 meshToRef = mulmm(convexToRef, meshToConvex);
+    const int lane = wave_lane();
+    F.nclip = Fc.y < CVX_MAX_FACE_VERTS ? Fc.y : CVX_MAX_FACE_VERTS;
+    const f3 cv = mulmv(convexToRef, mulv(scale, lane_face_vert(cm, Fc, F.nclip)));
+    F.clip = mk2(cv.z, cv.x);
+    const int4 ix = mc.tri(ci.tri);
+    const f3 v = mulmv(meshToRef, sub(mc.vert(lane == 0 ? ix.x : lane == 1 ? ix.y : ix.z), cpos));
+    F.p = mk2(v.z, v.x);
+    F.n = 3;
+    F.incOrig = mulmv(meshToRef, sub(mc.c(ci.tri), cpos));
+    F.incNormal = mulmv(meshToRef, mc.n(ci.tri));
+    F.polygon_frame(cpos, transpose(meshToRef), refOrig, u1);
+    m.normal = mulmv(mulmm(mat3_cast(meshOr), convexToMesh), u1);   // when the clip leaves contacts
 }
 
 // ------------------------------------------------------------------ one (body, mesh) pair
@@ -678,20 +630,24 @@ struct MeshOut {
     int triBase;     // same block in npTri
     int n;
     bool flip;
-    __device__ void emit(Mf& m, int tri) {
+    __device__ __forceinline__ void emit(Mf& m, int tri) {   // the same manifold in every lane; lane 0 stores
         if (m.numPoints <= 0) return;                  // simulate skips empty manifolds (Physecs.cpp:233)
         if (flip) {
             m.normal = neg(m.normal);
-            for (int i = 0; i < m.numPoints; ++i) { f3 t = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = t; }
+            swap_sides(m);
         }
-        size_t q = (size_t)base + n;
-        npNum[q] = m.numPoints;
-        npNormal[q] = f4(m.normal, 0.f);
-        for (int k = 0; k < m.numPoints; ++k) {
-            npPts[8 * q + 2 * k] = f4(m.pts[k].p0, 0.f);
-            npPts[8 * q + 2 * k + 1] = f4(m.pts[k].p1, 0.f);
+        if (wave_lane() == 0) {
+            const size_t q = (size_t)base + n;
+            npNum[q] = m.numPoints;
+            npNormal[q] = f4(m.normal, 0.f);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k < m.numPoints) {
+                    npPts[8 * q + 2 * k] = f4(m.pts[k].p0, 0.f);
+                    npPts[8 * q + 2 * k + 1] = f4(m.pts[k].p1, 0.f);
+                }
+            npTri[triBase + n] = tri;
         }
-        npTri[triBase + n] = tri;
         ++n;
     }
 };
@@ -710,11 +666,19 @@ __device__ void mesh_local(int t, float4 g, f3 pos0, qf or0, f3 pos1, qf or1, co
 }
 
 // The body's bounds in the mesh frame (getBounds(localPos, localOr, geom0),
-// src/BoundsUtil.cpp:35-69) and the mesh's triangles whose BVH leaves they overlap, depth
-// first, left child first (overlapBvh, src/TriangleMesh.cpp:163-192). Returns the number
-// of candidates, -1 on a capacity error.
-__device__ int mesh_query(int t, float4 g, f3 localPos, qf localOr, const ConvexView& cv, const MeshCtx& mc,
-                          MeshWs& ws) {
+// src/BoundsUtil.cpp:35-69) and the mesh's triangles whose BVH leaves they overlap, in
+// S.cand in the order of overlapBvh's depth-first walk, left child first
+// (src/TriangleMesh.cpp:163-192). Returns the number of candidates, -1 on a capacity error.
+//
+// The build partitions the triangles in place, so the left subtree's come before the right's
+// and the walk's order is that of the triangle indices (inOrder: checked for every mesh at
+// creation): the wave then visits up to 64 nodes at once, in any order, and sorts what it
+// found. A mesh stored in another order is walked node by node. The node list cannot
+// overflow: within two wave widths of its end nodes are taken one by one, depth first, and
+// the tree is at most TM_STACK deep.
+__device__ __forceinline__ int mesh_query(int t, float4 g, f3 localPos, qf localOr, const ConvexView& cv,
+                                          const MeshCtx& mc, bool inOrder, QueryMem& S) {
+    const int lane = wave_lane();
     f3 mn, mx;
     if (t == PGX_SPHERE) {
         mn = sub(localPos, s3(g.x)); mx = add(localPos, s3(g.x));
@@ -725,126 +689,203 @@ __device__ int mesh_query(int t, float4 g, f3 localPos, qf localOr, const Convex
         m3 u = mat3_cast(localOr);
         f3 w = mulmv(mk_m3(vabs(u.c0), vabs(u.c1), vabs(u.c2)), mk3(g.x, g.y, g.z));
         mn = sub(localPos, w); mx = add(localPos, w);
-    } else {
-        int4 ci = cv.mesh[(int)g.w];
-        f3 scale = mk3(g.x, g.y, g.z);
+    } else {   // a vertex per lane; which of equal values is kept does not reach the comparisons
+        const int4 ci = cv.mesh[(int)g.w];
+        const f3 scale = mk3(g.x, g.y, g.z);
         mn = s3(3.402823466e+38f); mx = s3(-3.402823466e+38f);
-        int np = (ci.y + 3) & ~3;
-        for (int i = 0; i < np; ++i) {
+        const int np = (ci.y + 3) & ~3;
+        for (int i = lane; i < np; i += WAVE) {
             f3 p = add(localPos, qrot(localOr, mulv(scale, xyz(cv.verts[ci.x + i]))));
             mn = vmin(mn, p); mx = vmax(mx, p);
         }
+        mn = mk3(-wave_max(-mn.x), -wave_max(-mn.y), -wave_max(-mn.z));
+        mx = mk3(wave_max(mx.x), wave_max(mx.y), wave_max(mx.z));
     }
-    int stack[TM_STACK];
-    int sp = 0, nc = 0;
-    stack[sp++] = 0;
+    static_assert(TM_NODES >= 4 * WAVE + TM_STACK, "room for a wide step and a depth-first descent");
     const float4* nodes = mc.tv->nodes + 2 * (size_t)mc.mi.w;
+    const uint64_t lt = lanes_below();
+    int sp = 1, nc = 0;
+    if (lane == 0) S.nodes[0] = 0;
+    wave_sync();
     while (sp > 0) {
-        int id = stack[--sp];
-        float4 lo = nodes[2 * id], hi = nodes[2 * id + 1];
-        bool over = !(mx.x < lo.x || mn.x > hi.x) && !(mx.y < lo.y || mn.y > hi.y) && !(mx.z < lo.z || mn.z > hi.z);
-        if (!over) continue;
-        int triCount = __float_as_int(lo.w), index = __float_as_int(hi.w);
-        if (triCount) {
-            for (int i = 0; i < triCount; ++i) {
-                if (nc >= TM_MAXCAND) return -1;
-                ws.cand(nc++) = index + i;
-            }
-        } else {
-            if (sp + 2 > TM_STACK) return -1;
-            stack[sp++] = index + 1;
-            stack[sp++] = index;
+        const int take = inOrder && sp <= TM_NODES - 2 * WAVE - TM_STACK ? min(sp, WAVE) : 1;
+        sp -= take;
+        int triCount = 0, index = 0;
+        bool over = false;
+        if (lane < take) {
+            const int id = S.nodes[sp + lane];
+            const float4 lo = nodes[2 * id], hi = nodes[2 * id + 1];
+            over = !(mx.x < lo.x || mn.x > hi.x) && !(mx.y < lo.y || mn.y > hi.y) && !(mx.z < lo.z || mn.z > hi.z);
+            triCount = __float_as_int(lo.w);
+            index = __float_as_int(hi.w);
         }
+        wave_sync();   // the nodes are read before their places are filled again
+        const bool leaf = over && triCount > 0, inner = over && triCount == 0;
+        if (__ballot(leaf)) {
+            int total;
+            const int at = nc + wave_scan(leaf ? triCount : 0, total);
+            if (nc + total > TM_MAXCAND) return -1;
+            if (leaf)
+                for (int i = 0; i < triCount; ++i) S.cand[at + i] = index + i;
+            nc += total;
+        }
+        const uint64_t im = __ballot(inner);
+        if (inner) {
+            const int at = sp + 2 * (int)__popcll(im & lt);
+            S.nodes[at] = index + 1;
+            S.nodes[at + 1] = index;
+        }
+        sp += 2 * (int)__popcll(im);
+        wave_sync();
+    }
+    if (inOrder && nc > 1) {   // ascending: each candidate's rank (they are distinct)
+        int mine[TM_MAXCAND / WAVE], rank[TM_MAXCAND / WAVE];
+#pragma unroll
+        for (int k = 0; k < TM_MAXCAND / WAVE; ++k) {
+            rank[k] = 0;
+            mine[k] = k * WAVE + lane < nc ? S.cand[k * WAVE + lane] : 0;
+        }
+        for (int j = 0; j < nc; ++j) {
+            const int other = S.cand[j];
+#pragma unroll
+            for (int k = 0; k < TM_MAXCAND / WAVE; ++k)
+                if (k * WAVE < nc) rank[k] += other < mine[k] ? 1 : 0;
+        }
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < TM_MAXCAND / WAVE; ++k)
+            if (k * WAVE + lane < nc) S.cand[rank[k]] = mine[k];
+        wave_sync();
     }
     return nc;
 }
 
 // the per-shape test of one candidate triangle ti (src/CollisionTriangleMesh.cpp:886-903):
 // the shapes with a closed form
-__device__ bool mesh_test_closed(int t, float4 g, f3 localPos, qf localOr, const MeshCtx& mc, int ti, TCI& ci) {
-    int4 ix = mc.tri(ti);
-    f3 a = mc.vert(ix.x), b = mc.vert(ix.y), c = mc.vert(ix.z);
-    f3 n = mc.n(ti);
+__device__ __forceinline__ bool mesh_test_closed(int t, float4 g, f3 localPos, qf localOr, f3 a, f3 b, f3 c, f3 n,
+                                                 TCI& ci) {
     ci.featureIndex = 0; ci.boxFeature = 0; ci.boxAxis = 0;
-    ci.tri = ti;
     if (t == PGX_SPHERE) return sphere_tri(localPos, g.x, a, b, c, n, ci);
     if (t == PGX_CAPSULE) return capsule_tri(localPos, localOr, g.x, g.y, a, b, c, n, ci);
     return box_tri(localPos, localOr, mk3(g.x, g.y, g.z), a, b, c, n, ci);
 }
 
-// and all shapes, in one lane
-__device__ bool mesh_test(int t, float4 g, f3 localPos, qf localOr, const SupConvex& sc, const MeshCtx& mc, int ti,
-                          EpaWs& ews, TCI& ci, bool& epaErr) {
-    if (t != PGX_CONVEX_MESH) return mesh_test_closed(t, g, localPos, localOr, mc, ti, ci);
-    int4 ix = mc.tri(ti);
-    ci.featureIndex = 0; ci.boxFeature = 0; ci.boxAxis = 0;
-    ci.tri = ti;
-    const bool hit = convex_tri(sc, mc.vert(ix.x), mc.vert(ix.y), mc.vert(ix.z), mc.c(ti), ews, ci);
-    if (ews.overflow) epaErr = true;
-    return hit;
+__device__ __forceinline__ bool is_voided(const EmitMem& S, int nv, int v) {
+    bool found = false;
+    for (int i = wave_lane(); i < nv; i += WAVE) found = found || S.voided[i] == v;
+    return __ballot(found) != 0;
+}
+__device__ __forceinline__ void cover(EmitMem& S, int& nv, int4 ix) {
+    const int lane = wave_lane();
+    if (lane < 3) S.voided[nv + lane] = lane == 0 ? ix.x : lane == 1 ? ix.y : ix.z;
+    nv += 3;
+    wave_sync();
 }
 
-__device__ __forceinline__ bool is_voided(MeshWs& ws, int nv, int v) {
-    for (int i = 0; i < nv; ++i)
-        if (ws.voided(i) == v) return true;
-    return false;
-}
-
-// the emission passes (:906-953) over the nct contact records ws.order(0 .. nct-1) lists
-// in candidate order; out.emit(manifold, triangle) takes each manifold in order
-template <class Out>
-__device__ void mesh_emit(int t, float4 g, f3 localPos, qf localOr, f3 pos1, qf or1, const MeshCtx& mc,
-                          const ConvexView& cv, MeshWs& ws, const MeshRecs& recs, int nct, Out& out) {
-    f3 he = mk3(g.x, g.y, g.z);
+// the emission passes (:906-953) over the nct contact records S.order lists in candidate
+// order; out.emit(manifold, triangle) takes each manifold in order
+template <bool CONVEX, class Out>
+__device__ __forceinline__ void mesh_emit(int t, float4 g, f3 localPos, qf localOr, f3 pos1, qf or1, const MeshCtx& mc,
+                                          const ConvexView& cv, EmitMem& S, const MeshRecs& recs, size_t base, int nct,
+                                          Out& out) {
+    const f3 he = mk3(g.x, g.y, g.z);
     MeshRef cm{&cv, make_int4(0, 0, 0, 0)};
-    if (t == PGX_CONVEX_MESH) cm.info = cv.mesh[(int)g.w];
-    int nv = 0;
-    int n = nct;
-    // first pass: face contacts, last to first, swap-removed
-    for (int i = n - 1; i >= 0; i--) {
-        int c = ws.order(i);
-        if (recs.feature(c) != TF_FACE) continue;
-        TCI ci = recs.load(c);
-        int4 ix = mc.tri(ci.tri);
-        ws.voided(nv++) = ix.x; ws.voided(nv++) = ix.y; ws.voided(nv++) = ix.z;
-        Mf m;
-        m.numPoints = 0;
-        if (t == PGX_SPHERE) { gen_sphere(pos1, or1, ci, m); out.emit(m, ci.tri); }
-        else if (t == PGX_CAPSULE) { if (gen_capsule_face(localPos, localOr, g.x, g.y, pos1, or1, mc, ci, m)) out.emit(m, ci.tri); }
-        else if (t == PGX_BOX) { gen_box_tri_face(localPos, localOr, he, pos1, or1, mc, ci, m); out.emit(m, ci.tri); }
-        else { gen_convex_tri_face(localPos, localOr, cm, he, pos1, or1, mc, ci, m); out.emit(m, ci.tri); }
-        int last = ws.order(n - 1);
-        ws.order(n - 1) = ws.order(i);
-        ws.order(i) = last;
-        --n;
-    }
-    OrderArr arr{&ws, &recs};
-    introsort(arr, n);
-    for (int k = 0; k < n; ++k) {
-        int c = ws.order(k);
-        TCI ci = recs.load(c);
-        int4 ix = mc.tri(ci.tri);
-        int iv[3] = {ix.x, ix.y, ix.z};
-        Mf m;
-        m.numPoints = 0;
-        if (ci.feature == TF_EDGE) {
-            if (is_voided(ws, nv, iv[(ci.featureIndex + 1) % 3]) && is_voided(ws, nv, iv[(ci.featureIndex + 2) % 3]))
+    if (CONVEX && t == PGX_CONVEX_MESH) cm.info = cv.mesh[(int)g.w];
+    // the other kinds of contact, sorted, follow the face contacts: one loop, so that each
+    // generator is in the kernel once
+    int nv = 0, n = nct;
+    int i = n - 1, k = 0;
+    bool faces = true;
+    while (true) {
+        int c;
+        if (faces) {   // first pass: face contacts, last to first, swap-removed
+            while (i >= 0 && S.feature[S.order[i]] != TF_FACE) --i;
+            if (i < 0) {
+                faces = false;
+                OrderArr arr{S};
+                introsort(arr, n);
+                wave_sync();
                 continue;
-            if (t == PGX_SPHERE || t == PGX_CAPSULE) gen_sphere(pos1, or1, ci, m);
-            else if (t == PGX_BOX) {
-                if (ci.boxFeature == BF_FACE) gen_box_face_tri(localPos, localOr, he, pos1, or1, mc, ci, m);
-                else gen_box_edge_tri_edge(localPos, localOr, he, pos1, or1, mc, ci, m);
-            } else gen_convex_face_tri(localPos, localOr, cm, he, pos1, or1, mc, ci, m);
-            out.emit(m, ci.tri);
-        } else if (ci.feature == TF_VERTEX) {
-            if (is_voided(ws, nv, iv[ci.featureIndex])) continue;
-            if (t == PGX_SPHERE || t == PGX_CAPSULE) gen_sphere(pos1, or1, ci, m);
-            else if (t == PGX_BOX) gen_box_face_tri(localPos, localOr, he, pos1, or1, mc, ci, m);
-            else gen_convex_face_tri(localPos, localOr, cm, he, pos1, or1, mc, ci, m);
-            out.emit(m, ci.tri);
+            }
+            c = S.order[i];
+        } else {
+            if (k >= n) break;
+            c = S.order[k++];
         }
-        ws.voided(nv++) = ix.x; ws.voided(nv++) = ix.y; ws.voided(nv++) = ix.z;
+        const TCI ci = recs.load(base + c);
+        const int4 ix = mc.tri(ci.tri);
+        Mf m;
+        m.numPoints = 0;
+        bool emit = true;
+        const bool box = !CONVEX || t == PGX_BOX;
+        bool clipped = false;      // the contacts come from the face clip,
+        bool local = false;        // in the mesh's frame (a triangle clipped by the body's face)
+        FaceClip F;
+        if (faces) {
+            cover(S, nv, ix);
+            if (t == PGX_SPHERE) {
+                gen_sphere(pos1, or1, ci, m);
+            } else if (t == PGX_CAPSULE) {
+                emit = gen_capsule_face(localPos, localOr, g.x, g.y, pos1, or1, mc, ci, m);
+            } else {
+                clipped = true;
+                if (box) clip_box_tri(localPos, localOr, he, pos1, or1, mc, ci, F, m);
+                else clip_convex_tri(localPos, localOr, cm, he, pos1, or1, mc, ci, F, m);
+            }
+        } else {
+            // (a face contact swapped behind the end of the face pass is not here: n excludes it)
+            const int v = ci.featureIndex;
+            const int v0 = v == 0 ? ix.x : v == 1 ? ix.y : ix.z;
+            const int v1 = v == 0 ? ix.y : v == 1 ? ix.z : ix.x, v2 = v == 0 ? ix.z : v == 1 ? ix.x : ix.y;
+            if (ci.feature == TF_EDGE) {
+                if (is_voided(S, nv, v1) && is_voided(S, nv, v2)) continue;
+            } else if (is_voided(S, nv, v0)) {
+                continue;
+            }
+            if (t == PGX_SPHERE || t == PGX_CAPSULE) {
+                gen_sphere(pos1, or1, ci, m);
+            } else if (box && ci.feature == TF_EDGE && ci.boxFeature != BF_FACE) {
+                gen_box_edge_tri_edge(localPos, localOr, he, pos1, or1, mc, ci, m);
+            } else {
+                clipped = local = true;
+                if (box) clip_tri_box(localPos, localOr, he, or1, mc, ci, F, m);
+                else clip_tri_convex(localPos, localOr, cm, he, or1, mc, ci, F, m);
+            }
+        }
+        if (clipped) {
+            wave_contacts(F, S.P, m.pts, m.numPoints);
+            if (!local) {
+                swap_sides(m);
+            } else {
+                const m3 meshToWorld = mat3_cast(or1);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (j < m.numPoints) {
+                        m.pts[j].p0 = add(pos1, mulmv(meshToWorld, m.pts[j].p0));
+                        m.pts[j].p1 = add(pos1, mulmv(meshToWorld, m.pts[j].p1));
+                    }
+                if (!box && !m.numPoints) {
+                    m.normal = mulmv(meshToWorld, ci.normal);
+                    m.numPoints = 1;
+                    m.pts[0].p0 = add(pos1, mulmv(meshToWorld, ci.cpBody));
+                    m.pts[0].p1 = add(pos1, mulmv(meshToWorld, ci.cpTri));
+                }
+            }
+        }
+        if (emit) out.emit(m, ci.tri);
+        if (faces) {
+            const int last = S.order[n - 1];
+            wave_sync();
+            S.order[n - 1] = c;
+            S.order[i] = last;
+            wave_sync();
+            --n;
+            --i;
+        } else {
+            cover(S, nv, ix);
+        }
     }
+    wave_sync();   // the order is read before the wave's next pair overwrites it
 }
 
 }  // namespace pgx

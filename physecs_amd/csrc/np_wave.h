@@ -12,24 +12,27 @@
 // - the polytope is in LDS (14 KB per wave, 11 waves per CU): distances and visibility of 64
 //   faces at a time, new faces one per lane, the horizon's edges in registers;
 // - faces of a hull are searched, and polygon corners clipped, one per lane.
+// The same pairs then take 44 us and 134 us. What is left is the longest pair's chain: some
+// 1.3 us per insertion, of LDS reads, wave maxima and 64-bit distances that wait on each other.
 // What every lane needs (simplex, directions, normals) is computed by all lanes alike, so
 // control flow is the same in the whole wave; a kernel using this has blocks of one wave.
 //
 // The sequential loops' ties are kept: the first of equal values wins (in SupConvex the
 // lowest vertex of the lowest class i % 4), edges keep the list order of EpaPolytope, and
 // findClosestFace's float running minimum is reproduced from its final value (closest_face).
-// Included by narrowphase.hip after np_trimesh.h.
+// Included by narrowphase.hip after np_convex.h.
 #pragma once
 
 namespace pgx {
 
 // ------------------------------------------------------------------ wave primitives
 __device__ __forceinline__ int wave_lane() { return (int)threadIdx.x & (WAVE - 1); }
-// The wave's LDS stores before it are seen by its loads after it. Everything here is inlined
-// into its kernel: through a pointer that has lost its address space the same accesses would
-// be flat ones, which are not ordered with each other.
+// The wave's LDS stores before it are seen by its loads after it: a wave's LDS operations
+// are performed in order, so this only keeps the compiler from moving them. Everything here
+// is inlined into its kernel: through a pointer that has lost its address space the same
+// accesses would be flat ones, which are not ordered with each other.
 __device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
 __device__ __forceinline__ float lane_read(float x, int lane) {
@@ -38,20 +41,38 @@ __device__ __forceinline__ float lane_read(float x, int lane) {
 __device__ __forceinline__ f3 lane_read(f3 v, int lane) {
     return mk3(lane_read(v.x, lane), lane_read(v.y, lane), lane_read(v.z, lane));
 }
+// floats in the order of ints (-0 below 0), and back
+__device__ __forceinline__ int ordered(int bits) { return bits ^ ((bits >> 31) & 0x7fffffff); }
 template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_max(float x) {
-    const int i = __float_as_int(x);
-    return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false)));
+__device__ __forceinline__ int dpp_max(int x) {
+    return max(x, __builtin_amdgcn_update_dpp(-2147483647 - 1, x, CTRL, ROWS, 0xf, false));
 }
-// the largest of the lanes' values (a NaN counts as none), in every lane
-__device__ __forceinline__ float wave_max(float x) {
+// the largest of the lanes' values (none a NaN), in every lane; as ints, whose maximum takes
+// its lane move as an operand
+__device__ __forceinline__ float wave_max(float v) {
+    int x = ordered(__float_as_int(v));
     x = dpp_max<0x111, 0xf>(x);   // row_shr 1, 2, 4, 8: a row's maximum in its last lane
     x = dpp_max<0x112, 0xf>(x);
     x = dpp_max<0x114, 0xf>(x);
     x = dpp_max<0x118, 0xf>(x);
     x = dpp_max<0x142, 0xa>(x);   // row_bcast 15, then 31: the wave's in lane 63
     x = dpp_max<0x143, 0xc>(x);
-    return lane_read(x, WAVE - 1);
+    return __int_as_float(ordered(__builtin_amdgcn_readlane(x, WAVE - 1)));
+}
+// x with lane l's value replaced
+__device__ __forceinline__ int lane_write(int value, int l, int x) {
+    return (int)(threadIdx.x & (WAVE - 1)) == l ? value : x;
+}
+// exclusive prefix of n over the wave and the wave's total
+__device__ __forceinline__ int wave_scan(int n, int& total) {
+    const int lane = wave_lane();
+    int incl = n;
+    for (int o = 1; o < WAVE; o <<= 1) {
+        int t = __shfl_up(incl, o);
+        if (lane >= o) incl += t;
+    }
+    total = __shfl(incl, WAVE - 1);
+    return incl - n;
 }
 __device__ __forceinline__ uint64_t lanes_below() { return (1ull << wave_lane()) - 1ull; }
 __device__ __forceinline__ int first_lane(uint64_t mask) { return __ffsll((unsigned long long)mask) - 1; }
@@ -138,6 +159,9 @@ __device__ __forceinline__ GV pick(bool c, const GV& a, const GV& b) {
     r.sp1 = mk3(c ? a.sp1.x : b.sp1.x, c ? a.sp1.y : b.sp1.y, c ? a.sp1.z : b.sp1.z);
     return r;
 }
+__device__ __forceinline__ GV lane_read(const GV& g, int lane) {
+    return GV{lane_read(g.pos, lane), lane_read(g.sp0, lane), lane_read(g.sp1, lane)};
+}
 template <class S0, class S1>
 __device__ __forceinline__ GV mdiff_w(const S0& s0, const S1& s1, f3 dir) {
     GV r;
@@ -146,79 +170,130 @@ __device__ __forceinline__ GV mdiff_w(const S0& s0, const S1& s1, f3 dir) {
     r.pos = sub(r.sp0, r.sp1);
     return r;
 }
-template <class S0, class S1>
-__device__ __forceinline__ bool check_direction_w(const S0& s0, const S1& s1, d3 dir, GV& v) {
-    dir = dnormalize(dir);
-    v = mdiff_w(s0, s1, narrow(dir));
-    return ddot(wide(v.pos), dir) >= 0;
-}
-template <class S0, class S1>
-__device__ __forceinline__ void complete_from_line_w(const S0& s0, const S1& s1, const GV& a, const GV& b, GV& c,
-                                                     GV& d) {
-    const d3 ab = dsub(wide(a.pos), wide(b.pos));
-    d3 dir = dcross(ab, mkd(0, 1, 0));
-    if (is_zero(narrow(dir))) dir = dcross(ab, mkd(0, 0, 1));
-    c = mdiff_w(s0, s1, narrow(dnormalize(dir)));
-    if (sqr_dist_point_line(c.pos, a.pos, b.pos) < 0.00001f) c = mdiff_w(s0, s1, narrow(dneg(dir)));
-    dir = dnormalize(dcross(dsub(wide(b.pos), wide(a.pos)), dsub(wide(c.pos), wide(a.pos))));
-    d = mdiff_w(s0, s1, narrow(dir));
-    if (dist_point_plane(d.pos, a.pos, narrow(dir)) < 0.0001f) d = mdiff_w(s0, s1, narrow(dneg(dir)));
-}
-// gjk (np_convex.h) with the simplex in named vertices: no indexed access, no scratch
+// gjk (np_convex.h) with the simplex in named vertices (no indexed access, no scratch) and
+// its support queries answered at one place in the code: written out where the algorithm asks
+// them, they are eleven copies of both support maps, and as fast (both within 2 us of each
+// other on 2.4 k hull pairs).
 template <class S0, class S1>
 __device__ __forceinline__ bool gjk_w(const S0& s0, const S1& s1, f3 startDir, GV& a, GV& b, GV& c, GV& d) {
-    d3 dir = wide(normalize(startDir));
-    a = mdiff_w(s0, s1, narrow(dir));
-    if (is_zero(a.pos)) {
-        b = mdiff_w(s0, s1, narrow(dneg(dir)));
-        complete_from_line_w(s0, s1, a, b, c, d);
-        return true;
+    // what the answer is for
+    enum { FIRST, SECOND_ZERO, SECOND, THIRD, LINE_THIRD, LINE_THIRD_BACK, LAST, LAST_BACK, FOURTH, LOOP };
+    int ask = FIRST, fi = 0, rounds = 0;
+    d3 dir = wide(normalize(startDir)), plain = dir;   // plain: a direction before its normalisation
+    bool unit = true;                                  // dir is used as it is
+    while (true) {
+        if (!unit) dir = dnormalize(dir);
+        const GV v = mdiff_w(s0, s1, narrow(dir));
+        // checkDirection (src/GJK.h:162-167) of the queries that must pass the origin
+        if ((ask == SECOND || ask == THIRD || ask == FOURTH || ask == LOOP) && !(ddot(wide(v.pos), dir) >= 0)) return false;
+        unit = false;
+        bool line = false, last = false;               // go on with the third vertex of a line, with the last one
+        switch (ask) {
+            case FIRST:
+                a = v;
+                if (is_zero(a.pos)) {
+                    dir = dneg(dir);
+                    unit = true;
+                    ask = SECOND_ZERO;
+                } else {
+                    dir = dneg(wide(a.pos));
+                    ask = SECOND;
+                }
+                break;
+            case SECOND_ZERO:
+                b = v;
+                line = true;
+                break;
+            case SECOND: {
+                b = v;
+                const d3 ab = dsub(wide(a.pos), wide(b.pos));
+                dir = dcross(dcross(ab, dneg(wide(b.pos))), ab);
+                if (is_zero(narrow(dir))) line = true;
+                else ask = THIRD;
+                break;
+            }
+            case THIRD: {
+                c = v;
+                dir = dcross(dsub(wide(b.pos), wide(a.pos)), dsub(wide(c.pos), wide(a.pos)));
+                const double sg = dsign(ddot(dneg(wide(a.pos)), dir));
+                if (!sg) {
+                    ask = LAST;
+                } else {
+                    dir = dmul(sg, dir);
+                    ask = FOURTH;
+                }
+                break;
+            }
+            case LINE_THIRD:
+                c = v;
+                if (sqr_dist_point_line(c.pos, a.pos, b.pos) < 0.00001f) {
+                    dir = dneg(plain);
+                    unit = true;
+                    ask = LINE_THIRD_BACK;
+                } else {
+                    last = true;
+                }
+                break;
+            case LINE_THIRD_BACK:
+                c = v;
+                last = true;
+                break;
+            case LAST:
+                d = v;
+                if (!(dist_point_plane(d.pos, a.pos, narrow(dir)) < 0.0001f)) return true;
+                dir = dneg(dir);
+                unit = true;
+                ask = LAST_BACK;
+                break;
+            case LAST_BACK:
+                d = v;
+                return true;
+            case FOURTH:
+                d = v;
+                ask = LOOP;
+                break;
+            default: {   // the new vertex replaces vertex fi, then changes places with vertex 3
+                a = pick(fi == 0, d, a);
+                b = pick(fi == 1, d, b);
+                c = pick(fi == 2, d, c);
+                d = v;
+                break;
+            }
+        }
+        if (line) {   // complete_from_line, src/GJK.h:233-243
+            const d3 ab = dsub(wide(a.pos), wide(b.pos));
+            dir = dcross(ab, mkd(0, 1, 0));
+            if (is_zero(narrow(dir))) dir = dcross(ab, mkd(0, 0, 1));
+            plain = dir;
+            ask = LINE_THIRD;
+        } else if (last) {
+            dir = dcross(dsub(wide(b.pos), wide(a.pos)), dsub(wide(c.pos), wide(a.pos)));
+            ask = LAST;
+        } else if (ask == LOOP) {   // simplexContainsOrigin (src/GJK.h:175-181)
+            if (rounds++ == 100) return false;
+            const d3 pa = wide(a.pos), pb = wide(b.pos), pc = wide(c.pos), pd = wide(d.pos);
+            fi = 2;
+            bool outside = check_face(pd, pa, pb, pc, dir);
+            if (!outside) { fi = 1; outside = check_face(pd, pc, pa, pb, dir); }
+            if (!outside) { fi = 0; outside = check_face(pd, pb, pc, pa, dir); }
+            if (!outside) return true;
+        }
     }
-    if (!check_direction_w(s0, s1, dneg(wide(a.pos)), b)) return false;
-    const d3 ab = dsub(wide(a.pos), wide(b.pos));
-    dir = dcross(dcross(ab, dneg(wide(b.pos))), ab);
-    if (is_zero(narrow(dir))) {
-        complete_from_line_w(s0, s1, a, b, c, d);
-        return true;
-    }
-    if (!check_direction_w(s0, s1, dir, c)) return false;
-    dir = dcross(dsub(wide(b.pos), wide(a.pos)), dsub(wide(c.pos), wide(a.pos)));
-    const double sg = dsign(ddot(dneg(wide(a.pos)), dir));
-    if (!sg) {
-        dir = dnormalize(dir);
-        d = mdiff_w(s0, s1, narrow(dir));
-        if (dist_point_plane(d.pos, a.pos, narrow(dir)) < 0.0001f) d = mdiff_w(s0, s1, narrow(dneg(dir)));
-        return true;
-    }
-    if (!check_direction_w(s0, s1, dmul(sg, dir), d)) return false;
-    for (int i = 0; i < 100; ++i) {
-        const d3 pa = wide(a.pos), pb = wide(b.pos), pc = wide(c.pos), pd = wide(d.pos);
-        int fi = 2;
-        bool outside = check_face(pd, pa, pb, pc, dir);
-        if (!outside) { fi = 1; outside = check_face(pd, pc, pa, pb, dir); }
-        if (!outside) { fi = 0; outside = check_face(pd, pb, pc, pa, dir); }
-        if (!outside) return true;
-        GV v;
-        if (!check_direction_w(s0, s1, dir, v)) return false;
-        // the new vertex replaces vertex fi, then changes places with vertex 3
-        a = pick(fi == 0, d, a);
-        b = pick(fi == 1, d, b);
-        c = pick(fi == 2, d, c);
-        d = v;
-    }
-    return false;
 }
 
 // ------------------------------------------------------------------ EPA
-struct WaveMem {
-    double n[4][EPA_MAXF];        // per face: unit normal, and its distance (EPA.h:41-43)
-    float v[EPA_MAXV * 9];        // per vertex: pos, sp0, sp1
-    int fi[EPA_MAXF];             // per face: its vertices, a byte each
+// a clipped polygon's corners
+struct WavePoly {
     f2 poly[CVX_MAXPOLY];
     f3 pen[CVX_MAXPOLY];
 };
-constexpr int EPA_CHUNKS = EPA_MAXF / WAVE;
-static_assert(EPA_MAXF % WAVE == 0 && EPA_MAXV < 256 && EPA_MAXE == 2 * WAVE, "faces by wave, edges in two registers");
+// and EPA's polytope
+struct WaveMem : WavePoly {
+    double n[4][EPA_MAXF];        // per face: unit normal, and its distance (EPA.h:41-43)
+    float v[EPA_MAXV * 9];        // per vertex: pos, sp0, sp1
+    int fi[EPA_MAXF];             // per face: its vertices, a byte each
+};
+static_assert(EPA_MAXV < 256 && EPA_MAXE == 2 * WAVE, "a vertex in a byte, edges in two registers");
 
 __device__ __forceinline__ d3 mem_pos(const WaveMem& M, int i) {
     return mkd(M.v[9 * i], M.v[9 * i + 1], M.v[9 * i + 2]);
@@ -273,26 +348,19 @@ __device__ __forceinline__ f3 epa_w(const S0& s0, const S1& s1, const GV& a, con
         // rounded distance; a face of that rounded distance is taken when it is the first
         // (m was above) or when its distance itself is below m (rounding was upward): the
         // last of these, or else the first, is the one left. None when nothing is below inf.
-        double dist[EPA_CHUNKS];
         float low = __builtin_inff();
-#pragma unroll
-        for (int k = 0; k < EPA_CHUNKS; ++k) {
-            dist[k] = __builtin_inf();
-            if (k * WAVE < nf) {
-                const int f = k * WAVE + lane;
-                if (f < nf) dist[k] = M.n[3][f];
-                low = fminf(low, (float)dist[k]);
-            }
-        }
-        minDist = -wave_max(-low);
         int taken = -1, first = -1;
-#pragma unroll
-        for (int k = EPA_CHUNKS - 1; k >= 0; --k) {
-            if (k * WAVE >= nf) continue;
-            const uint64_t below = __ballot(dist[k] < (double)minDist);
-            if (below && taken < 0) taken = k * WAVE + last_lane(below);
-            const uint64_t same = __ballot(k * WAVE + lane < nf && (float)dist[k] == minDist);
-            if (same) first = k * WAVE + first_lane(same);
+        double dist = __builtin_inf();
+        if (lane < nf) dist = M.n[3][lane];
+        low = fminf(low, (float)dist);
+        for (int f = WAVE + lane; f < nf; f += WAVE) low = fminf(low, (float)M.n[3][f]);
+        minDist = -wave_max(-low);
+        for (int k = 0; k < nf; k += WAVE) {
+            if (k) dist = k + lane < nf ? M.n[3][k + lane] : __builtin_inf();
+            const uint64_t below = __ballot(dist < (double)minDist);
+            if (below) taken = k + last_lane(below);
+            const uint64_t same = __ballot(k + lane < nf && (float)dist == minDist);
+            if (same && first < 0) first = k + first_lane(same);
         }
         if (taken < 0 && minDist < __builtin_inff()) taken = first;
         if (taken >= 0) {
@@ -300,73 +368,91 @@ __device__ __forceinline__ f3 epa_w(const S0& s0, const S1& s1, const GV& a, con
             normal = mem_normal(M, taken);
         }
         const GV v = mdiff_w(s0, s1, narrow(normal));
-        if (ddot(wide(v.pos), normal) - (double)minDist < (double)0.00001f) break;
+        if (__ballot(ddot(wide(v.pos), normal) - (double)minDist < (double)0.00001f)) break;
         // insertVertex (:81-120)
         if (nv >= EPA_MAXV) { overflow = true; break; }
-        uint64_t seen[EPA_CHUNKS];
-        int fr[EPA_CHUNKS];
-#pragma unroll
-        for (int k = 0; k < EPA_CHUNKS; ++k) {
-            seen[k] = 0;
-            fr[k] = 0;
-            if (k * WAVE < nf) {
-                const int f = k * WAVE + lane;
-                bool see = false;
-                if (f < nf) {
-                    fr[k] = M.fi[f];
-                    see = ddot(mem_normal(M, f), dsub(wide(v.pos), mem_pos(M, fr[k] & 255))) > 0;
-                }
-                seen[k] = __ballot(see);
+        // the faces that see the vertex, from the last to the first; the last face fills each
+        // one's place (it comes later, so it has been looked at: the faces still to come are in
+        // their places). Up to 64 faces only note where each place's face comes from.
+        int ne = 0, e0 = -1, e1 = -1;   // edge k in lane k & 63 of e0 or e1: first | second << 8
+        const bool small = nf <= WAVE;
+        int source = lane;
+        for (int k = (nf - 1) & ~(WAVE - 1); k >= 0; k -= WAVE) {
+            bool see = false;
+            int ixs = 0;
+            if (k + lane < nf) {
+                ixs = M.fi[k + lane];
+                see = ddot(mem_normal(M, k + lane), dsub(wide(v.pos), mem_pos(M, ixs & 255))) > 0;
             }
-        }
-        // the seen faces from the last to the first; the last face fills each one's place (it
-        // comes later, so it has been looked at: the faces read here are still in their places)
-        int ne = 0, e0 = 0, e1 = 0;   // edge k in lane k & 63 of e0 or e1: first | second << 8
-#pragma unroll
-        for (int k = EPA_CHUNKS - 1; k >= 0; --k) {
-            while (seen[k]) {
-                const int l = last_lane(seen[k]);
-                seen[k] &= ~(1ull << l);
-                const int f = k * WAVE + l, ix = __builtin_amdgcn_readlane(fr[k], l);
+            for (uint64_t seen = __ballot(see); seen;) {
+                const int l = last_lane(seen);
+                seen &= ~(1ull << l);
+                const int f = k + l, ix = __builtin_amdgcn_readlane(ixs, l);
                 const int v0 = ix & 255, v1 = (ix >> 8) & 255, v2 = ix >> 16;
-                const int from[3] = {v0, v1, v2}, to[3] = {v1, v2, v0};
+                const int edge[3] = {v0 | (v1 << 8), v1 | (v2 << 8), v2 | (v0 << 8)};
+                const int back[3] = {v1 | (v0 << 8), v2 | (v1 << 8), v0 | (v2 << 8)};
                 bool found[3];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    const int want = to[j] | (from[j] << 8);
-                    const uint64_t hi = __ballot(lane + WAVE < ne && e1 == want), lo = __ballot(lane < ne && e0 == want);
-                    found[j] = (hi | lo) != 0;
-                    if (found[j]) {   // the last edge takes its place
-                        const int end = ne - 1 >= WAVE ? __builtin_amdgcn_readlane(e1, ne - 1 - WAVE)
-                                                       : __builtin_amdgcn_readlane(e0, ne - 1);
-                        if (hi) { if (lane == last_lane(hi)) e1 = end; }
-                        else { if (lane == last_lane(lo)) e0 = end; }
-                        --ne;
+                for (int j = 0; j < 3; ++j) {   // a found edge's place is taken by the last one
+                    const uint64_t lo = __ballot(e0 == back[j]);
+                    if (ne <= WAVE) {
+                        found[j] = lo != 0;
+                        if (lo) {
+                            --ne;
+                            e0 = lane_write(__builtin_amdgcn_readlane(e0, ne), last_lane(lo), e0);
+                            e0 = lane_write(-1, ne, e0);
+                        }
+                    } else {
+                        const uint64_t hi = __ballot(e1 == back[j]);
+                        found[j] = (hi | lo) != 0;
+                        if (hi | lo) {
+                            --ne;
+                            const int end = __builtin_amdgcn_readlane(e1, ne - WAVE);
+                            if (hi) e1 = lane_write(end, last_lane(hi), e1);
+                            else e0 = lane_write(end, last_lane(lo), e0);
+                            e1 = lane_write(-1, ne - WAVE, e1);
+                        }
                     }
                 }
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
-                    if (found[j] || overflow) continue;
-                    if (ne >= EPA_MAXE) { overflow = true; continue; }
-                    const int edge = from[j] | (to[j] << 8);
-                    if (lane + WAVE == ne) e1 = edge;
-                    else if (lane == ne) e0 = edge;
+                    if (found[j]) continue;
+                    if (ne >= EPA_MAXE) { overflow = true; break; }
+                    if (ne < WAVE) e0 = lane_write(edge[j], ne, e0);
+                    else e1 = lane_write(edge[j], ne - WAVE, e1);
                     ++ne;
                 }
                 --nf;
-                if (f != nf) {
+                if (f == nf) continue;
+                if (small) {
+                    source = lane_write(__builtin_amdgcn_readlane(source, nf), f, source);
+                } else {
                     if (lane < 4) M.n[lane][f] = M.n[lane][nf];
                     else if (lane == 4) M.fi[f] = M.fi[nf];
+                    wave_sync();
                 }
-                wave_sync();
+            }
+        }
+        if (small && __ballot(lane < nf && source != lane)) {
+            const bool moved = lane < nf && source != lane;
+            const d3 n = mem_normal(M, source);
+            const double dn = M.n[3][source];
+            const int ix = M.fi[source];
+            wave_sync();
+            if (moved) {
+                M.n[0][lane] = n.x; M.n[1][lane] = n.y; M.n[2][lane] = n.z;
+                M.n[3][lane] = dn;
+                M.fi[lane] = ix;
             }
         }
         const int vi = nv++;
         if (lane == 0) mem_put(M, vi, v);
         wave_sync();
         if (nf + ne > EPA_MAXF) { overflow = true; break; }
-        if (lane < ne) mem_face(M, nf + lane, vi, e0 & 255, e0 >> 8);
-        if (lane + WAVE < ne) mem_face(M, nf + WAVE + lane, vi, e1 & 255, e1 >> 8);
+        for (int k = lane; k < ne; k += WAVE) {
+            const int e = k < WAVE ? e0 : e1;
+            mem_face(M, nf + k, vi, e & 255, e >> 8);
+        }
         nf += ne;
         wave_sync();
     }
@@ -412,7 +498,7 @@ __device__ __forceinline__ int wave_face(int n, F value) {
 
 // clip_polygon_n<CVX_MAXPOLY> (np_convex.h) with corner `lane` of the polygon (n of them)
 // and of the clip polygon (nclip) in the lanes
-__device__ __forceinline__ void wave_clip(f2& p, int& n, f2 clip, int nclip, WaveMem& M) {
+__device__ __forceinline__ void wave_clip(f2& p, int& n, f2 clip, int nclip, WavePoly& M) {
     const int lane = wave_lane();
     const uint64_t lt = lanes_below();
     for (int e = 0; e < nclip; ++e) {
@@ -436,73 +522,69 @@ __device__ __forceinline__ void wave_clip(f2& p, int& n, f2 clip, int nclip, Wav
     }
 }
 
-// The penetrating corners of a clipped face (keep: this lane's corner p3 is one), in order,
-// and the up to four of them that become contacts (src/ContactsUtil.cpp:9-204):
-// put(slot, corner). cx, cy: the axes of the face's plane.
-template <class Put>
-__device__ __forceinline__ void wave_contacts(f3 p3, bool keep, int cx, int cy, WaveMem& M, int& numPoints, Put put) {
-    const int lane = wave_lane();
+// A face of one shape clipped against a face of the other: corner `lane` of the incident
+// polygon and of the clip polygon in the reference face's plane, and the frame that the
+// contacts are taken back from. polygon_box_face_contacts (src/ContactsUtil.cpp:9-107) takes
+// the plane of a box's axis; polygon_polygon_face_contacts (:109-204) is the same arithmetic
+// for axis y, sign 1, plane (z, x) and the face's distance in place of the half extent.
+struct FaceClip {
+    f2 p, clip;
+    int n, nclip;
+    f3 refPos, incOrig, incNormal, he;
+    m3 basis;
+    int axis, axisSign;
+    __device__ __forceinline__ void polygon_frame(f3 pos, const m3& refToWorld, f3 refOrig, f3 refNormal) {
+        refPos = pos;
+        basis = refToWorld;
+        he = s3(dot(refOrig, refNormal));
+        axis = 1;
+        axisSign = 1;
+    }
+};
+
+__device__ __forceinline__ void wave_contacts(FaceClip& F, WavePoly& M, CPt* cps, int& numPoints) {
+    wave_clip(F.p, F.n, F.clip, F.nclip, M);
+    const int axis = F.axis, cx = (axis + 1) % 3, cy = (axis + 2) % 3, lane = wave_lane();
+    const float lim = at(F.he, axis);
+    f3 dir = s3(0.f), p3 = s3(0.f);
+    set(dir, axis, (float)F.axisSign);
+    const float denom = dot(dir, F.incNormal);
+    set(p3, cx, F.p.x);
+    set(p3, cy, F.p.y);
+    const float distance = dot(sub(F.incOrig, p3), F.incNormal) / denom;
+    const bool keep = lane < F.n && distance < lim + 1e-4f;
+    set(p3, axis, F.axisSign * distance);
+    // the penetrating corners, in order
     const uint64_t mask = __ballot(keep);
     const int np = (int)__popcll(mask);
     if (keep) M.pen[__popcll(mask & lanes_below())] = p3;
     wave_sync();
     const f3 pen = lane < np ? M.pen[lane] : s3(0.f);
     wave_sync();
+    int pick0 = 0, pick1 = 1, pick2 = 2, pick3 = 3;   // the up to four that become contacts
+    numPoints = np;
     if (np > 4) {
-        const f3 p0 = lane_read(pen, 0);
-        put(0, p0);
-        const f3 d = sub(pen, p0);
-        const f3 far = lane_read(pen, wave_first_max(dot(d, d), lane < np));
-        put(1, far);
-        const f3 ca = sub(p0, pen), cb = sub(far, pen);
+        const f3 p0 = lane_read(pen, 0), d = sub(pen, p0);
+        pick1 = wave_first_max(dot(d, d), lane < np);
+        const f3 ca = sub(p0, pen), cb = sub(lane_read(pen, pick1), pen);
         const float area = det2(mk2(at(ca, cx), at(ca, cy)), mk2(at(cb, cx), at(cb, cy)));
-        put(2, lane_read(pen, wave_first_max(area, lane < np)));
-        put(3, lane_read(pen, wave_first_max(-area, lane < np)));
+        pick2 = wave_first_max(area, lane < np);
+        pick3 = wave_first_max(-area, lane < np);
         numPoints = 4;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (i < np) put(i, lane_read(pen, i));
-        numPoints = np;
     }
-}
-
-// polygon_polygon_face_contacts (np_convex.h), corner `lane` of the clipped polygon
-__device__ __forceinline__ void wave_polygon_contacts(f3 refPos, const m3& refToWorld, f3 refOrig, f3 refNormal,
-                                                      f3 incOrig, f3 incNormal, f2 p, int n, WaveMem& M, CPt* cps,
-                                                      int& numPoints) {
-    const float distRef = dot(refOrig, refNormal);
-    const f3 dir = mk3(0.f, 1.f, 0.f);
-    f3 p3 = mk3(p.y, 0.f, p.x);
-    const float distance = dot(sub(incOrig, p3), incNormal) / dot(dir, incNormal);
-    const bool keep = wave_lane() < n && distance < distRef + 1e-4f;
-    p3.y = distance;
-    wave_contacts(p3, keep, 2, 0, M, numPoints, [&](int slot, f3 c) {
-        f3 on = c;
-        on.y = distRef;
-        cps[slot].p0 = add(refPos, mulmv(refToWorld, on));
-        cps[slot].p1 = add(refPos, mulmv(refToWorld, c));
-    });
-}
-
-// polygon_box_face_contacts_n (narrowphase.hip), corner `lane` of the clipped polygon
-__device__ __forceinline__ void wave_box_contacts(f3 boxCenter, const m3& basis, int axis, int axisSign, f3 he,
-                                                  f3 incOrig, f3 incNormal, f2 p, int n, int cx, int cy, WaveMem& M,
-                                                  CPt* cps, int& numPoints) {
-    f3 dir = s3(0.f), p3 = s3(0.f);
-    set(dir, axis, (float)axisSign);
-    const float denom = dot(dir, incNormal);
-    set(p3, cx, p.x);
-    set(p3, cy, p.y);
-    const float distance = dot(sub(incOrig, p3), incNormal) / denom;
-    const bool keep = wave_lane() < n && distance < at(he, axis) + 1e-4f;
-    set(p3, axis, axisSign * distance);
-    wave_contacts(p3, keep, cx, cy, M, numPoints, [&](int slot, f3 c) {
-        f3 on = c;
-        set(on, axis, axisSign * at(he, axis));
-        cps[slot].p0 = add(boxCenter, mulmv(basis, on));
-        cps[slot].p1 = add(boxCenter, mulmv(basis, c));
-    });
+    // contact `lane` in lanes 0-3, then in every lane
+    const f3 c = mk3(__shfl(pen.x, lane == 0 ? pick0 : lane == 1 ? pick1 : lane == 2 ? pick2 : pick3),
+                     __shfl(pen.y, lane == 0 ? pick0 : lane == 1 ? pick1 : lane == 2 ? pick2 : pick3),
+                     __shfl(pen.z, lane == 0 ? pick0 : lane == 1 ? pick1 : lane == 2 ? pick2 : pick3));
+    f3 on = c;
+    set(on, axis, F.axisSign * lim);
+    const f3 a = add(F.refPos, mulmv(F.basis, on)), b = add(F.refPos, mulmv(F.basis, c));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (i < numPoints) {
+            cps[i].p0 = lane_read(a, i);
+            cps[i].p1 = lane_read(b, i);
+        }
 }
 
 // vertex `lane` of a face (face vertices beyond the face's count are not read)
@@ -511,8 +593,8 @@ __device__ __forceinline__ f3 lane_face_vert(const MeshRef& m, int2 F, int n) {
 }
 
 // convex_convex_contacts, src/Collision.cpp:352-410
-__device__ __forceinline__ void convex_convex_contacts_w(f3 pos0, qf or0, const MeshRef& m0, f3 s0, f3 pos1, qf or1, const MeshRef& m1,
-                                         f3 s1, f3 normal, WaveMem& M, CPt* cps, int& numPoints) {
+__device__ __forceinline__ void convex_convex_clip(f3 pos0, qf or0, const MeshRef& m0, f3 s0, f3 pos1, qf or1,
+                                                   const MeshRef& m1, f3 s1, f3 normal, FaceClip& F) {
     const int f0 = wave_face(m0.nfaces(), [&](int i) { return dot(normal, world_face_normal(or0, m0.fnormal(i), s0)); });
     const int f1 = wave_face(m1.nfaces(), [&](int i) { return -dot(normal, world_face_normal(or1, m1.fnormal(i), s1)); });
     const int2 F0 = m0.face(f0), F1 = m1.face(f1);
@@ -523,15 +605,15 @@ __device__ __forceinline__ void convex_convex_contacts_w(f3 pos0, qf or0, const 
     const f3 u2 = cross(u0, u1);
     const m3 c0ToRef = transpose(mk_m3(u0, u1, u2));
     const m3 worldToRef = mulmm(c0ToRef, worldToC0);
-    const int nc = F0.y < 16 ? F0.y : 16;
-    int n = F1.y < 16 ? F1.y : 16;
-    const f3 cv = mulmv(c0ToRef, mulv(s0, lane_face_vert(m0, F0, nc)));
-    const f3 pv = mulmv(worldToRef, sub(add(pos1, qrot(or1, mulv(s1, lane_face_vert(m1, F1, n)))), pos0));
-    f2 p = mk2(pv.z, pv.x);
-    wave_clip(p, n, mk2(cv.z, cv.x), nc, M);
-    const f3 incOrig = mulmv(worldToRef, sub(add(pos1, qrot(or1, mulv(s1, m1.fcentroid(f1)))), pos0));
-    const f3 incNormal = mulmv(worldToRef, qrot(or1, normalize(divv(m1.fnormal(f1), s1))));
-    wave_polygon_contacts(pos0, transpose(worldToRef), refOrig, u1, incOrig, incNormal, p, n, M, cps, numPoints);
+    F.nclip = F0.y < 16 ? F0.y : 16;
+    F.n = F1.y < 16 ? F1.y : 16;
+    const f3 cv = mulmv(c0ToRef, mulv(s0, lane_face_vert(m0, F0, F.nclip)));
+    const f3 pv = mulmv(worldToRef, sub(add(pos1, qrot(or1, mulv(s1, lane_face_vert(m1, F1, F.n)))), pos0));
+    F.p = mk2(pv.z, pv.x);
+    F.clip = mk2(cv.z, cv.x);
+    F.incOrig = mulmv(worldToRef, sub(add(pos1, qrot(or1, mulv(s1, m1.fcentroid(f1)))), pos0));
+    F.incNormal = mulmv(worldToRef, qrot(or1, normalize(divv(m1.fnormal(f1), s1))));
+    F.polygon_frame(pos0, transpose(worldToRef), refOrig, u1);
 }
 
 // capsule_convex_contacts, src/Collision.cpp:694-785
@@ -588,9 +670,15 @@ __device__ __forceinline__ void capsule_convex_contacts_w(f3 p0L, f3 p1L, float 
     res.numPoints = (k0 ? 1 : 0) + (k1 ? 1 : 0);
 }
 
+// the clip rectangle (hx, hy), (hx, -hy), (-hx, -hy), (-hx, hy) of a box's face
+__device__ __forceinline__ f2 lane_rectangle(float hx, float hy) {
+    const int lane = wave_lane();
+    return mk2(lane < 2 ? hx : -hx, lane == 0 || lane == 3 ? hy : -hy);
+}
+
 // box_convex_contacts, src/Collision.cpp:808-871
-__device__ __forceinline__ void box_convex_contacts_w(f3 boxCenter, const m3& basis, f3 he, f3 cpos, qf cor, const MeshRef& m, f3 scale,
-                                      f3 normal, WaveMem& M, CPt* cps, int& numPoints) {
+__device__ __forceinline__ void box_convex_clip(f3 boxCenter, const m3& basis, f3 he, f3 cpos, qf cor, const MeshRef& m,
+                                                f3 scale, f3 normal, FaceClip& F) {
     int boxAxis = 0;
     float boxAxisSign = 0.f, maxDot = 0.f;
     for (int i = 0; i < 3; ++i) {
@@ -599,19 +687,21 @@ __device__ __forceinline__ void box_convex_contacts_w(f3 boxCenter, const m3& ba
         if (ad > maxDot) { maxDot = ad; boxAxis = i; boxAxisSign = d < 0 ? -1.f : 1.f; }
     }
     const int fi = wave_face(m.nfaces(), [&](int i) { return -dot(normal, world_face_normal(cor, m.fnormal(i), scale)); });
-    const int2 F = m.face(fi);
-    const int cx = (boxAxis + 1) % 3, cy = (boxAxis + 2) % 3, lane = wave_lane();
+    const int2 Fc = m.face(fi);
+    const int cx = (boxAxis + 1) % 3, cy = (boxAxis + 2) % 3;
     const m3 worldToBox = transpose(basis);
-    int n = F.y < 16 ? F.y : 16;
-    const f3 v = mulmv(worldToBox, sub(add(cpos, qrot(cor, mulv(scale, lane_face_vert(m, F, n)))), boxCenter));
-    f2 p = mk2(at(v, cx), at(v, cy));
-    const float hx = at(he, cx), hy = at(he, cy);
-    const f2 clip = mk2(lane < 2 ? hx : -hx, lane == 0 || lane == 3 ? hy : -hy);   // (+,+), (+,-), (-,-), (-,+)
-    wave_clip(p, n, clip, 4, M);
-    const f3 incOrig = mulmv(worldToBox, sub(add(cpos, qrot(cor, mulv(scale, m.fcentroid(fi)))), boxCenter));
-    const f3 incNormal = normalize(mulmv(worldToBox, qrot(cor, divv(m.fnormal(fi), scale))));
-    wave_box_contacts(boxCenter, basis, boxAxis, (int)boxAxisSign, he, incOrig, incNormal, p, n, cx, cy, M, cps,
-                      numPoints);
+    F.n = Fc.y < 16 ? Fc.y : 16;
+    const f3 v = mulmv(worldToBox, sub(add(cpos, qrot(cor, mulv(scale, lane_face_vert(m, Fc, F.n)))), boxCenter));
+    F.p = mk2(at(v, cx), at(v, cy));
+    F.clip = lane_rectangle(at(he, cx), at(he, cy));
+    F.nclip = 4;
+    F.incOrig = mulmv(worldToBox, sub(add(cpos, qrot(cor, mulv(scale, m.fcentroid(fi)))), boxCenter));
+    F.incNormal = normalize(mulmv(worldToBox, qrot(cor, divv(m.fnormal(fi), scale))));
+    F.refPos = boxCenter;
+    F.basis = basis;
+    F.he = he;
+    F.axis = boxAxis;
+    F.axisSign = (int)boxAxisSign;
 }
 
 // one pair with a convex mesh on either side (src/Collision.cpp:895-1016); flips as the
@@ -650,10 +740,18 @@ __device__ __forceinline__ bool collide_convex_w(int t0, float4 g0, f3 p0, qf q0
             const f3 axisLc = mulmv(w2c, axis);
             capsule_convex_contacts_w(add(p, mul(axisLc, g0.x)), sub(p, mul(axisLc, g0.x)), g0.y, p1, b.l2w, m1, b.scale,
                                       m);
-        } else if (t0 == PGX_BOX) {                          // src/Collision.cpp:873-887
-            box_convex_contacts_w(p0, a.hull.l2w, a.g, p1, q1, m1, b.scale, m.normal, M, m.pts, m.numPoints);
-        } else {                                             // src/Collision.cpp:412-426
-            convex_convex_contacts_w(p0, q0, m0, a.hull.scale, p1, q1, m1, b.scale, m.normal, M, m.pts, m.numPoints);
+        } else {                                             // src/Collision.cpp:412-426,873-887
+            FaceClip F;
+            if (t0 == PGX_BOX) box_convex_clip(p0, a.hull.l2w, a.g, p1, q1, m1, b.scale, m.normal, F);
+            else convex_convex_clip(p0, q0, m0, a.hull.scale, p1, q1, m1, b.scale, m.normal, F);
+            int n;
+            CPt pts[4];
+            wave_contacts(F, M, pts, n);
+            if (n) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) m.pts[i] = pts[i];
+                m.numPoints = n;
+            }
         }
         if (!m.numPoints) m.numPoints = 1;                   // the points of EPA
     }
@@ -664,21 +762,6 @@ __device__ __forceinline__ bool collide_convex_w(int t0, float4 g0, f3 p0, qf q0
             if (i < m.numPoints) { const f3 t = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = t; }
     }
     return hit;
-}
-
-// the test of a convex body against one triangle (convex_tri, np_trimesh.h)
-__device__ __forceinline__ bool mesh_test_convex_w(const SupConvex& sc, const MeshCtx& mc, int ti, WaveMem& M, TCI& ci, bool& overflow) {
-    const int4 ix = mc.tri(ti);
-    const f3 a = mc.vert(ix.x), b = mc.vert(ix.y), c = mc.vert(ix.z);
-    ci.featureIndex = 0; ci.boxFeature = 0; ci.boxAxis = 0;
-    ci.tri = ti;
-    const SupHull hull = hull_of(sc);
-    const SupTriangle st{a, b, c};
-    GV va, vb, vc, vd;
-    if (!gjk_w(hull, st, sub(mc.c(ti), hull.pos), va, vb, vc, vd)) return false;
-    ci.normal = epa_w(hull, st, va, vb, vc, vd, M, ci.cpBody, ci.cpTri, overflow);
-    convex_tri_feature(a, b, c, ci);
-    return true;
 }
 
 }  // namespace pgx

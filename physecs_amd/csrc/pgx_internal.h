@@ -111,12 +111,10 @@ constexpr int EPA_MAXV = 104;          // 4 simplex vertices + at most 100 inser
 constexpr int EPA_MAXF = 256;          // > 2 * EPA_MAXV - 4, the face count of a closed triangulation
 constexpr int EPA_MAXE = 128;          // horizon (loose) edges of one insertion
 constexpr int CVX_MAX_FACE_VERTS = 16;
-// triangle-mesh narrowphase: per-lane capacities and lanes
+// triangle-mesh narrowphase
 constexpr int TM_MAXCAND = 256;        // triangles overlapping one body's local bounds
-constexpr int TM_STACK = 64;           // BVH traversal stack (the build's depth is checked)
-constexpr int TM_CI_WORDS = 14;        // one triangle contact record (+ 1 word: the test hit)
-constexpr int TM_WS_WORDS = TM_MAXCAND * (2 + 3);   // per lane: candidates, order, covered vertices
-constexpr int TM_LANES = 16384;
+constexpr int TM_STACK = 64;           // depth of a BVH, checked at creation
+constexpr int TM_CI_WORDS = 14;        // one triangle contact record
 inline int div_up(long a, long b) { return (int)((a + b - 1) / b); }
 
 // ------------------------------------------------------------------ utilities (util.hip)
@@ -155,6 +153,15 @@ void fill_u64(hipStream_t s, uint64_t* p, uint64_t v, int n);
 // Collider flag bits
 enum { CF_ENABLE = 1, CF_TRIGGER = 2, CF_DYNAMIC = 4 };
 constexpr int LEAF_BIT = 0x40000000;
+
+// The triangle-mesh passes' buffers: candidates (triangle, pair), contact records
+// (TM_CI_WORDS and the hit each), each pair's block of candidates; the triangles that a
+// convex mesh's GJK hit, with its simplex.
+struct MeshBuffers {
+    int candCap = 0;
+    DBuf<int32_t> cand, pairOf, recs, candOff, candCount, hitList;
+    DBuf<float> simplex;
+};
 
 struct World {
     int device = 0;
@@ -231,7 +238,7 @@ struct World {
     DBuf<int32_t> worldRoot, worldStop;
     DBuf<uint64_t> pkeys;
     DBuf<int32_t> pvals;
-    DBuf<int32_t> counters;              // [0] pairs, [1] manifolds, [3] uncolored, [5] colour overflow, [6] bvh error, [7] refit ready
+    DBuf<int32_t> counters;              // [0] pairs, [1] manifolds, [2] triangles GJK hit, [3] uncolored, [5] colour overflow, [6] bvh error, [7] refit ready
     SortTemp sortT;
     ScanTemp scanT;
 
@@ -291,8 +298,6 @@ struct World {
     DBuf<int2> cvFace;
     DBuf<int32_t> cvFaceIdx;
     DBuf<int32_t> heavy;               // pairs with a convex mesh (filled by the primitive kernel)
-    DBuf<double> epaV, epaFN;          // the triangle-mesh MTD queries' polytopes, a lane each
-    DBuf<int32_t> epaFI, epaE;
     // static triangle meshes: vertices, triangles in the BVH build's order (mesh-local
     // vertex indices), triangle normals / centroids, BVH nodes (2 float4 each: {min,
     // triCount bits}, {max, index bits}), {first vertex, vertices, first triangle, first node}
@@ -301,12 +306,8 @@ struct World {
     DBuf<int4> tmMesh;
     DBuf<int4> tmTris;
     DBuf<int32_t> meshPairs;           // pairs with a triangle mesh (filled by the primitive kernel)
-    int meshLanes = 0;                 // lanes of the mesh kernel
-    DBuf<int32_t> tmWs;                // per-lane candidates, order, voided vertices
-    int tmCandCap = 0;                 // candidate triangles per step (all mesh pairs)
-    DBuf<int32_t> tmCand, tmPairOf;    // per candidate: triangle, mesh pair
-    DBuf<int32_t> tmRecs;              // per candidate: contact record (TM_CI_WORDS + hit)
-    DBuf<int32_t> tmCandOff, tmCandCount;   // per mesh pair: its candidates
+    bool tmInOrder = true;             // every mesh's BVH walk meets its triangles in index order
+    MeshBuffers stepMesh, qMesh;       // the mesh passes' buffers, the step's and the MTD queries'
     int mmCap = 0;                     // manifolds of mesh pairs, stored after the pair slots
     int lastMeshSlots = 0;
     DBuf<int32_t> npTri, meshFirst, meshCount;
@@ -393,7 +394,6 @@ struct World {
     DBuf<int32_t> qMtdN;
     DBuf<float4> qRes;
     DBuf<int2> qCvxPairs, qMeshPairs;
-    DBuf<int32_t> qRecs;                 // MTD triangle-mesh pairs: TM_MAXCAND contact records per lane
     std::vector<int32_t> worldListHost[2];   // worlds of at most WORLD_SMALL dynamic bodies, and the rest
     DBuf<int32_t> worldList[2];
     bool worldsContiguous = false;
@@ -482,15 +482,16 @@ struct OverlapArgs {
 
 // what the MTD overlap query kernels read and write
 struct MtdArgs {
-    int n, nLeaves, cap, cbits, listCap, recLanes;
-    int32_t* recs;        // the triangle-mesh pass's contact records, TM_MAXCAND per lane
+    int n, nLeaves, cap, cbits, listCap;
     const float4 *qPrm, *qPos, *qQuat;      // per query: params (.w mesh), position (.w world bits), orientation
     const int32_t* qType;
     const int32_t *worldRoot, *worldStop, *worldStaticStart, *staticCols, *mvals;
     const float4 *leafA, *nodeA, *nodeB;
     const float4 *cbmin, *cbmax, *cparams, *clpos, *clquat, *bpos, *bquat;
     const int32_t *cbody, *ctype;
-    int32_t* counts;      // [0] results, [1] convex pairs, [2] mesh pairs, [3] errors (device, zero before)
+    // [0] results, [1] convex pairs, [2] mesh pairs, [3] errors, [4] candidate triangles,
+    // [5] those that a convex shape's GJK hit (device, zero before)
+    int32_t* counts;
     uint64_t* keys;       // (query, collider, manifold) keys of the first `cap` results
     int32_t* vals;        // their result index (the sort's payload)
     float4* res;          // normal xyz, mtd
@@ -500,6 +501,7 @@ struct MtdArgs {
 
 // narrowphase.hip
 void np_run(World& w, int nPairs);
+void np_mesh_buffers(World& w, MeshBuffers& b, size_t pairs, size_t cands);
 // the MTD query's passes: the walk (primitive pairs solved, the others listed), the convex
 // pairs, the triangle-mesh pairs
 void np_mtd_launch(World& w, const MtdArgs& A);

@@ -265,6 +265,7 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
                    const float* orientations, const int32_t* queryWorld, int capacity, int32_t* offsets,
                    int32_t* colliders, float* normalMtd, int32_t* total, double* deviceUs) {
     constexpr int MBITS = 8;   // manifold index within a pair (the kernels' MTD_MBITS)
+    constexpr int MTD_COUNTS = 6;
     hipStream_t s = w.stream;
     int cbits = 1;
     while ((1L << cbits) < (long)w.C) ++cbits;
@@ -272,26 +273,12 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
     while ((1L << qbits) < (long)n) ++qbits;
     if (qbits + cbits + MBITS > 64) throw PgxError{PGX_ERR_UNSUPPORTED, "too many queries and colliders for one call"};
     upload_query_shapes(w, n, types, params, positions, orientations, queryWorld);
-    w.qMtdN.alloc(4);
+    w.qMtdN.alloc(MTD_COUNTS);
     w.qKeys.alloc(std::max(capacity, 1)); w.qVals.alloc(std::max(capacity, 1)); w.qRes.alloc(std::max(capacity, 1));
     if (!w.qEv[0])
         for (auto& e : w.qEv) PGX_HIP(hipEventCreate(&e));
     MtdArgs A;
     A.n = n; A.nLeaves = w.nDynCol; A.cap = capacity; A.cbits = cbits;
-    // triangle-mesh pairs: one lane each, with TM_MAXCAND contact records of its own
-    // (a buffer of the query's own, allocated on first use: 8192 lanes, 126 MB)
-    A.recLanes = 1;
-    A.recs = nullptr;
-    if (w.nTriMesh > 0) {
-        A.recLanes = std::max(1, std::min(w.meshLanes, 8192));
-        w.qRecs.alloc((size_t)(TM_CI_WORDS + 1) * TM_MAXCAND * A.recLanes);
-        if (w.nConvex > 0) {   // convex query shapes against triangles: a polytope per lane
-            const size_t L = (size_t)A.recLanes;
-            w.epaV.alloc(9 * EPA_MAXV * L); w.epaFN.alloc(3 * EPA_MAXF * L);
-            w.epaFI.alloc(3 * EPA_MAXF * L); w.epaE.alloc(2 * EPA_MAXE * L);
-        }
-        A.recs = w.qRecs.p;
-    }
     A.qPrm = w.qShape.p; A.qPos = w.qShape.p + n; A.qQuat = w.qShape.p + 2 * (size_t)n; A.qType = w.qType.p;
     A.worldRoot = w.worldRoot.p; A.worldStop = w.worldStop.p;
     A.worldStaticStart = w.worldStaticStart.p; A.staticCols = w.staticCols.p; A.mvals = w.mvals.p;
@@ -299,14 +286,17 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
     A.cbmin = w.cbmin.p; A.cbmax = w.cbmax.p; A.cparams = w.cparams.p; A.clpos = w.clpos.p; A.clquat = w.clquat.p;
     A.bpos = w.bpos.p; A.bquat = w.bquat.p; A.cbody = w.cbody.p; A.ctype = w.ctype.p;
     A.counts = w.qMtdN.p; A.keys = w.qKeys.p; A.vals = w.qVals.p; A.res = w.qRes.p;
-    int cnt[4] = {0, 0, 0, 0};
+    int cnt[MTD_COUNTS] = {};
     int listCap = (int)std::max<size_t>(std::max<size_t>(w.qCvxPairs.n, 4096), 4 * (size_t)n);
+    size_t cands = std::max<size_t>({(size_t)w.qMesh.candCap, (size_t)1 << 18, 2 * (size_t)n});
     float ms0 = 0.f;
-    for (int attempt = 0; attempt < 2; ++attempt) {   // the second with pair lists as long as the first needed
+    // the second attempt with pair lists, the third with candidate lists as long as was needed
+    for (int attempt = 0; attempt < 3; ++attempt) {
         w.qCvxPairs.alloc(listCap); w.qMeshPairs.alloc(listCap);
+        if (w.nTriMesh > 0) np_mesh_buffers(w, w.qMesh, listCap, cands);
         A.listCap = listCap; A.convexPairs = w.qCvxPairs.p; A.meshPairs = w.qMeshPairs.p;
         PGX_HIP(hipEventRecord(w.qEv[0], s));
-        fill_i32(s, w.qMtdN.p, 0, 4);
+        fill_i32(s, w.qMtdN.p, 0, MTD_COUNTS);
         fill_i32(s, w.counters.p + 7, 0, 1);   // the refit's work counter
         bp_build(w);
         if (w.nDynCol == 0) fill_i32(s, w.worldRoot.p, -1, w.W);   // no tree: static lists only
@@ -315,9 +305,11 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
         PGX_HIP(hipMemcpyAsync(cnt, w.qMtdN.p, sizeof cnt, hipMemcpyDeviceToHost, s));
         PGX_HIP(hipStreamSynchronize(s));
         PGX_HIP(hipEventElapsedTime(&ms0, w.qEv[0], w.qEv[1]));
-        if (std::max(cnt[1], cnt[2]) <= listCap) break;
-        if (attempt == 1) throw PgxError{PGX_ERR_HIP, "MTD query: pair lists overflowed twice"};
-        listCap = std::max(cnt[1], cnt[2]);
+        const bool pairs = std::max(cnt[1], cnt[2]) <= listCap;
+        if (pairs && (w.nTriMesh == 0 || cnt[4] <= w.qMesh.candCap)) break;
+        if (attempt == 2) throw PgxError{PGX_ERR_HIP, "MTD query: pair or candidate lists overflowed again"};
+        if (!pairs) listCap = std::max(cnt[1], cnt[2]);
+        else cands = (size_t)cnt[4];
     }
     if (cnt[3]) throw PgxError{PGX_ERR_CAPACITY, "MTD query: EPA or triangle-candidate workspace overflow in " +
                                                      std::to_string(cnt[3]) + " pairs"};

@@ -439,13 +439,8 @@ void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
             throw PgxError{PGX_ERR_UNSUPPORTED, "triangle mesh BVH depth " + std::to_string(w.tmMaxDepth) +
                                                     " exceeds the device traversal stack"};
         w.meshPairs.alloc(w.pairCap);
-        w.meshLanes = TM_LANES;
-        w.tmWs.alloc((size_t)TM_WS_WORDS * w.meshLanes);
-        // candidate triangles of all mesh pairs of a step, one contact record each
-        w.tmCandCap = std::max(1 << 18, 4 * w.mmCap);
-        w.tmCand.alloc(w.tmCandCap); w.tmPairOf.alloc(w.tmCandCap);
-        w.tmRecs.alloc((size_t)(TM_CI_WORDS + 1) * w.tmCandCap);
-        w.tmCandOff.alloc(w.pairCap); w.tmCandCount.alloc(w.pairCap);
+        // candidate triangles of all mesh pairs of a step
+        np_mesh_buffers(w, w.stepMesh, w.pairCap, std::max(1 << 18, 4 * w.mmCap));
     }
     // creation-time bounds: no margin (src/Physecs.cpp:32)
     bp_compute_bounds(w, false);
