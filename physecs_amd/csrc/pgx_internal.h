@@ -361,7 +361,9 @@ struct World {
     DBuf<int32_t> wDyn, sWorld, wcS, wcE;
     // scene queries: rays (origin + maxDistance, direction + world), rejected entities,
     // results, the events around a query's device work
-    DBuf<float4> qRays;
+    DBuf<float> qRays;                   // origins, directions, maxDistance
+    DBuf<int32_t> qRayWorld;
+    DBuf<float4> qRayNode, qRayLeaf;     // the walk's records, 4 x dynamic colliders
     DBuf<uint32_t> qIgnore;
     DBuf<int32_t> qHit;
     DBuf<float> qT;
