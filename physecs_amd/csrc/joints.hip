@@ -46,7 +46,7 @@ struct JointArgs {
     float4 *bvel, *pvel, *pang;
     const float4* brec;
     const int32_t* order;                                     // joints sorted by colour
-    float h;
+    float h, bias;                                            // substep, 0.2 / h
 };
 
 #define JROW(r, f) a.jRow[((size_t)((r) * JR_NF + (f))) * a.Jcap + j]
@@ -332,11 +332,66 @@ __device__ __forceinline__ JBodies joint_bodies(const JointArgs& a, int j) {
     return B;
 }
 
-__device__ void row_presolve_d(const JointArgs& a, int j, int r, int flags, bool simd, const JRow& d,
-                               const JBodies& B, float4& pv0, float4& pw0, float4& pv1, float4& pw1);
+// Constraint1D<flags>::preSolve / Constraint1DW<flags>::preSolve of one row: its products
+// with the bodies' inverse masses (written to the row), and whether and by how much its
+// multiplier moves the bodies' pseudo velocities. Nothing here depends on those velocities.
+struct JPush { f3 lin0t, lin1t, ang0t, ang1t; float lambda; bool moves; };
+__device__ __forceinline__ JPush row_products(const JointArgs& a, int j, int r, int flags, bool simd, const JRow& d,
+                                              const JBodies& B) {
+    JPush p;
+    const bool ang = flags & JF_ANGULAR;
+    const f3 lin = xyz(d.L), ang0 = xyz(d.G0), ang1 = xyz(d.G1);
+    const float c = d.G0.w;
+    float4 G1 = d.G1, L0 = d.L0, L1 = d.L1, T0 = d.T0, T1 = d.T1;
+    p.ang0t = mulmv(B.I0, ang0);
+    p.ang1t = mulmv(B.I1, ang1);
+    float invEff = dot(ang0, p.ang0t) + dot(ang1, p.ang1t);
+    p.lin0t = s3(0.f);
+    p.lin1t = s3(0.f);
+    if (!ang) {
+        invEff = invEff + dot(lin, lin) * (B.im0 + B.im1);
+        p.lin0t = mul(B.im0, lin);
+        p.lin1t = mul(B.im1, lin);
+        set_xyz(L0, p.lin0t);
+        set_xyz(L1, p.lin1t);
+    }
+    set_xyz(T0, p.ang0t);
+    set_xyz(T1, p.ang1t);
+    G1.w = invEff;
+    JROW(r, JR_ANG1) = G1; JROW(r, JR_LIN0T) = L0; JROW(r, JR_LIN1T) = L1; JROW(r, JR_ANG0T) = T0;
+    JROW(r, JR_ANG1T) = T1;
+    p.moves = !(flags & JF_SOFT) && !(c == 0.f || invEff == 0.f);
+    p.lambda = 0.f;
+    if (p.moves) {
+        p.lambda = c / invEff;
+        if (flags & JF_LIMITED) {
+            const float mn = L1.w, mx = T0.w;
+            if (simd) { p.lambda = p.lambda > mn ? p.lambda : mn; p.lambda = p.lambda < mx ? p.lambda : mx; }
+            else p.lambda = gclamp(p.lambda, mn, mx);
+        }
+    }
+    return p;
+}
 
-// Constraint1D<flags>::preSolve / Constraint1DW<flags>::preSolve for one row, on the
-// bodies' pseudo velocities held by the caller (pv, pw; pw.w = constraint count)
+// ... on the bodies' pseudo velocities held by the caller (pv, pw; pw.w = constraint count)
+__device__ void row_presolve_d(const JointArgs& a, int j, int r, int flags, bool simd, const JRow& d,
+                               const JBodies& B, float4& pv0, float4& pw0, float4& pv1, float4& pw1) {
+    const JPush p = row_products(a, j, r, flags, simd, d, B);
+    if (!p.moves) return;
+    const bool ang = flags & JF_ANGULAR;
+    if (B.b0 >= 0) {
+        if (!ang) set_xyz(pv0, add(xyz(pv0), mul(p.lambda, p.lin0t)));
+        set_xyz(pw0, add(xyz(pw0), mul(p.lambda, p.ang0t)));
+        pw0.w = pw0.w + 1.f;
+    }
+    if (B.b1 >= 0) {
+        if (!ang) set_xyz(pv1, sub(xyz(pv1), mul(p.lambda, p.lin1t)));
+        set_xyz(pw1, sub(xyz(pw1), mul(p.lambda, p.ang1t)));
+        pw1.w = pw1.w + 1.f;
+    }
+}
+
+// the same on a row and bodies read from memory
 __device__ void row_presolve(const JointArgs& a, int j, int r, int flags, bool simd, float4& pv0, float4& pw0,
                              float4& pv1, float4& pw1) {
     JBodies B;
@@ -345,52 +400,6 @@ __device__ void row_presolve(const JointArgs& a, int j, int r, int flags, bool s
     if (B.b0 >= 0) { B.im0 = a.dvel[B.b0].w; B.I0 = world_inv_inertia_j(a, B.b0); }
     if (B.b1 >= 0) { B.im1 = a.dvel[B.b1].w; B.I1 = world_inv_inertia_j(a, B.b1); }
     row_presolve_d(a, j, r, flags, simd, load_jrow(a, j, r), B, pv0, pw0, pv1, pw1);
-}
-
-__device__ void row_presolve_d(const JointArgs& a, int j, int r, int flags, bool simd, const JRow& d,
-                               const JBodies& B, float4& pv0, float4& pw0, float4& pv1, float4& pw1) {
-    const int b0 = B.b0, b1 = B.b1;
-    const float im0 = B.im0, im1 = B.im1;
-    const m3 &I0 = B.I0, &I1 = B.I1;
-    bool ang = flags & JF_ANGULAR;
-    float4 L = d.L, G0 = d.G0, G1 = d.G1;
-    f3 lin = xyz(L), ang0 = xyz(G0), ang1 = xyz(G1);
-    float c = G0.w;
-    f3 ang0t = mulmv(I0, ang0), ang1t = mulmv(I1, ang1);
-    float invEff = dot(ang0, ang0t) + dot(ang1, ang1t);
-    f3 lin0t = s3(0.f), lin1t = s3(0.f);
-    float4 L0 = d.L0, L1 = d.L1;
-    if (!ang) {
-        invEff = invEff + dot(lin, lin) * (im0 + im1);
-        lin0t = mul(im0, lin);
-        lin1t = mul(im1, lin);
-        set_xyz(L0, lin0t);
-        set_xyz(L1, lin1t);
-    }
-    float4 T0 = d.T0, T1 = d.T1;
-    set_xyz(T0, ang0t);
-    set_xyz(T1, ang1t);
-    G1.w = invEff;
-    JROW(r, JR_ANG1) = G1; JROW(r, JR_LIN0T) = L0; JROW(r, JR_LIN1T) = L1; JROW(r, JR_ANG0T) = T0;
-    JROW(r, JR_ANG1T) = T1;
-    if (flags & JF_SOFT) return;
-    if (c == 0.f || invEff == 0.f) return;
-    float lambda = c / invEff;
-    if (flags & JF_LIMITED) {
-        float mn = L1.w, mx = T0.w;
-        if (simd) { lambda = lambda > mn ? lambda : mn; lambda = lambda < mx ? lambda : mx; }
-        else lambda = gclamp(lambda, mn, mx);
-    }
-    if (b0 >= 0) {
-        if (!ang) set_xyz(pv0, add(xyz(pv0), mul(lambda, lin0t)));
-        set_xyz(pw0, add(xyz(pw0), mul(lambda, ang0t)));
-        pw0.w = pw0.w + 1.f;
-    }
-    if (b1 >= 0) {
-        if (!ang) set_xyz(pv1, sub(xyz(pv1), mul(lambda, lin1t)));
-        set_xyz(pw1, sub(xyz(pw1), mul(lambda, ang1t)));
-        pw1.w = pw1.w + 1.f;
-    }
 }
 
 // Constraint1DW<flags>::solve for one lane (src/Constraint1DW.cpp:117-233), on the bodies'
@@ -434,8 +443,7 @@ __device__ void row_solve_simd(const JointArgs& a, int j, int r, int flags, bool
         float beta = h * stiffness * gamma;
         lambda = (rv + beta * c / h) / (invEff + gamma / h);
     } else {
-        float bias = (float)(0.2 / (double)h);
-        lambda = (rv - L.w + bias * c) * effMass;
+        lambda = (rv - L.w + a.bias * c) * effMass;
     }
     float prev = lam;
     if (flags & JF_LIMITED) {
@@ -521,10 +529,8 @@ __device__ void row_solve_scalar(const JointArgs& a, int j, int r, int flags, bo
 
 // one joint of a SIMD colour, its rows in flag-type order. The joint's bodies belong to no
 // other joint of the colour, so their velocities (or pseudo velocities) stay in registers
-// across the joint's rows: one load and one store per body. UPFRONT loads every row of the
-// joint at once (the loads overlap; about 200 registers, for a kernel bounded to few
-// threads); otherwise each row is loaded while the one before it is solved.
-template <bool UPFRONT>
+// across the joint's rows: one load and one store per body. Each row is loaded while the one
+// before it is solved.
 __device__ void joint_color_one(const JointArgs& a, int j, int phase, int warm) {
     int n = a.jNRows[j];
     int b0 = a.jB0[j], b1 = a.jB1[j];
@@ -537,36 +543,18 @@ __device__ void joint_color_one(const JointArgs& a, int j, int phase, int warm) 
         for (int r = 0; r < n; ++r)
             if (((rowFlags >> (4 * r)) & 15) == kFlagOrder[f]) seq |= (uint32_t)r << (4 * cnt++);
     float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    // UPFRONT: rows[i] holds row i of the solve order; otherwise rows[0] the row being solved
-    // and rows[1] the next one, in flight meanwhile
-    constexpr int NR = UPFRONT ? JOINT_MAX_ROWS : 2;
-    JRow rows[NR];
-    if constexpr (UPFRONT) {
-#pragma unroll
-        for (int i = 0; i < NR; ++i)
-            if (i < cnt) rows[i] = load_jrow(a, j, (seq >> (4 * i)) & 15);
-    } else {
-        if (cnt) rows[0] = load_jrow(a, j, seq & 15);
-    }
+    JRow row, next;
+    if (cnt) row = load_jrow(a, j, seq & 15);
     if (phase == 0) {
         const JBodies B = joint_bodies(a, j);
         float4 pv0 = z, pw0 = z, pv1 = z, pw1 = z;
         if (b0 >= 0) { pv0 = a.pvel[b0]; pw0 = a.pang[b0]; }
         if (b1 >= 0) { pv1 = a.pvel[b1]; pw1 = a.pang[b1]; }
-        if constexpr (UPFRONT) {
-#pragma unroll
-            for (int i = 0; i < NR; ++i) {
-                if (i >= cnt) break;
-                const int r = (seq >> (4 * i)) & 15;
-                row_presolve_d(a, j, r, (rowFlags >> (4 * r)) & 15, true, rows[i], B, pv0, pw0, pv1, pw1);
-            }
-        } else {
-            for (int i = 0; i < cnt; ++i) {
-                const int r = (seq >> (4 * i)) & 15;
-                if (i + 1 < cnt) rows[1] = load_jrow(a, j, (seq >> (4 * (i + 1))) & 15);
-                row_presolve_d(a, j, r, (rowFlags >> (4 * r)) & 15, true, rows[0], B, pv0, pw0, pv1, pw1);
-                rows[0] = rows[1];
-            }
+        for (int i = 0; i < cnt; ++i) {
+            const int r = (seq >> (4 * i)) & 15;
+            if (i + 1 < cnt) next = load_jrow(a, j, (seq >> (4 * (i + 1))) & 15);
+            row_presolve_d(a, j, r, (rowFlags >> (4 * r)) & 15, true, row, B, pv0, pw0, pv1, pw1);
+            row = next;
         }
         if (b0 >= 0) { a.pvel[b0] = pv0; a.pang[b0] = pw0; }
         if (b1 >= 0) { a.pvel[b1] = pv1; a.pang[b1] = pw1; }
@@ -576,20 +564,11 @@ __device__ void joint_color_one(const JointArgs& a, int j, int phase, int warm) 
     if (b0 >= 0) { tv0 = a.bvel[bv(b0, BV_V)]; tw0 = a.bvel[bv(b0, BV_W)]; }
     if (b1 >= 0) { tv1 = a.bvel[bv(b1, BV_V)]; tw1 = a.bvel[bv(b1, BV_W)]; }
     f3 v0 = xyz(tv0), w0 = xyz(tw0), v1 = xyz(tv1), w1 = xyz(tw1);
-    if constexpr (UPFRONT) {
-#pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            if (i >= cnt) break;
-            const int r = (seq >> (4 * i)) & 15;
-            row_solve_simd(a, j, r, (rowFlags >> (4 * r)) & 15, warm != 0, rows[i], b0, b1, v0, w0, v1, w1);
-        }
-    } else {
-        for (int i = 0; i < cnt; ++i) {
-            const int r = (seq >> (4 * i)) & 15;
-            if (i + 1 < cnt) rows[1] = load_jrow(a, j, (seq >> (4 * (i + 1))) & 15);
-            row_solve_simd(a, j, r, (rowFlags >> (4 * r)) & 15, warm != 0, rows[0], b0, b1, v0, w0, v1, w1);
-            rows[0] = rows[1];
-        }
+    for (int i = 0; i < cnt; ++i) {
+        const int r = (seq >> (4 * i)) & 15;
+        if (i + 1 < cnt) next = load_jrow(a, j, (seq >> (4 * (i + 1))) & 15);
+        row_solve_simd(a, j, r, (rowFlags >> (4 * r)) & 15, warm != 0, row, b0, b1, v0, w0, v1, w1);
+        row = next;
     }
     if (b0 >= 0) { set_xyz(tv0, v0); set_xyz(tw0, w0); a.bvel[bv(b0, BV_V)] = tv0; a.bvel[bv(b0, BV_W)] = tw0; }
     if (b1 >= 0) { set_xyz(tv1, v1); set_xyz(tw1, w1); a.bvel[bv(b1, BV_V)] = tv1; a.bvel[bv(b1, BV_W)] = tw1; }
@@ -598,26 +577,256 @@ __device__ void joint_color_one(const JointArgs& a, int j, int phase, int warm) 
 // one SIMD colour: a thread per joint
 __global__ void k_joint_color(JointArgs a, int begin, int end, int phase, int warm) {
     int k = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < end) joint_color_one<false>(a, a.order[k], phase, warm);
+    if (k < end) joint_color_one(a, a.order[k], phase, warm);
 }
 
 // Every SIMD colour (0-7) of a joint pass in one launch: joints that share a dynamic body,
-// directly or through other joints, form an island, and one workgroup takes each island,
-// its joints colour by colour with a workgroup barrier between colours. Islands share no
-// dynamic body, so each body sees its joints in colour order, as with one launch per
-// colour, and the floats are the same. islandCS: per island, 9 offsets into islandJoint
-// (the start of each colour 0-7, then the island's end).
-constexpr int ISLAND_THREADS = 64;
-__global__ __launch_bounds__(ISLAND_THREADS) void k_joint_islands(JointArgs a, const int32_t* __restrict__ islandCS,
-                                                                  const int32_t* __restrict__ islandJoint, int phase,
-                                                                  int warm) {
-    const int32_t* cs = islandCS + 9 * blockIdx.x;
-    for (int c = 0; c < 8; ++c) {
-        const int b = cs[c], e = cs[c + 1];
-        if (b == e) continue;   // the same for the whole workgroup
-        for (int k = b + (int)threadIdx.x; k < e; k += ISLAND_THREADS)
-            joint_color_one<true>(a, islandJoint[k], phase, warm);
-        __syncthreads();        // this colour's velocity stores are seen by the next colour's loads
+// directly or through other joints, form an island, and one workgroup takes each island.
+// Islands share no dynamic body, so each body sees its joints in colour order, as with one
+// launch per colour, and the floats are the same.
+//
+// An island is a chain: colour after colour, row after row, each on the velocities that the
+// one before it left. What a row does not need those for is taken out of the chain and done
+// for all rows of up to ISLAND_CHUNK joints at once, a lane per row: its loads, its place in
+// the solve order, products with the inverse masses, effective mass, soft-row terms, limits
+// (with the preSolve everything but the sum itself). The results and the island's velocities
+// sit in LDS, and the first wave runs the chain with two lanes per joint, one per body, that
+// exchange their dot products. With a lane per joint for everything, on rows and velocities
+// in memory, a solve pass of 24 ragdolls of 12 joints took 19 us and one of 128 chains of 7
+// joints 14 us; now 11.5 and 8.5 us, and the preSolve 7 us.
+constexpr int ISLAND_CHUNK = WAVE / 2;
+// LDS words of a row, in solve order. Solve: {ang0, lambda} {ang1, lambda} {lin0t, bits}
+// {-lin1t, bits} {ang0t, -} {-ang1t, -} {lin, target} {k0, k1, lower, upper}; preSolve: the
+// pushes {linear 0, bits} {linear 1, bits} {angular 0, -} {angular 1, -}. Bits: the row in
+// 0-2, then JF_* flags and what the chain does with the row.
+constexpr int ROW_WORDS = 8, PUSH_WORDS = 4;
+constexpr int RB_FLAGS = 4, RB_WARM = 1 << 8, RB_MOVES = 1 << 9;
+struct IslandArgs {
+    const int32_t *cs, *bs, *body;   // per island: 9 colour offsets, first body; bodies
+    const int4* joint;               // joint, its bodies' places in the island or -1
+};
+__device__ __forceinline__ float other_lane(float x) {   // of a joint's two lanes
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));   // quad_perm 1,0,3,2
+}
+__device__ __forceinline__ f3 pick(bool c, f3 x, f3 y) { return mk3(c ? x.x : y.x, c ? x.y : y.y, c ? x.z : y.z); }
+// the place of row r among a joint's rows: flag type by flag type, creation order inside one
+__device__ __forceinline__ int row_place(int rowFlags, int n, int r) {
+    const uint32_t rank = 0xF5F34120u;   // kFlagOrder's index of each flag type, 4 bits each
+    const uint32_t mine = rank >> (4 * ((rowFlags >> (4 * r)) & 7)) & 15;
+    int place = 0;
+    for (int k = 0; k < n; ++k) {
+        const uint32_t o = rank >> (4 * ((rowFlags >> (4 * k)) & 7)) & 15;
+        place += o < mine || (o == mine && k < r);
+    }
+    return place;
+}
+// the chunk's joints: rows, and the bodies' places
+__device__ __forceinline__ void chunk_joint(const JointArgs& a, const int4& jl, int4* out) {
+    *out = make_int4(a.jNRows[jl.x], jl.y, jl.z, jl.x);
+}
+// waits for the wave's own LDS stores to be in order before its later loads
+__device__ __forceinline__ void chain_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(8 * ISLAND_CHUNK) void k_island_presolve(JointArgs a, IslandArgs is, int maxBodies, int maxJoints) {
+    extern __shared__ float4 lds[];
+    float4 *sv = lds, *sw = lds + maxBodies, *rows = lds + 2 * maxBodies;
+    int4* js = (int4*)(rows + PUSH_WORDS * JOINT_MAX_ROWS * maxJoints);
+    const int32_t* cs = is.cs + 9 * blockIdx.x;
+    const int b0 = is.bs[blockIdx.x], nb = is.bs[blockIdx.x + 1] - b0;
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+        const int b = is.body[b0 + i];
+        sv[i] = a.pvel[b];
+        sw[i] = a.pang[b];
+    }
+    const int starts = cs[min((int)threadIdx.x & (WAVE - 1), 8)];   // lane c: colour c's start
+    const int first = __builtin_amdgcn_readlane(starts, 0), last = __builtin_amdgcn_readlane(starts, 8);
+    for (int at = first; at < last; at += maxJoints) {
+        const int m = min(maxJoints, last - at);
+        const int jj = threadIdx.x / 8, r = threadIdx.x & 7;
+        if (jj < m) {
+            const int4 jl = is.joint[at + jj];
+            const int j = jl.x;
+            if (r == JOINT_MAX_ROWS) {
+                chunk_joint(a, jl, &js[jj]);
+            } else {
+                const JRow d = load_jrow(a, j, r);
+                const JBodies B = joint_bodies(a, j);
+                const int n = a.jNRows[j], rowFlags = a.jRowFlags[j];
+                if (r < n) {
+                    const int flags = (rowFlags >> (4 * r)) & 15;
+                    const JPush p = row_products(a, j, r, flags, true, d, B);
+                    float4* R = rows + PUSH_WORDS * (JOINT_MAX_ROWS * jj + row_place(rowFlags, n, r));
+                    const float bits = __int_as_float(flags << RB_FLAGS | (p.moves ? RB_MOVES : 0));
+                    R[0] = f4(mul(p.lambda, p.lin0t), bits);
+                    R[1] = f4(neg(mul(p.lambda, p.lin1t)), bits);
+                    R[2] = f4(mul(p.lambda, p.ang0t), 0.f);
+                    R[3] = f4(neg(mul(p.lambda, p.ang1t)), 0.f);
+                }
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < WAVE) {
+            const int side = threadIdx.x & 1;
+            for (int c = 0; c < 8; ++c) {
+                const int b = max(__builtin_amdgcn_readlane(starts, c) - at, 0);
+                const int e = min(__builtin_amdgcn_readlane(starts, c + 1) - at, m);
+                if (b >= e) continue;
+                const int k = b + (int)threadIdx.x / 2;
+                if (k < e) {
+                    const int4 J = js[k];
+                    const int body = side ? J.z : J.y;
+                    const float4* R = rows + PUSH_WORDS * JOINT_MAX_ROWS * k + side;
+                    if (body >= 0) {
+                        float4 v = sv[body], w = sw[body];
+                        float4 nl = R[0], na = R[2];   // the next row's, in flight meanwhile
+                        for (int i = 0; i < J.x; ++i) {
+                            const float4 pl = nl, pa = na;
+                            R += i + 1 < J.x ? PUSH_WORDS : 0;
+                            nl = R[0]; na = R[2];
+                            const int bits = __float_as_int(pl.w);
+                            if (!(bits & RB_MOVES)) continue;
+                            if (!(bits >> RB_FLAGS & JF_ANGULAR)) set_xyz(v, add(xyz(v), xyz(pl)));
+                            set_xyz(w, add(xyz(w), xyz(pa)));
+                            w.w = w.w + 1.f;
+                        }
+                        if (side || J.y != J.z) {   // a joint of a body with itself: side 1's
+                            sv[body] = v;
+                            sw[body] = w;
+                        }
+                    }
+                }
+                chain_sync();
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+        const int b = is.body[b0 + i];
+        a.pvel[b] = sv[i];
+        a.pang[b] = sw[i];
+    }
+}
+
+__global__ __launch_bounds__(8 * ISLAND_CHUNK) void k_island_solve(JointArgs a, IslandArgs is, int maxBodies, int maxJoints,
+                                                                   int warm) {
+    extern __shared__ float4 lds[];
+    float4 *sv = lds, *sw = lds + maxBodies, *rows = lds + 2 * maxBodies;
+    int4* js = (int4*)(rows + ROW_WORDS * JOINT_MAX_ROWS * maxJoints);
+    const int32_t* cs = is.cs + 9 * blockIdx.x;
+    const int b0 = is.bs[blockIdx.x], nb = is.bs[blockIdx.x + 1] - b0;
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+        const int b = is.body[b0 + i];
+        sv[i] = a.bvel[bv(b, BV_V)];
+        sw[i] = a.bvel[bv(b, BV_W)];
+    }
+    const int starts = cs[min((int)threadIdx.x & (WAVE - 1), 8)];   // lane c: colour c's start
+    const int first = __builtin_amdgcn_readlane(starts, 0), last = __builtin_amdgcn_readlane(starts, 8);
+    const float h = a.h;
+    for (int at = first; at < last; at += maxJoints) {
+        const int m = min(maxJoints, last - at);
+        const int jj = threadIdx.x / 8, r = threadIdx.x & 7;
+        if (jj < m) {
+            const int4 jl = is.joint[at + jj];
+            const int j = jl.x;
+            if (r == JOINT_MAX_ROWS) {
+                chunk_joint(a, jl, &js[jj]);
+            } else {
+                const JRow d = load_jrow(a, j, r);
+                const int n = a.jNRows[j], rowFlags = a.jRowFlags[j];
+                if (r < n) {
+                    const int flags = (rowFlags >> (4 * r)) & 15;
+                    const float c = d.G0.w, invEff = d.G1.w, lam = d.L0.w;
+                    const float effMass = 1.f / invEff;
+                    float k0 = effMass, k1 = a.bias * c;
+                    if (flags & JF_SOFT) {   // lambda = (rv + k1) / k0
+                        const float twoPi = 2.f * 3.14159265358979323846f;
+                        const float af = twoPi * d.T1.w;
+                        const float stiffness = af * af * effMass;
+                        const float damping = 2.f * af * d.EX.x * effMass;
+                        const float gamma = 1.f / (damping + h * stiffness);
+                        const float beta = h * stiffness * gamma;
+                        k1 = beta * c / h;
+                        k0 = invEff + gamma / h;
+                    }
+                    int bits = r | flags << RB_FLAGS;
+                    if (!(flags & JF_SOFT) && warm && fabsf(c) < 1e-4f && fabsf(lam) < 10000.f) bits |= RB_WARM;
+                    if (!(invEff == 0.f)) bits |= RB_MOVES;
+                    float4* R = rows + ROW_WORDS * (JOINT_MAX_ROWS * jj + row_place(rowFlags, n, r));
+                    R[0] = f4(xyz(d.G0), lam);
+                    R[1] = f4(xyz(d.G1), lam);
+                    R[2] = f4(xyz(d.L0), __int_as_float(bits));
+                    R[3] = f4(neg(xyz(d.L1)), __int_as_float(bits));   // body 1 is pushed the other way
+                    R[4] = d.T0;
+                    R[5] = f4(neg(xyz(d.T1)), 0.f);
+                    R[6] = d.L;
+                    R[7] = make_float4(k0, k1, d.L1.w * h, d.T0.w * h);
+                }
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < WAVE) {
+            const int side = threadIdx.x & 1;
+            for (int c = 0; c < 8; ++c) {
+                const int b = max(__builtin_amdgcn_readlane(starts, c) - at, 0);
+                const int e = min(__builtin_amdgcn_readlane(starts, c + 1) - at, m);
+                if (b >= e) continue;
+                const int k = b + (int)threadIdx.x / 2;
+                if (k < e) {
+                    const int4 J = js[k];
+                    const int body = side ? J.z : J.y;
+                    const float4* R = rows + ROW_WORDS * JOINT_MAX_ROWS * k + side;
+                    float4 tv = make_float4(0.f, 0.f, 0.f, 0.f), tw = tv;
+                    if (body >= 0) { tv = sv[body]; tw = sw[body]; }
+                    f3 bodyV = xyz(tv), bodyW = xyz(tw);
+                    float4 ng = R[0], nlt = R[2], nat = R[4], nl = R[6 - side], nq = R[7 - side];
+                    for (int i = 0; i < J.x; ++i) {
+                        const float4 g = ng, lt = nlt, at_ = nat, l = nl, q = nq;
+                        R += i + 1 < J.x ? ROW_WORDS : 0;   // the next row's, in flight meanwhile
+                        ng = R[0]; nlt = R[2]; nat = R[4]; nl = R[6 - side]; nq = R[7 - side];
+                        const int bits = __float_as_int(lt.w), flags = bits >> RB_FLAGS;
+                        // selects, not branches: a branch of one lane costs more than both sides
+                        const bool ang = flags & JF_ANGULAR, warmed = bits & RB_WARM, moves = bits & RB_MOVES;
+                        const f3 lint = xyz(lt), angt = xyz(at_);
+                        const float l2 = g.w * 0.5f, lam = warmed ? l2 : g.w;
+                        f3 v = pick(warmed && !ang, add(bodyV, mul(l2, lint)), bodyV);
+                        f3 w = pick(warmed, add(bodyW, mul(l2, angt)), bodyW);
+                        const float dw = dot(xyz(g), w), dv = dot(xyz(l), v);
+                        const float ow = other_lane(dw), ov = other_lane(dv);
+                        const float rw = side ? dw - ow : ow - dw;
+                        const float rv = ang ? rw : rw + (side ? dv - ov : ov - dv);
+                        float lambda = (rv - l.w + q.y) * q.x;
+                        if (flags & JF_SOFT) lambda = (rv + q.y) / q.x;
+                        const float sum = lam + lambda;
+                        float t = sum > q.z ? sum : q.z;
+                        t = t < q.w ? t : q.w;
+                        const bool limited = flags & JF_LIMITED;
+                        lambda = limited ? t - lam : lambda;
+                        const float newLam = moves ? (limited ? t : sum) : lam;
+                        v = add(v, mul(lambda, lint));
+                        w = add(w, mul(lambda, angt));
+                        bodyV = pick(moves && !ang && body >= 0, v, bodyV);
+                        bodyW = pick(moves && body >= 0, w, bodyW);
+                        const int j = J.w, row = bits & 7;
+                        if (side == 0) JROW(row, JR_LIN0T).w = newLam;
+                    }
+                    if (body >= 0 && (side || J.y != J.z)) {   // a joint of a body with itself: side 1's
+                        set_xyz(tv, bodyV); set_xyz(tw, bodyW);
+                        sv[body] = tv;
+                        sw[body] = tw;
+                    }
+                }
+                chain_sync();
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+        const int b = is.body[b0 + i];
+        a.bvel[bv(b, BV_V)] = sv[i];
+        a.bvel[bv(b, BV_W)] = sw[i];
     }
 }
 
@@ -658,6 +867,7 @@ static JointArgs make_jargs(World& w, float h) {
     a.bvel = w.bvel.p; a.brec = w.brec.p; a.pvel = w.pvel.p; a.pang = w.pang.p;
     a.order = w.jOrder.p;
     a.h = h;
+    a.bias = (float)(0.2 / (double)h);
     return a;
 }
 
@@ -747,8 +957,16 @@ void jt_colors(World& w, float h, int phase, bool warm) {
     if (!w.J) return;
     JointArgs a = make_jargs(w, h);
     if (w.jIslands > 0) {   // colours 0-7 by island in one launch, then the overflow colour
-        hipLaunchKernelGGL(k_joint_islands, dim3(w.jIslands), dim3(ISLAND_THREADS), 0, w.stream, a, w.jIslandCS.p,
-                           w.jIslandJoint.p, phase, warm ? 1 : 0);
+        const IslandArgs is{w.jIslandCS.p, w.jIslandBS.p, w.jIslandBody.p, w.jIslandJoint.p};
+        const int m = std::min(w.jIslandJoints, ISLAND_CHUNK), threads = div_up(8 * m, WAVE) * WAVE;
+        const size_t lds = 2 * sizeof(float4) * w.jIslandBodies + sizeof(int4) * m;
+        if (phase == 0)
+            hipLaunchKernelGGL(k_island_presolve, dim3(w.jIslands), dim3(threads),
+                               lds + sizeof(float4) * PUSH_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m);
+        else
+            hipLaunchKernelGGL(k_island_solve, dim3(w.jIslands), dim3(threads),
+                               lds + sizeof(float4) * ROW_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m,
+                               warm ? 1 : 0);
         const int b = w.jColorStart[8], e = w.jColorStart[9];
         if (e > b)
             hipLaunchKernelGGL(k_joint_overflow, dim3(1), dim3(64), 0, w.stream, a, b, e, phase, warm ? 1 : 0);

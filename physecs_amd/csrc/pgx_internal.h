@@ -321,7 +321,10 @@ struct World {
     std::vector<int> jColorStart;                // 10 offsets into jOrder
     DBuf<int32_t> jType, jA0, jA1, jB0, jB1, jRowFlags, jNRows, jOrder;
     int jIslands = 0;                    // islands of the one-launch joint passes (0: per-colour launches)
-    DBuf<int32_t> jIslandCS, jIslandJoint;   // per island 9 colour offsets; joints by island and colour
+    int jIslandJoints = 0, jIslandBodies = 0;   // of the largest island
+    DBuf<int32_t> jIslandCS, jIslandBS;  // per island: 9 colour offsets into jIslandJoint; its start in jIslandBody
+    DBuf<int32_t> jIslandBody;           // the islands' dynamic bodies
+    DBuf<int4> jIslandJoint;             // joints by island and colour: {joint, its bodies' places in the island or -1, 0}
     DBuf<float4> jP0, jQ0, jP1, jQ1, jDrive, jR0, jR1, jRow;
     DBuf<float4> jPar0, jPar1;           // (lower, upper, target, stiffness), (damping, gear ratio)
     DBuf<float4> jGear;                  // gear state: persistent angle 0, 1, virtual angle 0, 1

@@ -660,7 +660,7 @@ static void upload_joints(World& w, int keepState) {
         if (w.hjAlive[j]) order[fillp[w.hjColor[j]]++] = j;
     // islands of the SIMD colours (0-7): joints joined through dynamic bodies; each island's
     // joints by colour, in the colour order above inside a colour. One launch per joint pass
-    // solves them all (k_joint_islands) when no island holds more than ISLAND_MAX joints of
+    // solves them all (k_island_presolve, k_island_solve) when no island holds more than ISLAND_MAX joints of
     // one colour; per-colour launches otherwise.
     {
         std::vector<int> parent(w.D > 0 ? w.D : 1);
@@ -690,7 +690,8 @@ static void upload_joints(World& w, int keepState) {
         const int most = cnt.empty() ? 0 : *std::max_element(cnt.begin(), cnt.end());
         w.jIslands = 0;
         if (nIsl >= ISLAND_MIN && most <= ISLAND_MAX) {
-            std::vector<int32_t> cs((size_t)nIsl * 9), cursor((size_t)nIsl * 8), list(w.jColorStart[8]);
+            std::vector<int32_t> cs((size_t)nIsl * 9), cursor((size_t)nIsl * 8), bs((size_t)nIsl + 1), bodies;
+            std::vector<int4> list(w.jColorStart[8]);
             int at = 0;
             for (int i = 0; i < nIsl; ++i) {
                 for (int c = 0; c < 8; ++c) {
@@ -701,11 +702,30 @@ static void upload_joints(World& w, int keepState) {
             }
             for (int k = 0; k < w.jColorStart[8]; ++k) {   // colour order, creation order inside a colour
                 const int j = order[k];
-                list[cursor[(size_t)islandOf[k] * 8 + w.hjColor[j]]++] = j;
+                list[cursor[(size_t)islandOf[k] * 8 + w.hjColor[j]]++] = make_int4(j, -1, -1, 0);
             }
+            std::vector<int32_t> place(w.D > 0 ? w.D : 1, -1);
+            w.jIslandJoints = w.jIslandBodies = 0;
+            for (int i = 0; i < nIsl; ++i) {
+                bs[i] = (int32_t)bodies.size();
+                auto placed = [&](int b) {
+                    if (b < 0) return -1;
+                    if (place[b] < 0) { place[b] = (int)bodies.size() - bs[i]; bodies.push_back(b); }
+                    return (int)place[b];
+                };
+                for (int k = cs[(size_t)i * 9]; k < cs[(size_t)i * 9 + 8]; ++k) {
+                    list[k].y = placed(w.hjB0[list[k].x]);
+                    list[k].z = placed(w.hjB1[list[k].x]);
+                }
+                w.jIslandJoints = std::max(w.jIslandJoints, cs[(size_t)i * 9 + 8] - cs[(size_t)i * 9]);
+                w.jIslandBodies = std::max(w.jIslandBodies, (int)bodies.size() - bs[i]);
+            }
+            bs[nIsl] = (int32_t)bodies.size();
             w.jIslands = nIsl;
             upload(w.jIslandCS, cs, w.stream);
             upload(w.jIslandJoint, list, w.stream);
+            upload(w.jIslandBS, bs, w.stream);
+            upload(w.jIslandBody, bodies, w.stream);
         }
     }
     hipStream_t s = w.stream;
