@@ -61,3 +61,13 @@ def test_sort_empty_and_one(api):
     for n in (0, 1):
         ko, vo = api.sort_u64(np.arange(n, dtype=np.uint64), np.arange(n, dtype=np.int32), 8)
         assert len(ko) == n
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 2048, 2049, 8191, 8192, 8193])
+@pytest.mark.parametrize("bits", [4, 33])
+def test_sort_around_the_single_workgroup(api, n, bits):
+    """Sizes at which the one-workgroup sort changes its waves or its items per wave, and its limit."""
+    log(f"[sort] one workgroup n={n} bits={bits}")
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << bits, n).astype(np.uint64)
+    _check(api, keys, bits)
