@@ -269,7 +269,8 @@ struct World {
     DBuf<int2> sB, sA;                   // per slot: its sides' dynamic bodies (-1: none) and internal bodies
     DBuf<int32_t> sFlags, sMode;         // sFlags: numPoints | soft<<8 | color<<16; sMode: the substep's
     DBuf<int32_t> sCanon;                // canonical index
-    DBuf<int32_t> batchLoc, batchList, batchN;   // runs of small colours: LDS slots of their bodies
+    DBuf<int32_t> batchLoc, batchList;   // runs of small colours: LDS slots of their bodies
+    DBuf<int2> batchTurns;               // and their turns
     DBuf<int32_t> colorPack;             // the colouring's read-back, packed by k_color_start
     PinnedInts readHost;                 // pinned host memory for the step's read-backs (READ_HOST_INTS)
     bool batchLdsSet = false;            // k_solve_batch's LDS limit raised on this world's device

@@ -410,7 +410,7 @@ static_assert(2 * RS_NF + 1 == CONTACT_ROW_FIELDS, "sRow holds CONTACT_ROW_FIELD
 #define LAM(k) a.sLam[(size_t)(k) * a.Mcap + s]
 // sMode: what the solve has to know of a slot this substep: points, softness, and the points
 // whose normal or friction row has no mass (invN or invT is 0) and is left out
-enum { MODE_NUM = 255, MODE_SOFT = 256, MODE_SKIP_N = 1 << 16, MODE_SKIP_T = 1 << 20 };
+enum { MODE_NUM = 255, MODE_SOFT = 256, MODE_N = 1 << 16, MODE_T = 1 << 20 };
 // a pass over the contacts: with the bias; without the soft contacts (relaxation); the
 // substep's first (the lambdas are 0) and last (nothing reads them afterwards)
 enum { PASS_BIAS = 1, PASS_SKIP_SOFT = 2, PASS_FIRST = 4, PASS_LAST = 8 };
@@ -522,8 +522,8 @@ __device__ void prepare_side(const SubArgs& a, int i) {
         // the friction impulse of one pass, on the component velocities
         const float ct = dot(signed_of(t, side), cv), cr = dot(signed_of(rxt, side), cw);
         const float rvT = side0(ct + cr) + side1(ct) + side1(cr);
-        if (invN == 0.f) mode |= MODE_SKIP_N << k;
-        if (invT == 0.f) mode |= MODE_SKIP_T << k;
+        if (!(invN == 0.f)) mode |= MODE_N << k;
+        if (!(invT == 0.f)) mode |= MODE_T << k;
         ROW(RS_N, k) = f4(signed_of(rxn, side), anchor.w);
         ROW(RS_NT, k) = f4(signed_of(rxnt, side), termA);
         ROW(RS_TT, k) = f4(signed_of(rxtt, side), termB);
@@ -574,13 +574,12 @@ __device__ void integrate_velocity(const SubArgs& a, int d, float4 vv, f3 ang) {
 }
 
 // Everything one side's solve reads except its body's solver velocities: the manifold's
-// mode, normal (with the side's sign) and friction, and its rows, tangents and lambdas. All
+// mode, normal and friction, and its rows, tangents and lambdas. All
 // of it is fixed for the whole pass.
 struct SideIn {
     int num, mode, b;
     bool soft;
-    f3 sn;
-    float friction;
+    float4 n;         // normal, friction
     float4 row[4][RS_NF], t[4];
     float2 lam[4];
 };
@@ -589,16 +588,13 @@ struct SideIn {
 // mode and body index, without waiting for the point count; slots 1-3 wait for the count,
 // in the same round of loads as the body's velocities (which wait for the body index
 // anyway), so unused slots cost no traffic and the solve still takes two dependent rounds.
+// the rest of a side whose mode and body index are known
 template <bool EAGER = false>
-__device__ __forceinline__ void load_side(const SubArgs& a, int i, int pass, SideIn& in) {
+__device__ __forceinline__ void load_rows(const SubArgs& a, int i, int pass, SideIn& in) {
     const int s = i >> 1;
-    in.mode = a.sMode[s];
     in.soft = (in.mode & MODE_SOFT) != 0;
     in.num = in.mode & MODE_NUM;
-    in.b = a.sB[i];
-    const float4 nf = a.sN[s];
-    in.sn = signed_of(xyz(nf), i & 1);
-    in.friction = nf.w;
+    in.n = a.sN[s];
     // all rows of the side are loaded before any dependent arithmetic (memory-level
     // parallelism); unused point slots are never read back
 #pragma unroll
@@ -611,60 +607,65 @@ __device__ __forceinline__ void load_side(const SubArgs& a, int i, int pass, Sid
         }
     }
 }
+template <bool EAGER = false>
+__device__ __forceinline__ void load_side(const SubArgs& a, int i, int pass, SideIn& in) {
+    in.mode = a.sMode[i >> 1];
+    in.b = a.sB[i];
+    load_rows<EAGER>(a, i, pass, in);
+}
 
 // ContactConstraints::solve (src/ContactConstraints.cpp:33-124) of one side of a manifold,
 // normal then friction rows, on its body's solver velocities (v.w = invMass; updated in
 // place); the even lane stores the accumulated lambdas. Manifolds of one colour touch
 // disjoint dynamic bodies, so a colour is solved in parallel exactly as a sequential pass
 // over it would be. Both lanes of the pair run it together.
-__device__ __forceinline__ void solve_side(const SubArgs& a, int i, const SideIn& in, int pass, float4& v4, f3& w) {
-    const int s = i >> 1, num = in.num;
+//
+// A pass is a chain of these, each a chain of points on its body's velocities, so what counts
+// is the instructions a wave issues one after the other: one branch per point and row (soft
+// rows, rare, have theirs only in waves that hold one), selects for the rest. With a branch
+// for each condition a colour of four-point manifolds took 1.7 us of a run's workgroup.
+__device__ __forceinline__ void solve_side(int i, SideIn& in, int pass, float4& v4, f3& w) {
     const bool moves = in.b >= 0;
     const float im = (i & 1) ? v4.w : -v4.w;
+    const f3 n = xyz(in.n), sn = signed_of(n, i & 1);
+    const bool anySoft = __ballot(in.soft) != 0;
     f3 v = xyz(v4);
-    float lN[4], lT[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        if (k >= num) break;
+        if (!(in.mode & (MODE_N << k))) continue;
         const float4* r = in.row[k];
-        lN[k] = in.lam[k].x;
-        if (in.mode & (MODE_SKIP_N << k)) continue;
-        const float p = dot(in.sn, v), q = dot(xyz(r[RS_N]), w);
+        const float p = dot(sn, v), q = dot(xyz(r[RS_N]), w);
         const float rv = side0(p + q) + side1(p) + side1(q);
-        float lambda;
-        if (in.soft) lambda = (rv + r[RS_TT].w) / r[RS_NT].w;
-        else lambda = (rv - r[RS_N].w + ((pass & PASS_BIAS) ? r[RS_TT].w : 0.f)) * r[RS_NT].w;
-        const float prev = lN[k];
-        lN[k] = lN[k] + lambda;
-        lN[k] = gmin(lN[k], 0.f);
-        lambda = lN[k] - prev;
-        if (moves) {   // the normal with side 1's sign times -im or im: the side's own sign
-            v = sub(v, mul(lambda * im, signed_of(in.sn, i & 1)));
-            w = sub(w, mul(lambda, xyz(r[RS_NT])));
+        float lambda = (rv - r[RS_N].w + ((pass & PASS_BIAS) ? r[RS_TT].w : 0.f)) * r[RS_NT].w;
+        if (anySoft) {
+            if (in.soft) lambda = (rv + r[RS_TT].w) / r[RS_NT].w;
         }
+        const float prev = in.lam[k].x;
+        in.lam[k].x = gmin(prev + lambda, 0.f);
+        // a side that does not move has zero velocities, which a zero push leaves as they are
+        lambda = moves ? in.lam[k].x - prev : 0.f;
+        v = sub(v, mul(lambda * im, n));   // the normal with side 1's sign times -im or im: the side's own sign
+        w = sub(w, mul(lambda, xyz(r[RS_NT])));
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        if (k >= num) break;
-        lT[k] = in.lam[k].y;
-        if (in.mode & (MODE_SKIP_T << k)) continue;
-        const float limit = in.friction * lN[k];
-        const float prev = lT[k];
-        lT[k] = lT[k] + in.t[k].w;
-        lT[k] = gclamp(lT[k], limit, -limit);
-        const float lambda = lT[k] - prev;
-        if (moves) {
-            v = sub(v, mul(lambda * im, xyz(in.t[k])));
-            w = sub(w, mul(lambda, xyz(in.row[k][RS_TT])));
-        }
+        if (!(in.mode & (MODE_T << k))) continue;
+        const float limit = in.n.w * in.lam[k].x;
+        const float prev = in.lam[k].y;
+        in.lam[k].y = gclamp(prev + in.t[k].w, limit, -limit);
+        const float lambda = moves ? in.lam[k].y - prev : 0.f;
+        v = sub(v, mul(lambda * im, xyz(in.t[k])));
+        w = sub(w, mul(lambda, xyz(in.row[k][RS_TT])));
     }
     v4 = f4(v, v4.w);
+}
+// the manifold's accumulated lambdas, by its even lane, once the velocities are handed on
+__device__ __forceinline__ void store_lambdas(const SubArgs& a, int i, const SideIn& in, int pass) {
     if ((i & 1) || (pass & PASS_LAST)) return;
+    const int s = i >> 1;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (k >= num) break;
-        LAM(k) = make_float2(lN[k], lT[k]);
-    }
+    for (int k = 0; k < 4; ++k)
+        if (k < in.num) LAM(k) = in.lam[k];
 }
 
 // one side of a manifold of a colour launch: every other manifold touching its body is in
@@ -677,8 +678,9 @@ __device__ void solve_lane(const SubArgs& a, int i, int pass) {
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     f3 w = s3(0.f);
     if (in.b >= 0) { v = a.bvel[bv(in.b, BV_V)]; w = xyz(a.bvel[bv(in.b, BV_W)]); }
-    solve_side(a, i, in, pass, v, w);
+    solve_side(i, in, pass, v, w);
     if (in.b >= 0) { a.bvel[bv(in.b, BV_V)] = v; a.bvel[bv(in.b, BV_W)] = f4(w, 0.f); }
+    store_lambdas(a, i, in, pass);
 }
 
 // integrate positions of one body, src/Physecs.cpp:494-511
@@ -780,7 +782,7 @@ __device__ __forceinline__ void st_agent3(float4* p, f3 v) {
 
 // the solve of one side whose fixed inputs are loaded, on velocities at the coherence point
 // (the inverse mass beside them never changes)
-__device__ __forceinline__ void solve_coherent(const SubArgs& a, int i, const SideIn& in, int pass) {
+__device__ __forceinline__ void solve_coherent(const SubArgs& a, int i, SideIn& in, int pass) {
     if ((pass & PASS_SKIP_SOFT) && in.soft) return;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     f3 w = s3(0.f);
@@ -788,8 +790,9 @@ __device__ __forceinline__ void solve_coherent(const SubArgs& a, int i, const Si
         v = f4(ld_agent3(&a.bvel[bv(in.b, BV_V)]), a.bvel[bv(in.b, BV_V)].w);
         w = ld_agent3(&a.bvel[bv(in.b, BV_W)]);
     }
-    solve_side(a, i, in, pass, v, w);
+    solve_side(i, in, pass, v, w);
     if (in.b >= 0) { st_agent3(&a.bvel[bv(in.b, BV_V)], xyz(v)); st_agent3(&a.bvel[bv(in.b, BV_W)], w); }
+    store_lambdas(a, i, in, pass);
 }
 
 // grid barrier number `target` / gridDim.x of the substep: every workgroup has arrived
@@ -856,7 +859,7 @@ constexpr int XPASS_MAX_GRID = 248; // at most 31 workgroups per XCD: a byte nev
 
 __device__ __forceinline__ f3 ld_l2_3(const float4* p) { return ld_agent3(p); }
 
-__device__ __forceinline__ void solve_xcd(const SubArgs& a, int i, const SideIn& in, int pass) {
+__device__ __forceinline__ void solve_xcd(const SubArgs& a, int i, SideIn& in, int pass) {
     if ((pass & PASS_SKIP_SOFT) && in.soft) return;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     f3 w = s3(0.f);
@@ -864,8 +867,9 @@ __device__ __forceinline__ void solve_xcd(const SubArgs& a, int i, const SideIn&
         v = f4(ld_l2_3(&a.bvel[bv(in.b, BV_V)]), a.bvel[bv(in.b, BV_V)].w);
         w = ld_l2_3(&a.bvel[bv(in.b, BV_W)]);
     }
-    solve_side(a, i, in, pass, v, w);
+    solve_side(i, in, pass, v, w);
     if (in.b >= 0) { a.bvel[bv(in.b, BV_V)] = v; a.bvel[bv(in.b, BV_W)] = f4(w, 0.f); }
+    store_lambdas(a, i, in, pass);
 }
 
 __global__ __launch_bounds__(XPASS_THREADS) void k_solve_xpass(SubArgs a, int nColors, int pass, int32_t* ctl) {
@@ -934,12 +938,16 @@ constexpr int BATCH_THREADS = 1024;     // two lanes per manifold; 4 waves per S
 constexpr int BATCH_MAP_THREADS = 1024;
 constexpr int BATCH_HASH = 8192;        // LDS hash of body -> slot: at least twice a run's bodies
 constexpr int BATCH_MAX_GROUPS = 16;
-constexpr int BATCH_MAX_MANIFOLDS = 1264;   // 2 x 1264 bodies x 32 B of velocities in LDS
+constexpr int BATCH_MAX_MANIFOLDS = 2400;   // 2 x 2400 bodies x 32 B of velocities in LDS
 constexpr int BATCH_MAX_COLOURS = 128;
+constexpr int BATCH_LANES = BATCH_THREADS / 2;   // a team's
+constexpr int BATCH_MAX_TURNS = BATCH_MAX_COLOURS + 2 * BATCH_MAX_MANIFOLDS / BATCH_LANES + 1;
 
 struct BatchGroups {
     int n;
     int S[BATCH_MAX_GROUPS], E[BATCH_MAX_GROUPS];
+    int c0[BATCH_MAX_GROUPS], c1[BATCH_MAX_GROUPS];   // colours
+    int turns[BATCH_MAX_GROUPS];
 };
 
 __device__ __forceinline__ uint32_t batch_hash(int b) { return ((uint32_t)b * 2654435761u) >> (32 - 13); }
@@ -949,44 +957,60 @@ __device__ __forceinline__ uint32_t batch_hash(int b) { return ((uint32_t)b * 26
 __global__ __launch_bounds__(BATCH_MAP_THREADS) void k_batch_map(BatchGroups g, const int32_t* __restrict__ sB,
                                                                  int32_t* __restrict__ batchLoc,
                                                                  int32_t* __restrict__ batchList,
-                                                                 int32_t* __restrict__ batchN) {
+                                                                 const int32_t* __restrict__ colorStart,
+                                                                 int2* __restrict__ batchTurns) {
     static_assert(BATCH_HASH == 1 << 13, "batch_hash gives 13 bits");
     __shared__ int32_t hk[BATCH_HASH], hv[BATCH_HASH];
     __shared__ int32_t count;
-    for (int q = 0; q < g.n; ++q) {
-        const int S = g.S[q], E = g.E[q], sides = 2 * (E - S);
-        for (int i = threadIdx.x; i < BATCH_HASH; i += BATCH_MAP_THREADS) hk[i] = -1;
-        if (threadIdx.x == 0) count = 0;
-        __syncthreads();
-        for (int i = threadIdx.x; i < sides; i += BATCH_MAP_THREADS) {
-            const int b = sB[2 * S + i];
-            if (b < 0) continue;
+    const int q = blockIdx.x;
+    const int S = g.S[q], E = g.E[q], sides = 2 * (E - S);
+    for (int i = threadIdx.x; i < BATCH_HASH; i += BATCH_MAP_THREADS) hk[i] = -1;
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < sides; i += BATCH_MAP_THREADS) {
+        const int b = sB[2 * S + i];
+        if (b < 0) continue;
+        uint32_t h = batch_hash(b);
+        for (int probe = 0; probe < BATCH_HASH; ++probe) {   // the table is never full
+            const int prev = atomicCAS(&hk[h], -1, b);
+            if (prev == -1) {
+                const int slot = atomicAdd(&count, 1);
+                hv[h] = slot;
+                batchList[2 * S + slot] = b;
+                break;
+            }
+            if (prev == b) break;
+            h = (h + 1) & (BATCH_HASH - 1);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < sides; i += BATCH_MAP_THREADS) {
+        const int b = sB[2 * S + i];
+        int slot = -1;
+        if (b >= 0) {
             uint32_t h = batch_hash(b);
-            for (int probe = 0; probe < BATCH_HASH; ++probe) {   // the table is never full
-                const int prev = atomicCAS(&hk[h], -1, b);
-                if (prev == -1) {
-                    const int slot = atomicAdd(&count, 1);
-                    hv[h] = slot;
-                    batchList[2 * S + slot] = b;
-                    break;
-                }
-                if (prev == b) break;
-                h = (h + 1) & (BATCH_HASH - 1);
-            }
+            for (int probe = 0; probe < BATCH_HASH && hk[h] != b; ++probe) h = (h + 1) & (BATCH_HASH - 1);
+            slot = hv[h];
         }
-        __syncthreads();
-        for (int i = threadIdx.x; i < sides; i += BATCH_MAP_THREADS) {
-            const int b = sB[2 * S + i];
-            int slot = -1;
-            if (b >= 0) {
-                uint32_t h = batch_hash(b);
-                for (int probe = 0; probe < BATCH_HASH && hk[h] != b; ++probe) h = (h + 1) & (BATCH_HASH - 1);
-                slot = hv[h];
+        batchLoc[2 * S + i] = slot;
+    }
+    for (int i = count + threadIdx.x; i < sides; i += BATCH_MAP_THREADS) batchList[2 * S + i] = -1;
+    if (threadIdx.x < WAVE) {   // the turns, in colour order
+        int2* turns = batchTurns + (size_t)BATCH_MAX_TURNS * q;
+        int at = 0;
+        for (int c = g.c0[q]; c < g.c1[q]; c += WAVE) {
+            const int k = c + (int)threadIdx.x;
+            int b = 0, e = 0;
+            if (k < g.c1[q]) { b = 2 * colorStart[k]; e = 2 * colorStart[k + 1]; }
+            const int mine = (e - b + BATCH_LANES - 1) / BATCH_LANES;
+            int x = mine;
+            for (int o = 1; o < WAVE; o <<= 1) {
+                const int y = __shfl_up(x, o);
+                if ((int)threadIdx.x >= o) x += y;
             }
-            batchLoc[2 * S + i] = slot;
+            for (int j = 0; j < mine; ++j) turns[at + x - mine + j] = make_int2(b + j * BATCH_LANES, min(b + (j + 1) * BATCH_LANES, e));
+            at += __shfl(x, WAVE - 1);
         }
-        if (threadIdx.x == 0) batchN[q] = count;
-        __syncthreads();
     }
 }
 
@@ -999,57 +1023,94 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // The run's bodies' velocities (solver v with the inverse mass, and w) are gathered into
-// LDS once per launch, so a manifold's solve needs only its own rows from global memory:
-// slot 0's with the mode, slots 1-3 once the point count is known (one CU's load bandwidth
-// bounds these launches, so unused slots are not read). Each colour's rows are loaded
-// before the barrier that waits for the previous colour's velocities, so their latency
-// overlaps the wait.
-__global__ __launch_bounds__(BATCH_THREADS) void k_solve_batch(SubArgs a, int c0, int c1, int S,
+// LDS once per launch, so a manifold's solve needs only its own rows from global memory.
+// Those are two dependent rounds of loads (the mode, then as many slots as the mode has
+// points), longer than the solve itself, so the workgroup's waves form two teams that take
+// turns: while one team solves a turn (a colour, or 512 lanes of a larger one), the other
+// stores its lambdas and loads the rows of its next turn (their modes were loaded a turn
+// earlier). A barrier between turns orders LDS only. The first rows and the bodies' velocities
+// are fetched together. 415 manifolds in eight colours: 11.5 us, 18.5 with one team that loads
+// a colour after the one before it; four teams of 256 lanes take 12.2 and eight of 128 15.4
+// (more turns), two of 256 11.6 there and 13.0 for 11.9 on 789 manifolds.
+// FIRST: the substep's first pass, whose lambdas are not read (a branch on the pass would wait
+// for the loads).
+template <bool FIRST>
+__global__ __launch_bounds__(BATCH_THREADS) void k_solve_batch(SubArgs a, int S, int E, int total,
+                                                               const int2* __restrict__ turnsIn,
                                                                const int32_t* __restrict__ batchLoc,
-                                                               const int32_t* __restrict__ batchList,
-                                                               const int32_t* __restrict__ batchN, int pass) {
+                                                               const int32_t* __restrict__ batchList, int flags) {
+    const int pass = FIRST ? flags | PASS_FIRST : flags & ~PASS_FIRST;
     extern __shared__ float4 rec[];       // [n] solver v, then [n] solver w of the run's bodies
-    __shared__ int32_t cs[BATCH_MAX_COLOURS + 1];   // the run's colour starts, in side lanes
-    const int n = *batchN;
-    const int32_t* list = batchList + 2 * S;
-    for (int i = threadIdx.x; i <= c1 - c0; i += BATCH_THREADS) cs[i] = 2 * a.colorStart[c0 + i];
-    for (int i = threadIdx.x; i < n; i += BATCH_THREADS) {
-        const int b = list[i];
-        rec[i] = a.bvel[bv(b, BV_V)];
-        rec[n + i] = a.bvel[bv(b, BV_W)];
+    __shared__ int2 turns[BATCH_MAX_TURNS];   // side lanes [x, y), in colour order
+    const int n = 2 * (E - S);
+    const int team = __builtin_amdgcn_readfirstlane((int)threadIdx.x / BATCH_LANES), t = (int)threadIdx.x - team * BATCH_LANES;
+    constexpr int GATHER = (2 * BATCH_MAX_MANIFOLDS + BATCH_THREADS - 1) / BATCH_THREADS;
+    int body[GATHER];   // the bodies this thread gathers and writes back: slots threadIdx.x + 1024 j
+#pragma unroll
+    for (int j = 0; j < GATHER; ++j) {
+        const int i = threadIdx.x + j * BATCH_THREADS;
+        body[j] = i < n ? batchList[2 * S + i] : -1;
     }
-    __syncthreads();
-    auto solve = [&](int i, const SideIn& in, int l) {
-        if ((pass & PASS_SKIP_SOFT) && in.soft) return;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        f3 w = s3(0.f);
-        if (in.b >= 0) { v = rec[l]; w = xyz(rec[n + l]); }
-        solve_side(a, i, in, pass, v, w);
-        if (in.b >= 0) { rec[l] = v; rec[n + l] = f4(w, 0.f); }
+    if ((int)threadIdx.x < total) turns[threadIdx.x] = turnsIn[threadIdx.x];
+    lds_barrier();
+    // a side's turn: its place, and what is loaded a turn ahead of its rows
+    struct Turn { int i, mode, b, l; };
+    auto turn = [&](int k, Turn& h) {
+        h.i = -1;
+        if (k >= total) return;
+        const int2 range = turns[k];
+        if (range.x + t >= range.y) return;
+        h.i = range.x + t;
+        h.mode = a.sMode[h.i >> 1];
+        h.b = a.sB[h.i];
+        h.l = batchLoc[h.i];
     };
-    for (int c = 0; c < c1 - c0; ++c) {
-        const int e = cs[c + 1];
-        int i = cs[c] + (int)threadIdx.x;
-        SideIn in;
-        int l = -1;
-        const bool have = i < e;
-        if (have) {
-            load_side(a, i, pass, in);
-            l = batchLoc[i];
+    auto rows = [&](const Turn& h, SideIn& in) {
+        SideIn x;   // slots that are not loaded hold nothing, not the last turn's rows
+        x.mode = h.mode;
+        x.b = h.b;
+        if (h.i >= 0) load_rows(a, h.i, pass, x);
+        in = x;
+    };
+    Turn now, next;
+    SideIn in;
+    turn(team, now);
+#pragma unroll
+    for (int j = 0; j < GATHER; ++j) {
+        if (body[j] < 0) continue;
+        const int i = threadIdx.x + j * BATCH_THREADS;
+        rec[i] = a.bvel[bv(body[j], BV_V)];
+        rec[n + i] = a.bvel[bv(body[j], BV_W)];
+    }
+    rows(now, in);
+    turn(team + 2, next);
+    for (int k = 0; k <= total; ++k) {
+        lds_barrier();   // the previous turn's velocities are in LDS
+        if (k < total && (k & 1) == team && now.i >= 0 && !((pass & PASS_SKIP_SOFT) && in.soft)) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            f3 w = s3(0.f);
+            if (in.b >= 0) { v = rec[now.l]; w = xyz(rec[n + now.l]); }
+            solve_side(now.i, in, pass, v, w);
+            if (in.b >= 0) { rec[now.l] = v; rec[n + now.l] = f4(w, 0.f); }
         }
-        lds_barrier();   // the previous colour's velocities are in LDS
-        if (have) solve(i, in, l);
-        // colours larger than the workgroup: a lane's manifolds of one colour share no body
-        for (i += BATCH_THREADS; i < e; i += BATCH_THREADS) {
-            load_side(a, i, pass, in);
-            solve(i, in, batchLoc[i]);
+        // after its turn, while the next team solves
+        if (k > 0 && ((k - 1) & 1) == team) {
+            if (now.i >= 0 && !((pass & PASS_SKIP_SOFT) && in.soft)) store_lambdas(a, now.i, in, pass);
+            now = next;
+            // arrived a turn ago: taken before the rows' loads, which a later wait for them
+            // would wait for too
+            asm volatile("" : "+v"(now.i), "+v"(now.mode), "+v"(now.b), "+v"(now.l));
+            rows(now, in);
+            turn(k + 3, next);
         }
     }
     lds_barrier();
-    for (int i = threadIdx.x; i < n; i += BATCH_THREADS) {
-        const int b = list[i];
-        a.bvel[bv(b, BV_V)] = rec[i];
-        a.bvel[bv(b, BV_W)] = rec[n + i];
+#pragma unroll
+    for (int j = 0; j < GATHER; ++j) {
+        if (body[j] < 0) continue;
+        const int i = threadIdx.x + j * BATCH_THREADS;
+        a.bvel[bv(body[j], BV_V)] = rec[i];
+        a.bvel[bv(body[j], BV_W)] = rec[n + i];
     }
 }
 
@@ -1101,8 +1162,9 @@ __global__ __launch_bounds__(WORLD_THREADS) void k_world_pass(SubArgs a, WorldPa
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             f3 w = s3(0.f);
             if (in.b >= 0) { v = wv[l]; w = xyz(wv[n + l]); }
-            solve_side(a, i, in, pass, v, w);
+            solve_side(i, in, pass, v, w);
             if (in.b >= 0) { wv[l] = v; wv[n + l] = f4(w, 0.f); }
+            store_lambdas(a, i, in, pass);
         }
         __syncthreads();
     }
@@ -1242,8 +1304,10 @@ __global__ __launch_bounds__(256) void k_solve_flow(SubArgs a, FlowArgs f) {
                 const bool both = __builtin_amdgcn_mov_dpp((int)have, 0xB1, 0xf, 0xf, true) != 0 && have;   // quad_perm 1,0,3,2
                 if (both) {
                     // a soft manifold in the relaxation passes its bodies' velocities on
-                    if (!((f.pass & PASS_SKIP_SOFT) && in.soft)) solve_side(a, i, in, f.pass, v, w);
+                    const bool solved = !((f.pass & PASS_SKIP_SOFT) && in.soft);
+                    if (solved) solve_side(i, in, f.pass, v, w);
                     if (in.b >= 0) hand_on(a, f, in.b, last, vbase | (uint32_t)(r + 1), v, w);
+                    if (solved) store_lambdas(a, i, in, f.pass);
                     pending = false;
                     done += lane & 1;
                 } else if (++spins > FLOW_SPIN_LIMIT) {
@@ -1562,8 +1626,6 @@ bool sv_world_pass_fits(World& w) {
     return 2 * sizeof(float4) * (size_t)std::max(1, w.maxWorldDyn) <= (size_t)w.ldsMax;
 }
 
-// one colour [b, e) in workgroups of `block` threads; with events, stamped from the
-// launch's own dispatch packet
 // Workgroups of a colour launch over side lanes [b, e) in chunks of bs homed on their XCD
 // (homed_chunk): 8 per round, as many rounds as the XCD with the most chunks needs.
 static int homed_blocks(int b, int e, int bs) {
@@ -1577,6 +1639,8 @@ static int homed_blocks(int b, int e, int bs) {
     return 8 * most;
 }
 
+// one colour [b, e) in workgroups of `block` threads; with events, stamped from the
+// launch's own dispatch packet
 static void launch_solve(int block, bool eager, hipStream_t s, hipEvent_t e0, hipEvent_t e1, const SubArgs& a, int b,
                          int e, int pass) {
     auto go = [&](auto kernel, int bs) {
@@ -1602,10 +1666,11 @@ void sv_presize(World& w) {
     if (w.tune.colorBatch > 0) {
         w.batchLoc.alloc(2 * (size_t)w.manifoldCap);
         w.batchList.alloc(2 * (size_t)w.manifoldCap);
-        w.batchN.alloc(BATCH_MAX_GROUPS);
+        w.batchTurns.alloc((size_t)BATCH_MAX_GROUPS * BATCH_MAX_TURNS);
         if (!w.batchLdsSet) {
-            PGX_HIP(hipFuncSetAttribute((const void*)k_solve_batch, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)(4 * sizeof(float4) * BATCH_MAX_MANIFOLDS)));
+            for (const void* k : {(const void*)k_solve_batch<true>, (const void*)k_solve_batch<false>})
+                PGX_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)(4 * sizeof(float4) * BATCH_MAX_MANIFOLDS)));
             w.batchLdsSet = true;
         }
     }
@@ -1686,6 +1751,11 @@ void sv_substeps(World& w, int M, float dt) {
             if (c1 - c >= 2) {
                 bg.S[bg.n] = w.colorStartHost[c];
                 bg.E[bg.n] = w.colorStartHost[c1];
+                bg.c0[bg.n] = c;
+                bg.c1[bg.n] = c1;
+                bg.turns[bg.n] = 0;
+                for (int k = c; k < c1; ++k)
+                    bg.turns[bg.n] += div_up(2 * (w.colorStartHost[k + 1] - w.colorStartHost[k]), BATCH_LANES);
                 groups.push_back(make_int3(c, c1, ++bg.n));
                 c = c1;
                 continue;
@@ -1696,8 +1766,8 @@ void sv_substeps(World& w, int M, float dt) {
     }
     if (bg.n > 0) {   // the runs' body slots, fixed for the step
         sv_presize(w);
-        hipLaunchKernelGGL(k_batch_map, dim3(1), dim3(BATCH_MAP_THREADS), 0, s, bg, a.sB, w.batchLoc.p,
-                           w.batchList.p, w.batchN.p);
+        hipLaunchKernelGGL(k_batch_map, dim3(bg.n), dim3(BATCH_MAP_THREADS), 0, s, bg, a.sB, w.batchLoc.p,
+                           w.batchList.p, a.colorStart, w.batchTurns.p);
         PGX_LAUNCH_CHECK();
     }
     int passIndex = 0;
@@ -1780,14 +1850,16 @@ void sv_substeps(World& w, int M, float dt) {
                 const int q = g.z - 1;
                 // 2 bodies per manifold at most
                 const size_t lds = 4 * sizeof(float4) * (size_t)(bg.E[q] - bg.S[q]);
+                const int2* turns = w.batchTurns.p + (size_t)BATCH_MAX_TURNS * q;
+                auto* kernel = (flags & PASS_FIRST) ? k_solve_batch<true> : k_solve_batch<false>;
                 if (rec) {   // a run of colours [g.x, g.y), stamped from its dispatch packet
                     hipEvent_t e0, e1;
                     solve_events(w, g.x, &e0, &e1, g.y);
-                    hipExtLaunchKernelGGL(k_solve_batch, dim3(1), dim3(BATCH_THREADS), lds, s, e0, e1, 0, a, g.x, g.y,
-                                          bg.S[q], w.batchLoc.p, w.batchList.p, w.batchN.p + q, flags);
+                    hipExtLaunchKernelGGL(kernel, dim3(1), dim3(BATCH_THREADS), lds, s, e0, e1, 0, a, bg.S[q],
+                                          bg.E[q], bg.turns[q], turns, w.batchLoc.p, w.batchList.p, flags);
                 } else {
-                    hipLaunchKernelGGL(k_solve_batch, dim3(1), dim3(BATCH_THREADS), lds, s, a, g.x, g.y, bg.S[q],
-                                       w.batchLoc.p, w.batchList.p, w.batchN.p + q, flags);
+                    hipLaunchKernelGGL(kernel, dim3(1), dim3(BATCH_THREADS), lds, s, a, bg.S[q], bg.E[q],
+                                       bg.turns[q], turns, w.batchLoc.p, w.batchList.p, flags);
                 }
                 continue;
             }
