@@ -538,8 +538,10 @@ __device__ bool capsule_box(f3 p0, qf q0, float hh0, float r0, f3 p1, qf q1, f3 
     return true;
 }
 
-// src/Collision.cpp:135-350
-__device__ bool box_box(f3 p0, qf q0, f3 he0, f3 p1, qf q1, f3 he1, Mf& m) {
+// src/Collision.cpp:135-350. LATER: a face contact's polygon is left to k_box_faces: face is
+// set to 3 * the face's box + its axis, m untouched.
+template <bool LATER>
+__device__ bool box_box(f3 p0, qf q0, f3 he0, f3 p1, qf q1, f3 he1, Mf& m, int& face) {
     float edgeOffset = 0.1f;
     const float edgeLimit = 0.999f;
     bool isEdge = false;
@@ -585,7 +587,9 @@ __device__ bool box_box(f3 p0, qf q0, f3 he0, f3 p1, qf q1, f3 he1, Mf& m) {
             }
         }
     }
-    if (!isEdge) {
+    if (LATER && !isEdge) {
+        face = 3 * faceBox + faceAxis;
+    } else if (!isEdge) {
         CPt cps[4];
         int np = 0;
         f3 axis;
@@ -604,16 +608,16 @@ __device__ bool box_box(f3 p0, qf q0, f3 he0, f3 p1, qf q1, f3 he1, Mf& m) {
         f3 a0 = col(u0, e0), a1 = col(u1, e1);
         f3 axis = cross(a0, a1);
         m.normal = normalize(dot(axis, sub(p1, p0)) < 0 ? neg(axis) : axis);
-        float s0[3] = {-1.f, -1.f, -1.f}, s1[3] = {-1.f, -1.f, -1.f};
-        s0[(e0 + 1) % 3] = dot(col(u0, (e0 + 1) % 3), m.normal) < 0 ? -1.f : 1.f;
-        s0[(e0 + 2) % 3] = dot(col(u0, (e0 + 2) % 3), m.normal) < 0 ? -1.f : 1.f;
+        float s0[3], s1[3];   // the edges' start corners
+        for (int i = 0; i < 3; ++i) {
+            s0[i] = i == e0 || dot(col(u0, i), m.normal) < 0 ? -1.f : 1.f;
+            s1[i] = i == e1 || dot(col(u1, i), m.normal) > 0 ? -1.f : 1.f;
+        }
         f3 c0 = add(add(add(p0, mul(s0[0] * h0[0], u0.c0)), mul(s0[1] * h0[1], u0.c1)), mul(s0[2] * h0[2], u0.c2));
-        s1[(e1 + 1) % 3] = dot(col(u1, (e1 + 1) % 3), m.normal) > 0 ? -1.f : 1.f;
-        s1[(e1 + 2) % 3] = dot(col(u1, (e1 + 2) % 3), m.normal) > 0 ? -1.f : 1.f;
         f3 c1 = add(add(add(p1, mul(s1[0] * h1[0], u1.c0)), mul(s1[1] * h1[1], u1.c1)), mul(s1[2] * h1[2], u1.c2));
         m.numPoints = 1;
         f3 a, b;
-        closest_points_segments(c0, a0, 0.f, h0[e0] * 2, c1, a1, 0.f, h1[e1] * 2, a, b);
+        closest_points_segments(c0, a0, 0.f, at(he0, e0) * 2, c1, a1, 0.f, at(he1, e1) * 2, a, b);
         m.pts[0].p0 = a;
         m.pts[0].p1 = b;
     }
@@ -625,8 +629,9 @@ __device__ void flip(Mf& m) {
     for (int i = 0; i < m.numPoints; ++i) { f3 a = m.pts[i].p0; m.pts[i].p0 = m.pts[i].p1; m.pts[i].p1 = a; }
 }
 
-// src/Collision.cpp:895-1016 for primitive shapes
-__device__ bool collide(int t0, float4 g0, f3 p0, qf q0, int t1, float4 g1, f3 p1, qf q1, Mf& m) {
+// src/Collision.cpp:895-1016 for primitive shapes; face and LATER as box_box
+template <bool LATER>
+__device__ bool collide(int t0, float4 g0, f3 p0, qf q0, int t1, float4 g1, f3 p1, qf q1, Mf& m, int& face) {
     m.numPoints = 0;
     bool hit = false;
     f3 he0 = mk3(g0.x, g0.y, g0.z), he1 = mk3(g1.x, g1.y, g1.z);
@@ -642,7 +647,7 @@ __device__ bool collide(int t0, float4 g0, f3 p0, qf q0, int t1, float4 g1, f3 p
     }
     if (t1 == PGX_SPHERE) { hit = sphere_box(p1, g1.x, p0, q0, he0, m); flip(m); return hit; }
     if (t1 == PGX_CAPSULE) { hit = capsule_box(p1, q1, g1.x, g1.y, p0, q0, he0, m); flip(m); return hit; }
-    return box_box(p0, q0, he0, p1, q1, he1, m);
+    return box_box<LATER>(p0, q0, he0, p1, q1, he1, m, face);
 }
 
 }  // namespace pgx
@@ -705,7 +710,7 @@ __global__ __launch_bounds__(256) void k_narrowphase(
     int32_t* __restrict__ heavy, int32_t* __restrict__ nHeavy, int32_t* __restrict__ meshPairs,
     int32_t* __restrict__ nMesh, int32_t* __restrict__ meshCount, int32_t* __restrict__ trigList,
     int32_t* __restrict__ nTrig, const int32_t* __restrict__ filterClass, const uint8_t* __restrict__ filterTable,
-    int filterK) {
+    int filterK, int32_t* __restrict__ nFaces, int32_t* __restrict__ facesEnd) {
     // pairs per lane = pairs / (grid size): a lane takes every grid-size'th pair of the
     // class order; results are stored at the pair's own slot
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nPairs; i += gridDim.x * blockDim.x) {
@@ -717,7 +722,7 @@ __global__ __launch_bounds__(256) void k_narrowphase(
         int base = worldColStart[wd];
         int c0 = colOfLocal[base + (int)((key >> localBits) & lmask)];
         int c1 = colOfLocal[base + (int)(key & lmask)];
-        int num = 0;
+        int num = 0, face = -1;
         // the contact filter on (collider of the lower entity, other collider): TRIGGER makes
         // a trigger pair, not a contact (src/Physecs.cpp:200-207); defaultContactFilter is a
         // trigger on either side (:20-23). Joint-connected / setCanCollide pairs are skipped (:209)
@@ -756,10 +761,14 @@ __global__ __launch_bounds__(256) void k_narrowphase(
             qf q0 = qmul(bq0, q4(clquat[c0]));
             f3 p1 = add(bp1, qrot(bq1, xyz(clpos[c1])));
             qf q1 = qmul(bq1, q4(clquat[c1]));
-            bool hit = collide(ctype[c0], cparams[c0], p0, q0, ctype[c1], cparams[c1], p1, q1, m);
+            bool hit = collide<true>(ctype[c0], cparams[c0], p0, q0, ctype[c1], cparams[c1], p1, q1, m, face);
             num = hit ? m.numPoints : 0;
         }
-        npNum[p] = num;
+        if (__ballot(face >= 0)) {
+            const int k = wave_append(nFaces, face >= 0);
+            if (face >= 0) facesEnd[-1 - k] = p;
+        }
+        npNum[p] = face >= 0 ? face : num;
         if (num) {
             npNormal[p] = f4(m.normal, 0.f);
             for (int k = 0; k < 4; ++k) {
@@ -776,6 +785,175 @@ __global__ __launch_bounds__(256) void k_narrowphase(
 // what the chip holds of their 14 KB of LDS each, walks the list. The list length is read on
 // the device, so no host round trip.
 constexpr int CONVEX_WAVES = 2816;
+// The face contacts of box pairs (box_face_contacts and polygon_box_face_contacts_n,
+// operation for operation): the other box's face clipped by the four sides of the reference
+// face, its penetrating corners, four of them picked. Eight lanes per pair, a polygon corner
+// each (a second round of corners where a clip leaves more than eight), the corners in LDS.
+// With a lane per pair in k_narrowphase this was a chain of some thirty corners, each with a
+// branch and a division, on polygons in scratch memory: 58 us for the 585 pairs of a pyramid
+// of boxes however few they were, 17 us now with k_narrowphase; 177 and 111 us for 662k mixed
+// pairs.
+constexpr int BOX_LANES = 8, BOX_GROUPS = 256 / BOX_LANES, BOX_BLOCKS = 2048;
+struct BoxClip { f2 poly[2][MAXPOLY]; f3 pen[MAXPOLY]; };
+__device__ __forceinline__ uint32_t group_ballot(bool b) {
+    return (uint32_t)(__ballot(b) >> (threadIdx.x & (WAVE - BOX_LANES))) & ((1u << BOX_LANES) - 1);
+}
+template <int CTRL>
+__device__ __forceinline__ float larger_lane(float x) {
+    const float y = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+    return y > x ? y : x;
+}
+// the first index whose value (v[c] of lane l: element 8 c + l, below n) is the largest and
+// above 0, else 0: the sequential loop that keeps what is greater than the best so far
+__device__ __forceinline__ int first_largest(const float (&v)[2], int n) {
+    const int l = threadIdx.x & (BOX_LANES - 1);
+    float best = l < n && v[0] > 0.f ? v[0] : 0.f;
+    if (BOX_LANES + l < n && v[1] > best) best = v[1];
+    best = larger_lane<0xB1>(best);    // quad_perm 1,0,3,2
+    best = larger_lane<0x4E>(best);    // quad_perm 2,3,0,1
+    best = larger_lane<0x141>(best);   // row_half_mirror
+    const uint32_t e0 = group_ballot(l < n && v[0] == best), e1 = group_ballot(BOX_LANES + l < n && v[1] == best);
+    if (!(best > 0.f)) return 0;
+    return e0 ? __ffs(e0) - 1 : BOX_LANES + __ffs(e1) - 1;
+}
+__global__ __launch_bounds__(256) void k_box_faces(
+    const int32_t* __restrict__ nFacesP, const int32_t* __restrict__ facesEnd, const uint64_t* __restrict__ pkeys,
+    int localBits, const int32_t* __restrict__ worldColStart, const int32_t* __restrict__ colOfLocal,
+    const int32_t* __restrict__ cbody, const float4* __restrict__ cparams, const float4* __restrict__ clpos,
+    const float4* __restrict__ clquat, const float4* __restrict__ bpos, const float4* __restrict__ bquat,
+    int32_t* __restrict__ npNum, float4* __restrict__ npNormal, float4* __restrict__ npPts) {
+    __shared__ BoxClip clips[BOX_GROUPS];
+    const int group = threadIdx.x / BOX_LANES, l = threadIdx.x & (BOX_LANES - 1);
+    BoxClip& C = clips[group];
+    const uint32_t before = (1u << l) - 1;
+    const int nFaces = *nFacesP;
+    const uint64_t lmask = (1ull << localBits) - 1;
+    for (int base = blockIdx.x * BOX_GROUPS; base < nFaces; base += gridDim.x * BOX_GROUPS) {
+        const bool live = base + group < nFaces;   // the block's last groups repeat its first pair, unstored
+        const int p = facesEnd[-1 - (live ? base + group : base)];
+        const int code = live ? npNum[p] : 0;
+        const uint64_t key = pkeys[p];
+        const int cols = worldColStart[(int)(key >> (2 * localBits))];
+        const int c0 = colOfLocal[cols + (int)((key >> localBits) & lmask)], c1 = colOfLocal[cols + (int)(key & lmask)];
+        const int b0 = cbody[c0], b1 = cbody[c1];
+        const qf bq0 = q4(bquat[b0]), bq1 = q4(bquat[b1]);
+        const f3 p0 = add(xyz(bpos[b0]), qrot(bq0, xyz(clpos[c0]))), p1 = add(xyz(bpos[b1]), qrot(bq1, xyz(clpos[c1])));
+        const m3 m0 = mat3_cast(qmul(bq0, q4(clquat[c0]))), m1 = mat3_cast(qmul(bq1, q4(clquat[c1])));
+        const bool second = code >= 3;   // the reference face's box
+        const int refAxis = second ? code - 3 : code;
+        auto of = [&](f3 x, f3 y) { return mk3(second ? y.x : x.x, second ? y.y : x.y, second ? y.z : x.z); };
+        const m3 uRef = mk_m3(of(m0.c0, m1.c0), of(m0.c1, m1.c1), of(m0.c2, m1.c2));
+        const m3 uInc = mk_m3(of(m1.c0, m0.c0), of(m1.c1, m0.c1), of(m1.c2, m0.c2));
+        const f3 posRef = of(p0, p1), posInc = of(p1, p0);
+        const f3 heRef = xyz(cparams[second ? c1 : c0]), heInc = xyz(cparams[second ? c0 : c1]);
+        // box_face_contacts: the incident face
+        const f3 axis = col(uRef, refAxis);
+        const float refSign = dot(axis, sub(posInc, posRef)) < 0 ? -1.f : 1.f;
+        float maxDot = 0.f, incSign = 1.f;
+        int incAxis = 0;
+        for (int i = 0; i < 3; ++i) {
+            const float d = dot(mul(-refSign, axis), col(uInc, i)), ad = gabs(d);
+            if (ad > maxDot) { maxDot = ad; incAxis = i; incSign = d < 0 ? -1.f : 1.f; }
+        }
+        const int ia1 = incAxis == 2 ? 0 : incAxis + 1, ia2 = incAxis == 0 ? 2 : incAxis - 1;
+        const m3 inv = inverse(uRef);
+        const f3 ui = col(uInc, incAxis), u1 = col(uInc, ia1), u2 = col(uInc, ia2);
+        const float h1 = at(heInc, ia1), h2 = at(heInc, ia2);
+        const f3 incOrig = mulmv(inv, sub(add(posInc, mul(mul(ui, at(heInc, incAxis)), incSign)), posRef));
+        const f3 a = mul(u1, h1), b = mul(u2, h2), na = mul(neg(u1), h1);
+        const int cx = refAxis == 2 ? 0 : refAxis + 1, cy = refAxis == 0 ? 2 : refAxis - 1;
+        {
+            const f3 x = l == 1 || l == 2 ? na : a;
+            const f3 corner = add(incOrig, mulmv(inv, l < 2 ? add(x, b) : sub(x, b)));
+            if (l < 4) C.poly[0][l] = mk2(at(corner, cx), at(corner, cy));
+        }
+        wave_sync();
+        // clip_polygon: an edge's outputs, in the order of the corners
+        const float hx = at(heRef, cx), hy = at(heRef, cy);
+        int n = 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const f2 ca = mk2(e < 2 ? hx : -hx, e == 0 || e == 3 ? hy : -hy);
+            const f2 cb = mk2(e == 0 || e == 3 ? hx : -hx, e < 2 ? -hy : hy);
+            const f2* in = C.poly[e & 1];
+            f2* out = C.poly[1 - (e & 1)];
+            int m = 0;
+            for (int k = 0; k < MAXPOLY && __ballot(k < n); k += BOX_LANES) {
+                const int i = k + l;
+                const bool have = i < n;
+                const f2 me = in[have ? i : 0], next = in[have && i + 1 < n ? i + 1 : 0];
+                const bool ii = have && inside(me, ca, cb), ji = have && inside(next, ca, cb);
+                const uint32_t one = group_ballot(ii || ji), two = group_ballot(!ii && ji);
+                int at_ = m + __popc(one & before) + __popc(two & before);
+                if (ii != ji) {
+                    if (at_ < MAXPOLY) out[at_] = intersect2(me, next, ca, cb);
+                    ++at_;
+                }
+                if (ji && at_ < MAXPOLY) out[at_] = next;
+                m += __popc(one) + __popc(two);
+            }
+            n = min(m, MAXPOLY);
+            wave_sync();
+        }
+        // polygon_box_face_contacts_n: the corners under the face
+        const f3 incNormal = mulmv(inv, ui);
+        const int axisSign = (int)refSign;
+        f3 dir = s3(0.f);
+        set(dir, refAxis, (float)axisSign);
+        const float denom = dot(dir, incNormal), heAxis = at(heRef, refAxis), lim = heAxis + 1e-4f;
+        int np = 0;
+        for (int k = 0; k < MAXPOLY && __ballot(k < n); k += BOX_LANES) {
+            const bool have = k + l < n;
+            const f2 q = C.poly[0][have ? k + l : 0];
+            f3 p3 = s3(0.f);
+            set(p3, cx, q.x);
+            set(p3, cy, q.y);
+            const float distance = dot(sub(incOrig, p3), incNormal) / denom;
+            const bool keep = have && distance < lim;
+            const uint32_t kept = group_ballot(keep);
+            set(p3, refAxis, axisSign * distance);
+            if (keep) C.pen[np + __popc(kept & before)] = p3;
+            np += __popc(kept);
+        }
+        wave_sync();
+        int pick = l;   // the corner of contact l
+        if (np > 4) {
+            const f3 first = C.pen[0];
+            f3 pen[2];
+            float v[2];
+            for (int c = 0; c < 2; ++c) {
+                pen[c] = C.pen[min(BOX_LANES * c + l, np - 1)];
+                const f3 d = sub(pen[c], first);
+                v[c] = dot(d, d);
+            }
+            const int far = first_largest(v, np);
+            const f3 second_ = C.pen[far];
+            for (int c = 0; c < 2; ++c) {
+                const f3 da = sub(first, pen[c]), db = sub(second_, pen[c]);
+                v[c] = det2(mk2(at(da, cx), at(da, cy)), mk2(at(db, cx), at(db, cy)));
+            }
+            const int left = first_largest(v, np);
+            for (int c = 0; c < 2; ++c) v[c] = -v[c];
+            const int right = first_largest(v, np);
+            pick = l == 0 ? 0 : l == 1 ? far : l == 2 ? left : right;
+            np = 4;
+        }
+        if (live && l < np) {
+            const f3 pen = C.pen[pick];
+            f3 on = pen;
+            set(on, refAxis, axisSign * heAxis);
+            const f3 onRef = add(posRef, mulmv(uRef, on)), onInc = add(posRef, mulmv(uRef, pen));
+            npPts[8 * (size_t)p + 2 * l] = f4(second ? onInc : onRef, 0.f);
+            npPts[8 * (size_t)p + 2 * l + 1] = f4(second ? onRef : onInc, 0.f);
+        }
+        if (live && l == 0) {
+            npNum[p] = np;
+            if (np) npNormal[p] = f4(dot(axis, sub(p1, p0)) < 0 ? neg(axis) : axis, 0.f);
+        }
+        wave_sync();
+    }
+}
+
 __global__ __launch_bounds__(64) void k_narrowphase_convex(
     const int32_t* __restrict__ nHeavyP, const int32_t* __restrict__ heavy, const uint64_t* __restrict__ pkeys,
     int localBits, const int32_t* __restrict__ worldColStart, const int32_t* __restrict__ colOfLocal,
@@ -1457,7 +1635,8 @@ __global__ __launch_bounds__(64) void k_mtd_walk(MtdArgs A, ConvexView cv) {
                 f3 cp;
                 qf cq;
                 mtd_collider_pose(A, c, cp, cq);
-                hit = collide(ct, A.cparams[c], cp, cq, t, g, pos, q, m) && m.numPoints > 0;
+                int face;
+                hit = collide<false>(ct, A.cparams[c], cp, cq, t, g, pos, q, m, face) && m.numPoints > 0;
             }
         }
         if (__ballot(hit)) {
@@ -1650,7 +1829,12 @@ void np_run(World& w, int nPairs) {
                        w.nNonColliding, w.npNum.p, w.npNormal.p, w.npPts.p, w.heavy.p, w.counters.p + 8,
                        w.meshPairs.p, w.counters.p + 10, w.meshCount.p,
                        w.hasTriggers ? w.trigList.p : nullptr, w.trigN.p + 2 * w.trigCur, w.filterClass.p,
-                       w.filterTable.p, w.filterK);
+                       w.filterTable.p, w.filterK, w.counters.p + 4, w.heavy.p + w.pairCap);
+    PGX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_box_faces, dim3(std::min(div_up(nPairs, BOX_GROUPS), BOX_BLOCKS)), dim3(256), 0, w.stream,
+                       w.counters.p + 4, w.heavy.p + w.pairCap, w.pkeys.p, w.localBits, w.worldColStart.p, w.colOfLocal.p,
+                       w.cbody.p, w.cparams.p, w.clpos.p, w.clquat.p, w.bpos.p, w.bquat.p, w.npNum.p, w.npNormal.p,
+                       w.npPts.p);
     PGX_LAUNCH_CHECK();
     if (w.hasTriggers) {
         ConvexView cv{w.cvVerts.p, w.cvMesh.p, w.cvFace.p, w.cvFaceIdx.p, w.cvFaceN.p, w.cvFaceC.p};

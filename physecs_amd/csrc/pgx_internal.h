@@ -238,7 +238,7 @@ struct World {
     DBuf<int32_t> worldRoot, worldStop;
     DBuf<uint64_t> pkeys;
     DBuf<int32_t> pvals;
-    DBuf<int32_t> counters;              // [0] pairs, [1] manifolds, [2] triangles GJK hit, [3] uncolored, [5] colour overflow, [6] bvh error, [7] refit ready
+    DBuf<int32_t> counters;              // [0] pairs, [1] manifolds, [2] triangles GJK hit, [3] uncolored, [4] box faces, [5] colour overflow, [6] bvh error, [7] refit ready
     SortTemp sortT;
     ScanTemp scanT;
 
@@ -298,7 +298,7 @@ struct World {
     DBuf<int4> cvMesh;
     DBuf<int2> cvFace;
     DBuf<int32_t> cvFaceIdx;
-    DBuf<int32_t> heavy;               // pairs with a convex mesh (filled by the primitive kernel)
+    DBuf<int32_t> heavy;               // from its start: pairs with a convex mesh; from its end: pairs of boxes touching with a face (filled by the primitive kernel)
     // static triangle meshes: vertices, triangles in the BVH build's order (mesh-local
     // vertex indices), triangle normals / centroids, BVH nodes (2 float4 each: {min,
     // triCount bits}, {max, index bits}), {first vertex, vertices, first triangle, first node}
