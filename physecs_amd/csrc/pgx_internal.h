@@ -136,6 +136,19 @@ struct RadixScratch {
     size_t keys = 0, vals = 0, hist = 0, sums = 0;
 };
 RadixScratch radix_sort_scratch(int n, int bits);
+// rank of the lane's element among the wave's elements of the same digit so far; bumps the
+// wave's count of the digit (counts: this wave's counters in LDS, one per digit value)
+__device__ __forceinline__ int32_t rs_rank(uint32_t d, bool ok, int dbits, uint64_t lt, int32_t* counts) {
+    uint64_t same = __ballot(ok);
+    for (int b = 0; b < dbits; ++b) {
+        const uint64_t bal = __ballot((d >> b) & 1u);
+        same &= ((d >> b) & 1u) ? bal : ~bal;
+    }
+    const int32_t prior = counts[d];
+    if (ok && (same & lt) == 0ull) counts[d] = prior + (int32_t)__popcll(same);
+    return prior + (int32_t)__popcll(same & lt);
+}
+
 // The same sort with caller-provided scratch of radix_sort_scratch(n, bits) elements; it
 // needs no zeroed memory (every table it reads it has written first) and allocates nothing.
 void radix_sort_u64_into(hipStream_t s, uint64_t* keys, int32_t* vals, int n, int bits, uint64_t* kalt,
@@ -238,7 +251,7 @@ struct World {
     DBuf<int32_t> worldRoot, worldStop;
     DBuf<uint64_t> pkeys;
     DBuf<int32_t> pvals;
-    DBuf<int32_t> counters;              // [0] pairs, [1] manifolds, [2] triangles GJK hit, [3] uncolored, [4] box faces, [5] colour overflow, [6] bvh error, [7] refit ready
+    DBuf<int32_t> counters;              // [0] pairs, [1] manifolds, [2] triangles GJK hit, [3] the flow passes' error flag, [4] box faces, [5] colour overflow, [6] bvh error, [7] refit ready
     SortTemp sortT;
     ScanTemp scanT;
 
@@ -274,6 +287,7 @@ struct World {
     DBuf<int32_t> colorPack;             // the colouring's read-back, packed by k_color_start
     PinnedInts readHost;                 // pinned host memory for the step's read-backs (READ_HOST_INTS)
     bool batchLdsSet = false;            // k_solve_batch's LDS limit raised on this world's device
+    bool colorLdsSet = false;            // k_color_small's, likewise
     DBuf<float4> sN;                     // normal, friction
     DBuf<float2> sSoft;                  // frequency, damping
     DBuf<float4> sR;                     // 4 x M x 2 sides: local anchor + targetVelocity

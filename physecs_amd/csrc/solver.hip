@@ -26,8 +26,10 @@ namespace pgx {
 // ------------------------------------------------------------------ compaction
 // manifolds of pair p: one for a pair with points, meshCount[p] for a triangle-mesh pair
 __global__ void k_flag_manifolds(int nPairs, const int32_t* __restrict__ npNum, const int32_t* __restrict__ meshCount,
-                                 int32_t* __restrict__ flag) {
+                                 int32_t* __restrict__ flag, const int32_t* __restrict__ flowErr,
+                                 int32_t* __restrict__ counters) {
     int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == 0) counters[3] = *flowErr;
     if (p < nPairs) flag[p] = (npNum[p] > 0 ? 1 : 0) + meshCount[p];
 }
 
@@ -43,33 +45,77 @@ __device__ __forceinline__ void pair_colliders(uint64_t key, int localBits, cons
 // Manifold list in pair order; a triangle-mesh pair contributes its manifolds in the order
 // collisionTriangleMesh emitted them. mfSrc is the narrowphase data slot (the pair's own
 // slot, or pairCap + the mesh manifold's slot), mfTri the triangle index (-1 otherwise).
-__global__ void k_compact(int nPairs, const int32_t* __restrict__ npNum, const int32_t* __restrict__ npIndex,
-                          const int32_t* __restrict__ meshFirst, const int32_t* __restrict__ meshCount,
-                          const int32_t* __restrict__ npTri, int pairCap,
-                          const uint64_t* __restrict__ pkeys, int localBits, const int32_t* __restrict__ worldColStart,
-                          const int32_t* __restrict__ colOfLocal, const int32_t* __restrict__ cbody,
-                          const int32_t* __restrict__ cflags, int32_t* __restrict__ mfPair,
-                          uint64_t* __restrict__ mfKey, int32_t* __restrict__ mfB0, int32_t* __restrict__ mfB1,
-                          int32_t* __restrict__ mfSrc, int32_t* __restrict__ mfTri) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nPairs) return;
-    int nm = meshCount[p];
-    if (npNum[p] == 0 && nm == 0) return;
-    int m = npIndex[p];
-    uint64_t key = pkeys[p];
+struct CompactArgs {
+    const int32_t *npNum, *meshFirst, *meshCount, *npTri;
+    int pairCap, localBits;
+    const uint64_t* pkeys;
+    const int32_t *worldColStart, *colOfLocal, *cbody, *cflags;
+    int32_t* mfPair;
+    uint64_t* mfKey;
+    int32_t *mfB0, *mfB1, *mfSrc, *mfTri;
+};
+// pair p's manifolds, the first of them at m
+__device__ __forceinline__ void compact_pair(const CompactArgs& a, int p, int m) {
+    const int nm = a.meshCount[p];
+    const uint64_t key = a.pkeys[p];
     int c0, c1, wd;
-    pair_colliders(key, localBits, worldColStart, colOfLocal, c0, c1, wd);
-    int b0 = (cflags[c0] & CF_DYNAMIC) ? cbody[c0] : -1;
-    int b1 = (cflags[c1] & CF_DYNAMIC) ? cbody[c1] : -1;
+    pair_colliders(key, a.localBits, a.worldColStart, a.colOfLocal, c0, c1, wd);
+    const int b0 = (a.cflags[c0] & CF_DYNAMIC) ? a.cbody[c0] : -1;
+    const int b1 = (a.cflags[c1] & CF_DYNAMIC) ? a.cbody[c1] : -1;
     if (nm == 0) {
-        mfPair[m] = p; mfKey[m] = key; mfB0[m] = b0; mfB1[m] = b1; mfSrc[m] = p; mfTri[m] = -1;
+        a.mfPair[m] = p; a.mfKey[m] = key; a.mfB0[m] = b0; a.mfB1[m] = b1; a.mfSrc[m] = p; a.mfTri[m] = -1;
         return;
     }
-    int first = meshFirst[p];
+    const int first = a.meshFirst[p];
     for (int j = 0; j < nm; ++j) {
-        mfPair[m + j] = p; mfKey[m + j] = key; mfB0[m + j] = b0; mfB1[m + j] = b1;
-        mfSrc[m + j] = pairCap + first + j;
-        mfTri[m + j] = npTri[first + j];
+        a.mfPair[m + j] = p; a.mfKey[m + j] = key; a.mfB0[m + j] = b0; a.mfB1[m + j] = b1;
+        a.mfSrc[m + j] = a.pairCap + first + j;
+        a.mfTri[m + j] = a.npTri[first + j];
+    }
+}
+__global__ void k_compact(int nPairs, CompactArgs a, const int32_t* __restrict__ npIndex) {
+    int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= nPairs || (a.npNum[p] == 0 && a.meshCount[p] == 0)) return;
+    compact_pair(a, p, npIndex[p]);
+}
+
+// k_flag_manifolds, the scan and k_compact of at most MANIFOLDS_SMALL pairs in one workgroup,
+// the scan in registers: five launches of a microsecond or two of work each. 585 pairs: 16 us
+// of kernels before, 3.5 us now; 4,912 pairs 17 us.
+constexpr int MANIFOLDS_THREADS = 1024, MANIFOLDS_ITEMS = 8, MANIFOLDS_SMALL = MANIFOLDS_THREADS * MANIFOLDS_ITEMS;
+__global__ __launch_bounds__(MANIFOLDS_THREADS) void k_manifolds_small(int nPairs, int items, CompactArgs a,
+                                                                       int32_t* __restrict__ npIndex,
+                                                                       const int32_t* __restrict__ flowErr,
+                                                                       int32_t* __restrict__ counters) {
+    __shared__ int32_t waveSum[MANIFOLDS_THREADS / WAVE];
+    const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE, base = threadIdx.x * items;
+    int n[MANIFOLDS_ITEMS], sum = 0;
+#pragma unroll
+    for (int k = 0; k < MANIFOLDS_ITEMS; ++k) {
+        const int p = base + k;
+        n[k] = k < items && p < nPairs ? (a.npNum[p] > 0 ? 1 : 0) + a.meshCount[p] : 0;
+        sum += n[k];
+    }
+    int x = sum;
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == WAVE - 1) waveSum[wv] = x;
+    __syncthreads();
+    int m = x - sum;
+    for (int w = 0; w < wv; ++w) m += waveSum[w];
+    if (threadIdx.x == MANIFOLDS_THREADS - 1) {
+        counters[1] = m + sum;
+        counters[3] = *flowErr;
+    }
+#pragma unroll
+    for (int k = 0; k < MANIFOLDS_ITEMS; ++k) {
+        const int p = base + k;
+        if (k >= items || p >= nPairs) continue;
+        npIndex[p] = m;
+        if (n[k]) compact_pair(a, p, m);
+        m += n[k];
     }
 }
 
@@ -161,6 +207,19 @@ __global__ void k_color_round(int M, int round, const uint64_t* __restrict__ mfK
 // inherited colour (the step colours from scratch). Only new manifolds go through the
 // claim rounds.
 constexpr int CACHE_NUM_MASK = 255, CACHE_COLOR_SHIFT = 8, CACHE_HAS_COLOR = 0x8000;
+// the manifold's place in the previous step's cache, or -1
+__device__ __forceinline__ int cached_manifold(uint64_t key, int tri, const uint64_t* __restrict__ prevKey,
+                                               const int32_t* __restrict__ prevTri, int prevCount) {
+    // the cache is in manifold order, so a pair's manifolds are one run of equal keys
+    int lo = 0, hi = prevCount;
+    while (lo < hi) {
+        int mid = (lo + hi) >> 1;
+        if (prevKey[mid] < key) lo = mid + 1; else hi = mid;
+    }
+    for (; lo < prevCount && prevKey[lo] == key; ++lo)
+        if (prevTri[lo] == tri) return lo;
+    return -1;
+}
 __global__ void k_color_inherit(int M, const uint64_t* __restrict__ mfKey, const int32_t* __restrict__ mfTri,
                                 const uint64_t* __restrict__ prevKey, const int32_t* __restrict__ prevTri,
                                 const int32_t* __restrict__ prevNum, int prevCount, const int32_t* __restrict__ b0,
@@ -171,16 +230,7 @@ __global__ void k_color_inherit(int M, const uint64_t* __restrict__ mfKey, const
     if (m >= M) return;
     const uint64_t key = mfKey[m];
     const int tri = mfTri[m];
-    int prev = -1;
-    {   // the cache is in manifold order, so a pair's manifolds are one run of equal keys
-        int lo = 0, hi = prevCount;
-        while (lo < hi) {
-            int mid = (lo + hi) >> 1;
-            if (prevKey[mid] < key) lo = mid + 1; else hi = mid;
-        }
-        for (; lo < prevCount && prevKey[lo] == key; ++lo)
-            if (prevTri[lo] == tri) { prev = lo; break; }
-    }
+    const int prev = cached_manifold(key, tri, prevKey, prevTri, prevCount);
     mfPrev[m] = prev;
     int c = -1;
     if (prev >= 0) {
@@ -245,6 +295,173 @@ __global__ void k_color_start(int M, int n, const uint64_t* __restrict__ keys, i
         const uint64_t last = M > 0 ? keys[M - 1] : 0ull;
         pack[n + 1] = (int32_t)(uint32_t)last;
         pack[n + 2] = (int32_t)(uint32_t)(last >> 32);
+    }
+}
+
+// The whole colouring of a small scene in one workgroup: k_color_begin, k_color_inherit,
+// k_color_clash, k_color_claim, as many k_color_rounds as are needed, the stable sort into
+// solve order (k_color_keys and the radix sort, here one counting pass over colour and point
+// count), k_color_start and k_color_rank, with the same colours and the same order. The
+// bodies' claims and colour masks are in LDS; one claim buffer does, as a round's losers
+// claim again only after a barrier. Each of those kernels is a microsecond or two of work
+// behind a launch of five, and the host waits for the last: 415 manifolds took thirteen
+// launches, 35 us of kernels and about 5 us of launch each, and take one of 11 us now (3,543
+// manifolds 37 us). The limit is what fits a
+// workgroup's registers and LDS; larger colourings have work for more than one workgroup.
+constexpr int COLOR_THREADS = 1024, COLOR_WAVES = COLOR_THREADS / WAVE, COLOR_ITEMS = 4;
+constexpr int COLOR_SMALL = COLOR_THREADS * COLOR_ITEMS;
+constexpr int COLOR_BINS = 128 << COLOR_KEY_SHIFT, COLOR_STARTS = 130;
+__global__ __launch_bounds__(COLOR_THREADS) void k_color_small(
+    int M, int D, int items, int maxRounds, const uint64_t* __restrict__ mfKey, int worldShift, int32_t* __restrict__ wstart,
+    const int32_t* __restrict__ mfTri, const uint64_t* __restrict__ prevKey, const int32_t* __restrict__ prevTri,
+    const int32_t* __restrict__ prevNum, int prevCount, const int32_t* __restrict__ b0, const int32_t* __restrict__ b1,
+    const int32_t* __restrict__ npNum, const int32_t* __restrict__ mfSrc, int byPoints, int32_t* __restrict__ mfColor,
+    int32_t* __restrict__ mfPrev, uint64_t* __restrict__ usedOut, int32_t* __restrict__ perm, int32_t* __restrict__ rank,
+    int32_t* __restrict__ start, int32_t* __restrict__ pack) {
+    extern __shared__ unsigned long long bodies[];
+    unsigned long long *used = bodies, *claim = bodies + 2 * D;
+    __shared__ int32_t waveCnt[COLOR_WAVES][COLOR_BINS];
+    __shared__ int32_t off[COLOR_BINS], wsum[COLOR_BINS / WAVE];
+    __shared__ int32_t clash, overflow, lastBin;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
+    const int run = wv * WAVE * items + lane;   // the wave's manifolds: run + 64 k, in manifold order
+    for (int i = tid; i < 3 * D; i += COLOR_THREADS) bodies[i] = 0ull;
+    if (tid == 0) { clash = 0; overflow = 0; }
+    int color[COLOR_ITEMS], ba[COLOR_ITEMS], bb[COLOR_ITEMS], world[COLOR_ITEMS];
+#pragma unroll
+    for (int k = 0; k < COLOR_ITEMS; ++k) {
+        color[k] = 0;   // no manifold: nothing to colour
+        const int m = run + k * WAVE;
+        if (k >= items || m >= M) continue;
+        const uint64_t key = mfKey[m];
+        world[k] = (int)(key >> worldShift);
+        if (m == 0 || (int)(mfKey[m - 1] >> worldShift) != world[k]) wstart[world[k]] = m;
+        ba[k] = b0[m];
+        bb[k] = b1[m];
+        const int prev = cached_manifold(key, mfTri[m], prevKey, prevTri, prevCount);
+        mfPrev[m] = prev;
+        color[k] = -1;
+        if (prev >= 0) {
+            const int pn = prevNum[prev];
+            if (pn & CACHE_HAS_COLOR) color[k] = (pn >> CACHE_COLOR_SHIFT) & 127;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < COLOR_ITEMS; ++k) {
+        if (k >= items || run + k * WAVE >= M || color[k] < 0) continue;
+        const unsigned long long bit = 1ull << (color[k] & 63);
+        const int word = color[k] >> 6;
+        bool twice = false;
+        if (ba[k] >= 0) twice |= (atomicOr(&used[2 * ba[k] + word], bit) & bit) != 0;
+        if (bb[k] >= 0) twice |= (atomicOr(&used[2 * bb[k] + word], bit) & bit) != 0;
+        if (twice) clash = 1;
+    }
+    __syncthreads();
+    if (clash) {
+        for (int i = tid; i < 2 * D; i += COLOR_THREADS) used[i] = 0ull;
+        for (int k = 0; k < COLOR_ITEMS; ++k)
+            if (k < items && run + k * WAVE < M) color[k] = -1;
+    }
+    uint32_t prio[COLOR_ITEMS];
+    auto claims = [&](int k, int round) {
+        const unsigned long long v = ((unsigned long long)round << 32) | prio[k];
+        if (ba[k] >= 0) atomicMax(&claim[ba[k]], v);
+        if (bb[k] >= 0) atomicMax(&claim[bb[k]], v);
+    };
+#pragma unroll
+    for (int k = 0; k < COLOR_ITEMS; ++k) {
+        prio[k] = 0;
+        if (color[k] >= 0) continue;
+        prio[k] = mix32((uint32_t)(run + k * WAVE - wstart[world[k]]));
+        claims(k, 1);
+    }
+    int rounds = 0;
+    for (int round = 1; round <= maxRounds; ++round) {
+        __syncthreads();
+        bool lost = false;
+#pragma unroll
+        for (int k = 0; k < COLOR_ITEMS; ++k) {
+            if (color[k] >= 0) continue;
+            const unsigned long long v = ((unsigned long long)round << 32) | prio[k];
+            const int a = ba[k], b = bb[k];
+            if ((a >= 0 && claim[a] != v) || (b >= 0 && claim[b] != v)) { lost = true; continue; }
+            uint64_t lo = 0, hi = 0;
+            if (a >= 0) { lo |= used[2 * a]; hi |= used[2 * a + 1]; }
+            if (b >= 0) { lo |= used[2 * b]; hi |= used[2 * b + 1]; }
+            int c;
+            if (~lo) c = __ffsll((long long)~lo) - 1;
+            else if (~hi) c = 64 + __ffsll((long long)~hi) - 1;
+            else { c = 127; overflow = 1; }   // reported as an error by the host
+            color[k] = c;
+            const uint64_t bl = c < 64 ? (1ull << c) : 0ull, bh = c >= 64 ? (1ull << (c - 64)) : 0ull;
+            if (a >= 0) { used[2 * a] |= bl; used[2 * a + 1] |= bh; }
+            if (b >= 0) { used[2 * b] |= bl; used[2 * b + 1] |= bh; }
+        }
+        if (!__syncthreads_or(lost)) { rounds = round; break; }
+#pragma unroll
+        for (int k = 0; k < COLOR_ITEMS; ++k)
+            if (color[k] < 0) claims(k, round + 1);
+    }
+    for (int i = tid; i < 2 * D; i += COLOR_THREADS) usedOut[i] = used[i];
+    // solve order, as k_rs_single ranks and places one digit
+    const uint64_t lt = (1ull << lane) - 1ull;
+    for (int d = lane; d < COLOR_BINS; d += WAVE) waveCnt[wv][d] = 0;
+    uint32_t bin[COLOR_ITEMS];
+    int32_t place[COLOR_ITEMS];
+#pragma unroll
+    for (int k = 0; k < COLOR_ITEMS; ++k) {
+        const int m = run + k * WAVE;
+        const bool have = k < items && m < M;
+        bin[k] = 0;
+        if (have) {
+            mfColor[m] = color[k];
+            const int num = byPoints ? min(max(npNum[mfSrc[m]], 1), 4) : 1;
+            bin[k] = (uint32_t)(max(color[k], 0) << COLOR_KEY_SHIFT | (num - 1));
+        }
+        if (k < items) place[k] = rs_rank(bin[k], have, 7 + COLOR_KEY_SHIFT, lt, waveCnt[wv]);
+    }
+    __syncthreads();
+    int32_t total = 0, x = 0;
+    if (tid < COLOR_BINS) {
+#pragma unroll
+        for (int w = 0; w < COLOR_WAVES; ++w) {
+            const int32_t c = waveCnt[w][tid];
+            waveCnt[w][tid] = total;
+            total += c;
+        }
+        x = total;
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const int32_t y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        if (lane == WAVE - 1) wsum[wv] = x;
+    }
+    __syncthreads();
+    if (tid < COLOR_BINS) {
+        int32_t before = 0;
+        for (int w = 0; w < COLOR_BINS / WAVE; ++w) before += w < wv ? wsum[w] : 0;
+        off[tid] = before + x - total;
+        if (total > 0 && before + x == M) lastBin = tid;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < COLOR_ITEMS; ++k) {
+        const int m = run + k * WAVE;
+        if (k >= items || m >= M) continue;
+        const int pos = off[bin[k]] + waveCnt[wv][bin[k]] + place[k];
+        perm[pos] = m;
+        rank[m] = pos;
+    }
+    if (tid < COLOR_STARTS) {
+        const int at = tid < 128 ? off[tid << COLOR_KEY_SHIFT] : M;
+        start[tid] = at;
+        pack[tid] = at;
+    }
+    if (tid == 0) {   // after the starts: the overflow flag, the colours, the rounds (0: too many)
+        pack[COLOR_STARTS] = overflow;
+        pack[COLOR_STARTS + 1] = (lastBin >> COLOR_KEY_SHIFT) + 1;
+        pack[COLOR_STARTS + 2] = rounds;
     }
 }
 
@@ -1397,9 +1614,18 @@ int sv_setup_manifolds(World& w, int nPairs) {
     if (nPairs == 0) return 0;
     // manifold index of every pair with points: exclusive scan of the hit flags (the pair
     // sort's value buffer is free at this point and holds the flags)
-    hipLaunchKernelGGL(k_flag_manifolds, dim3(div_up(nPairs, 256)), dim3(256), 0, s, nPairs, w.npNum.p,
-                       w.meshCount.p, w.pvals.p);
-    exclusive_scan_i32(s, w.pvals.p, w.npIndex.p, nPairs, w.counters.p + 1, w.scanT);
+    const CompactArgs ca{w.npNum.p, w.meshFirst.p, w.meshCount.p, w.npTri.p, w.pairCap, w.localBits, w.pkeys.p,
+                         w.worldColStart.p, w.colOfLocal.p, w.cbody.p, w.cflags.p, w.mfPair.p, w.mfKey.p, w.mfB0.p,
+                         w.mfB1.p, w.mfSrc.p, w.mfTri.p};
+    const bool small = nPairs <= MANIFOLDS_SMALL;
+    if (small) {
+        hipLaunchKernelGGL(k_manifolds_small, dim3(1), dim3(MANIFOLDS_THREADS), 0, s, nPairs,
+                           div_up(nPairs, MANIFOLDS_THREADS), ca, w.npIndex.p, w.flowErr.p, w.counters.p);
+    } else {
+        hipLaunchKernelGGL(k_flag_manifolds, dim3(div_up(nPairs, 256)), dim3(256), 0, s, nPairs, w.npNum.p,
+                           w.meshCount.p, w.pvals.p, w.flowErr.p, w.counters.p);
+        exclusive_scan_i32(s, w.pvals.p, w.npIndex.p, nPairs, w.counters.p + 1, w.scanT);
+    }
     int M = 0, epaErrors = 0, flowErr = 0;
     int meshInfo[3] = {0, 0, 0};   // mesh pairs, mesh manifold slots, mesh capacity errors
     // the counters (manifold total, EPA and mesh counts) and the previous step's
@@ -1410,18 +1636,16 @@ int sv_setup_manifolds(World& w, int nPairs) {
     w.readHost.alloc(READ_HOST_INTS);
     int32_t* rb = w.readHost.p;
     PGX_HIP(hipMemcpyAsync(rb, w.counters.p, 16 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    PGX_HIP(hipMemcpyAsync(rb + 16, w.flowErr.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     if (lastQueues) {
         PGX_HIP(hipMemcpyAsync(qDone, w.qDone.p, sizeof(qDone), hipMemcpyDeviceToHost, s));
         PGX_HIP(hipMemcpyAsync(qStart, w.qStart.p, sizeof(int) * (lastQueues + 1), hipMemcpyDeviceToHost, s));
     }
-    hipLaunchKernelGGL(k_compact, dim3(div_up(nPairs, 256)), dim3(256), 0, s, nPairs, w.npNum.p, w.npIndex.p,
-                       w.meshFirst.p, w.meshCount.p, w.npTri.p, w.pairCap, w.pkeys.p, w.localBits, w.worldColStart.p, w.colOfLocal.p, w.cbody.p, w.cflags.p,
-                       w.mfPair.p, w.mfKey.p, w.mfB0.p, w.mfB1.p, w.mfSrc.p, w.mfTri.p);
+    if (!small)
+        hipLaunchKernelGGL(k_compact, dim3(div_up(nPairs, 256)), dim3(256), 0, s, nPairs, ca, w.npIndex.p);
     PGX_LAUNCH_CHECK();
     PGX_HIP(hipStreamSynchronize(s));
     M = rb[1];
-    flowErr = rb[16];
+    flowErr = rb[3];
     if (w.nConvex) epaErrors = rb[9];
     if (w.nTriMesh) std::copy(rb + 10, rb + 13, meshInfo);
     if (flowErr)
@@ -1442,6 +1666,36 @@ int sv_setup_manifolds(World& w, int nPairs) {
     return M;
 }
 
+constexpr int MAX_ROUNDS = 1024;
+
+// The colouring of at most COLOR_SMALL manifolds and bodies: one launch and the read-back.
+static int color_small(World& w, int M, std::vector<int32_t>& starts, int& nColors) {
+    hipStream_t s = w.stream;
+    w.colorPack.alloc(133 + MAX_ROUNDS + 1);
+    w.readHost.alloc(READ_HOST_INTS);
+    w.mfPrev.alloc(w.manifoldCap);
+    if (!w.colorLdsSet) {
+        PGX_HIP(hipFuncSetAttribute((const void*)k_color_small, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)(3 * sizeof(uint64_t) * COLOR_SMALL)));
+        w.colorLdsSet = true;
+    }
+    const int prv = w.cacheCur;
+    hipLaunchKernelGGL(k_color_small, dim3(1), dim3(COLOR_THREADS), 3 * sizeof(uint64_t) * (size_t)w.D, s, M, w.D,
+                       div_up(M, COLOR_THREADS), MAX_ROUNDS, w.mfKey.p, 2 * w.localBits, w.worldMStart.p, w.mfTri.p,
+                       w.cacheKey[prv].p, w.cacheTri[prv].p, w.cacheNum[prv].p, w.cacheCount[prv], w.mfB0.p, w.mfB1.p,
+                       w.npNum.p, w.mfSrc.p, w.execMode == EXEC_WORLDS ? 0 : 1, w.mfColor.p, w.mfPrev.p, w.usedMask.p,
+                       w.colorPerm.p, w.colorRank.p, w.colorCount.p, w.colorPack.p);
+    PGX_LAUNCH_CHECK();
+    PGX_HIP(hipMemcpyAsync(w.readHost.p, w.colorPack.p, sizeof(int32_t) * 133, hipMemcpyDeviceToHost, s));
+    PGX_HIP(hipStreamSynchronize(s));
+    const int32_t* rb = w.readHost.p;
+    if (rb[130]) throw PgxError{PGX_ERR_CAPACITY, "a body touches more than 127 contact colours"};
+    if (rb[132] == 0) throw PgxError{PGX_ERR_INVALID, "graph colouring did not converge"};
+    std::copy(rb, rb + 130, starts.begin());
+    nColors = rb[131];
+    return rb[132];
+}
+
 int sv_color(World& w, int M) {
     hipStream_t s = w.stream;
     const int prevRounds = w.lastRounds;
@@ -1452,78 +1706,83 @@ int sv_color(World& w, int M) {
     }
     int worldShift = 2 * w.localBits;
     int nb = div_up(M, 256);
-    constexpr int MAX_ROUNDS = 1024;
-    static_assert(133 + MAX_ROUNDS + 1 <= READ_HOST_INTS, "the colouring's read-back fits the pinned buffer");
-    w.colorUncol.alloc(MAX_ROUNDS + 1);
-    w.colorPack.alloc(133 + MAX_ROUNDS + 1);
-    w.readHost.alloc(READ_HOST_INTS);
-    w.claim2.alloc(std::max(w.D, 1));
-    w.mfPrev.alloc(w.manifoldCap);
-    w.colorFlag.alloc(1);
-    hipLaunchKernelGGL(k_color_begin, dim3(div_up(std::max({M, 2 * w.D, MAX_ROUNDS + 1}), 256)), dim3(256), 0, s, M,
-                       w.D, MAX_ROUNDS + 1, w.mfKey.p, worldShift, w.worldMStart.p, w.mfColor.p, w.claim.p,
-                       w.claim2.p, w.usedMask.p, w.colorUncol.p, w.counters.p + 5, w.colorFlag.p);
-    unsigned long long* claims[2] = {(unsigned long long*)w.claim.p, (unsigned long long*)w.claim2.p};
-    // colours of the manifolds that persist from the previous step; only new ones are
-    // coloured in the rounds below
-    const int prevCache = w.cacheCur;
-    hipLaunchKernelGGL(k_color_inherit, dim3(nb), dim3(256), 0, s, M, w.mfKey.p, w.mfTri.p, w.cacheKey[prevCache].p,
-                       w.cacheTri[prevCache].p, w.cacheNum[prevCache].p, w.cacheCount[prevCache], w.mfB0.p, w.mfB1.p,
-                       w.mfColor.p,
-                       w.mfPrev.p, (unsigned long long*)w.usedMask.p, w.colorFlag.p);
-    hipLaunchKernelGGL(k_color_clash, dim3(div_up(std::max(M, 2 * w.D), 256)), dim3(256), 0, s, M, w.D, w.colorFlag.p,
-                       w.mfColor.p, w.usedMask.p);
-    // round-1 claims
-    hipLaunchKernelGGL(k_color_claim, dim3(nb), dim3(256), 0, s, M, 1, w.mfKey.p, worldShift, w.worldMStart.p,
-                       w.mfColor.p, w.mfB0.p, w.mfB1.p, claims[1]);
-    // Rounds are queued in batches sized from the last step's count (a round after the last
-    // one needed exits at once); the sort into colour order and the colour starts follow,
-    // and one read-back tells whether the batch finished, with the counts and starts. Only
-    // a batch that ran short is followed by another (and the sort is redone).
-    int round = 0;
-    int batch = std::min(MAX_ROUNDS, std::max(w.tune.colorRounds, prevRounds + 4));
-    std::vector<int32_t> starts(130, 0), uc;
-    uint64_t lastKey = 0;
-    while (true) {
-        for (int r = 0; r < batch && round < MAX_ROUNDS; ++r) {
-            ++round;
-            hipLaunchKernelGGL(k_color_round, dim3(nb), dim3(256), 0, s, M, round, w.mfKey.p, worldShift,
-                               w.worldMStart.p, w.mfColor.p, w.mfB0.p, w.mfB1.p,
-                               (const unsigned long long*)claims[round & 1], claims[(round + 1) & 1], w.usedMask.p,
-                               w.colorUncol.p, w.counters.p);
+    std::vector<int32_t> starts(130, 0);
+    int nColors = 0;
+    if (M <= COLOR_SMALL && w.D <= COLOR_SMALL) {
+        w.lastRounds = color_small(w, M, starts, nColors);
+    } else {
+        static_assert(133 + MAX_ROUNDS + 1 <= READ_HOST_INTS, "the colouring's read-back fits the pinned buffer");
+        w.colorUncol.alloc(MAX_ROUNDS + 1);
+        w.colorPack.alloc(133 + MAX_ROUNDS + 1);
+        w.readHost.alloc(READ_HOST_INTS);
+        w.claim2.alloc(std::max(w.D, 1));
+        w.mfPrev.alloc(w.manifoldCap);
+        w.colorFlag.alloc(1);
+        hipLaunchKernelGGL(k_color_begin, dim3(div_up(std::max({M, 2 * w.D, MAX_ROUNDS + 1}), 256)), dim3(256), 0, s, M,
+                           w.D, MAX_ROUNDS + 1, w.mfKey.p, worldShift, w.worldMStart.p, w.mfColor.p, w.claim.p,
+                           w.claim2.p, w.usedMask.p, w.colorUncol.p, w.counters.p + 5, w.colorFlag.p);
+        unsigned long long* claims[2] = {(unsigned long long*)w.claim.p, (unsigned long long*)w.claim2.p};
+        // colours of the manifolds that persist from the previous step; only new ones are
+        // coloured in the rounds below
+        const int prevCache = w.cacheCur;
+        hipLaunchKernelGGL(k_color_inherit, dim3(nb), dim3(256), 0, s, M, w.mfKey.p, w.mfTri.p, w.cacheKey[prevCache].p,
+                           w.cacheTri[prevCache].p, w.cacheNum[prevCache].p, w.cacheCount[prevCache], w.mfB0.p, w.mfB1.p,
+                           w.mfColor.p,
+                           w.mfPrev.p, (unsigned long long*)w.usedMask.p, w.colorFlag.p);
+        hipLaunchKernelGGL(k_color_clash, dim3(div_up(std::max(M, 2 * w.D), 256)), dim3(256), 0, s, M, w.D, w.colorFlag.p,
+                           w.mfColor.p, w.usedMask.p);
+        // round-1 claims
+        hipLaunchKernelGGL(k_color_claim, dim3(nb), dim3(256), 0, s, M, 1, w.mfKey.p, worldShift, w.worldMStart.p,
+                           w.mfColor.p, w.mfB0.p, w.mfB1.p, claims[1]);
+        // Rounds are queued in batches sized from the last step's count (a round after the last
+        // one needed exits at once); the sort into colour order and the colour starts follow,
+        // and one read-back tells whether the batch finished, with the counts and starts. Only
+        // a batch that ran short is followed by another (and the sort is redone).
+        int round = 0;
+        int batch = std::min(MAX_ROUNDS, std::max(w.tune.colorRounds, prevRounds + 4));
+        std::vector<int32_t> uc;
+        uint64_t lastKey = 0;
+        while (true) {
+            for (int r = 0; r < batch && round < MAX_ROUNDS; ++r) {
+                ++round;
+                hipLaunchKernelGGL(k_color_round, dim3(nb), dim3(256), 0, s, M, round, w.mfKey.p, worldShift,
+                                   w.worldMStart.p, w.mfColor.p, w.mfB0.p, w.mfB1.p,
+                                   (const unsigned long long*)claims[round & 1], claims[(round + 1) & 1], w.usedMask.p,
+                                   w.colorUncol.p, w.counters.p);
+            }
+            // stable sort by colour and point count -> solve order
+            hipLaunchKernelGGL(k_color_keys, dim3(nb), dim3(256), 0, s, M, w.mfColor.p, w.npNum.p, w.mfSrc.p,
+                               w.execMode == EXEC_WORLDS ? 0 : 1, w.colorKeys.p, w.colorPerm.p);
+            radix_sort_u64(s, w.colorKeys.p, w.colorPerm.p, M, 7 + COLOR_KEY_SHIFT, w.sortT);
+            hipLaunchKernelGGL(k_color_start, dim3(1), dim3(256), 0, s, M, 130, w.colorKeys.p, w.colorCount.p, round,
+                               w.colorUncol.p, w.counters.p + 5, w.colorPack.p);
+            PGX_LAUNCH_CHECK();
+            // one copy to pinned host memory brings the starts, the overflow flag, the last key
+            // and the per-round counts
+            const size_t packed = 133 + (size_t)round + 1;
+            PGX_HIP(hipMemcpyAsync(w.readHost.p, w.colorPack.p, sizeof(int32_t) * packed, hipMemcpyDeviceToHost, s));
+            PGX_HIP(hipStreamSynchronize(s));
+            const int32_t* rb = w.readHost.p;
+            const int ovf = rb[130];
+            lastKey = (uint64_t)(uint32_t)rb[131] | ((uint64_t)(uint32_t)rb[132] << 32);
+            std::copy(rb, rb + 130, starts.begin());
+            uc.assign(rb + 133, rb + 133 + round + 1);
+            if (ovf) throw PgxError{PGX_ERR_CAPACITY, "a body touches more than 127 contact colours"};
+            if (uc[round] == 0) break;
+            if (round >= MAX_ROUNDS) throw PgxError{PGX_ERR_INVALID, "graph colouring did not converge"};
+            batch = 16;
         }
-        // stable sort by colour and point count -> solve order
-        hipLaunchKernelGGL(k_color_keys, dim3(nb), dim3(256), 0, s, M, w.mfColor.p, w.npNum.p, w.mfSrc.p,
-                           w.execMode == EXEC_WORLDS ? 0 : 1, w.colorKeys.p, w.colorPerm.p);
-        radix_sort_u64(s, w.colorKeys.p, w.colorPerm.p, M, 7 + COLOR_KEY_SHIFT, w.sortT);
-        hipLaunchKernelGGL(k_color_start, dim3(1), dim3(256), 0, s, M, 130, w.colorKeys.p, w.colorCount.p, round,
-                           w.colorUncol.p, w.counters.p + 5, w.colorPack.p);
-        PGX_LAUNCH_CHECK();
-        // one copy to pinned host memory brings the starts, the overflow flag, the last key
-        // and the per-round counts
-        const size_t packed = 133 + (size_t)round + 1;
-        PGX_HIP(hipMemcpyAsync(w.readHost.p, w.colorPack.p, sizeof(int32_t) * packed, hipMemcpyDeviceToHost, s));
-        PGX_HIP(hipStreamSynchronize(s));
-        const int32_t* rb = w.readHost.p;
-        const int ovf = rb[130];
-        lastKey = (uint64_t)(uint32_t)rb[131] | ((uint64_t)(uint32_t)rb[132] << 32);
-        std::copy(rb, rb + 130, starts.begin());
-        uc.assign(rb + 133, rb + 133 + round + 1);
-        if (ovf) throw PgxError{PGX_ERR_CAPACITY, "a body touches more than 127 contact colours"};
-        if (uc[round] == 0) break;
-        if (round >= MAX_ROUNDS) throw PgxError{PGX_ERR_INVALID, "graph colouring did not converge"};
-        batch = 16;
+        // rounds actually used: the first whose count of uncoloured manifolds is zero
+        int used = round;
+        for (int r = 1; r <= round; ++r)
+            if (uc[r] == 0) { used = r; break; }
+        nColors = (int)(lastKey >> COLOR_KEY_SHIFT) + 1;
+        w.lastRounds = used;
+        hipLaunchKernelGGL(k_color_rank, dim3(nb), dim3(256), 0, s, M, w.colorPerm.p, w.colorRank.p);
     }
-    // rounds actually used: the first whose count of uncoloured manifolds is zero
-    int used = round;
-    for (int r = 1; r <= round; ++r)
-        if (uc[r] == 0) { used = r; break; }
-    int nColors = (int)(lastKey >> COLOR_KEY_SHIFT) + 1;
     w.colorStartHost.assign(starts.begin(), starts.begin() + nColors + 1);
-    w.lastRounds = used;
     // contact setup, written in solve order
     int cur = w.cacheCur ^ 1, prv = w.cacheCur;
-    hipLaunchKernelGGL(k_color_rank, dim3(nb), dim3(256), 0, s, M, w.colorPerm.p, w.colorRank.p);
     hipLaunchKernelGGL(k_setup, dim3(nb), dim3(256), 0, s, M, w.manifoldCap, w.colorRank.p, w.mfSrc.p, w.mfTri.p,
                        w.mfKey.p,
                        w.localBits, w.worldColStart.p, w.colOfLocal.p, w.cbody.p, w.cflags.p, w.cmat.p, w.npNum.p,

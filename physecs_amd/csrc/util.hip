@@ -29,19 +29,6 @@ __device__ __forceinline__ uint32_t rs_digit(uint64_t k, int shift, int dbits) {
     return (uint32_t)(k >> shift) & ((1u << dbits) - 1u);
 }
 
-// rank of the lane's element among the wave's elements of the same digit so far; bumps the
-// wave's count of the digit (counts: this wave's RS_BINS counters in LDS)
-__device__ __forceinline__ int32_t rs_rank(uint32_t d, bool ok, int dbits, uint64_t lt, int32_t* counts) {
-    uint64_t same = __ballot(ok);
-    for (int b = 0; b < dbits; ++b) {
-        const uint64_t bal = __ballot((d >> b) & 1u);
-        same &= ((d >> b) & 1u) ? bal : ~bal;
-    }
-    const int32_t prior = counts[d];
-    if (ok && (same & lt) == 0ull) counts[d] = prior + (int32_t)__popcll(same);
-    return prior + (int32_t)__popcll(same & lt);
-}
-
 // The tile's digit counts with LDS atomics, every key load issued before the counting. (A
 // ballot-ranked count per wave, free of the atomics' bank conflicts on nearly sorted keys,
 // measured slower: 11.9 against 6.4 us per pass on the 32k scene's 16-key tiles.)

@@ -1,0 +1,39 @@
+"""Small scenes list and colour their manifolds in one workgroup; larger ones in a launch per
+phase. A world's colouring does not depend on the worlds beside it, so the same worlds alone
+(one workgroup) and in a batch of more than 4,096 bodies (a launch per phase) must step to the
+same bits; and a pile on either side of the limits must be coloured properly and match the
+oracle fed its order."""
+import numpy as np
+import pytest
+
+from gpu_util import bits, lockstep, log
+from physecs_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def test_worlds_alone_and_in_a_large_batch():
+    from physecs_amd import api
+    sc = scenes.batched_worlds(8, n_worlds=60, lo=60, hi=140, ragdoll_frac=0.3)
+    assert sc.n_dyn > 4096
+    log(f"[small] {sc.n_dyn} bodies in 60 worlds against worlds alone")
+    big = api.World(sc, substeps=4, iterations=2)
+    arr = sc.arrays()
+    picks = {w: api.World(sc.world_subscene(w), substeps=4, iterations=2) for w in (0, 7, 33, 59)}
+    for k in range(40):
+        big.step(1 / 60)
+        for g in picks.values():
+            g.step(1 / 60)
+    pos = big.state()[0]
+    for w, g in picks.items():
+        assert np.array_equal(bits(pos[arr["world"] == w]), bits(g.state()[0])), w
+        assert 0 < g.counts()["manifolds"] < 4096
+        g.close()
+    big.close()
+
+
+@pytest.mark.parametrize("side", [1, 2, 10, 15, 17])
+def test_piles_lockstep_bitexact(side):
+    """1 to 4,913 bodies: one to four manifolds a thread, and beyond the limit."""
+    log(f"[small] a pile of {side ** 3} bodies")
+    lockstep(scenes.mixed_lattice(5, side=side), 30 if side < 15 else 12, check_every=6)
