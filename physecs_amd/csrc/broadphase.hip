@@ -8,6 +8,7 @@
 // src/BoundsUtil.cpp:35-59 with the reference's margin rule: none at creation, +0.01 for
 // the colliders of non-kinematic dynamic bodies after every step (Physecs.cpp:32,79-90).
 #include "pgx_internal.h"
+#include "radix_block.h"
 #include "shape_bounds.h"
 
 namespace pgx {
@@ -150,21 +151,23 @@ __global__ void k_scene_bounds_init(uint32_t* wb, double* mom, int32_t* counters
     if (counters && threadIdx.x < 16) counters[threadIdx.x] = 0;
 }
 
-// The dynamic colliders' centres: their box (min, max per axis) and their sums and sums of
-// squares per axis (the Morton box and the grid below); and the colliders' largest extent
-// per axis (wb[6..8], as float bits: extents are >= 0, so the bits order like the values). One block of 1024 threads reduces its share with
-// wave shuffles and per-wave partials in LDS, then 6 integer and 6 double atomics per block.
-__global__ __launch_bounds__(1024) void k_scene_bounds(int n, const int32_t* __restrict__ dynCols,
-                                                       const float4* __restrict__ bmin,
-                                                       const float4* __restrict__ bmax, uint32_t* __restrict__ wb,
-                                                       double* __restrict__ mom) {
-    __shared__ uint32_t red[9];
-    __shared__ double part[1024 / WAVE][6];
-    if (threadIdx.x < 3) { red[threadIdx.x] = 0xffffffffu; red[3 + threadIdx.x] = 0u; red[6 + threadIdx.x] = 0u; }
+struct BoundsLds {
+    uint32_t red[9];
+    double part[1024 / WAVE][6];
+    __device__ double moment(int k) const {
+        double t = 0.0;
+        for (int w = 0; w < (int)blockDim.x / WAVE; ++w) t += part[w][k];
+        return t;
+    }
+};
+// one workgroup's share (first, first + stride, ...) of k_scene_bounds
+__device__ __forceinline__ void block_bounds(BoundsLds& L, int first, int stride, int n, const int32_t* __restrict__ dynCols,
+                                             const float4* __restrict__ bmin, const float4* __restrict__ bmax) {
+    if (threadIdx.x < 3) { L.red[threadIdx.x] = 0xffffffffu; L.red[3 + threadIdx.x] = 0u; L.red[6 + threadIdx.x] = 0u; }
     __syncthreads();
     uint32_t mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u}, ex[3] = {0u, 0u, 0u};
     double sm[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = first; i < n; i += stride) {
         int c = dynCols[i];
         float4 a = bmin[c], b = bmax[c];
         const float cc[3] = {0.5f * (a.x + b.x), 0.5f * (a.y + b.y), 0.5f * (a.z + b.z)};
@@ -188,20 +191,28 @@ __global__ __launch_bounds__(1024) void k_scene_bounds(int n, const int32_t* __r
     }
     const int wv = threadIdx.x / WAVE;
     if ((threadIdx.x & (WAVE - 1)) == 0) {
-        for (int k = 0; k < 3; ++k) { atomicMin(&red[k], mn[k]); atomicMax(&red[3 + k], mx[k]); atomicMax(&red[6 + k], ex[k]); }
-        for (int k = 0; k < 6; ++k) part[wv][k] = sm[k];
+        for (int k = 0; k < 3; ++k) { atomicMin(&L.red[k], mn[k]); atomicMax(&L.red[3 + k], mx[k]); atomicMax(&L.red[6 + k], ex[k]); }
+        for (int k = 0; k < 6; ++k) L.part[wv][k] = sm[k];
     }
     __syncthreads();
+}
+
+// The dynamic colliders' centres: their box (min, max per axis) and their sums and sums of
+// squares per axis (the Morton box and the grid below); and the colliders' largest extent
+// per axis (wb[6..8], as float bits: extents are >= 0, so the bits order like the values). One block of 1024 threads reduces its share with
+// wave shuffles and per-wave partials in LDS, then 6 integer and 6 double atomics per block.
+__global__ __launch_bounds__(1024) void k_scene_bounds(int n, const int32_t* __restrict__ dynCols,
+                                                       const float4* __restrict__ bmin,
+                                                       const float4* __restrict__ bmax, uint32_t* __restrict__ wb,
+                                                       double* __restrict__ mom) {
+    __shared__ BoundsLds L;
+    block_bounds(L, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, n, dynCols, bmin, bmax);
     if (threadIdx.x < 3) {
-        atomicMin(&wb[threadIdx.x], red[threadIdx.x]);
-        atomicMax(&wb[3 + threadIdx.x], red[3 + threadIdx.x]);
-        atomicMax(&wb[6 + threadIdx.x], red[6 + threadIdx.x]);
+        atomicMin(&wb[threadIdx.x], L.red[threadIdx.x]);
+        atomicMax(&wb[3 + threadIdx.x], L.red[3 + threadIdx.x]);
+        atomicMax(&wb[6 + threadIdx.x], L.red[6 + threadIdx.x]);
     }
-    if (threadIdx.x < 6) {
-        double t = 0.0;
-        for (int w = 0; w < (int)blockDim.x / WAVE; ++w) t += part[w][threadIdx.x];
-        atomicAdd(&mom[threadIdx.x], t);
-    }
+    if (threadIdx.x < 6) atomicAdd(&mom[threadIdx.x], L.moment(threadIdx.x));
 }
 
 __device__ __forceinline__ uint32_t spread10(uint32_t v) {
@@ -310,6 +321,16 @@ __device__ __forceinline__ void grid_frame(const uint32_t* __restrict__ wb, cons
     }
 }
 
+// collider c's cell key
+__device__ __forceinline__ uint64_t cell_key(int c, const float lo[3], const float h[3], const int32_t* __restrict__ cworld,
+                                             const float4* __restrict__ bmin, const float4* __restrict__ bmax) {
+    const float4 a = bmin[c], b = bmax[c];
+    const float cc[3] = {0.5f * (a.x + b.x), 0.5f * (a.y + b.y), 0.5f * (a.z + b.z)};
+    uint32_t q[3];
+    for (int k = 0; k < 3; ++k) q[k] = (uint32_t)fminf(fmaxf(floorf((cc[k] - lo[k]) / h[k]), 0.f), 1023.f);
+    return ((uint64_t)cworld[c] << 30) | (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
+}
+
 __global__ void k_cell_codes(int n, const int32_t* __restrict__ dynCols, const int32_t* __restrict__ cworld,
                              const float4* __restrict__ bmin, const float4* __restrict__ bmax,
                              const uint32_t* __restrict__ wb, const double* __restrict__ mom, uint64_t* __restrict__ keys,
@@ -319,12 +340,8 @@ __global__ void k_cell_codes(int n, const int32_t* __restrict__ dynCols, const i
     if (i >= n) return;
     float lo[3], h[3];
     grid_frame(wb, mom, n, lo, h);
-    int c = dynCols[i];
-    float4 a = bmin[c], b = bmax[c];
-    const float cc[3] = {0.5f * (a.x + b.x), 0.5f * (a.y + b.y), 0.5f * (a.z + b.z)};
-    uint32_t q[3];
-    for (int k = 0; k < 3; ++k) q[k] = (uint32_t)fminf(fmaxf(floorf((cc[k] - lo[k]) / h[k]), 0.f), 1023.f);
-    keys[i] = ((uint64_t)cworld[c] << 30) | (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
+    const int c = dynCols[i];
+    keys[i] = cell_key(c, lo, h, cworld, bmin, bmax);
     vals[i] = c;
 }
 
@@ -392,29 +409,107 @@ __global__ __launch_bounds__(256) void k_cell_ends(int n, const uint64_t* __rest
 // {min xyz, world-local index}, {max xyz, entity}; a disabled collider gets an empty box, so
 // it overlaps nothing. And the world's non-dynamic colliders, as k_pack writes them for the
 // tree walk.
+__device__ __forceinline__ void grid_record(int t, int c, const float4* __restrict__ cbmin, const float4* __restrict__ cbmax,
+                                            const int32_t* __restrict__ cflags, const uint32_t* __restrict__ centity,
+                                            const int32_t* __restrict__ clocal, float4* __restrict__ gridRec) {
+    float4 a = cbmin[c], b = cbmax[c];
+    if (!(cflags[c] & CF_ENABLE)) {
+        a = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+        b = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    }
+    gridRec[2 * t] = make_float4(a.x, a.y, a.z, __int_as_float(clocal[c]));
+    gridRec[2 * t + 1] = make_float4(b.x, b.y, b.z, __int_as_float((int)centity[c]));
+}
+__device__ __forceinline__ void static_record(int t, int c, const float4* __restrict__ cbmin, const float4* __restrict__ cbmax,
+                                              const int32_t* __restrict__ cflags, const uint32_t* __restrict__ centity,
+                                              const int32_t* __restrict__ clocal, float4* __restrict__ statA,
+                                              float4* __restrict__ statB, int32_t* __restrict__ statL) {
+    const float4 a = cbmin[c], b = cbmax[c];
+    statA[t] = make_float4(a.x, a.y, a.z, __int_as_float(cflags[c]));
+    statB[t] = make_float4(b.x, b.y, b.z, __int_as_float((int)centity[c]));
+    statL[t] = clocal[c];
+}
+
 __global__ void k_grid_pack(int n, const int32_t* __restrict__ order, const float4* __restrict__ cbmin,
                             const float4* __restrict__ cbmax, const int32_t* __restrict__ cflags,
                             const uint32_t* __restrict__ centity, const int32_t* __restrict__ clocal,
                             float4* __restrict__ gridRec, int nStatic, const int32_t* __restrict__ staticCols,
                             float4* __restrict__ statA, float4* __restrict__ statB, int32_t* __restrict__ statL) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) {
-        const int c = order[t];
-        float4 a = cbmin[c], b = cbmax[c];
-        if (!(cflags[c] & CF_ENABLE)) {
-            a = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
-            b = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    if (t < n) grid_record(t, order[t], cbmin, cbmax, cflags, centity, clocal, gridRec);
+    if (t < nStatic) static_record(t, staticCols[t], cbmin, cbmax, cflags, centity, clocal, statA, statB, statL);
+}
+
+// The grid of at most GRID_SMALL dynamic colliders in one workgroup: k_scene_bounds_init,
+// k_scene_bounds, k_cell_codes, the sort, k_grid_pack, k_cell_insert and k_cell_ends, each a
+// microsecond or two of work behind a launch of five. The keys stay in registers and LDS; a
+// run's first collider finds the run's end in them, so the table is not read back. (The sums
+// behind the cells' frame are added in another order than k_scene_bounds adds them over
+// several workgroups; the pairs do not depend on the frame.) 210 colliders: seven launches and
+// 29 us of kernels before, 17 us now. 3,072 colliders take 57 us, no less than the launches.
+constexpr int GRID_SMALL = 2048;
+__global__ __launch_bounds__(RS_SINGLE_THREADS) void k_grid_small(
+    int n, int items, int bits, const int32_t* __restrict__ dynCols, const int32_t* __restrict__ cworld,
+    const float4* __restrict__ cbmin, const float4* __restrict__ cbmax, const int32_t* __restrict__ cflags,
+    const uint32_t* __restrict__ centity, const int32_t* __restrict__ clocal, uint64_t* __restrict__ keys,
+    int32_t* __restrict__ vals, uint32_t mask, uint64_t* __restrict__ tabKey, int32_t* __restrict__ tabStart,
+    int32_t* __restrict__ tabEnd, float4* __restrict__ gridRec, int nStatic, const int32_t* __restrict__ staticCols,
+    float4* __restrict__ statA, float4* __restrict__ statB, int32_t* __restrict__ statL, int32_t* __restrict__ counters) {
+    __shared__ RsBlock B;
+    __shared__ BoundsLds L;
+    __shared__ double mom[6];
+    __shared__ int32_t longest;
+    const int tid = threadIdx.x;
+    for (uint32_t i = tid; i <= mask; i += blockDim.x) tabKey[i] = GRID_EMPTY;
+    if (tid < 16) counters[tid] = 0;
+    if (tid == 0) longest = 0;
+    for (int t = tid; t < nStatic; t += blockDim.x)
+        static_record(t, staticCols[t], cbmin, cbmax, cflags, centity, clocal, statA, statB, statL);
+    block_bounds(L, tid, blockDim.x, n, dynCols, cbmin, cbmax);
+    if (tid < 6) mom[tid] = L.moment(tid);
+    __threadfence();   // the cleared table, before the claims
+    __syncthreads();
+    float lo[3], h[3];
+    grid_frame(L.red, mom, n, lo, h);
+    RsItems x;
+#pragma unroll
+    for (int k = 0; k < RS_SINGLE_ITEMS; ++k) {
+        const int i = rs_index(items, k);
+        if (k >= items || i >= n) continue;
+        x.val[k] = dynCols[i];
+        x.key[k] = cell_key(x.val[k], lo, h, cworld, cbmin, cbmax);
+    }
+    rs_block_sort(B, x, n, bits, items);
+    rs_block_exchange(B, x, n, items);
+    int run = 0;
+#pragma unroll
+    for (int k = 0; k < RS_SINGLE_ITEMS; ++k) {
+        const int i = rs_index(items, k);
+        if (k >= items || i >= n) continue;
+        const uint64_t key = x.key[k];
+        keys[i] = key;
+        vals[i] = x.val[k];
+        grid_record(i, x.val[k], cbmin, cbmax, cflags, centity, clocal, gridRec);
+        if (i > 0 && B.sk[i - 1] == key) continue;
+        int from = i + 1, to = n;   // the first collider after the run
+        while (from < to) {
+            const int mid = (from + to) >> 1;
+            if (B.sk[mid] <= key) from = mid + 1; else to = mid;
         }
-        gridRec[2 * t] = make_float4(a.x, a.y, a.z, __int_as_float(clocal[c]));
-        gridRec[2 * t + 1] = make_float4(b.x, b.y, b.z, __int_as_float((int)centity[c]));
+        run = max(run, from - i);
+        uint32_t slot = cell_hash(key) & mask;
+        for (uint32_t probe = 0; probe <= mask; ++probe) {   // the table is at least twice the cells
+            if (atomicCAS((unsigned long long*)&tabKey[slot], GRID_EMPTY, key) == GRID_EMPTY) {
+                tabStart[slot] = i;
+                tabEnd[slot] = from;
+                break;
+            }
+            slot = (slot + 1) & mask;
+        }
     }
-    if (t < nStatic) {
-        const int c = staticCols[t];
-        const float4 a = cbmin[c], b = cbmax[c];
-        statA[t] = make_float4(a.x, a.y, a.z, __int_as_float(cflags[c]));
-        statB[t] = make_float4(b.x, b.y, b.z, __int_as_float((int)centity[c]));
-        statL[t] = clocal[c];
-    }
+    if (run) atomicMax(&longest, run);
+    __syncthreads();
+    if (tid == 0) counters[15] = longest;
 }
 
 // GRID_LANES lanes per enabled dynamic collider s (sorted order): lane 0 its own cell after
@@ -987,23 +1082,30 @@ static void bp_grid(World& w) {
     hipStream_t s = w.stream;
     const int n = w.nDynCol;
     const uint32_t T = grid_table_size(n);
-    hipLaunchKernelGGL(k_scene_bounds_init, dim3(1), dim3(64), 0, s, w.worldBoundsI.p, w.sceneMoments.p,
-                       w.counters.p);
-    hipLaunchKernelGGL(k_scene_bounds, dim3(std::min(64, div_up(n, 1024))), dim3(1024), 0, s, n, w.dynCols.p,
-                       w.cbmin.p, w.cbmax.p, w.worldBoundsI.p, w.sceneMoments.p);
-    hipLaunchKernelGGL(k_cell_codes, dim3(div_up(std::max<int>(n, (int)T), 256)), dim3(256), 0, s, n, w.dynCols.p,
-                       w.cworld.p, w.cbmin.p, w.cbmax.p, w.worldBoundsI.p, w.sceneMoments.p, w.mkeys.p, w.mvals.p,
-                       (int)T, w.gridKey.p);
-    PGX_LAUNCH_CHECK();
-    radix_sort_u64(s, w.mkeys.p, w.mvals.p, n, 30 + w.worldBits, w.sortT);
     const int nStatic = w.C - w.nDynCol;
-    hipLaunchKernelGGL(k_grid_pack, dim3(div_up(std::max(n, nStatic), 256)), dim3(256), 0, s, n, w.mvals.p,
-                       w.cbmin.p, w.cbmax.p, w.cflags.p, w.centity.p, w.clocal.p, w.gridRec.p, nStatic, w.staticCols.p,
-                       w.statA.p, w.statB.p, w.statL.p);
-    hipLaunchKernelGGL(k_cell_insert, dim3(div_up(n, 256)), dim3(256), 0, s, n, w.mkeys.p, T - 1, w.gridKey.p,
-                       w.gridStart.p);
-    hipLaunchKernelGGL(k_cell_ends, dim3(div_up(n, 256)), dim3(256), 0, s, n, w.mkeys.p, T - 1, w.gridKey.p,
-                       w.gridStart.p, w.gridEnd.p, w.counters.p);
+    if (n <= GRID_SMALL) {
+        hipLaunchKernelGGL(k_grid_small, dim3(1), dim3(rs_threads(n)), 0, s, n, rs_item_count(n), 30 + w.worldBits,
+                           w.dynCols.p, w.cworld.p, w.cbmin.p, w.cbmax.p, w.cflags.p, w.centity.p, w.clocal.p, w.mkeys.p,
+                           w.mvals.p, T - 1, w.gridKey.p, w.gridStart.p, w.gridEnd.p, w.gridRec.p, nStatic,
+                           w.staticCols.p, w.statA.p, w.statB.p, w.statL.p, w.counters.p);
+    } else {
+        hipLaunchKernelGGL(k_scene_bounds_init, dim3(1), dim3(64), 0, s, w.worldBoundsI.p, w.sceneMoments.p,
+                           w.counters.p);
+        hipLaunchKernelGGL(k_scene_bounds, dim3(std::min(64, div_up(n, 1024))), dim3(1024), 0, s, n, w.dynCols.p,
+                           w.cbmin.p, w.cbmax.p, w.worldBoundsI.p, w.sceneMoments.p);
+        hipLaunchKernelGGL(k_cell_codes, dim3(div_up(std::max<int>(n, (int)T), 256)), dim3(256), 0, s, n, w.dynCols.p,
+                           w.cworld.p, w.cbmin.p, w.cbmax.p, w.worldBoundsI.p, w.sceneMoments.p, w.mkeys.p, w.mvals.p,
+                           (int)T, w.gridKey.p);
+        PGX_LAUNCH_CHECK();
+        radix_sort_u64(s, w.mkeys.p, w.mvals.p, n, 30 + w.worldBits, w.sortT);
+        hipLaunchKernelGGL(k_grid_pack, dim3(div_up(std::max(n, nStatic), 256)), dim3(256), 0, s, n, w.mvals.p,
+                           w.cbmin.p, w.cbmax.p, w.cflags.p, w.centity.p, w.clocal.p, w.gridRec.p, nStatic, w.staticCols.p,
+                           w.statA.p, w.statB.p, w.statL.p);
+        hipLaunchKernelGGL(k_cell_insert, dim3(div_up(n, 256)), dim3(256), 0, s, n, w.mkeys.p, T - 1, w.gridKey.p,
+                           w.gridStart.p);
+        hipLaunchKernelGGL(k_cell_ends, dim3(div_up(n, 256)), dim3(256), 0, s, n, w.mkeys.p, T - 1, w.gridKey.p,
+                           w.gridStart.p, w.gridEnd.p, w.counters.p);
+    }
     // 16 lanes per collider at every size: fewer lanes, each opening several cells one after
     // another, measured slower on the 857k-collider batch (506 against 390 us)
     const long long lanes = (long long)n * GRID_LANES;
@@ -1053,8 +1155,10 @@ int bp_find_pairs(World& w) {
     if (cnt[6]) throw PgxError{PGX_ERR_INVALID, "broadphase traversal exceeded its visit bound (malformed tree)"};
     if (nPairs > w.pairCap) throw PgxError{PGX_ERR_CAPACITY, "pair capacity exceeded: " + std::to_string(nPairs) +
                                                                  " > " + std::to_string(w.pairCap)};
-    // canonical order: (world, local collider of the smaller entity, other local collider)
-    radix_sort_u64(s, w.pkeys.p, w.pvals.p, nPairs, w.worldBits + 2 * w.localBits, w.sortT);
+    // canonical order: (world, local collider of the smaller entity, other local collider); up
+    // to NP_ORDER_SMALL pairs are sorted with their classes (np_run)
+    if (nPairs > NP_ORDER_SMALL)
+        radix_sort_u64(s, w.pkeys.p, w.pvals.p, nPairs, w.worldBits + 2 * w.localBits, w.sortT);
     return nPairs;
 }
 

@@ -136,19 +136,6 @@ struct RadixScratch {
     size_t keys = 0, vals = 0, hist = 0, sums = 0;
 };
 RadixScratch radix_sort_scratch(int n, int bits);
-// rank of the lane's element among the wave's elements of the same digit so far; bumps the
-// wave's count of the digit (counts: this wave's counters in LDS, one per digit value)
-__device__ __forceinline__ int32_t rs_rank(uint32_t d, bool ok, int dbits, uint64_t lt, int32_t* counts) {
-    uint64_t same = __ballot(ok);
-    for (int b = 0; b < dbits; ++b) {
-        const uint64_t bal = __ballot((d >> b) & 1u);
-        same &= ((d >> b) & 1u) ? bal : ~bal;
-    }
-    const int32_t prior = counts[d];
-    if (ok && (same & lt) == 0ull) counts[d] = prior + (int32_t)__popcll(same);
-    return prior + (int32_t)__popcll(same & lt);
-}
-
 // The same sort with caller-provided scratch of radix_sort_scratch(n, bits) elements; it
 // needs no zeroed memory (every table it reads it has written first) and allocates nothing.
 void radix_sort_u64_into(hipStream_t s, uint64_t* keys, int32_t* vals, int n, int bits, uint64_t* kalt,

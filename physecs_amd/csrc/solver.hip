@@ -18,6 +18,7 @@
 #include <hip/hip_cooperative_groups.h>
 #include <hip/hip_ext.h>
 #include "pgx_internal.h"
+#include "radix_block.h"
 
 namespace cg = cooperative_groups;
 

@@ -1,6 +1,7 @@
 // Device-wide primitives: a stable LSD radix sort of 64-bit keys with 32-bit values, and an
 // exclusive scan, both written for 64-lane CDNA wavefronts.
 #include "pgx_internal.h"
+#include "radix_block.h"
 
 namespace pgx {
 
@@ -21,13 +22,8 @@ namespace pgx {
 // whose exclusive scan is the offset table, scanned in place before the scatter reads it.
 constexpr int RS_THREADS = 256;
 constexpr int RS_WAVES = RS_THREADS / WAVE;
-constexpr int RS_BINS = 256;
 // up to this many tiles, every block sums its offsets from the histogram table itself
 constexpr int RS_SUM_TILES = 64;
-
-__device__ __forceinline__ uint32_t rs_digit(uint64_t k, int shift, int dbits) {
-    return (uint32_t)(k >> shift) & ((1u << dbits) - 1u);
-}
 
 // The tile's digit counts with LDS atomics, every key load issued before the counting. (A
 // ballot-ranked count per wave, free of the atomics' bank conflicts on nearly sorted keys,
@@ -126,94 +122,24 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t* __res
 }
 
 // Up to RS_SINGLE keys: every digit pass in one workgroup, in one launch instead of two per
-// digit, each pass ranked and placed as k_rs_scatter places a single tile (no other tile's
-// counts), so the output is the same stable order. A pass is a chain (rank, scan, place) that
-// costs the more the more keys a wave ranks one after the other, so the keys go to as many
-// waves as there are: each takes an equal run of whole 64s. 500 keys: 17 us with four waves
-// of 16 items each, 5 us with this. The limit: 6,000 keys of 30 bits take 26 us here and 36 us
-// in tiles, with eight launches; the chain of 16 items a wave that twice as many would be is
-// no faster than tiles any more.
-constexpr int RS_SINGLE_THREADS = 1024, RS_SINGLE_WAVES = RS_SINGLE_THREADS / WAVE;
-constexpr int RS_SINGLE_ITEMS = 8;
-constexpr int RS_SINGLE = RS_SINGLE_THREADS * RS_SINGLE_ITEMS;
+// digit (rs_block_sort), so the output is the same stable order. The limit: 6,000 keys of 30
+// bits take 26 us here and 36 us in tiles, with eight launches; the chain of 16 items a wave
+// that twice as many would be is no faster than tiles any more.
 __global__ __launch_bounds__(RS_SINGLE_THREADS) void k_rs_single(uint64_t* __restrict__ keys, int32_t* __restrict__ vals,
                                                                  int n, int bits, int items) {
-    constexpr int ITEMS = RS_SINGLE_ITEMS;
-    __shared__ uint64_t sk[RS_SINGLE];
-    __shared__ int32_t sv[RS_SINGLE];
-    __shared__ int32_t waveCnt[RS_SINGLE_WAVES][RS_BINS];
-    __shared__ int32_t off[RS_BINS];
-    __shared__ int32_t wsum[RS_BINS / WAVE];
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE, waves = blockDim.x / WAVE;
-    const int runBase = wv * WAVE * items;   // the wave's elements: item k covers [k * 64, k * 64 + 64) of its run
-    const uint64_t lt = (1ull << lane) - 1ull;
-    const int passes = (bits + 7) / 8;
-    uint64_t key[ITEMS];
-    int32_t val[ITEMS], rank[ITEMS];
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        if (k >= items) break;
-        const int i = runBase + k * WAVE + lane;
-        key[k] = i < n ? keys[i] : 0ull;
-        val[k] = i < n ? vals[i] : 0;
+    __shared__ RsBlock B;
+    RsItems x;
+    for (int k = 0; k < RS_SINGLE_ITEMS; ++k) {
+        const int i = rs_index(items, k);
+        if (k >= items || i >= n) continue;
+        x.key[k] = keys[i];
+        x.val[k] = vals[i];
     }
-    for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p, dbits = min(8, bits - 8 * p);
-        for (int d = lane; d < RS_BINS; d += WAVE) waveCnt[wv][d] = 0;   // the wave's own counters
-#pragma unroll
-        for (int k = 0; k < ITEMS; ++k) {
-            if (k >= items) break;
-            rank[k] = rs_rank(rs_digit(key[k], shift, dbits), runBase + k * WAVE + lane < n, dbits, lt, waveCnt[wv]);
-        }
-        __syncthreads();
-        // digit tid: the waves' counts to exclusive prefixes across waves, and the digit's
-        // offset, the exclusive scan of the totals over the digits
-        int32_t total = 0, x = 0;
-        if (tid < RS_BINS) {
-#pragma unroll 4
-            for (int w = 0; w < waves; ++w) {
-                const int32_t c = waveCnt[w][tid];
-                waveCnt[w][tid] = total;
-                total += c;
-            }
-            x = total;
-            for (int o = 1; o < WAVE; o <<= 1) {
-                const int32_t y = __shfl_up(x, o);
-                if (lane >= o) x += y;
-            }
-            if (lane == WAVE - 1) wsum[wv] = x;
-        }
-        __syncthreads();
-        if (tid < RS_BINS) {
-            int32_t before = 0;
-            for (int w = 0; w < RS_BINS / WAVE; ++w) before += w < wv ? wsum[w] : 0;
-            off[tid] = before + x - total;
-        }
-        __syncthreads();
-        const bool last = p + 1 == passes;
-#pragma unroll
-        for (int k = 0; k < ITEMS; ++k) {
-            if (k >= items) break;
-            if (runBase + k * WAVE + lane >= n) continue;
-            const uint32_t d = rs_digit(key[k], shift, dbits);
-            const int pos = off[d] + waveCnt[wv][d] + rank[k];
-            if (last) {
-                keys[pos] = key[k];
-                vals[pos] = val[k];
-            } else {
-                sk[pos] = key[k];
-                sv[pos] = val[k];
-            }
-        }
-        if (last) break;
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < ITEMS; ++k) {
-            if (k >= items) break;
-            const int i = runBase + k * WAVE + lane;
-            key[k] = i < n ? sk[i] : 0ull;
-            val[k] = i < n ? sv[i] : 0;
-        }
+    rs_block_sort(B, x, n, bits, items);
+    for (int k = 0; k < RS_SINGLE_ITEMS; ++k) {
+        if (k >= items || rs_index(items, k) >= n) continue;
+        keys[x.pos[k]] = x.key[k];
+        vals[x.pos[k]] = x.val[k];
     }
 }
 
@@ -268,8 +194,7 @@ void radix_sort_u64_into(hipStream_t s, uint64_t* keys, int32_t* vals, int n, in
     if (n <= 1 || bits <= 0) return;
     bits = std::min(bits, 64);
     if (n <= RS_SINGLE) {   // every pass in one launch
-        const int threads = std::min(RS_SINGLE_THREADS, div_up(n, RS_THREADS) * RS_THREADS);
-        hipLaunchKernelGGL(k_rs_single, dim3(1), dim3(threads), 0, s, keys, vals, n, bits, div_up(n, threads));
+        hipLaunchKernelGGL(k_rs_single, dim3(1), dim3(rs_threads(n)), 0, s, keys, vals, n, bits, rs_item_count(n));
         PGX_LAUNCH_CHECK();
         return;
     }
