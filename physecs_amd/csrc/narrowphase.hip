@@ -778,7 +778,7 @@ __global__ __launch_bounds__(256) void k_narrowphase(
         }
         Mf m;
         m.numPoints = 0;
-        // pairs with a triangle mesh go to k_narrowphase_mesh, pairs with a convex mesh to
+        // pairs with a triangle mesh go to the mesh passes, pairs with a convex mesh to
         // k_narrowphase_convex: appended with one atomic per wave
         const bool toMesh = !skip && (ctype[c0] == PGX_TRIANGLE_MESH || ctype[c1] == PGX_TRIANGLE_MESH);
         const bool toHeavy = !skip && !toMesh && (ctype[c0] == PGX_CONVEX_MESH || ctype[c1] == PGX_CONVEX_MESH);

@@ -607,7 +607,7 @@ void sv_color_points(World& w, int nColors) {
 // ten SIMDs, so its time is one wave's chain of instructions: k_solve is 718 of them instead
 // of 1,076 with a lane per manifold, at 98 registers instead of 208, and took 4.26 us per
 // colour launch of the settled 32k scene instead of 5.63 (a run of small colours in
-// k_solve_batch 17.1 us instead of 24.8; a large colour of 1,024 worlds 8.4 instead of 10.4).
+// k_solve_batch 17.1 us instead of 24.8 (before its two teams); a large colour of 1,024 worlds 8.4 instead of 10.4).
 //
 // Contact rows of point k of side lane i, field f at ((k * RS_NF + f) * Mcap) * 2 + i, so
 // a wave's loads are contiguous: r x n (.w = target velocity), the row times the body's
