@@ -630,6 +630,9 @@ __device__ __forceinline__ void chain_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// UPDATE: k_joint_update's work of the chunk's joints first, a lane per joint: 10.9 us for 24
+// ragdolls instead of 5.8 in a launch of its own and 7.2.
+template <bool UPDATE>
 __global__ __launch_bounds__(8 * ISLAND_CHUNK) void k_island_presolve(JointArgs a, IslandArgs is, int maxBodies, int maxJoints) {
     extern __shared__ float4 lds[];
     float4 *sv = lds, *sw = lds + maxBodies, *rows = lds + 2 * maxBodies;
@@ -645,6 +648,10 @@ __global__ __launch_bounds__(8 * ISLAND_CHUNK) void k_island_presolve(JointArgs 
     const int first = __builtin_amdgcn_readlane(starts, 0), last = __builtin_amdgcn_readlane(starts, 8);
     for (int at = first; at < last; at += maxJoints) {
         const int m = min(maxJoints, last - at);
+        if (UPDATE) {
+            if ((int)threadIdx.x < m) joint_update(a, is.joint[at + threadIdx.x].x);
+            __syncthreads();   // the rows are in memory
+        }
         const int jj = threadIdx.x / 8, r = threadIdx.x & 7;
         if (jj < m) {
             const int4 jl = is.joint[at + jj];
@@ -944,8 +951,14 @@ void jt_step_setup(World& w) {
     if (!w.custList.empty()) custom_layouts(w, a);
 }
 
+// Whether the islands' preSolve updates the rows itself: every live joint is in an island, and
+// none waits for the host's rows.
+static bool islands_update(const World& w) {
+    return w.jIslands > 0 && w.jColorStart[9] == w.jColorStart[8] && w.custList.empty();
+}
+
 void jt_update(World& w, float h) {
-    if (!w.J) return;
+    if (!w.J || islands_update(w)) return;
     JointArgs a = make_jargs(w, h);
     hipLaunchKernelGGL(k_joint_update, dim3(div_up(w.J, 256)), dim3(256), 0, w.stream, a);
     PGX_LAUNCH_CHECK();
@@ -961,8 +974,8 @@ void jt_colors(World& w, float h, int phase, bool warm) {
         const int m = std::min(w.jIslandJoints, ISLAND_CHUNK), threads = div_up(8 * m, WAVE) * WAVE;
         const size_t lds = 2 * sizeof(float4) * w.jIslandBodies + sizeof(int4) * m;
         if (phase == 0)
-            hipLaunchKernelGGL(k_island_presolve, dim3(w.jIslands), dim3(threads),
-                               lds + sizeof(float4) * PUSH_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m);
+            hipLaunchKernelGGL(islands_update(w) ? k_island_presolve<true> : k_island_presolve<false>,
+                               dim3(w.jIslands), dim3(threads), lds + sizeof(float4) * PUSH_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m);
         else
             hipLaunchKernelGGL(k_island_solve, dim3(w.jIslands), dim3(threads),
                                lds + sizeof(float4) * ROW_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m,
