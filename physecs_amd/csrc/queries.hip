@@ -130,6 +130,7 @@ struct RayScene {
     int W, nLeaves;
     const int32_t *worldRoot, *worldStop, *worldStaticStart, *staticCols, *mvals;
     const int32_t* inOrder;
+    const float* near;                 // RaySkip::near
     const float4 *rayNode, *rayLeaf;   // k_ray_records
     const float4 *leafA, *nodeA, *nodeB;
     const float4 *cbmin, *cbmax, *cparams, *clpos, *clquat, *bpos, *bquat;
@@ -174,13 +175,25 @@ __device__ __forceinline__ void test_collider(const RayScene& S, int c, f3 o, f3
 // capsule's or plane's direction), and a direction component under 0.001 counts as parallel
 // (intersectRayAABB, a drift of up to 0.001 t per axis). m and t are at most the distance to
 // the far corner of the tree's box.
+//
+// A capsule is the exception (src/Raycast.cpp:65-100): where the ray's line leaves its cylinder
+// behind the origin, carried on beyond the caps, the hit counts as one at 0 if the origin lies
+// between the caps' planes, however far ahead the ray enters the capsule's box. How far that is:
+// with H the distance from the capsule's centre to the farthest corner of its box, half its
+// half height, the ray moves away from the axis from its origin on and is at most H from it
+// where it enters the box, so its origin is at most H from the axis and half <= H from the
+// centre along it, sqrt(2) H from the centre, and the entry at most (1 + sqrt(2)) H from the
+// origin. Boxes that the ray enters within 2.5 H of the tree's largest capsule are not skipped
+// (the rest is for rounding and drift, which are under a hundredth of such a distance).
 struct RaySkip {
     f3 inv;          // 1 / d, 0 on a parallel axis
     float margin;    // negative: the bound does not hold, walk without skipping
+    float near;      // what is entered up to here is not skipped
 };
 // The formulas take directions as unit vectors, and their squares stay finite up to 1e9.
-__device__ __forceinline__ RaySkip ray_skip(f3 o, f3 d, f3 inv, f3 mn, f3 mx) {
+__device__ __forceinline__ RaySkip ray_skip(f3 o, f3 d, f3 inv, f3 mn, f3 mx, float near) {
     RaySkip r;
+    r.near = near;
     r.inv = mk3(fabsf(d.x) < 0.001f ? 0.f : inv.x, fabsf(d.y) < 0.001f ? 0.f : inv.y, fabsf(d.z) < 0.001f ? 0.f : inv.z);
     const f3 far = mk3(fmaxf(fabsf(mn.x - o.x), fabsf(mx.x - o.x)), fmaxf(fabsf(mn.y - o.y), fabsf(mx.y - o.y)),
                        fmaxf(fabsf(mn.z - o.z), fabsf(mx.z - o.z)));
@@ -198,25 +211,9 @@ __device__ __forceinline__ float widened_entry(const RaySkip& r, f3 o, f3 mn, f3
     return t * (1.f - 1e-5f);
 }
 
-// The walk's records, 64 bytes each so that a visit takes one line: per inner node
-// {left box min, left}, {left max, right}, {right min}, {right max}; per leaf
-// {position, type}, {orientation}, {params}, {collider, entity}.
-// Sets *inOrder (0 before) if a dynamic collider is one for which the margin does not hold
-// or whose hit distance could be a NaN, which makes the result depend on the order of the
-// tests: bounds that are not finite, or an orientation that is not a unit quaternion.
-__global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __restrict__ child, RayScene S,
-                                                     const float4* __restrict__ leafB, const float4* __restrict__ clquat,
-                                                     float4* __restrict__ rayNode, float4* __restrict__ rayLeaf,
-                                                     int32_t* __restrict__ inOrder) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n - 1) {
-        const int l = child[2 * i], r = child[2 * i + 1], ll = l & ~LEAF_BIT, rl = r & ~LEAF_BIT;
-        rayNode[4 * (size_t)i] = f4(xyz(l & LEAF_BIT ? S.leafA[ll] : S.nodeA[ll]), __int_as_float(l));
-        rayNode[4 * (size_t)i + 1] = f4(xyz(l & LEAF_BIT ? leafB[ll] : S.nodeB[ll]), __int_as_float(r));
-        rayNode[4 * (size_t)i + 2] = f4(xyz(r & LEAF_BIT ? S.leafA[rl] : S.nodeA[rl]), 0.f);
-        rayNode[4 * (size_t)i + 3] = f4(xyz(r & LEAF_BIT ? leafB[rl] : S.nodeB[rl]), 0.f);
-    }
-    if (i >= n) return;
+// leaf i's record; what it asks of RaySkip::near
+__device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4* __restrict__ clquat,
+                                          float4* __restrict__ rayLeaf, int32_t* __restrict__ inOrder) {
     const int c = S.mvals[i], b = S.cbody[c];
     const float4 mn = S.cbmin[c], mx = S.cbmax[c], l = clquat[c], q = S.bquat[b];
     const bool bounded = mn.x > -1e9f && mn.y > -1e9f && mn.z > -1e9f && mx.x < 1e9f && mx.y < 1e9f && mx.z < 1e9f;
@@ -224,10 +221,40 @@ __global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __res
                        fabsf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w - 1.f) < 1e-5f;
     if (!(bounded && units)) *inOrder = 1;
     const qf lq = qmul(q4(q), q4(l));
-    rayLeaf[4 * (size_t)i] = f4(add(xyz(S.bpos[b]), qrot(q4(q), xyz(S.clpos[c]))), __int_as_float(S.ctype[c]));
+    const f3 pos = add(xyz(S.bpos[b]), qrot(q4(q), xyz(S.clpos[c])));
+    rayLeaf[4 * (size_t)i] = f4(pos, __int_as_float(S.ctype[c]));
     rayLeaf[4 * (size_t)i + 1] = f4(mk3(lq.x, lq.y, lq.z), lq.w);
     rayLeaf[4 * (size_t)i + 2] = S.cparams[c];
     rayLeaf[4 * (size_t)i + 3] = make_float4(__int_as_float(c), __uint_as_float(S.centity[c]), 0.f, 0.f);
+    if (S.ctype[c] != PGX_CAPSULE) return 0.f;
+    const f3 far = mk3(fmaxf(pos.x - mn.x, mx.x - pos.x), fmaxf(pos.y - mn.y, mx.y - pos.y), fmaxf(pos.z - mn.z, mx.z - pos.z));
+    return 2.5f * length(far);
+}
+
+// The walk's records, 64 bytes each so that a visit takes one line: per inner node
+// {left box min, left}, {left max, right}, {right min}, {right max}; per leaf
+// {position, type}, {orientation}, {params}, {collider, entity}.
+// Sets *inOrder (0 before) if a dynamic collider is one for which the margin does not hold
+// or whose hit distance could be a NaN, which makes the result depend on the order of the
+// tests: bounds that are not finite, or an orientation that is not a unit quaternion. Raises
+// *near (0 before) to RaySkip::near.
+__global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __restrict__ child, RayScene S,
+                                                     const float4* __restrict__ leafB, const float4* __restrict__ clquat,
+                                                     float4* __restrict__ rayNode, float4* __restrict__ rayLeaf,
+                                                     int32_t* __restrict__ inOrder, float* __restrict__ near) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    float reach = 0.f;
+    if (i < n - 1) {
+        const int l = child[2 * i], r = child[2 * i + 1], ll = l & ~LEAF_BIT, rl = r & ~LEAF_BIT;
+        rayNode[4 * (size_t)i] = f4(xyz(l & LEAF_BIT ? S.leafA[ll] : S.nodeA[ll]), __int_as_float(l));
+        rayNode[4 * (size_t)i + 1] = f4(xyz(l & LEAF_BIT ? leafB[ll] : S.nodeB[ll]), __int_as_float(r));
+        rayNode[4 * (size_t)i + 2] = f4(xyz(r & LEAF_BIT ? S.leafA[rl] : S.nodeA[rl]), 0.f);
+        rayNode[4 * (size_t)i + 3] = f4(xyz(r & LEAF_BIT ? leafB[rl] : S.nodeB[rl]), 0.f);
+    }
+    if (i < n) reach = ray_leaf(i, S, clquat, rayLeaf, inOrder);
+    // one atomic a wave at most: the floats are not negative, so their bits order like them
+    for (int o = WAVE / 2; o >= 1; o >>= 1) reach = fmaxf(reach, __shfl_xor(reach, o));
+    if ((threadIdx.x & (WAVE - 1)) == 0 && reach > *near) atomicMax((unsigned int*)near, __float_as_uint(reach));
 }
 
 // Ray i: origin, direction and maxDistance as the caller holds them (3, 3 and 1 floats), the
@@ -261,8 +288,9 @@ __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __r
     float bestT = 0.f;
     int best = -1;
     const int root = S.worldRoot[wd];
-    RaySkip skip{s3(0.f), -1.f};
-    if (root != -1 && !(root & LEAF_BIT) && !*S.inOrder) skip = ray_skip(o, d, inv, xyz(S.nodeA[root]), xyz(S.nodeB[root]));
+    RaySkip skip{s3(0.f), -1.f, 0.f};
+    if (root != -1 && !(root & LEAF_BIT) && !*S.inOrder) 
+        skip = ray_skip(o, d, inv, xyz(S.nodeA[root]), xyz(S.nodeB[root]), *S.near);
     auto statics = [&]() {
         for (int st = S.worldStaticStart[wd]; st < S.worldStaticStart[wd + 1]; ++st)
             test_collider(S, S.staticCols[st], o, d, inv, maxDist, ig, bestT, best);
@@ -272,7 +300,7 @@ __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __r
         if (!ray_aabb(o, d, inv, xyz(mn), xyz(mx), t) || !(t <= maxDist)) return false;
         if (skip.margin < 0.f) return true;
         t = widened_entry(skip, o, xyz(mn), xyz(mx));
-        return best < 0 || !(t > bestT);
+        return best < 0 || !(t > fmaxf(bestT, skip.near));
     };
     int visits = 0;   // a walk visits at most 2n - 1 nodes
     float t;
@@ -292,7 +320,7 @@ __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __r
     auto pop = [&]() {   // the next waiting subtree that is not beyond the best hit by now
         while (sp > 0) {
             --sp;
-            if (best < 0 || !(entry[sp][threadIdx.x] > bestT)) return waiting[sp][threadIdx.x];
+            if (best < 0 || !(entry[sp][threadIdx.x] > fmaxf(bestT, skip.near))) return waiting[sp][threadIdx.x];
         }
         return -1;
     };
@@ -367,7 +395,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
     if (!w.qEv[0])
         for (auto& e : w.qEv) PGX_HIP(hipEventCreate(&e));
     PGX_HIP(hipEventRecord(w.qEv[0], s));
-    fill_i32(s, w.counters.p + 7, 0, 2);   // the refit's work counter, the walks' order
+    fill_i32(s, w.counters.p + 7, 0, 3);   // the refit's work counter, the walks' order and near
     bp_build(w);
     RayScene S;
     S.W = w.W;
@@ -375,7 +403,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
     S.worldRoot = w.worldRoot.p; S.worldStop = w.worldStop.p;
     S.worldStaticStart = w.worldStaticStart.p; S.staticCols = w.staticCols.p; S.mvals = w.mvals.p;
     w.qRayNode.alloc(4 * (size_t)std::max(w.nDynCol, 1)); w.qRayLeaf.alloc(4 * (size_t)std::max(w.nDynCol, 1));
-    S.inOrder = w.counters.p + 8; S.rayNode = w.qRayNode.p; S.rayLeaf = w.qRayLeaf.p;
+    S.inOrder = w.counters.p + 8; S.near = (const float*)(w.counters.p + 9); S.rayNode = w.qRayNode.p; S.rayLeaf = w.qRayLeaf.p;
     S.leafA = w.leafA.p; S.nodeA = w.nodeA.p; S.nodeB = w.nodeB.p;
     S.cbmin = w.cbmin.p; S.cbmax = w.cbmax.p; S.cparams = w.cparams.p; S.clpos = w.clpos.p; S.clquat = w.clquat.p;
     S.bpos = w.bpos.p; S.bquat = w.bquat.p; S.cbody = w.cbody.p; S.ctype = w.ctype.p; S.centity = w.centity.p;
@@ -384,7 +412,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
         fill_i32(s, w.worldRoot.p, -1, w.W);   // no tree: static lists only
     } else {
         hipLaunchKernelGGL(k_ray_records, dim3(div_up(w.nDynCol, 256)), dim3(256), 0, s, w.nDynCol, w.nodeChild.p, S,
-                           w.leafB.p, w.clquat.p, w.qRayNode.p, w.qRayLeaf.p, w.counters.p + 8);
+                           w.leafB.p, w.clquat.p, w.qRayNode.p, w.qRayLeaf.p, w.counters.p + 8, (float*)(w.counters.p + 9));
         PGX_LAUNCH_CHECK();
     }
     hipLaunchKernelGGL(k_raycast, dim3(div_up(n, RAY_THREADS)), dim3(RAY_THREADS), 0, s, n, w.qRays.p, w.qRays.p + n3,

@@ -1,7 +1,8 @@
 """The raycast walk at the places where its order or its skipping could show: trees deeper
 than its stack, grazing rays, distant origins, directions and orientations that are not
-normalised (walked in the tree's order), batches that end within a wave. Against the
-oracle's Scene::raycastClosest on the same state, bit for bit."""
+normalised (walked in the tree's order), batches that end within a wave, capsules whose
+bounds reach far from them. Against the oracle's Scene::raycastClosest on the same state, bit
+for bit."""
 import numpy as np
 import pytest
 
@@ -53,6 +54,14 @@ def _rays(kind, sc, rng, n):
     return (target + away * reach + side * offset).astype(np.float32), d.astype(np.float32)
 
 
+def _same(g, o, origins, dirs, maxd):
+    gc, gt, _ = g.raycast(origins, dirs, maxd)
+    oc, ot = o.raycast(origins, dirs, np.full(len(origins), maxd, np.float32))
+    assert np.array_equal(gc, oc), np.flatnonzero(gc != oc)
+    assert np.array_equal(bits(gt[gc >= 0]), bits(ot[gc >= 0]))
+    return oc, ot
+
+
 @pytest.mark.parametrize("scene,kind,n", [("deep", "near", 1), ("deep", "near", 257), ("deep", "length", 65),
                                           ("mixed", "graze", 1023), ("mixed", "far", 1000), ("mixed", "length", 300),
                                           ("loose", "near", 500)])
@@ -62,8 +71,48 @@ def test_walk_matches_oracle(scene, kind, n):
     g, o = lockstep(sc, 10 if scene == "mixed" else 0)
     origins, dirs = _rays(kind, sc, np.random.default_rng(n), n)
     for maxd in (3e5, 20.0):
-        gc, gt, _ = g.raycast(origins, dirs, maxd)
-        oc, ot = o.raycast(origins, dirs, np.full(n, maxd, np.float32))
-        assert np.array_equal(gc, oc)
-        assert np.array_equal(bits(gt[gc >= 0]), bits(ot[gc >= 0]))
-    assert (gc >= 0).any() or kind == "far"
+        c, _ = _same(g, o, origins, dirs, maxd)
+    assert (c >= 0).any() or kind == "far"
+
+
+def test_capsule_met_behind_the_origin():
+    """The line meets the tilted capsule behind the origin, which is a hit at 0; its bounds are
+    entered 8.5 m ahead, behind a sphere that is met at 2.7 m."""
+    sc = scenes.Scene()
+    d = np.array([-1, -1.5, 0]) / np.hypot(1, 1.5)
+    o = np.array([12.0, 1, 0])
+    sc.add_body(scenes.CAPSULE, [10, 0.1], [0, 0, 0], [0, 0, np.sin(-np.pi / 8), np.cos(-np.pi / 8)])
+    sc.add_body(scenes.SPHERE, [0.3], o + 3 * d)
+    c, t = _same(*lockstep(sc, 0), np.array([o], np.float32), np.array([d], np.float32), 200.0)
+    assert c[0] == 0 and t[0] == 0
+
+
+@pytest.mark.parametrize("half", [0.5, 1.0, 6.0, 10.0])
+def test_rays_that_start_beside_poles(half):
+    """The same of many poles: rays from beside a pole, on a line that comes from its axis beyond
+    the end, each with a ball a little way ahead."""
+    rng = np.random.default_rng(int(10 * half))
+    sc = scenes.Scene()
+    origins, dirs = [], []
+    poles, n = rng.uniform(-40 * half, 40 * half, (60, 3)), 12
+    for at in poles:
+        a, p = rng.normal(size=(2, 3))
+        a /= np.linalg.norm(a)
+        q = np.array([a[2], 0, -a[0], 1 + a[1]])      # the turn that takes the y axis to a
+        sc.add_body(scenes.CAPSULE, [half, 0.02 * half], at, q / np.linalg.norm(q))
+        for _ in range(n):
+            p = rng.normal(size=3)
+            p -= p.dot(a) * a
+            end = rng.choice([-1, 1])
+            o = a * half * end * rng.uniform(0, 0.9) + p / np.linalg.norm(p) * half * rng.uniform(0.05, 0.6)
+            d = o - a * half * end * rng.uniform(1.05, 2.0)
+            d /= np.linalg.norm(d)
+            origins.append(at + o)
+            dirs.append(d)
+            sc.add_body(scenes.SPHERE, [0.01 * half], at + o + d * half * rng.uniform(0.02, 0.2))
+    g, o = lockstep(sc, 0)
+    origins, dirs = np.array(origins, np.float32), np.array(dirs, np.float32)
+    c, t = _same(g, o, origins, dirs, 200.0)
+    mn, mx = o.bounds()[c, :3], o.bounds()[c, 3:]
+    ahead = (np.minimum((mn - origins) / dirs, (mx - origins) / dirs)).max(1)
+    assert ((c >= 0) & (t == 0) & (ahead > 0.3 * half)).sum() > 5
