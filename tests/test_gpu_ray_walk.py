@@ -89,30 +89,28 @@ def test_capsule_met_behind_the_origin():
 
 @pytest.mark.parametrize("half", [0.5, 1.0, 6.0, 10.0])
 def test_rays_that_start_beside_poles(half):
-    """The same of many poles: rays from beside a pole, on a line that comes from its axis beyond
-    the end, each with a ball a little way ahead."""
+    """The same of random poles, each alone with 48 balls: rays from beside the pole, on a line
+    that comes from its axis beyond the end, each with a ball a little way ahead."""
     rng = np.random.default_rng(int(10 * half))
-    sc = scenes.Scene()
-    origins, dirs = [], []
-    poles, n = rng.uniform(-40 * half, 40 * half, (60, 3)), 12
-    for at in poles:
-        a, p = rng.normal(size=(2, 3))
+    ahead = 0
+    for _ in range(20):
+        sc = scenes.Scene()
+        a = rng.normal(size=3)
         a /= np.linalg.norm(a)
         q = np.array([a[2], 0, -a[0], 1 + a[1]])      # the turn that takes the y axis to a
-        sc.add_body(scenes.CAPSULE, [half, 0.02 * half], at, q / np.linalg.norm(q))
-        for _ in range(n):
-            p = rng.normal(size=3)
-            p -= p.dot(a) * a
-            end = rng.choice([-1, 1])
-            o = a * half * end * rng.uniform(0, 0.9) + p / np.linalg.norm(p) * half * rng.uniform(0.05, 0.6)
-            d = o - a * half * end * rng.uniform(1.05, 2.0)
-            d /= np.linalg.norm(d)
-            origins.append(at + o)
-            dirs.append(d)
-            sc.add_body(scenes.SPHERE, [0.01 * half], at + o + d * half * rng.uniform(0.02, 0.2))
-    g, o = lockstep(sc, 0)
-    origins, dirs = np.array(origins, np.float32), np.array(dirs, np.float32)
-    c, t = _same(g, o, origins, dirs, 200.0)
-    mn, mx = o.bounds()[c, :3], o.bounds()[c, 3:]
-    ahead = (np.minimum((mn - origins) / dirs, (mx - origins) / dirs)).max(1)
-    assert ((c >= 0) & (t == 0) & (ahead > 0.3 * half)).sum() > 5
+        sc.add_body(scenes.CAPSULE, [half, 0.02 * half], [0, 0, 0], q / np.linalg.norm(q))
+        p = np.cross(rng.normal(size=(48, 3)), a)
+        end = a * half * rng.choice([-1, 1], (48, 1))
+        origins = end * rng.uniform(0, 0.9, (48, 1)) + \
+            p / np.linalg.norm(p, axis=1, keepdims=True) * half * rng.uniform(0.05, 0.6, (48, 1))
+        dirs = origins - end * rng.uniform(1.05, 2.0, (48, 1))
+        dirs /= np.linalg.norm(dirs, axis=1, keepdims=True)
+        for at in origins + dirs * half * rng.uniform(0.02, 0.2, (48, 1)):
+            sc.add_body(scenes.SPHERE, [0.01 * half], at)
+        origins, dirs = origins.astype(np.float32), dirs.astype(np.float32)
+        g, o = lockstep(sc, 0)
+        c, t = _same(g, o, origins, dirs, 200.0)
+        mn, mx = o.bounds()[0, :3], o.bounds()[0, 3:]
+        entry = (np.minimum((mn - origins) / dirs, (mx - origins) / dirs)).max(1)
+        ahead += ((c == 0) & (t == 0) & (entry > 0.3 * half)).sum()
+    assert ahead > 5
