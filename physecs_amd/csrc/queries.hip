@@ -8,6 +8,7 @@
 // reference settles them by its tree's shape). The filter rejects one entity per ray.
 #include <cstring>
 #include "pgx_internal.h"
+#include "shape_bounds.h"
 
 using namespace pgx;
 
@@ -137,6 +138,7 @@ struct RayScene {
     const int32_t *cbody, *ctype;
     const uint32_t* centity;
     ConvexFaces cv;
+    const float4* cvVerts;
 };
 
 __device__ __forceinline__ bool ray_shape(int type, const float4& prm, f3 pos, qf q, const ConvexFaces& cv, f3 o, f3 d,
@@ -169,8 +171,9 @@ __device__ __forceinline__ void test_collider(const RayScene& S, int c, f3 o, f3
 // What a walk may skip once it has a hit: the boxes that the ray enters beyond it. A shape's
 // hit distance comes from its own formula and can lie before the float entry distance of its
 // box, so a box is skipped by the entry into itself widened by a margin. The computed hit
-// point is within the margin of the shape, and so of every box around it: with m the distance
-// to the shape the formulas' error is that of a difference of squares (sqrt(8 eps m^2), and
+// point is within the margin of the shape, and so of every box around it (k_ray_records sees
+// to it that they are: poses may be written without the bounds): with m the distance to the
+// shape the formulas' error is that of a difference of squares (sqrt(8 eps m^2), and
 // sqrt(2e-6 m^2) for a direction that is a unit vector to 2e-6: under 2e-3 m, in a sphere's,
 // capsule's or plane's direction), and a direction component under 0.001 counts as parallel
 // (intersectRayAABB, a drift of up to 0.001 t per axis). m and t are at most the distance to
@@ -219,14 +222,22 @@ __device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4
     const bool bounded = mn.x > -1e9f && mn.y > -1e9f && mn.z > -1e9f && mx.x < 1e9f && mx.y < 1e9f && mx.z < 1e9f;
     const bool units = fabsf(l.x * l.x + l.y * l.y + l.z * l.z + l.w * l.w - 1.f) < 1e-5f &&
                        fabsf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w - 1.f) < 1e-5f;
-    if (!(bounded && units)) *inOrder = 1;
     const qf lq = qmul(q4(q), q4(l));
     const f3 pos = add(xyz(S.bpos[b]), qrot(q4(q), xyz(S.clpos[c])));
-    rayLeaf[4 * (size_t)i] = f4(pos, __int_as_float(S.ctype[c]));
+    const int type = S.ctype[c];
+    bool around = true;   // the bounds hold the shape as it is now (rays never hit a triangle mesh)
+    if (type != PGX_TRIANGLE_MESH) {
+        f3 lo, hi;
+        shape_bounds(type, S.cparams[c], pos, lq, S.cvVerts, S.cv.mesh, nullptr, nullptr, lo, hi);
+        around = mn.x <= lo.x && mn.y <= lo.y && mn.z <= lo.z && lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z &&
+                 hi.x <= mx.x && hi.y <= mx.y && hi.z <= mx.z;
+    }
+    if (!(bounded && units && around)) *inOrder = 1;
+    rayLeaf[4 * (size_t)i] = f4(pos, __int_as_float(type));
     rayLeaf[4 * (size_t)i + 1] = f4(mk3(lq.x, lq.y, lq.z), lq.w);
     rayLeaf[4 * (size_t)i + 2] = S.cparams[c];
     rayLeaf[4 * (size_t)i + 3] = make_float4(__int_as_float(c), __uint_as_float(S.centity[c]), 0.f, 0.f);
-    if (S.ctype[c] != PGX_CAPSULE) return 0.f;
+    if (type != PGX_CAPSULE) return 0.f;
     const f3 far = mk3(fmaxf(pos.x - mn.x, mx.x - pos.x), fmaxf(pos.y - mn.y, mx.y - pos.y), fmaxf(pos.z - mn.z, mx.z - pos.z));
     return 2.5f * length(far);
 }
@@ -236,8 +247,8 @@ __device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4
 // {position, type}, {orientation}, {params}, {collider, entity}.
 // Sets *inOrder (0 before) if a dynamic collider is one for which the margin does not hold
 // or whose hit distance could be a NaN, which makes the result depend on the order of the
-// tests: bounds that are not finite, or an orientation that is not a unit quaternion. Raises
-// *near (0 before) to RaySkip::near.
+// tests: bounds that are not finite or do not hold the shape, or an orientation that is not a
+// unit quaternion. Raises *near (0 before) to RaySkip::near.
 __global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __restrict__ child, RayScene S,
                                                      const float4* __restrict__ leafB, const float4* __restrict__ clquat,
                                                      float4* __restrict__ rayNode, float4* __restrict__ rayLeaf,
@@ -408,6 +419,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
     S.cbmin = w.cbmin.p; S.cbmax = w.cbmax.p; S.cparams = w.cparams.p; S.clpos = w.clpos.p; S.clquat = w.clquat.p;
     S.bpos = w.bpos.p; S.bquat = w.bquat.p; S.cbody = w.cbody.p; S.ctype = w.ctype.p; S.centity = w.centity.p;
     S.cv = ConvexFaces{w.cvMesh.p, w.cvFaceN.p, w.cvFaceC.p};
+    S.cvVerts = w.cvVerts.p;
     if (w.nDynCol == 0) {
         fill_i32(s, w.worldRoot.p, -1, w.W);   // no tree: static lists only
     } else {

@@ -6,6 +6,7 @@ for bit."""
 import numpy as np
 import pytest
 
+import oracle_lib as ol
 from gpu_util import bits, lockstep, log
 from physecs_amd import scenes
 
@@ -114,3 +115,33 @@ def test_rays_that_start_beside_poles(half):
         entry = (np.minimum((mn - origins) / dirs, (mx - origins) / dirs)).max(1)
         ahead += ((c == 0) & (t == 0) & (entry > 0.3 * half)).sum()
     assert ahead > 5
+
+
+def test_poses_written_without_bounds():
+    """write_state moves bodies and leaves their bounds, which rays go on to enter, as they were:
+    a hit can lie far before its collider's box."""
+    rng = np.random.default_rng(4)
+    sc = scenes.Scene()
+    n = 60
+    for at in rng.uniform(-6, 6, (n, 3)):
+        sc.add_body(scenes.SPHERE, [0.5], at)
+    g, o = lockstep(sc, 0)
+    box = o.bounds()
+    pos = g.state()[0]
+    pos[:, 0] -= rng.uniform(0, 6, n).astype(np.float32)
+    g.write_state(pos=pos)
+    origins = rng.uniform(-8, 8, (400, 3)).astype(np.float32)
+    origins[:, 0] = -20
+    dirs = np.tile(np.float32([[1, 0, 0]]), (400, 1))
+    gc, gt, _ = g.raycast(origins, dirs, 200.0)
+    jumps = 0
+    for k in range(len(origins)):
+        best, dist, first = -1, 0.0, np.inf
+        for c in range(n):
+            met, entry = ol.ray_aabb("orc", origins[k], dirs[k], box[c, :3], box[c, 3:])
+            hit, t = ol.ray_geometry("orc", origins[k], dirs[k], scenes.SPHERE, [0.5], pos[c], [0, 0, 0, 1])
+            if met and hit and (best < 0 or t < dist):
+                best, dist, first = c, t, entry
+        assert gc[k] == best and bits(gt[k]) == bits(np.float32(dist)), k
+        jumps += best >= 0 and first > dist + 1
+    assert jumps > 20
