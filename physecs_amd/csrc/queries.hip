@@ -177,7 +177,9 @@ __device__ __forceinline__ void test_collider(const RayScene& S, int c, f3 o, f3
 // sqrt(2e-6 m^2) for a direction that is a unit vector to 2e-6: under 2e-3 m, in a sphere's,
 // capsule's or plane's direction), and a direction component under 0.001 counts as parallel
 // (intersectRayAABB, a drift of up to 0.001 t per axis). m and t are at most the distance to
-// the far corner of the tree's box.
+// the far corner of the tree's box. Far from the world's origin the boxes' corners and the
+// entry are rounded at the size of the coordinates (2^-24 of them each), the shapes' distances
+// are not: the margin grows with the coordinates too.
 //
 // A capsule is the exception (src/Raycast.cpp:65-100): where the ray's line leaves its cylinder
 // behind the origin, carried on beyond the caps, the hit counts as one at 0 if the origin lies
@@ -201,8 +203,10 @@ __device__ __forceinline__ RaySkip ray_skip(f3 o, f3 d, f3 inv, f3 mn, f3 mx, fl
     const f3 far = mk3(fmaxf(fabsf(mn.x - o.x), fabsf(mx.x - o.x)), fmaxf(fabsf(mn.y - o.y), fabsf(mx.y - o.y)),
                        fmaxf(fabsf(mn.z - o.z), fabsf(mx.z - o.z)));
     const float reach = far.x + far.y + far.z;
+    const float size = fmaxf(fabsf(mn.x), fabsf(mx.x)) + fmaxf(fabsf(mn.y), fabsf(mx.y)) +
+                       fmaxf(fabsf(mn.z), fabsf(mx.z)) + fabsf(o.x) + fabsf(o.y) + fabsf(o.z);
     const bool unit = fabsf(dot(d, d) - 1.f) < 2e-6f;
-    r.margin = unit && reach < 1e9f && dot(o, o) < 1e18f ? 4e-3f * reach : -1.f;
+    r.margin = unit && reach < 1e9f && dot(o, o) < 1e18f ? 4e-3f * reach + 4e-6f * size : -1.f;
     return r;
 }
 // a lower bound of the distance at which the ray enters the widened box

@@ -117,6 +117,18 @@ def test_rays_that_start_beside_poles(half):
     assert ahead > 5
 
 
+@pytest.mark.parametrize("at", [2.0 ** 20, -2.0 ** 20, 2.0 ** 23, 1e8])
+def test_far_from_the_worlds_origin(at):
+    """The nearer sphere's box is rounded to begin behind the other sphere's surface: 9.75 or 10
+    for 9.7, with a hit at 9.72 before it (both at 2^20 and 2^23; rounded further at 1e8)."""
+    sc = scenes.Scene()
+    sc.add_body(scenes.SPHERE, [1.3], [at + 11, 0, 0])
+    sc.add_body(scenes.SPHERE, [0.28], [at + 10, 0, 0])
+    g, o = lockstep(sc, 0)
+    for origin, d in ((at, 1), (at + 21, -1)):
+        _same(g, o, np.array([[origin, 0, 0]], np.float32), np.array([[d, 0, 0]], np.float32), 200.0)
+
+
 def test_poses_written_without_bounds():
     """write_state moves bodies and leaves their bounds, which rays go on to enter, as they were:
     a hit can lie far before its collider's box."""
