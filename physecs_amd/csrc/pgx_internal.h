@@ -299,6 +299,7 @@ struct World {
     DBuf<int4> cvMesh;
     DBuf<int2> cvFace;
     DBuf<int32_t> cvFaceIdx;
+    DBuf<float> cvSlender;             // per mesh: hull_slenderness
     DBuf<int32_t> heavy;               // from its start: pairs with a convex mesh; from its end: pairs of boxes touching with a face (filled by the primitive kernel)
     // static triangle meshes: vertices, triangles in the BVH build's order (mesh-local
     // vertex indices), triangle normals / centroids, BVH nodes (2 float4 each: {min,

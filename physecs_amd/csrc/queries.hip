@@ -139,6 +139,7 @@ struct RayScene {
     const uint32_t* centity;
     ConvexFaces cv;
     const float4* cvVerts;
+    const float* cvSlender;
 };
 
 __device__ __forceinline__ bool ray_shape(int type, const float4& prm, f3 pos, qf q, const ConvexFaces& cv, f3 o, f3 d,
@@ -235,8 +236,15 @@ __device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4
         shape_bounds(type, S.cparams[c], pos, lq, S.cvVerts, S.cv.mesh, nullptr, nullptr, lo, hi);
         around = mn.x <= lo.x && mn.y <= lo.y && mn.z <= lo.z && lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z &&
                  hi.x <= mx.x && hi.y <= mx.y && hi.z <= mx.z;
+        if (type == PGX_CAPSULE) around = around && S.cparams[c].y >= 0.f;   // a radius below 0 narrows the bounds alone
     }
-    if (!(bounded && units && around)) *inOrder = 1;
+    bool closed = true;   // a hull's half-spaces end at its vertices
+    if (type == PGX_CONVEX_MESH) {
+        const float4 s = S.cparams[c];
+        const float x = fabsf(s.x), y = fabsf(s.y), z = fabsf(s.z);
+        closed = S.cvSlender[(int)s.w] * fmaxf(x, fmaxf(y, z)) <= 32.f * fminf(x, fminf(y, z)) && x > 0.f;
+    }
+    if (!(bounded && units && around && closed)) *inOrder = 1;
     rayLeaf[4 * (size_t)i] = f4(pos, __int_as_float(type));
     rayLeaf[4 * (size_t)i + 1] = f4(mk3(lq.x, lq.y, lq.z), lq.w);
     rayLeaf[4 * (size_t)i + 2] = S.cparams[c];
@@ -251,8 +259,10 @@ __device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4
 // {position, type}, {orientation}, {params}, {collider, entity}.
 // Sets *inOrder (0 before) if a dynamic collider is one for which the margin does not hold
 // or whose hit distance could be a NaN, which makes the result depend on the order of the
-// tests: bounds that are not finite or do not hold the shape, or an orientation that is not a
-// unit quaternion. Raises *near (0 before) to RaySkip::near.
+// tests: bounds that are not finite or do not hold the shape, an orientation that is not a unit
+// quaternion, or a hull whose half-spaces go on beyond its vertices (hull_slenderness; up to 32
+// the planes' rounding, some 1e-6 of the distance and 2^-23 of the coordinates, stays within
+// the margin). Raises *near (0 before) to RaySkip::near.
 __global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __restrict__ child, RayScene S,
                                                      const float4* __restrict__ leafB, const float4* __restrict__ clquat,
                                                      float4* __restrict__ rayNode, float4* __restrict__ rayLeaf,
@@ -423,7 +433,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
     S.cbmin = w.cbmin.p; S.cbmax = w.cbmax.p; S.cparams = w.cparams.p; S.clpos = w.clpos.p; S.clquat = w.clquat.p;
     S.bpos = w.bpos.p; S.bquat = w.bquat.p; S.cbody = w.cbody.p; S.ctype = w.ctype.p; S.centity = w.centity.p;
     S.cv = ConvexFaces{w.cvMesh.p, w.cvFaceN.p, w.cvFaceC.p};
-    S.cvVerts = w.cvVerts.p;
+    S.cvVerts = w.cvVerts.p; S.cvSlender = w.cvSlender.p;
     if (w.nDynCol == 0) {
         fill_i32(s, w.worldRoot.p, -1, w.W);   // no tree: static lists only
     } else {

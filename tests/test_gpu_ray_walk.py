@@ -129,6 +129,41 @@ def test_far_from_the_worlds_origin(at):
         _same(g, o, np.array([[origin, 0, 0]], np.float32), np.array([[d, 0, 0]], np.float32), 200.0)
 
 
+def _prism():
+    """A box's faces without the top one: the half-spaces of the others have no upper end."""
+    v, f, n, c = scenes.convex_hull(np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)], float))
+    keep = [k for k in range(len(f)) if n[k][1] < 0.5]
+    return v, [f[k] for k in keep], n[keep], c[keep]
+
+
+def test_hull_that_its_faces_do_not_close():
+    """The ray meets a side's plane above the bounds, at 4.12 m, and enters them 7.2 m ahead,
+    behind a sphere that is met at 5.2 m."""
+    sc = scenes.Scene()
+    sc.add_convex_body(sc.add_convex_mesh(*_prism()), [0, 0, 0])
+    sc.add_body(scenes.SPHERE, [0.2], [-0.7, 2.8, 0])
+    d = np.array([1, -4, 0.01]) / np.sqrt(17.0001)
+    c, t = _same(*lockstep(sc, 0), np.array([[-2, 8, 0]], np.float32), d[None].astype(np.float32), 200.0)
+    assert c[0] == 0 and 4 < t[0] < 4.2
+
+
+@pytest.mark.parametrize("scale", [(1, 1, 1), (1, -0.5, 2), (1, 0.002, 1), (0.001, 1, 0.001)])
+def test_hulls_of_any_scale(scale):
+    """Rays past the rims of hulls, flat and needle-like ones too, with spheres around them."""
+    rng = np.random.default_rng(9)
+    sc = scenes.Scene()
+    mesh = sc.add_convex_mesh(*scenes.ellipsoid_hull(rng))
+    at, q = rng.uniform(-3, 3, (40, 3)), scenes.random_quats(rng, 40)
+    for k in range(40):
+        sc.add_convex_body(mesh, at[k], q[k], scale)
+        sc.add_body(scenes.SPHERE, [0.1], at[k] + rng.uniform(-0.8, 0.8, 3))
+    g, o = lockstep(sc, 0)
+    origins = rng.uniform(-8, 8, (2000, 3))
+    dirs = at[rng.integers(0, 40, 2000)] + rng.uniform(-0.4, 0.4, (2000, 3)) * np.abs(scale) - origins
+    dirs /= np.linalg.norm(dirs, axis=1, keepdims=True)
+    _same(g, o, origins.astype(np.float32), dirs.astype(np.float32), 200.0)
+
+
 def test_poses_written_without_bounds():
     """write_state moves bodies and leaves their bounds, which rays go on to enter, as they were:
     a hit can lie far before its collider's box."""
