@@ -1432,8 +1432,9 @@ __global__ __launch_bounds__(MESH_BLOCK_WAVES * 64) void k_mesh_query(MeshArgs A
         }
         const int base = block_reserve<MESH_BLOCK_WAVES>(A.candTotal, nc);
         if (h >= n) continue;
-        if (base + nc > A.candCap) {
+        if (base + nc > A.candCap) {   // the last slots, some of the pair's, stay empty
             if (!QUERY && lane == 0) atomicAdd(A.errors, 1);
+            for (int i = base + lane; i < A.candCap; i += WAVE) A.pairOf[i] = -1;
             nc = 0;
         }
         for (int i = lane; i < nc; i += WAVE) {
@@ -1448,7 +1449,8 @@ __global__ __launch_bounds__(MESH_BLOCK_WAVES * 64) void k_mesh_query(MeshArgs A
 }
 
 // pass 2, a lane per (pair, candidate triangle): the closed forms and their contact records;
-// for a convex mesh GJK, its hits listed with their simplex
+// for a convex mesh GJK, its hits listed with their simplex. Slots without a candidate (pair
+// -1) are skipped; no pair's records are among them.
 constexpr int MESH_TEST_BLOCKS = 2048;
 template <bool QUERY, bool CONVEX>
 __global__ __launch_bounds__(64) void k_mesh_test(MeshArgs A) {
@@ -1456,12 +1458,13 @@ __global__ __launch_bounds__(64) void k_mesh_test(MeshArgs A) {
     // whole waves go round together, so the appends see whole waves
     for (int base = blockIdx.x * WAVE; base < total; base += gridDim.x * WAVE) {
         const int k = base + (int)threadIdx.x;
+        const int h = k < total ? A.pairOf[k] : -1;
         bool solved = false;
         GV va, vb, vc, vd;
-        if (k < total) {
+        if (h >= 0) {
             MeshPair m;
             SupConvex sc;
-            mesh_pair<QUERY>(A, A.pairOf[k], m, sc);
+            mesh_pair<QUERY>(A, h, m, sc);
             const MeshCtx mc{&A.tv, m.mi};
             TCI ci;
             ci.tri = A.cand[k];
