@@ -1387,6 +1387,9 @@ __device__ __forceinline__ bool mesh_pair(const MeshArgs& A, int h, MeshPair& m,
 // Places in a list for the waves of a block, n[wave] each: one atomic per block. (One per
 // wave, on one address, served some 65 per us: 47 us for the 3,071 pairs of 2,048 hulls and
 // 1,024 capsules on a terrain, more than the query itself.) Every wave of the block calls it.
+// A list counts on past its end, up to RESERVE_MAX places and what the blocks then at work ask
+// for, so that places never wrap: a block that comes after takes its count back.
+constexpr int RESERVE_MAX = 1 << 30;
 template <int WAVES>
 __device__ __forceinline__ int block_reserve(int32_t* counter, int n) {
     __shared__ int count[WAVES], first;
@@ -1397,6 +1400,7 @@ __device__ __forceinline__ int block_reserve(int32_t* counter, int n) {
         int total = 0;
         for (int k = 0; k < WAVES; ++k) total += count[k];
         first = total ? atomicAdd(counter, total) : 0;
+        if (first > RESERVE_MAX) atomicSub(counter, total);
     }
     __syncthreads();
     int at = first;
@@ -1786,6 +1790,8 @@ static MeshArgs mesh_args(World& w, MeshBuffers& b) {
 
 // buffers for the mesh pairs' passes: `pairs` pairs, `cands` candidate triangles
 void np_mesh_buffers(World& w, MeshBuffers& b, size_t pairs, size_t cands) {
+    if (cands > (size_t)RESERVE_MAX)
+        throw PgxError{PGX_ERR_CAPACITY, std::to_string(cands) + " candidate triangles are more than a call's list can hold"};
     b.candOff.alloc(pairs); b.candCount.alloc(pairs);
     if ((size_t)b.candCap >= cands) return;
     b.cand.alloc(cands); b.pairOf.alloc(cands);

@@ -7,6 +7,7 @@
 // hits the closest is kept; equal distances go to the lower collider index (the
 // reference settles them by its tree's shape). The filter rejects one entity per ray.
 #include <cstring>
+#include <limits>
 #include "pgx_internal.h"
 #include "shape_bounds.h"
 
@@ -475,9 +476,15 @@ static void upload_query_shapes(World& w, int n, const int32_t* types, const flo
     PGX_HIP(hipStreamSynchronize(w.stream));   // hs is released on return
 }
 
-int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, const float* positions,
-                   const float* orientations, const int32_t* queryWorld, int capacity, int32_t* offsets,
-                   int32_t* colliders, float* normalMtd, int32_t* total, double* deviceUs) {
+// Candidate triangles of one pass over the queries: 72 bytes each, and 144 more in a world with
+// hulls, so at most 1.2 or 3.6 GB. A call with more of them is made of several passes.
+constexpr int MTD_MAX_CANDS = 1 << 24;
+
+// One pass: PGX_OK or PGX_ERR_CAPACITY, or, with *candidates set, MTD_TOO_MANY.
+constexpr int MTD_TOO_MANY = 1;
+static int overlap_mtd_pass(World& w, int n, const int32_t* types, const float* params, const float* positions,
+                            const float* orientations, const int32_t* queryWorld, int capacity, int32_t* offsets,
+                            int32_t* colliders, float* normalMtd, int32_t* total, double* deviceUs, int* candidates) {
     constexpr int MBITS = 8;   // manifold index within a pair (the kernels' MTD_MBITS)
     constexpr int MTD_COUNTS = 6;
     hipStream_t s = w.stream;
@@ -502,7 +509,8 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
     A.counts = w.qMtdN.p; A.keys = w.qKeys.p; A.vals = w.qVals.p; A.res = w.qRes.p;
     int cnt[MTD_COUNTS] = {};
     int listCap = (int)std::max<size_t>(std::max<size_t>(w.qCvxPairs.n, 4096), 4 * (size_t)n);
-    size_t cands = std::max<size_t>({(size_t)w.qMesh.candCap, (size_t)1 << 18, 2 * (size_t)n});
+    size_t cands = std::max<size_t>({(size_t)w.qMesh.candCap, (size_t)1 << 18,
+                                     std::min<size_t>(2 * (size_t)n, MTD_MAX_CANDS)});
     float ms0 = 0.f;
     // the second attempt with pair lists, the third with candidate lists as long as was needed
     for (int attempt = 0; attempt < 3; ++attempt) {
@@ -521,6 +529,10 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
         PGX_HIP(hipEventElapsedTime(&ms0, w.qEv[0], w.qEv[1]));
         const bool pairs = std::max(cnt[1], cnt[2]) <= listCap;
         if (pairs && (w.nTriMesh == 0 || cnt[4] <= w.qMesh.candCap)) break;
+        if (w.nTriMesh > 0 && cnt[4] > std::max(w.qMesh.candCap, MTD_MAX_CANDS) && n > 1) {
+            *candidates = cnt[4];
+            return MTD_TOO_MANY;
+        }
         if (attempt == 2) throw PgxError{PGX_ERR_HIP, "MTD query: pair or candidate lists overflowed again"};
         if (!pairs) listCap = std::max(cnt[1], cnt[2]);
         else cands = (size_t)cnt[4];
@@ -563,6 +575,46 @@ int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, c
     }
     offsets[n] = k;
     if (k != m) throw PgxError{PGX_ERR_HIP, "MTD query: result keys out of order"};
+    return PGX_OK;
+}
+
+int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, const float* positions,
+                   const float* orientations, const int32_t* queryWorld, int capacity, int32_t* offsets,
+                   int32_t* colliders, float* normalMtd, int32_t* total, double* deviceUs) {
+    int candidates = 0;
+    const int rc = overlap_mtd_pass(w, n, types, params, positions, orientations, queryWorld, capacity, offsets,
+                                    colliders, normalMtd, total, deviceUs, &candidates);
+    if (rc != MTD_TOO_MANY) return rc;
+    // parts of the queries with about half of what a pass may have each, and their results one
+    // after the other; the caller's arrays are written only when all of them fit
+    const int part = (int)std::max<long long>(1, (long long)n * (MTD_MAX_CANDS / 2) / candidates);
+    std::vector<int32_t> off((size_t)n + 1), cols((size_t)capacity);
+    std::vector<float> nm(4 * (size_t)capacity);
+    long long found = 0;
+    double us = 0.0;
+    for (int lo = 0; lo < n; lo += part) {
+        const int m = std::min(part, n - lo);
+        const int room = (int)std::max<long long>(0, capacity - found);
+        int32_t t = 0;
+        double partUs = 0.0;
+        const size_t at = (size_t)(capacity - room);
+        const int r = qr_overlap_mtd(w, m, types + lo, params + 4 * (size_t)lo, positions + 3 * (size_t)lo,
+                                     orientations + 4 * (size_t)lo, queryWorld ? queryWorld + lo : nullptr, room,
+                                     off.data() + lo, cols.data() + at, nm.data() + 4 * at, &t, &partUs);
+        if (r != PGX_OK && r != PGX_ERR_CAPACITY) return r;
+        if (r == PGX_OK)
+            for (int i = 0; i <= m; ++i) off[lo + i] += (int32_t)found;
+        found += t;
+        us += partUs;
+    }
+    if (found > std::numeric_limits<int32_t>::max())
+        throw PgxError{PGX_ERR_CAPACITY, "MTD query: " + std::to_string(found) + " hits are more than a call can return"};
+    *total = (int32_t)found;
+    if (deviceUs) *deviceUs = us;
+    if (found > capacity) return PGX_ERR_CAPACITY;
+    std::copy(off.begin(), off.end(), offsets);
+    std::copy(cols.begin(), cols.begin() + found, colliders);
+    std::copy(nm.begin(), nm.begin() + 4 * found, normalMtd);
     return PGX_OK;
 }
 

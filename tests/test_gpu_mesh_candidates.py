@@ -1,6 +1,7 @@
 """The triangle-mesh passes keep the candidate triangles of all pairs in one list. Where it is
-too short for a call's candidates, an MTD query asks again with a longer one and must give what
-the same queries give in smaller calls; a step raises the capacity error."""
+too short for a call's candidates, an MTD query asks again with a longer one, and beyond 2^24 of
+them query by query range; it must give what the same queries give in smaller calls. A step
+raises the capacity error."""
 import numpy as np
 import pytest
 
@@ -53,24 +54,40 @@ def _world(hulls):
     return api.World(sc)
 
 
-def _same_in_parts(n, part, hulls, candidates):
-    q = _queries(n, hulls)
-    pos = q[2]
-    assert _under(pos - 0.24, pos + 0.24) > candidates     # within every shape's bounds
+def _same_in_parts(q, part, hulls):
+    n = len(q[0])
     log(f"[candidates] {n} queries, hulls {hulls}, in one call and in calls of {part}")
     whole, parts = _world(hulls), _world(hulls)
     got, _ = whole.overlap_mtd(*q)
     for lo in range(0, n, part):
         for k, (c, m) in enumerate(parts.overlap_mtd(*(x[lo:lo + part] for x in q))[0]):
             assert np.array_equal(c, got[lo + k][0]) and np.array_equal(bits(m), bits(got[lo + k][1])), lo + k
-    assert sum(len(c) for c, _ in got) > n
     whole.close()
     parts.close()
+    total = sum(len(c) for c, _ in got)
+    assert total > n
+    return total
 
 
 @pytest.mark.parametrize("hulls", [0, 1])
 def test_more_candidates_than_the_first_list_holds(hulls):
-    _same_in_parts(12007, 1000, hulls, INITIAL)
+    q = _queries(12007, hulls)
+    assert _under(q[2] - 0.24, q[2] + 0.24) > INITIAL     # within every shape's bounds
+    _same_in_parts(q, 1000, hulls)
+
+
+def test_more_candidates_than_a_pass_takes():
+    """Spheres of 1.8 m, which overlap some 180 triangles and touch few."""
+    from physecs_amd import api
+    n = 105001
+    pos = np.random.default_rng(2).uniform((-4, 0.7, -4), (4, 0.8, 4), (n, 3)).astype(np.float32)
+    assert _under(pos - 0.9, pos + 0.9) > 1 << 24
+    q = np.full(n, scenes.SPHERE), np.tile(np.float32([0.9]), (n, 1)), pos, np.tile(np.float32([0, 0, 0, 1]), (n, 1))
+    total = _same_in_parts(q, 20000, 0)
+    w = _world(0)
+    with pytest.raises(api.PgxError, match=f"{total} hits exceed the capacity {total - 1}"):
+        w.overlap_mtd(*q, capacity=total - 1)
+    w.close()
 
 
 def test_a_step_with_too_many_candidates_says_so():
