@@ -1792,12 +1792,7 @@ static MeshArgs mesh_args(World& w, MeshBuffers& b) {
 void np_mesh_buffers(World& w, MeshBuffers& b, size_t pairs, size_t cands) {
     if (cands > (size_t)RESERVE_MAX)
         throw PgxError{PGX_ERR_CAPACITY, std::to_string(cands) + " candidate triangles are more than a call's list can hold"};
-    b.candOff.alloc(pairs); b.candCount.alloc(pairs);
-    if ((size_t)b.candCap >= cands) return;
-    b.cand.alloc(cands); b.pairOf.alloc(cands);
-    b.recs.alloc((size_t)(TM_CI_WORDS + 1) * cands);
-    if (w.nConvex > 0) { b.hitList.alloc(cands); b.simplex.alloc(36 * cands); }
-    b.candCap = (int)cands;
+    b.reserve(pairs, cands, w.nConvex > 0);
 }
 
 void np_mtd_launch(World& w, const MtdArgs& A) {

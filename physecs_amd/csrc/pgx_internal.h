@@ -161,6 +161,20 @@ struct MeshBuffers {
     int candCap = 0;
     DBuf<int32_t> cand, pairOf, recs, candOff, candCount, hitList;
     DBuf<float> simplex;
+    void reserve(size_t pairs, size_t cands, bool hulls) {
+        candOff.alloc(pairs);
+        candCount.alloc(pairs);
+        if ((size_t)candCap >= cands) return;
+        candCap = 0;   // none, if one of these fails: each frees what it had first
+        cand.alloc(cands);
+        pairOf.alloc(cands);
+        recs.alloc((size_t)(TM_CI_WORDS + 1) * cands);
+        if (hulls) {
+            hitList.alloc(cands);
+            simplex.alloc(36 * cands);
+        }
+        candCap = (int)cands;
+    }
 };
 
 struct World {
