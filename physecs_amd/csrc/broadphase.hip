@@ -447,7 +447,13 @@ __global__ void k_grid_pack(int n, const int32_t* __restrict__ order, const floa
 // behind the cells' frame are added in another order than k_scene_bounds adds them over
 // several workgroups; the pairs do not depend on the frame.) 210 colliders: seven launches and
 // 29 us of kernels before, 17 us now. 3,072 colliders take 57 us, no less than the launches.
-constexpr int GRID_SMALL = 2048;
+// The non-dynamic colliders are packed here too, at about a microsecond for each of the
+// workgroup's rounds, or in a launch of their own (k_grid_pack) when there are more than
+// GRID_STATICS rounds of them and more than GRID_APART dynamic ones. A step of 500 worlds of
+// two bodies takes 170 us here and 167 apart with 16 non-dynamic colliders each (eight rounds),
+// 337 and 250 with 200, 1,040 and 607 with 1,000; of ten such worlds with 600 each, whose pair
+// search is a block or two that finds the records in the L2 they were written to, 252 and 300.
+constexpr int GRID_SMALL = 2048, GRID_STATICS = 8, GRID_APART = 64;
 __global__ __launch_bounds__(RS_SINGLE_THREADS) void k_grid_small(
     int n, int items, int bits, const int32_t* __restrict__ dynCols, const int32_t* __restrict__ cworld,
     const float4* __restrict__ cbmin, const float4* __restrict__ cbmax, const int32_t* __restrict__ cflags,
@@ -1084,9 +1090,14 @@ static void bp_grid(World& w) {
     const uint32_t T = grid_table_size(n);
     const int nStatic = w.C - w.nDynCol;
     if (n <= GRID_SMALL) {
+        const bool apart = n > GRID_APART && nStatic > GRID_STATICS * rs_threads(n);
+        if (apart)
+            hipLaunchKernelGGL(k_grid_pack, dim3(div_up(nStatic, 256)), dim3(256), 0, s, 0, w.mvals.p, w.cbmin.p,
+                               w.cbmax.p, w.cflags.p, w.centity.p, w.clocal.p, w.gridRec.p, nStatic, w.staticCols.p,
+                               w.statA.p, w.statB.p, w.statL.p);
         hipLaunchKernelGGL(k_grid_small, dim3(1), dim3(rs_threads(n)), 0, s, n, rs_item_count(n), 30 + w.worldBits,
                            w.dynCols.p, w.cworld.p, w.cbmin.p, w.cbmax.p, w.cflags.p, w.centity.p, w.clocal.p, w.mkeys.p,
-                           w.mvals.p, T - 1, w.gridKey.p, w.gridStart.p, w.gridEnd.p, w.gridRec.p, nStatic,
+                           w.mvals.p, T - 1, w.gridKey.p, w.gridStart.p, w.gridEnd.p, w.gridRec.p, apart ? 0 : nStatic,
                            w.staticCols.p, w.statA.p, w.statB.p, w.statL.p, w.counters.p);
     } else {
         hipLaunchKernelGGL(k_scene_bounds_init, dim3(1), dim3(64), 0, s, w.worldBoundsI.p, w.sceneMoments.p,

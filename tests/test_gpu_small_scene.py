@@ -39,6 +39,22 @@ def test_piles_lockstep_bitexact(side):
     lockstep(scenes.mixed_lattice(5, side=side), 30 if side < 15 else 12, check_every=6)
 
 
+@pytest.mark.parametrize("bodies,statics", [(64, 2100), (65, 2048), (65, 2049), (300, 4097), (3, 7000)])
+def test_statics_packed_in_the_grid_or_apart(bodies, statics):
+    """The grid's workgroup (256 threads for up to 256 bodies, 512 for up to 512) packs the
+    non-dynamic colliders of up to 64 bodies, and up to eight a thread of more bodies; beyond,
+    they have a launch of their own."""
+    sc = scenes.Scene()
+    side = int(np.ceil(statics ** 0.5))
+    for i in range(statics):
+        sc.add_static(scenes.BOX, [0.5, 0.3, 0.5], [i % side - side / 2, -0.3, i // side - side / 2])
+    for i in range(bodies):
+        sc.add_body((scenes.SPHERE, scenes.BOX)[i % 2], [[0.4], [0.3, 0.3, 0.3]][i % 2],
+                    [0.9 * (i % 16) - 7, 0.35, 0.9 * (i // 16) - 9])
+    g, _ = lockstep(sc, 4)
+    assert g.counts()["pairs"] >= bodies
+
+
 def test_a_full_cell_hands_the_step_to_the_tree_walk():
     """729 small bodies in one cell, made large by one large body: more than a cell may hold."""
     sc = scenes.Scene()
