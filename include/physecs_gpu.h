@@ -286,6 +286,8 @@ int pgx_world_write_state(pgx_world* w, const float* pos, const float* quat, con
 
 /* Introspection of the last step (for tests and tools). */
 int pgx_world_get_counts(pgx_world* w, pgx_counts* out);
+/* Steps since creation whose pairs the tree walk found because a cell of the grid was too full. */
+int pgx_world_get_grid_fallbacks(pgx_world* w, long* out);
 /* Bounds of every collider, descriptor order: min xyz, max xyz. */
 int pgx_world_get_bounds(pgx_world* w, float* out);
 /* Candidate pairs as descriptor collider indices (collider of the smaller entity first),

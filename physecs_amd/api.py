@@ -28,7 +28,7 @@ ERRORS = {-1: "PGX_ERR_INVALID", -2: "PGX_ERR_HIP", -3: "PGX_ERR_CAPACITY", -4: 
 EXPORTS = [
     "pgx_last_error", "pgx_device_count", "pgx_sort_u64", "pgx_sort_u64_noalloc", "pgx_world_create", "pgx_world_destroy", "pgx_world_set_params", "pgx_world_set_contact_filter",
     "pgx_world_set_can_collide", "pgx_world_step", "pgx_world_sync", "pgx_world_read_state",
-    "pgx_world_write_state", "pgx_world_get_counts", "pgx_world_get_bounds", "pgx_world_get_pairs",
+    "pgx_world_write_state", "pgx_world_get_counts", "pgx_world_get_grid_fallbacks", "pgx_world_get_bounds", "pgx_world_get_pairs",
     "pgx_world_get_manifolds", "pgx_world_enable_timing", "pgx_world_get_timing", "pgx_world_reset_stats",
     "pgx_world_get_stats", "pgx_world_set_exec", "pgx_world_add_joints", "pgx_world_set_joint_params",
     "pgx_world_destroy_joint", "pgx_world_set_graph", "pgx_world_set_tuning", "pgx_world_get_tuning",
@@ -193,6 +193,7 @@ def lib():
         L.pgx_world_read_state.argtypes = [vp, F, F, F, F]
         L.pgx_world_write_state.argtypes = [vp, F, F, F, F]
         L.pgx_world_get_counts.argtypes = [vp, ctypes.POINTER(PgxCounts)]
+        L.pgx_world_get_grid_fallbacks.argtypes = [vp, ctypes.POINTER(ctypes.c_long)]
         L.pgx_world_get_bounds.argtypes = [vp, F]
         L.pgx_world_get_pairs.argtypes = [vp, I32, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
         L.pgx_world_get_manifolds.argtypes = [vp, I32, I32, F, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
@@ -441,6 +442,12 @@ class World:
             return
         self._joint_fns = joint_callbacks(layout, rows)   # kept alive with the world
         check(self.L.pgx_world_set_joint_callbacks(self.h, self._joint_fns[0], self._joint_fns[1], None))
+
+    def grid_fallbacks(self):
+        """pgx_world_get_grid_fallbacks: steps whose pairs came from the tree walk, for a full cell."""
+        n = ctypes.c_long(0)
+        check(self.L.pgx_world_get_grid_fallbacks(self.h, ctypes.byref(n)))
+        return n.value
 
     def counts(self):
         c = PgxCounts()

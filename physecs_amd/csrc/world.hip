@@ -1633,6 +1633,12 @@ int pgx_world_patch_transforms(pgx_world* h, int n, const int32_t* actors, const
     });
 }
 
+int pgx_world_get_grid_fallbacks(pgx_world* h, long* out) {
+    if (!h || !out) return fail(PGX_ERR_INVALID, "NULL argument");
+    *out = h->w.gridFallbacks;
+    return PGX_OK;
+}
+
 int pgx_world_get_counts(pgx_world* h, pgx_counts* out) {
     if (!h || !out) return fail(PGX_ERR_INVALID, "NULL argument");
     out->pairs = h->w.lastPairs;

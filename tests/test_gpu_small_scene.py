@@ -36,7 +36,8 @@ def test_worlds_alone_and_in_a_large_batch():
 def test_piles_lockstep_bitexact(side):
     """1 to 4,913 bodies: one to four manifolds a thread, and beyond the limit."""
     log(f"[small] a pile of {side ** 3} bodies")
-    lockstep(scenes.mixed_lattice(5, side=side), 30 if side < 15 else 12, check_every=6)
+    g, _ = lockstep(scenes.mixed_lattice(5, side=side), 30 if side < 15 else 12, check_every=6)
+    assert g.grid_fallbacks() == 0
 
 
 @pytest.mark.parametrize("bodies,statics", [(64, 2100), (65, 2048), (65, 2049), (300, 4097), (3, 7000)])
@@ -62,4 +63,5 @@ def test_a_full_cell_hands_the_step_to_the_tree_walk():
         sc.add_body(scenes.SPHERE, [0.3], [0.7 * (i % 9), 0.7 * (i // 9 % 9), 0.7 * (i // 81)])
     sc.add_body(scenes.SPHERE, [4.0], [20, 3, 3])
     sc.add_static(scenes.BOX, [30, 0.5, 30], [0, -0.85, 0])
-    lockstep(sc, 6, check_every=3)
+    g, _ = lockstep(sc, 6, check_every=3)
+    assert g.grid_fallbacks() == 6
