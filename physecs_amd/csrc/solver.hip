@@ -1154,9 +1154,10 @@ __global__ __launch_bounds__(XPASS_THREADS) void k_solve_xpass(SubArgs a, int nC
 // step: a run's slots never change within the step.
 constexpr int BATCH_THREADS = 1024;     // two lanes per manifold; 4 waves per SIMD at 128 registers
 constexpr int BATCH_MAP_THREADS = 1024;
-constexpr int BATCH_HASH = 8192;        // LDS hash of body -> slot: at least twice a run's bodies
+constexpr int BATCH_HASH = 8192;        // LDS hash of body -> slot, at most 59% full
 constexpr int BATCH_MAX_GROUPS = 16;
 constexpr int BATCH_MAX_MANIFOLDS = 2400;   // 2 x 2400 bodies x 32 B of velocities in LDS
+static_assert(10 * 2 * BATCH_MAX_MANIFOLDS <= 6 * BATCH_HASH, "a run's bodies fill at most six tenths of the hash");
 constexpr int BATCH_MAX_COLOURS = 128;
 constexpr int BATCH_LANES = BATCH_THREADS / 2;   // a team's
 constexpr int BATCH_MAX_TURNS = BATCH_MAX_COLOURS + 2 * BATCH_MAX_MANIFOLDS / BATCH_LANES + 1;
