@@ -600,6 +600,12 @@ constexpr int ISLAND_CHUNK = WAVE / 2;
 // pushes {linear 0, bits} {linear 1, bits} {angular 0, -} {angular 1, -}. Bits: the row in
 // 0-2, then JF_* flags and what the chain does with the row.
 constexpr int ROW_WORDS = 8, PUSH_WORDS = 4;
+// what a pass keeps in LDS: the bodies' velocities, a chunk's joints and rows
+constexpr size_t island_lds(int bodies, int joints, int words) {
+    return 2 * sizeof(float4) * bodies + sizeof(int4) * joints + sizeof(float4) * words * JOINT_MAX_ROWS * joints;
+}
+// eight colours, a body more than joints: 45 KB; the launches ask for no raised limit
+static_assert(island_lds(8 * ISLAND_MAX + 1, ISLAND_CHUNK, ROW_WORDS) <= 64 * 1024, "an island's pass fits the LDS");
 constexpr int RB_FLAGS = 4, RB_WARM = 1 << 8, RB_MOVES = 1 << 9;
 struct IslandArgs {
     const int32_t *cs, *bs, *body;   // per island: 9 colour offsets, first body; bodies
@@ -972,13 +978,13 @@ void jt_colors(World& w, float h, int phase, bool warm) {
     if (w.jIslands > 0) {   // colours 0-7 by island in one launch, then the overflow colour
         const IslandArgs is{w.jIslandCS.p, w.jIslandBS.p, w.jIslandBody.p, w.jIslandJoint.p};
         const int m = std::min(w.jIslandJoints, ISLAND_CHUNK), threads = div_up(8 * m, WAVE) * WAVE;
-        const size_t lds = 2 * sizeof(float4) * w.jIslandBodies + sizeof(int4) * m;
         if (phase == 0)
             hipLaunchKernelGGL(islands_update(w) ? k_island_presolve<true> : k_island_presolve<false>,
-                               dim3(w.jIslands), dim3(threads), lds + sizeof(float4) * PUSH_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m);
+                               dim3(w.jIslands), dim3(threads), island_lds(w.jIslandBodies, m, PUSH_WORDS), w.stream, a, is,
+                               w.jIslandBodies, m);
         else
             hipLaunchKernelGGL(k_island_solve, dim3(w.jIslands), dim3(threads),
-                               lds + sizeof(float4) * ROW_WORDS * JOINT_MAX_ROWS * m, w.stream, a, is, w.jIslandBodies, m,
+                               island_lds(w.jIslandBodies, m, ROW_WORDS), w.stream, a, is, w.jIslandBodies, m,
                                warm ? 1 : 0);
         const int b = w.jColorStart[8], e = w.jColorStart[9];
         if (e > b)

@@ -701,7 +701,6 @@ static void grow_keep(DBuf<T>& b, int keep, int n, hipStream_t s) {
     b.n = (size_t)std::max(n, 1);
 }
 
-constexpr int ISLAND_MAX = 64;   // joints of one colour in one island: one wave's lanes
 constexpr int ISLAND_MIN = 1;
 
 // The live joints grouped by colour, creation order inside a colour, and the per-joint
