@@ -23,7 +23,7 @@ import pytest
 from physecs_amd import api, scenes
 import shim_lib
 
-pytestmark = pytest.mark.skipif(not os.path.isdir(shim_lib.REFERENCE), reason="needs the reference's headers")
+pytestmark = pytest.mark.skipif(not os.path.isdir(os.path.join(shim_lib.REFERENCE, "include")), reason="needs the reference's headers")
 
 HEADER = 48   # bytes of a triangle-mesh cache's header
 
