@@ -5,8 +5,8 @@
 // :54-107,135-350, capsule-box :501-692), src/GeomUtil.cpp (segment distances and the
 // segment-AABB regions :7-59,129-467), src/Clipping.cpp (:10-71) and
 // src/ContactsUtil.cpp (:9-107), operation for operation, so the manifold is bit-identical
-// to the reference's for the same poses. The polygon clip buffers live in registers
-// (a quad clipped by four edges has at most 8 vertices).
+// to the reference's for the same poses. Face contacts of boxes, hulls and triangles are
+// clipped by several lanes a pair, the polygons in LDS (k_box_faces, np_wave.h).
 #include "pgx_internal.h"
 #include "radix_block.h"
 #include "shape_bounds.h"

@@ -1,5 +1,5 @@
-// The convex narrowphase with one wave per pair: GJK, EPA and the convex contact generators
-// of np_convex.h, operation for operation, their loops spread over the wave's 64 lanes.
+// The convex narrowphase with one wave per pair: GJK, EPA and the convex contact generators,
+// operation for operation with the reference, their loops spread over the wave's 64 lanes.
 //
 // A pair is a chain of some ten support queries (GJK), up to a hundred EPA insertions of one
 // support query, one pass over all faces and one horizon each, then a search over the hulls'
@@ -320,7 +320,7 @@ __device__ __forceinline__ void mem_face(WaveMem& M, int f, int i0, int i1, int 
     M.n[3][f] = ddot(p0, n);
 }
 
-// epa (np_convex.h) over the wave
+// src/EPA.h:9-186 over the wave
 template <class S0, class S1>
 __device__ __forceinline__ f3 epa_w(const S0& s0, const S1& s1, const GV& a, const GV& b, const GV& c, const GV& d, WaveMem& M,
                     f3& cp0, f3& cp1, bool& overflow) {
@@ -496,7 +496,7 @@ __device__ __forceinline__ int wave_face(int n, F value) {
     return -(int)wave_max(best == m ? -(float)at : -3.402823466e+38f);
 }
 
-// clip_polygon_n<CVX_MAXPOLY> (np_convex.h) with corner `lane` of the polygon (n of them)
+// clipPolygon (src/Clipping.cpp:21-53), at most CVX_MAXPOLY corners, with corner `lane` of the polygon (n of them)
 // and of the clip polygon (nclip) in the lanes
 __device__ __forceinline__ void wave_clip(f2& p, int& n, f2 clip, int nclip, WavePoly& M) {
     const int lane = wave_lane();
