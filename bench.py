@@ -15,9 +15,10 @@ timed ones, so a short run times the settled pile, not the first fall.
 
 roofline: the dominant kernel is k_solve, the contact solve of one graph colour (one launch
 per colour and pass: numIterations biased passes + 1 relaxation, every substep). Its
-algorithmic bytes per launch are 284 B per contact point + 12 B per manifold of the colour
-(rows 108 + scalars 24 + both bodies' solver and component v,w 96 read; lambdas 8 + both
-bodies' v,w 48 written). Its duration comes from HIP start/stop events that
+algorithmic bytes per launch are 122.7 B per contact point (7 rows of 16 B; the lambdas, 8 B
+read in two of the substep's three passes and written in two) + 156 B per manifold (mode,
+normal, friction and bodies 28; both bodies' solver v,w 64 read and 64 written) of the
+colour. Its duration comes from HIP start/stop events that
 hipExtLaunchKernelGGL stamps from each launch's own dispatch packet, for every launch of the
 first substep of every 16th timed step (--timing-period), on the world's stream: the events
 and their reads slow the step that carries them (2.33 against 1.89 ms on the settled

@@ -308,14 +308,14 @@ int pgx_world_get_timing(pgx_world* w, float* broadphase_us, float* narrowphase_
 
 /* Cumulative timing since pgx_world_reset_stats, collected on the timed steps.
  * Default (per-colour) mode: every k_solve launch of the first substep of each step is
- * bracketed by HIP events on the world's stream; solve_bytes is their algorithmic traffic,
- * 284 B per contact point + 12 B per manifold of the launched colour (rows 108 + scalars
- * 24 + solver and component velocities of both bodies 96 read; lambdas 8 + velocities 48
- * written). Persistent mode: the substep-loop kernel (one cooperative launch per step) is
- * bracketed instead, and solve_bytes follows the per-substep phase model (update rows
- * 164 B/manifold + 96 B/point, integrate velocities 168 B/body, preSolve 80 B/manifold +
- * 116 B/point, each solve pass 284 B/point + 12 B/manifold, integrate positions 120 B/body,
- * write-back 48 B/body; per substep). */
+ * bracketed by HIP events on the world's stream; solve_bytes is their algorithmic traffic
+ * over the launched colour: per contact point 7 rows of 16 B, and the lambdas, 8 B read but
+ * in a substep's first pass and written but in its last (122.7 B on average at 2 iterations);
+ * per manifold 156 B (mode, normal, friction and bodies 28, both bodies' solver velocities
+ * 64 read and 64 written). Persistent mode: the substep-loop kernel (one cooperative launch
+ * per step) is bracketed instead, and solve_bytes follows the per-substep phase model (rows
+ * 264 B/manifold + 144 B/point, each solve pass as above, velocities 336 B/body, positions
+ * 144 B/body). */
 typedef struct pgx_stats {
     long steps;
     long solve_launches;

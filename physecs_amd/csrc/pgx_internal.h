@@ -569,6 +569,7 @@ constexpr int READ_HOST_INTS = 2048;
 void sv_presize(World& w);
 void sv_substeps(World& w, int nManifolds, float dt);
 void sv_finish_step(World& w, int nManifolds);
+double sv_pass_bytes(const World& w, double points, double manifolds);
 double sv_step_bytes(const World& w, int M, long points);
 bool sv_world_pass_fits(World& w);                  // per-world passes possible for this world
 

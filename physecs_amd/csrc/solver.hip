@@ -2152,12 +2152,21 @@ void sv_substeps(World& w, int M, float dt) {
     }
 }
 
-// algorithmic bytes of one step's substep loop (per-phase model in the measurement notes)
+// Algorithmic bytes of a contact pass over so many points and manifolds, both sides dynamic,
+// averaged over a substep's passes. Per point 7 rows of 16 B, and the lambdas, 8 B read but in
+// the first pass and written but in the last; per manifold its mode, normal, friction and
+// bodies (28 B) and both bodies' solver v and w, read and written (128 B).
+double sv_pass_bytes(const World& w, double points, double manifolds) {
+    return (112.0 + 16.0 * w.iterations / (w.iterations + 1)) * points + 156.0 * manifolds;
+}
+
+// Algorithmic bytes of one step's substep loop. Rows: per manifold both bodies' records (7
+// fields of 16 B each), bodies, flags, normal and softness read, the mode written; per point
+// two anchors of 16 B read, 7 rows of 16 B written. Per body: velocity integration with the
+// write-back before it (336 B), position integration (144 B).
 double sv_step_bytes(const World& w, int M, long points) {
-    double N = w.D, C = (double)points, Mm = M;
-    double perSub = 164 * Mm + 96 * C + 168 * N + 80 * Mm + 116 * C + (w.iterations + 1) * (284 * C + 12 * Mm) +
-                    120 * N + 48 * N;
-    return w.substeps * perSub;
+    const double N = w.D, C = (double)points;
+    return w.substeps * (264.0 * M + 144.0 * C + (w.iterations + 1) * sv_pass_bytes(w, C, M) + 480.0 * N);
 }
 
 void sv_finish_step(World& w, int M) {

@@ -1494,21 +1494,21 @@ void world_step(World& w, float dt) {
             ++w.statSolveLaunches;
         }
         for (int j = 0; !coop && j < w.solveEvUsed; ++j) {
-            // k_solve: 284 B per contact point + 12 B per manifold of the launched colour;
-            // k_solve_flow (colour -1): the same over every colour of the pass
+            // k_solve: the launched colour's points and manifolds; k_solve_flow (colour -1):
+            // every colour's of the pass
             float ms = 0.f;
             PGX_HIP(hipEventElapsedTime(&ms, w.solveEv[2 * j], w.solveEv[2 * j + 1]));
             int c = w.solveEvColor[j], ce = w.solveEvColorEnd[j];
-            if (ce > 0) {   // k_solve_batch: the same per-point model over its run of colours
+            if (ce > 0) {   // k_solve_batch: the same over its run of colours
                 double bytes = 0;
-                for (int k = c; k < ce; ++k) bytes += 284.0 * pts[k] + 12.0 * (w.colorStartHost[k + 1] - w.colorStartHost[k]);
+                for (int k = c; k < ce; ++k) bytes += sv_pass_bytes(w, pts[k], w.colorStartHost[k + 1] - w.colorStartHost[k]);
                 w.statBatchUs += 1000.0 * ms;
                 w.statBatchBytes += bytes;
                 ++w.statBatchLaunches;
                 continue;
             }
-            double bytes = c >= 0 ? 284.0 * pts[c] + 12.0 * (w.colorStartHost[c + 1] - w.colorStartHost[c])
-                                  : 284.0 * points + 12.0 * M;
+            double bytes = c >= 0 ? sv_pass_bytes(w, pts[c], w.colorStartHost[c + 1] - w.colorStartHost[c])
+                                  : sv_pass_bytes(w, (double)points, M);
             w.statSolveUs += 1000.0 * ms;
             w.statSolveBytes += bytes;
             ++w.statSolveLaunches;

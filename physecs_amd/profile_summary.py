@@ -4,8 +4,8 @@
         [--marker k_scene_bounds_init] [--fetch-scale F --write-scale W] --out summary.md
 
 A step of the library starts with one k_scene_bounds_init launch (the broadphase's scene
-bounds), so the last K steps of a run are the dispatches from the K-th last
-k_scene_bounds_init on. The summary gives, over the whole run and over that window, each
+bounds; k_grid_small in a scene of at most 2,048 dynamic colliders: --marker k_grid_small),
+so the last K steps of a run are the dispatches from the K-th last of them on. The summary gives, over the whole run and over that window, each
 kernel's dispatch count, total and average duration from the kernel trace
 (*kernel_trace.csv), and, where a counter run's *counter_collection.csv is in the folder,
 each counter's mean per dispatch over the window. FETCH_SIZE and WRITE_SIZE (KiB per
