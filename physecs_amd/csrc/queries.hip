@@ -128,11 +128,18 @@ __device__ bool ray_convex(f3 o, f3 d, f3 pos, qf ori, const ConvexFaces& cv, in
     return true;
 }
 
+// What the colliders of a tree allow its walks: whether only the tree's own order will do,
+// what is not skipped however far (RaySkip::near), whether nothing may be skipped.
+struct RayRules {
+    int32_t inOrder;
+    float near;
+    int32_t noSkip;
+};
+
 struct RayScene {
     int W, nLeaves;
     const int32_t *worldRoot, *worldStop, *worldStaticStart, *staticCols, *mvals;
-    const int32_t* inOrder;
-    const float* near;                 // RaySkip::near
+    const RayRules* rules;
     const float4 *rayNode, *rayLeaf;   // k_ray_records
     const float4 *leafA, *nodeA, *nodeB;
     const float4 *cbmin, *cbmax, *cparams, *clpos, *clquat, *bpos, *bquat;
@@ -194,11 +201,13 @@ __device__ __forceinline__ void test_collider(const RayScene& S, int c, f3 o, f3
 // (the rest is for rounding and drift, which are under a hundredth of such a distance).
 struct RaySkip {
     f3 inv;          // 1 / d, 0 on a parallel axis
-    float margin;    // negative: the bound does not hold, walk without skipping
+    float margin;    // negative: nothing is skipped
     float near;      // what is entered up to here is not skipped
+    bool numbers;    // false: a hit distance could be a NaN, walk in the tree's order
 };
-// The formulas take directions as unit vectors, and their squares stay finite up to 1e9.
-__device__ __forceinline__ RaySkip ray_skip(f3 o, f3 d, f3 inv, f3 mn, f3 mx, float near) {
+// The formulas take directions as unit vectors, of which the margin holds, and their squares
+// stay finite up to 1e9. Directions of other lengths give numbers too, up to 1e6.
+__device__ __forceinline__ RaySkip ray_skip(f3 o, f3 d, f3 inv, f3 mn, f3 mx, float near, bool skips) {
     RaySkip r;
     r.near = near;
     r.inv = mk3(fabsf(d.x) < 0.001f ? 0.f : inv.x, fabsf(d.y) < 0.001f ? 0.f : inv.y, fabsf(d.z) < 0.001f ? 0.f : inv.z);
@@ -207,8 +216,9 @@ __device__ __forceinline__ RaySkip ray_skip(f3 o, f3 d, f3 inv, f3 mn, f3 mx, fl
     const float reach = far.x + far.y + far.z;
     const float size = fmaxf(fabsf(mn.x), fabsf(mx.x)) + fmaxf(fabsf(mn.y), fabsf(mx.y)) +
                        fmaxf(fabsf(mn.z), fabsf(mx.z)) + fabsf(o.x) + fabsf(o.y) + fabsf(o.z);
-    const bool unit = fabsf(dot(d, d) - 1.f) < 2e-6f;
-    r.margin = unit && reach < 1e9f && dot(o, o) < 1e18f ? 4e-3f * reach + 4e-6f * size : -1.f;
+    const float dd = dot(d, d);
+    r.numbers = dd < 1e12f && reach < 1e9f && dot(o, o) < 1e18f;
+    r.margin = skips && fabsf(dd - 1.f) < 2e-6f ? 4e-3f * reach + 4e-6f * size : -1.f;
     return r;
 }
 // a lower bound of the distance at which the ray enters the widened box
@@ -222,33 +232,36 @@ __device__ __forceinline__ float widened_entry(const RaySkip& r, f3 o, f3 mn, f3
 
 // leaf i's record; what it asks of RaySkip::near
 __device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4* __restrict__ clquat,
-                                          float4* __restrict__ rayLeaf, int32_t* __restrict__ inOrder) {
+                                          float4* __restrict__ rayLeaf, RayRules* __restrict__ rules) {
     const int c = S.mvals[i], b = S.cbody[c];
     const float4 mn = S.cbmin[c], mx = S.cbmax[c], l = clquat[c], q = S.bquat[b];
     const bool bounded = mn.x > -1e9f && mn.y > -1e9f && mn.z > -1e9f && mx.x < 1e9f && mx.y < 1e9f && mx.z < 1e9f;
-    const bool units = fabsf(l.x * l.x + l.y * l.y + l.z * l.z + l.w * l.w - 1.f) < 1e-5f &&
-                       fabsf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w - 1.f) < 1e-5f;
+    const float ll = l.x * l.x + l.y * l.y + l.z * l.z + l.w * l.w, qq = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
     const qf lq = qmul(q4(q), q4(l));
     const f3 pos = add(xyz(S.bpos[b]), qrot(q4(q), xyz(S.clpos[c])));
     const int type = S.ctype[c];
-    bool around = true;   // the bounds hold the shape as it is now (rays never hit a triangle mesh)
-    if (type != PGX_TRIANGLE_MESH) {
+    const float4 prm = S.cparams[c];
+    bool numbers = bounded && ll > 0.25f && ll < 4.f && qq > 0.25f && qq < 4.f;
+    bool skips = fabsf(ll - 1.f) < 1e-5f && fabsf(qq - 1.f) < 1e-5f;
+    if (type != PGX_TRIANGLE_MESH) {   // the bounds hold the shape as it is now (rays never hit a mesh)
         f3 lo, hi;
-        shape_bounds(type, S.cparams[c], pos, lq, S.cvVerts, S.cv.mesh, nullptr, nullptr, lo, hi);
-        around = mn.x <= lo.x && mn.y <= lo.y && mn.z <= lo.z && lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z &&
-                 hi.x <= mx.x && hi.y <= mx.y && hi.z <= mx.z;
-        if (type == PGX_CAPSULE) around = around && S.cparams[c].y >= 0.f;   // a radius below 0 narrows the bounds alone
+        shape_bounds(type, prm, pos, lq, S.cvVerts, S.cv.mesh, nullptr, nullptr, lo, hi);
+        numbers = numbers && lo.x > -1e9f && lo.y > -1e9f && lo.z > -1e9f && hi.x < 1e9f && hi.y < 1e9f && hi.z < 1e9f;
+        skips = skips && mn.x <= lo.x && mn.y <= lo.y && mn.z <= lo.z && lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z &&
+                hi.x <= mx.x && hi.y <= mx.y && hi.z <= mx.z;
+        if (type == PGX_CAPSULE) skips = skips && prm.y >= 0.f;   // a radius below 0 narrows the bounds alone
     }
-    bool closed = true;   // a hull's half-spaces end at its vertices
-    if (type == PGX_CONVEX_MESH) {
-        const float4 s = S.cparams[c];
-        const float x = fabsf(s.x), y = fabsf(s.y), z = fabsf(s.z);
-        closed = S.cvSlender[(int)s.w] * fmaxf(x, fmaxf(y, z)) <= 32.f * fminf(x, fminf(y, z)) && x > 0.f;
+    if (type == PGX_CONVEX_MESH) {   // its half-spaces end at its vertices
+        const float x = fabsf(prm.x), y = fabsf(prm.y), z = fabsf(prm.z);
+        const float least = fminf(x, fminf(y, z)), most = fmaxf(x, fmaxf(y, z)), slender = S.cvSlender[(int)prm.w];
+        numbers = numbers && least >= 1e-6f && most <= 1e6f && slender == slender;
+        skips = skips && slender * most <= 32.f * least;
     }
-    if (!(bounded && units && around && closed)) *inOrder = 1;
+    if (!numbers) rules->inOrder = 1;
+    if (!skips) rules->noSkip = 1;
     rayLeaf[4 * (size_t)i] = f4(pos, __int_as_float(type));
     rayLeaf[4 * (size_t)i + 1] = f4(mk3(lq.x, lq.y, lq.z), lq.w);
-    rayLeaf[4 * (size_t)i + 2] = S.cparams[c];
+    rayLeaf[4 * (size_t)i + 2] = prm;
     rayLeaf[4 * (size_t)i + 3] = make_float4(__int_as_float(c), __uint_as_float(S.centity[c]), 0.f, 0.f);
     if (type != PGX_CAPSULE) return 0.f;
     const f3 far = mk3(fmaxf(pos.x - mn.x, mx.x - pos.x), fmaxf(pos.y - mn.y, mx.y - pos.y), fmaxf(pos.z - mn.z, mx.z - pos.z));
@@ -258,16 +271,17 @@ __device__ __forceinline__ float ray_leaf(int i, const RayScene& S, const float4
 // The walk's records, 64 bytes each so that a visit takes one line: per inner node
 // {left box min, left}, {left max, right}, {right min}, {right max}; per leaf
 // {position, type}, {orientation}, {params}, {collider, entity}.
-// Sets *inOrder (0 before) if a dynamic collider is one for which the margin does not hold
-// or whose hit distance could be a NaN, which makes the result depend on the order of the
-// tests: bounds that are not finite or do not hold the shape, an orientation that is not a unit
-// quaternion, or a hull whose half-spaces go on beyond its vertices (hull_slenderness; up to 32
-// the planes' rounding, some 1e-6 of the distance and 2^-23 of the coordinates, stays within
-// the margin). Raises *near (0 before) to RaySkip::near.
+// And the rules, 0 before: nothing is skipped if the margin does not hold for a dynamic
+// collider (its bounds do not hold the shape, its orientation is not a unit quaternion, or it
+// is a hull whose half-spaces go on beyond its vertices: hull_slenderness; up to 32 the planes'
+// rounding, some 1e-6 of the distance and 2^-23 of the coordinates, stays within the margin);
+// and the tree's order is kept if a hit distance could be a NaN, which makes the result depend
+// on the order of the tests (bounds, orientations or scales that are not finite or are far
+// from 1).
 __global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __restrict__ child, RayScene S,
                                                      const float4* __restrict__ leafB, const float4* __restrict__ clquat,
                                                      float4* __restrict__ rayNode, float4* __restrict__ rayLeaf,
-                                                     int32_t* __restrict__ inOrder, float* __restrict__ near) {
+                                                     RayRules* __restrict__ rules) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     float reach = 0.f;
     if (i < n - 1) {
@@ -277,10 +291,10 @@ __global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __res
         rayNode[4 * (size_t)i + 2] = f4(xyz(r & LEAF_BIT ? S.leafA[rl] : S.nodeA[rl]), 0.f);
         rayNode[4 * (size_t)i + 3] = f4(xyz(r & LEAF_BIT ? leafB[rl] : S.nodeB[rl]), 0.f);
     }
-    if (i < n) reach = ray_leaf(i, S, clquat, rayLeaf, inOrder);
+    if (i < n) reach = ray_leaf(i, S, clquat, rayLeaf, rules);
     // one atomic a wave at most: the floats are not negative, so their bits order like them
     for (int o = WAVE / 2; o >= 1; o >>= 1) reach = fmaxf(reach, __shfl_xor(reach, o));
-    if ((threadIdx.x & (WAVE - 1)) == 0 && reach > *near) atomicMax((unsigned int*)near, __float_as_uint(reach));
+    if ((threadIdx.x & (WAVE - 1)) == 0 && reach > rules->near) atomicMax((unsigned int*)&rules->near, __float_as_uint(reach));
 }
 
 // Ray i: origin, direction and maxDistance as the caller holds them (3, 3 and 1 floats), the
@@ -292,11 +306,17 @@ __global__ __launch_bounds__(256) void k_ray_records(int n, const int32_t* __res
 // other one waits in an LDS stack with its entry distance) and boxes beyond the best hit are
 // skipped; the lanes of a wave descend together, then test their leaves together; a visit
 // reads one 64-byte record. Which order the colliders are tested in does not reach the result
-// (least distance, then least index) while every distance is a number. A ray whose stack is
-// full, and one without a margin, walks along the escape links, which need no stack.
-// 262,144 rays into 32k bodies: 1,616 us along the links, 560 us nearest first with skipping
-// (nine loads of three arrays a visit), 390 us with the records, which take 7 us to write.
-constexpr int RAY_THREADS = 256, RAY_STACK = 20;   // 40 KB: four blocks per CU
+// (least distance, then least index) while every distance is a number, so a ray that may not
+// skip takes the same walk, entering every box; a subtree that finds the stack full, and a ray
+// whose result could depend on the order, are walked along the escape links, which need no
+// stack. 262,144 rays into 32k bodies: 1,616 us along the links, 560 us nearest first with
+// skipping (nine loads of three arrays a visit), 390 us with the records, 407 us with the boxes
+// near the origin kept; the records take 12 us to write. 1,048,576 rays of directions that are
+// not unit vectors: 6.4 ms with the tree in a kernel that only follows the links, 8.6 ms where
+// they did that here, 6.9 ms in this walk, 5.8 ms with a stack of 12 instead of 20 (six blocks
+// of 24 KB a CU, not four; ten measure the same); half of them unit vectors, which wait for the
+// others of their wave: 6.3, 8.0, 5.8 and 4.8 ms.
+constexpr int RAY_THREADS = 256, RAY_STACK = 12;
 __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __restrict__ ro, const float* __restrict__ rd,
                                                  const float* __restrict__ rmax, const int32_t* __restrict__ rworld,
                                                  const uint32_t* __restrict__ ignore, RayScene S,
@@ -314,9 +334,9 @@ __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __r
     float bestT = 0.f;
     int best = -1;
     const int root = S.worldRoot[wd];
-    RaySkip skip{s3(0.f), -1.f, 0.f};
-    if (root != -1 && !(root & LEAF_BIT) && !*S.inOrder) 
-        skip = ray_skip(o, d, inv, xyz(S.nodeA[root]), xyz(S.nodeB[root]), *S.near);
+    RaySkip skip{s3(0.f), -1.f, 0.f, false};
+    if (root != -1 && !(root & LEAF_BIT) && !S.rules->inOrder)
+        skip = ray_skip(o, d, inv, xyz(S.nodeA[root]), xyz(S.nodeB[root]), S.rules->near, !S.rules->noSkip);
     auto statics = [&]() {
         for (int st = S.worldStaticStart[wd]; st < S.worldStaticStart[wd + 1]; ++st)
             test_collider(S, S.staticCols[st], o, d, inv, maxDist, ig, bestT, best);
@@ -324,7 +344,7 @@ __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __r
     // enter: the box is met within maxDistance, and not beyond the best hit; t: where it may be met
     auto enter = [&](const float4& mn, const float4& mx, float& t) {
         if (!ray_aabb(o, d, inv, xyz(mn), xyz(mx), t) || !(t <= maxDist)) return false;
-        if (skip.margin < 0.f) return true;
+        if (skip.margin < 0.f) { t = 0.f; return true; }
         t = widened_entry(skip, o, xyz(mn), xyz(mx));
         return best < 0 || !(t > fmaxf(bestT, skip.near));
     };
@@ -358,9 +378,9 @@ __global__ __launch_bounds__(RAY_THREADS) void k_raycast(int n, const float* __r
         if (!ray_shape(__float_as_int(p.w), prm, xyz(p), q4(q), S.cv, o, d, t) || t > maxDist) return;
         if (best < 0 || t < bestT || (t == bestT && c < best)) { best = c; bestT = t; }
     };
-    if (skip.margin >= 0.f) statics();   // a wall behind the ray's pile ends its walk early
+    if (skip.numbers) statics();   // a wall behind the ray's pile ends its walk early
     // NaN: a static's, kept as the first hit; the order decides then
-    if (skip.margin < 0.f || bestT != bestT) {
+    if (!skip.numbers || bestT != bestT) {
         skip.margin = -1.f;
         best = -1; bestT = 0.f;
         if (root != -1) follow(root, S.worldStop[wd]);
@@ -421,7 +441,8 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
     if (!w.qEv[0])
         for (auto& e : w.qEv) PGX_HIP(hipEventCreate(&e));
     PGX_HIP(hipEventRecord(w.qEv[0], s));
-    fill_i32(s, w.counters.p + 7, 0, 3);   // the refit's work counter, the walks' order and near
+    fill_i32(s, w.counters.p + 7, 0, 4);   // the refit's work counter and the walks' rules
+    RayRules* const rules = (RayRules*)(w.counters.p + 8);
     bp_build(w);
     RayScene S;
     S.W = w.W;
@@ -429,7 +450,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
     S.worldRoot = w.worldRoot.p; S.worldStop = w.worldStop.p;
     S.worldStaticStart = w.worldStaticStart.p; S.staticCols = w.staticCols.p; S.mvals = w.mvals.p;
     w.qRayNode.alloc(4 * (size_t)std::max(w.nDynCol, 1)); w.qRayLeaf.alloc(4 * (size_t)std::max(w.nDynCol, 1));
-    S.inOrder = w.counters.p + 8; S.near = (const float*)(w.counters.p + 9); S.rayNode = w.qRayNode.p; S.rayLeaf = w.qRayLeaf.p;
+    S.rules = rules; S.rayNode = w.qRayNode.p; S.rayLeaf = w.qRayLeaf.p;
     S.leafA = w.leafA.p; S.nodeA = w.nodeA.p; S.nodeB = w.nodeB.p;
     S.cbmin = w.cbmin.p; S.cbmax = w.cbmax.p; S.cparams = w.cparams.p; S.clpos = w.clpos.p; S.clquat = w.clquat.p;
     S.bpos = w.bpos.p; S.bquat = w.bquat.p; S.cbody = w.cbody.p; S.ctype = w.ctype.p; S.centity = w.centity.p;
@@ -439,7 +460,7 @@ void qr_raycast(World& w, int n, const float* origins, const float* dirs, const 
         fill_i32(s, w.worldRoot.p, -1, w.W);   // no tree: static lists only
     } else {
         hipLaunchKernelGGL(k_ray_records, dim3(div_up(w.nDynCol, 256)), dim3(256), 0, s, w.nDynCol, w.nodeChild.p, S,
-                           w.leafB.p, w.clquat.p, w.qRayNode.p, w.qRayLeaf.p, w.counters.p + 8, (float*)(w.counters.p + 9));
+                           w.leafB.p, w.clquat.p, w.qRayNode.p, w.qRayLeaf.p, rules);
         PGX_LAUNCH_CHECK();
     }
     hipLaunchKernelGGL(k_raycast, dim3(div_up(n, RAY_THREADS)), dim3(RAY_THREADS), 0, s, n, w.qRays.p, w.qRays.p + n3,

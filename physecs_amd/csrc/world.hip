@@ -375,7 +375,8 @@ void world_alloc_derived(World& w, const pgx_config* cfg, int nTrimesh) {
 // mesh: their planes hold every vertex, every edge is met once in either direction, and the
 // volume that the faces enclose is at least a ball's of that radius (which a surface folded
 // onto itself does not). Meshes come with faces, normals and centroids as given, so they may
-// not; infinite then, and for meshes too large to look at here.
+// not; infinite then, and for meshes too large to look at here, and a NaN if the planes are
+// not numbers below 1e9.
 static float hull_slenderness(const pgx_scene_desc* sc, int m) {
     struct V { double x, y, z; };
     auto at = [](const float* p) { return V{p[0], p[1], p[2]}; };
@@ -385,6 +386,9 @@ static float hull_slenderness(const pgx_scene_desc* sc, int m) {
     constexpr float OPEN = std::numeric_limits<float>::infinity();
     const int v0 = sc->convex_vert_start[m], nv = sc->convex_vert_start[m + 1] - v0;
     const int f0 = sc->convex_face_start[m], nf = sc->convex_face_start[m + 1] - f0;
+    for (int k = 3 * f0; k < 3 * (f0 + nf); ++k)
+        if (!(std::fabs(sc->face_normal[k]) < 1e9f && std::fabs(sc->face_centroid[k]) < 1e9f))
+            return std::numeric_limits<float>::quiet_NaN();
     if (nv < 4 || nf < 4 || (long)nv * nf > 1 << 24) return OPEN;
     std::vector<V> v(nv);
     V mean{0, 0, 0}, lo = at(sc->convex_verts + 3 * (size_t)v0), hi = lo;

@@ -1,6 +1,6 @@
 """The raycast walk at the places where its order or its skipping could show: trees deeper
 than its stack, grazing rays, distant origins, directions and orientations that are not
-normalised (walked in the tree's order), batches that end within a wave, capsules whose
+normalised (nothing is skipped) or very long (walked in the tree's order), batches that end within a wave, capsules whose
 bounds reach far from them. Against the oracle's Scene::raycastClosest on the same state, bit
 for bit."""
 import numpy as np
@@ -52,6 +52,9 @@ def _rays(kind, sc, rng, n):
     reach = 10.0 ** rng.uniform(0, 5 if kind == "far" else 1.5, (n, 1))
     offset = {"graze": 0.5 + 1e-4 * rng.normal(size=(n, 1))}.get(kind, rng.uniform(0, 0.5, (n, 1)))
     d = -away * (rng.uniform(0.5, 2.0, (n, 1)) if kind == "length" else 1.0)
+    if kind == "odd":     # lengths of 1 among very short and long ones and none at all
+        d *= 10.0 ** np.where(rng.random((n, 1)) < 0.3, 0, rng.uniform(-4, 8, (n, 1)))
+        d[::17] = 0
     return (target + away * reach + side * offset).astype(np.float32), d.astype(np.float32)
 
 
@@ -65,7 +68,7 @@ def _same(g, o, origins, dirs, maxd):
 
 @pytest.mark.parametrize("scene,kind,n", [("deep", "near", 1), ("deep", "near", 257), ("deep", "length", 65),
                                           ("mixed", "graze", 1023), ("mixed", "far", 1000), ("mixed", "length", 300),
-                                          ("loose", "near", 500)])
+                                          ("loose", "near", 500), ("mixed", "odd", 900), ("deep", "odd", 200)])
 def test_walk_matches_oracle(scene, kind, n):
     log(f"[ray walk] {scene}, {kind}, {n} rays")
     sc = {"deep": _deep, "mixed": _mixed, "loose": _loose}[scene]()
