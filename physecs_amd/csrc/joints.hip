@@ -594,7 +594,6 @@ __global__ void k_joint_color(JointArgs a, int begin, int end, int phase, int wa
 // exchange their dot products. With a lane per joint for everything, on rows and velocities
 // in memory, a solve pass of 24 ragdolls of 12 joints took 19 us and one of 128 chains of 7
 // joints 14 us; now 11.5 and 8.5 us, and the preSolve 7 us.
-constexpr int ISLAND_CHUNK = WAVE / 2;
 // LDS words of a row, in solve order. Solve: {ang0, lambda} {ang1, lambda} {lin0t, bits}
 // {-lin1t, bits} {ang0t, -} {-ang1t, -} {lin, target} {k0, k1, lower, upper}; preSolve: the
 // pushes {linear 0, bits} {linear 1, bits} {angular 0, -} {angular 1, -}. Bits: the row in
@@ -604,8 +603,9 @@ constexpr int ROW_WORDS = 8, PUSH_WORDS = 4;
 constexpr size_t island_lds(int bodies, int joints, int words) {
     return 2 * sizeof(float4) * bodies + sizeof(int4) * joints + sizeof(float4) * words * JOINT_MAX_ROWS * joints;
 }
-// eight colours, a body more than joints: 45 KB; the launches ask for no raised limit
-static_assert(island_lds(8 * ISLAND_MAX + 1, ISLAND_CHUNK, ROW_WORDS) <= 64 * 1024, "an island's pass fits the LDS");
+// at most as many chunks as colours, eight (upload_joints), and a body more than joints: 37 KB;
+// the launches ask for no raised limit
+static_assert(island_lds(8 * ISLAND_CHUNK + 1, ISLAND_CHUNK, ROW_WORDS) <= 64 * 1024, "an island's pass fits the LDS");
 constexpr int RB_FLAGS = 4, RB_WARM = 1 << 8, RB_MOVES = 1 << 9;
 struct IslandArgs {
     const int32_t *cs, *bs, *body;   // per island: 9 colour offsets, first body; bodies

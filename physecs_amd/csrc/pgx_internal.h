@@ -99,9 +99,7 @@ enum { BR_COM = 0, BR_Q, BR_V, BR_W, BR_I0, BR_I1, BR_I2, BR_WORDS = 8 };
 __host__ __device__ __forceinline__ int br(int body, int field) { return BR_WORDS * body + field; }
 constexpr int CONTACT_ROW_FIELDS = 7;   // float4 rows per contact point (sRow)
 constexpr int JOINT_MAX_ROWS = 7;      // a prismatic joint with its limit and drive rows
-// joints of one colour in an island of the joint passes: bounds their LDS, which holds the
-// velocities of an island's bodies (joints.hip)
-constexpr int ISLAND_MAX = 64;
+constexpr int ISLAND_CHUNK = WAVE / 2;   // joints that an island's pass takes at a time (joints.hip)
 // substep-loop execution: one launch per colour and pass; one cooperative launch per step
 // (grid barriers between colours); one dependency-driven launch per pass
 // (one device-wide queue), the same with a queue per XCD

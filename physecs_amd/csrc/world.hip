@@ -705,8 +705,6 @@ static void grow_keep(DBuf<T>& b, int keep, int n, hipStream_t s) {
     b.n = (size_t)std::max(n, 1);
 }
 
-constexpr int ISLAND_MIN = 1;
-
 // The live joints grouped by colour, creation order inside a colour, and the per-joint
 // arrays, to the device.
 static void upload_joints(World& w, int keepState) {
@@ -723,8 +721,12 @@ static void upload_joints(World& w, int keepState) {
         if (w.hjAlive[j]) order[fillp[w.hjColor[j]]++] = j;
     // islands of the SIMD colours (0-7): joints joined through dynamic bodies; each island's
     // joints by colour, in the colour order above inside a colour. One launch per joint pass
-    // solves them all (k_island_presolve, k_island_solve) when no island holds more than ISLAND_MAX joints of
-    // one colour; per-colour launches otherwise.
+    // solves them all (k_island_presolve, k_island_solve) while the largest island is at most as
+    // many chunks of ISLAND_CHUNK joints, which take turns, as there are colours; per-colour
+    // launches otherwise. A chunk takes about as long as a colour's launch: a step of a chain of
+    // 60 (two colours, two chunks) takes 282 us so and 326 in per-colour launches, of 70 326
+    // and 320, of 120 387 and 328; a cloth of 9 x 9 (145 joints, 5 chunks) 378 and 387, of 10 x
+    // 10 (181, 6 chunks) 419 and 389.
     {
         std::vector<int> parent(w.D > 0 ? w.D : 1);
         std::iota(parent.begin(), parent.end(), 0);
@@ -750,9 +752,12 @@ static void upload_joints(World& w, int keepState) {
         }
         std::vector<int32_t> cnt((size_t)nIsl * 8, 0);   // joints per island and colour
         for (int k = 0; k < w.jColorStart[8]; ++k) ++cnt[(size_t)islandOf[k] * 8 + w.hjColor[order[k]]];
-        const int most = cnt.empty() ? 0 : *std::max_element(cnt.begin(), cnt.end());
+        int most = 0, colours = 0;   // joints of the largest island
+        for (int i = 0; i < nIsl; ++i)
+            most = std::max(most, std::accumulate(cnt.begin() + 8 * (size_t)i, cnt.begin() + 8 * ((size_t)i + 1), 0));
+        for (int c = 0; c < 8; ++c) colours += w.jColorStart[c + 1] > w.jColorStart[c];
         w.jIslands = 0;
-        if (nIsl >= ISLAND_MIN && most <= ISLAND_MAX) {
+        if (nIsl > 0 && div_up(most, ISLAND_CHUNK) <= colours) {
             std::vector<int32_t> cs((size_t)nIsl * 9), cursor((size_t)nIsl * 8), bs((size_t)nIsl + 1), bodies;
             std::vector<int4> list(w.jColorStart[8]);
             int at = 0;

@@ -34,10 +34,21 @@ def _web(n, seed):
     return sc
 
 
-@pytest.mark.parametrize("n", [1, 26, 27, 33, 62])
+@pytest.mark.parametrize("n", [1, 26, 27, 33, 62, 250])
 def test_islands_lockstep_bitexact(n):
     log(f"[islands] a web of {n} bodies")
     lockstep(_web(n, n), 25, check_every=5)
+
+
+@pytest.mark.parametrize("n", [33, 34, 65, 66, 140])
+def test_chains_lockstep_bitexact(n):
+    """Two colours: up to 64 joints are two chunks of an island's pass, more are solved in a
+    launch per colour."""
+    log(f"[islands] a chain of {n} bodies")
+    sc = scenes.Scene()
+    sc.add_static(scenes.BOX, [60, 0.5, 20], [0, -0.5, 0])
+    scenes.capsule_chain(sc, [-n / 4, 0.6, 0], n=n)
+    lockstep(sc, 20, check_every=5)
 
 
 def test_islands_of_different_sizes_lockstep_bitexact():
