@@ -314,7 +314,7 @@ struct World {
     DBuf<int4> cvMesh;
     DBuf<int2> cvFace;
     DBuf<int32_t> cvFaceIdx;
-    DBuf<float> cvSlender;             // per mesh: hull_slenderness
+    DBuf<float> cvSlender;             // per mesh: qr_hull_slenderness
     DBuf<int32_t> heavy;               // from its start: pairs with a convex mesh; from its end: pairs of boxes touching with a face (filled by the primitive kernel)
     // static triangle meshes: vertices, triangles in the BVH build's order (mesh-local
     // vertex indices), triangle normals / centroids, BVH nodes (2 float4 each: {min,
@@ -471,6 +471,7 @@ int qr_overlap(World& w, int n, const int32_t* types, const float* params, const
 void qr_character_move(World& w, int n, pgx_character* chars, const float* translations, uint8_t* flags);
 // queries.hip: Scene::overlapWithMinTranslationalDistance for n query shapes; returns PGX_OK
 // or PGX_ERR_CAPACITY (only *total set) when the hits exceed `capacity`
+void qr_hull_slenderness(World& w);   // cvSlender, once the hulls are uploaded
 int qr_overlap_mtd(World& w, int n, const int32_t* types, const float* params, const float* positions,
                    const float* orientations, const int32_t* queryWorld, int capacity, int32_t* offsets,
                    int32_t* colliders, float* normalMtd, int32_t* total, double* deviceUs);

@@ -2,14 +2,11 @@
 // the component state, and the per-step orchestration of Scene::simulate
 // (src/Physecs.cpp:112-561) on one HIP stream.
 #include <chrono>
-#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <functional>
-#include <limits>
 #include <numeric>
-#include <set>
 #include <unordered_map>
 #include "pgx_internal.h"
 
@@ -369,64 +366,6 @@ void world_alloc_derived(World& w, const pgx_config* cfg, int nTrimesh) {
 
 // (Re)initialises a world from a validated descriptor on w's device and stream. Device
 // buffers are reused where they are large enough.
-// How far convex mesh m's half-spaces, which are what a ray is tested against, reach beyond its
-// vertices when their planes are moved out: by at most this factor (and one) times the move.
-// It is the diameter over the inner radius about the vertices' mean, if the faces close the
-// mesh: their planes hold every vertex, every edge is met once in either direction, and the
-// volume that the faces enclose is at least a ball's of that radius (which a surface folded
-// onto itself does not). Meshes come with faces, normals and centroids as given, so they may
-// not; infinite then, and for meshes too large to look at here, and a NaN if the planes are
-// not numbers below 1e9.
-static float hull_slenderness(const pgx_scene_desc* sc, int m) {
-    struct V { double x, y, z; };
-    auto at = [](const float* p) { return V{p[0], p[1], p[2]}; };
-    auto minus = [](V a, V b) { return V{a.x - b.x, a.y - b.y, a.z - b.z}; };
-    auto dot3 = [](V a, V b) { return a.x * b.x + a.y * b.y + a.z * b.z; };
-    auto cross3 = [](V a, V b) { return V{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; };
-    constexpr float OPEN = std::numeric_limits<float>::infinity();
-    const int v0 = sc->convex_vert_start[m], nv = sc->convex_vert_start[m + 1] - v0;
-    const int f0 = sc->convex_face_start[m], nf = sc->convex_face_start[m + 1] - f0;
-    for (int k = 3 * f0; k < 3 * (f0 + nf); ++k)
-        if (!(std::fabs(sc->face_normal[k]) < 1e9f && std::fabs(sc->face_centroid[k]) < 1e9f))
-            return std::numeric_limits<float>::quiet_NaN();
-    if (nv < 4 || nf < 4 || (long)nv * nf > 1 << 24) return OPEN;
-    std::vector<V> v(nv);
-    V mean{0, 0, 0}, lo = at(sc->convex_verts + 3 * (size_t)v0), hi = lo;
-    for (int i = 0; i < nv; ++i) {
-        const V p = v[i] = at(sc->convex_verts + 3 * (size_t)(v0 + i));
-        mean = V{mean.x + p.x / nv, mean.y + p.y / nv, mean.z + p.z / nv};
-        lo = V{std::min(lo.x, p.x), std::min(lo.y, p.y), std::min(lo.z, p.z)};
-        hi = V{std::max(hi.x, p.x), std::max(hi.y, p.y), std::max(hi.z, p.z)};
-    }
-    const V box = minus(hi, lo);
-    const double diameter = std::sqrt(dot3(box, box));
-    double inner = std::numeric_limits<double>::infinity(), volume = 0.0;
-    std::set<std::pair<int, int>> edges;
-    for (int f = f0; f < f0 + nf; ++f) {
-        const V c = at(sc->face_centroid + 3 * (size_t)f);
-        V n = at(sc->face_normal + 3 * (size_t)f);
-        const double length = std::sqrt(dot3(n, n));
-        n = V{n.x / length, n.y / length, n.z / length};
-        const double depth = dot3(minus(c, mean), n);
-        if (!(depth > 0.0)) return OPEN;   // a NaN among them
-        inner = std::min(inner, depth);
-        for (const V& p : v)
-            if (!(dot3(minus(p, c), n) <= 1e-5 * diameter)) return OPEN;
-        const int k0 = sc->face_idx_start[f], k1 = sc->face_idx_start[f + 1];
-        if (k1 - k0 < 3) return OPEN;
-        for (int k = k0; k < k1; ++k) {
-            const int a = sc->face_idx[k], b = sc->face_idx[k + 1 < k1 ? k + 1 : k0];
-            if (a < 0 || a >= nv || b < 0 || b >= nv || !(dot3(minus(v[a], c), n) >= -1e-5 * diameter)) return OPEN;
-            if (!edges.insert({a, b}).second) return OPEN;
-            volume += dot3(minus(c, mean), cross3(minus(v[a], mean), minus(v[b], mean))) / 6.0;
-        }
-    }
-    for (const auto& e : edges)
-        if (!edges.count({e.second, e.first})) return OPEN;
-    if (!(std::fabs(volume) >= 4.0 * inner * inner * inner)) return OPEN;
-    return (float)(diameter / inner);
-}
-
 void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
     world_reset_host(w);
     SceneArrays o;
@@ -471,7 +410,6 @@ void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
         std::vector<int4> cvm;
         std::vector<int2> cvf;
         std::vector<int32_t> cvfi;
-        std::vector<float> slender;
         for (int m = 0; m < sc->n_convex; ++m) {
             int v0 = sc->convex_vert_start[m], nv = sc->convex_vert_start[m + 1] - v0;
             int first = (int)cvv.size();
@@ -481,7 +419,6 @@ void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
             while ((cvv.size() - first) % 4) cvv.push_back(cvv.back());
             int f0 = sc->convex_face_start[m], nf = sc->convex_face_start[m + 1] - f0;
             cvm.push_back(make_int4(first, nv, (int)cvf.size(), nf));
-            slender.push_back(hull_slenderness(sc, m));
             for (int f = f0; f < f0 + nf; ++f) {
                 int k0 = sc->face_idx_start[f], k1 = sc->face_idx_start[f + 1];
                 cvf.push_back(make_int2((int)cvfi.size(), k1 - k0));
@@ -495,7 +432,7 @@ void world_init(World& w, const pgx_config* cfg, const pgx_scene_desc* sc) {
         w.nConvex = sc->n_convex;
         upload(w.cvVerts, cvv, s); upload(w.cvMesh, cvm, s); upload(w.cvFace, cvf, s);
         upload(w.cvFaceIdx, cvfi, s); upload(w.cvFaceN, cvn, s); upload(w.cvFaceC, cvc, s);
-        upload(w.cvSlender, slender, s);
+        qr_hull_slenderness(w);
     }
     if (sc->n_trimesh > 0) {
         w.tmMaxDepth = upload_triangle_meshes(w, sc, s);
