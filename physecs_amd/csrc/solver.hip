@@ -1422,14 +1422,18 @@ __device__ __forceinline__ int colours_below(const uint64_t* used, int b, int c)
 // microseconds between XCDs.
 //
 // The solve order is the colour order's, so the arithmetic is exactly that of one launch
-// per colour. Waves take 32 manifolds at a time, in solve order, from the pass's ticket: a
-// manifold waits only on manifolds of lower solve positions held by waves already running,
-// so the waits resolve in order. Every wait is bounded; one that runs out sets flowErr and
+// per colour. Waves take manifolds in solve order from the pass's ticket, 32, or 64 that they
+// solve in two turns (more than FLOW_RESIDENT in all): a
+// manifold waits only on manifolds of lower solve positions, which are solved, or held by waves
+// already running that solve lower ones first, so the waits resolve in order. Every wait is bounded; one that runs out sets flowErr and
 // gives up (the host reports the error) rather than hang.
 constexpr int FLOW_SPIN_LIMIT = 1 << 18;   // ~0.5 s of polling: a wait this long is a bug
 
+constexpr int FLOW_RESIDENT = 131072;      // 32 manifolds each of the waves that fit the chip, four a SIMD (128 registers)
+
 struct FlowArgs {
     int index;                             // the pass within its substep
+    int take;                              // manifolds per ticket, a multiple of 32
     int pass;                              // PASS_* flags
     uint32_t epoch;                        // unique per launch (24 bits used)
     uint64_t* pub;                         // 6 words per body
@@ -1476,7 +1480,7 @@ __device__ __forceinline__ void hand_on(const SubArgs& a, const FlowArgs& f, int
     __hip_atomic_store(p + 5, pub_word(w.z, ver), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(256) void k_solve_flow(SubArgs a, FlowArgs f) {
+__global__ __launch_bounds__(256, 4) void k_solve_flow(SubArgs a, FlowArgs f) {
     const int lane = threadIdx.x & (WAVE - 1);
     int queue = 0;
     if (f.xcdScope) {
@@ -1485,11 +1489,13 @@ __global__ __launch_bounds__(256) void k_solve_flow(SubArgs a, FlowArgs f) {
     }
     const int qb = f.qStart[queue], qn = f.qStart[queue + 1] - qb;
     const uint32_t vbase = (f.epoch & 0xffffffu) << 8;
-    int done = 0;
+    int done = 0, base = -WAVE / 2, taken = 0;
     for (;;) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(a.tickets + f.index * FLOW_QUEUES + queue, WAVE / 2);
-        base = __shfl(base, 0);
+        if ((base += WAVE / 2) == taken) {   // the next manifolds of the pass
+            if (lane == 0) base = atomicAdd(a.tickets + f.index * FLOW_QUEUES + queue, f.take);
+            base = __shfl(base, 0);
+            taken = base + f.take;
+        }
         if (base >= qn) break;
         const int idx = base + (lane >> 1);
         bool pending = idx < qn;           // the same in both lanes of a pair
@@ -1994,9 +2000,14 @@ void sv_substeps(World& w, int M, float dt) {
                                     (int)worldLds[1]));
     w.lastQueues = flow && M > 0 ? f.nQueues : 0;
     w.lastFlowPasses = flow && M > 0 ? w.substeps * (w.iterations + 1) : 0;
-    // waves of the dependency-driven pass: enough to hold every manifold at once, at most
-    // what the chip keeps resident comfortably; on XCD queues, 64 workgroups per XCD
-    const int flowBlocks = f.xcdScope ? 64 * w.nXcd : std::max(1, std::min(div_up(2 * (long)std::max(M, 1), 256), 2048));
+    // Waves of the dependency-driven pass: all manifolds at once while they fit the chip; of more,
+    // two waves a SIMD with 64 manifolds each in turn, since what more waves would solve next
+    // waits for what these hold, and their polling is in its way. 4,096 worlds, 1.4 M manifolds:
+    // 405 M body-substeps/s; 317 with 8,192 waves of 32 manifolds, 305 of 64, 343 with 2,048 of 32.
+    // On XCD queues, 64 workgroups per XCD: 348, and 321 with 32 manifolds a wave.
+    const bool resident = M <= FLOW_RESIDENT;
+    f.take = resident ? WAVE / 2 : WAVE;
+    const int flowBlocks = f.xcdScope ? 64 * w.nXcd : resident ? div_up(2 * (long)std::max(M, 1), 256) : 512;
     // launch groups of the colour passes: (first colour, end colour, batched run index + 1);
     // a run holds consecutive colours of at most colorBatch manifolds each, at most
     // BATCH_MAX_MANIFOLDS in all (its bodies' velocities fit in LDS), two colours or more

@@ -61,3 +61,27 @@ def test_ragdoll_world_lockstep_with_oracle(api):
     log(f"[batched] ragdoll world alone vs oracle: {sub.n_dyn} bodies, {len(sub.joints)} joints")
     assert len(sub.joints) == 14
     lockstep(sub, 60)
+
+
+def test_flow_with_more_manifolds_than_the_chip_holds():
+    """147,852 manifolds of touching spheres: the dependency-driven pass takes 64 a wave."""
+    from physecs_amd import api
+    side = 37
+    n = side ** 3
+    at = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3) * 0.98 + [0, 0.49, 0]
+    sc = scenes.Scene()
+    sc.add_static(scenes.BOX, [30, 0.5, 30], [18, -0.5, 18])
+    sc.add_bodies_bulk(np.zeros(n, int), np.tile([0.5, 0, 0, 0], (n, 1)), at, np.tile([0, 0, 0, 1.0], (n, 1)),
+                       np.random.default_rng(1).normal(size=(n, 3)), np.zeros(n, int))
+    states = []
+    for mode in ("colors", "flow"):
+        log(f"[batched] {n} touching spheres, {mode}")
+        g = api.World(sc, pair_capacity=1 << 20)
+        g.set_exec(mode)
+        for _ in range(3):
+            g.step(1 / 60)
+            assert g.counts()["manifolds"] > 131072
+        states.append(g.state())
+        g.close()
+    for a, b in zip(*states):
+        assert np.array_equal(bits(a), bits(b))
