@@ -21,7 +21,7 @@ normal, friction and bodies 28; both bodies' solver v,w 64 read and 64 written) 
 colour. Its duration comes from HIP start/stop events that
 hipExtLaunchKernelGGL stamps from each launch's own dispatch packet, for every launch of the
 first substep of every 16th timed step (--timing-period), on the world's stream: the events
-and their reads slow the step that carries them (2.33 against 1.89 ms on the settled
+and their reads slow the step that carries them (2.01 against 1.43 ms on the settled
 default workload), so the steps between run without them, and p50/p99 are taken over
 those (config.p99_step_ms_all over all timed steps). --exec flow launches one
 k_solve_flow per pass instead (every colour in one launch: a manifold solves once its
